@@ -83,7 +83,7 @@ int check_shape(int b, int h, int64_t n, int d, int e, int dtype) {
   return 0;
 }
 
-int default_seg_len(int b, int h, int64_t n) {
+int default_seg_len(int b, int h, int64_t n, bool narrow64) {
   const int64_t bh = (int64_t)b * h;
   const int64_t want = (kTargetGroups + bh - 1) / bh;  // segments per (b, h)
   // rounded up, so that no more than `want` segments result: one workgroup more than the chip
@@ -92,7 +92,9 @@ int default_seg_len(int b, int h, int64_t n) {
   len = ((len + kMinSeg - 1) / kMinSeg) * kMinSeg;
   // Segments shorter than kPreferredSeg spend a visible share of their time on the 64 KiB
   // state each one loads and the scan has to carry; one workgroup per CU of longer
-  // segments measured faster than two of shorter ones.
+  // segments measured faster than two of shorter ones (also at d = e = 64, where two share a CU: forward +
+  // backward, b*h = 64, n = 4096: 4 segments of 1024 tokens 107 us against 115 for 8 of 512; b*h = 32, n = 8192: 8 of
+  // 1024 111 against 115).
   if (len < kPreferredSeg && bh * ((n + kPreferredSeg - 1) / kPreferredSeg) >= kMinGroups)
     len = kPreferredSeg;
   // Small problems that leave the chip under-filled even in the backward sweep (three workgroups per
@@ -103,10 +105,11 @@ int default_seg_len(int b, int h, int64_t n) {
   // Only where the shorter segments do not cost the backward sweep (one workgroup per CU) another round:
   // b*h = 4, n = 4096: 22 segments of 192 tokens are 264 workgroups, 56 us against 51 for 16 of 256; b*h = 8,
   // n = 2048: 52 against 49; b*h = 6, n = 3072: 54 against 52 -- and the other way round wherever the rounds
-  // stay the same (b*h = 3 ... 14, n = 2048 ... 4096: 2-6 us faster on 192).
+  // stay the same (b*h = 3 ... 14, n = 2048 ... 4096: 2-6 us faster on 192).  Not at d = e = 64, where twice the workgroups
+  // fit the chip (b*h = 12, n = 4096: 256 tokens 47 us against 52 for 192; b*h = 24, n = 2048: 44 against 49).
   constexpr int kShortSeg = 3 * kSegQuantum;
   auto bwd_rounds = [&](int64_t l) { return (3 * bh * ((n + l - 1) / l) + kMinGroups - 1) / kMinGroups; };
-  if (len == kMinSeg && bh >= 3 && n > 3 * kMinSeg && 3 * bh * ((n + kShortSeg - 1) / kShortSeg) <= kTargetGroups &&
+  if (len == kMinSeg && !narrow64 && bh >= 3 && n > 3 * kMinSeg && 3 * bh * ((n + kShortSeg - 1) / kShortSeg) <= kTargetGroups &&
       bwd_rounds(kShortSeg) <= bwd_rounds(kMinSeg))
     len = kShortSeg;
   // The backward sweep runs three workgroups per segment.  When those exceed what the chip holds at
@@ -134,11 +137,12 @@ int default_seg_len(int b, int h, int64_t n) {
   return (int)len;
 }
 
-// The 16-bit MFMA kernels work on 128 features and read narrower rows zero-extended; their
+// The 16-bit MFMA kernels work on 128 features, or 64 where neither d nor e is larger, and read narrower rows zero-extended; their
 // 8-byte loads and 16-byte stores need every row to start on such a boundary.
 bool mfma_eligible(int d, int e, int dtype) {
   return (dtype == LASP_DTYPE_BF16 || dtype == LASP_DTYPE_F16) && d % 8 == 0 && e % 8 == 0;
 }
+int sweep_width(int d, int e) { return d <= 64 && e <= 64 ? 64 : kMaxFeature; }
 bool mfma_f32_eligible(int d, int e, int dtype) {
   return dtype == LASP_DTYPE_F32 && d == kMaxFeature && e == kMaxFeature;
 }
@@ -201,7 +205,8 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   int rc = check_shape(b, h, n, d, e, dtype);
   if (rc) return rc;
   const int seg_len_arg = seg_len;
-  if (seg_len == 0) seg_len = mfma_eligible(d, e, dtype) ? default_seg_len(b, h, n) : two_per_cu_seg_len(b, h, n);
+  const int width = sweep_width(d, e);
+  if (seg_len == 0) seg_len = mfma_eligible(d, e, dtype) ? default_seg_len(b, h, n, width == 64) : two_per_cu_seg_len(b, h, n);
   if (seg_len < 0 || seg_len % kSegQuantum != 0) {
     set_error("seg_len=%d must be a positive multiple of %d (or 0 for the default)", seg_len,
               kSegQuantum);
@@ -249,7 +254,7 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
       // 208 of 256 CUs: 380 against 360).
       const bool few = fit <= kCombineMaxSeg;
       const bool few_fills = few && bh * fit * 8 >= kMinGroups * r * 7;
-      if (few && (fit < 2 || r > (few_fills ? 2 : 1) || d != kMaxFeature || e != kMaxFeature)) continue;
+      if (few && (fit < 2 || r > (few_fills ? 2 : 1) || d != width || e != width)) continue;
       const int64_t len = (n + fit - 1) / fit;
       int64_t stretched = 0;
       if (r > 1) {  // (more than one round: the pre-pass takes whole segments, see pre_len below)
@@ -308,7 +313,7 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   g->seg_len = seg_len;
   g->n_seg = (int)n_seg_final;
   g->fused = fused_eligible(n, d, e, dtype, seg_len_arg, seg_len, n_seg_final) ? 1 : 0;
-  g->combine = (!g->fused && mfma_eligible(d, e, dtype) && d == kMaxFeature && e == kMaxFeature &&
+  g->combine = (!g->fused && mfma_eligible(d, e, dtype) && d == width && e == width &&
                 n_seg_final <= kCombineMaxSeg) ? 1 : 0;
   // heads whose state dies within a segment skip the scan (16-bit MFMA kernels on the pre-pass / scan / sweep path)
   g->bypass = (mfma_eligible(d, e, dtype) && !g->fused && !g->combine && n_seg_final >= 2) ? 1 : 0;
@@ -330,8 +335,9 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   }
   g->pre_n = (int)((n + g->pre_len - 1) / g->pre_len);
   const bool padded_states = mfma_eligible(d, e, dtype) || mfma_f32_eligible(d, e, dtype);
-  g->sd = padded_states ? kMaxFeature : d;
-  g->se = padded_states ? kMaxFeature : e;
+  g->sd = mfma_eligible(d, e, dtype) ? width : padded_states ? kMaxFeature : d;
+  g->se = mfma_eligible(d, e, dtype) ? width : padded_states ? kMaxFeature : e;
+  g->width = mfma_eligible(d, e, dtype) ? width : 0;
   return 0;
 }
 
@@ -434,8 +440,10 @@ int static_scratch(float **out) {
   return 0;
 }
 
+// (a state of the 64-wide kernels takes a quarter of its slot: every caller sizes the array for 128 x 128)
 size_t state_bytes_of(const Geom &g) {
-  return sizeof(float) * (size_t)g.b * g.h * g.pre_n * g.sd * g.se;
+  const size_t one = g.width == 64 ? (size_t)kMaxFeature * kMaxFeature : (size_t)g.sd * g.se;
+  return sizeof(float) * (size_t)g.b * g.h * g.pre_n * one;
 }
 
 }  // namespace

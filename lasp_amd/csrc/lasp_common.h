@@ -56,7 +56,8 @@ struct Geom {
   int seg_len;  // tokens per segment (multiple of 64)
   int n_seg;    // ceil(n / seg_len)
   int sd, se;   // rows and columns of one segment state as stored in the workspace: d x e for the
-                // generic kernels, 128 x 128 (zero beyond d, e) for the MFMA kernels
+                // generic kernels, 128 x 128 or 64 x 64 (zero beyond d, e) for the MFMA kernels
+  int width;    // 16-bit MFMA kernels: the width they are laid out for, 128 or 64; else 0
   int fused;    // the chunk is served by the single-launch kernels, which use no workspace
   int combine;  // few segments: no scan launch, the sweep workgroups gather the segments' own states
   int bypass;   // the scan leaves out heads whose state dies within one segment (see state_dies_in_segment)
@@ -108,6 +109,8 @@ int generic_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st);
 int generic_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st);
 int mfma_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st);  // bf16 or fp16
 int mfma_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st);
+int mfma_f16_fwd(const FwdArgs &a, const Geom &g, hipStream_t st);
+int mfma_f16_bwd(const BwdArgs &a, const Geom &g, hipStream_t st);
 int mfma_f32_fwd(const FwdArgs &a, const Geom &g, hipStream_t st);
 int mfma_f32_bwd(const BwdArgs &a, const Geom &g, hipStream_t st);
 

@@ -1,7 +1,7 @@
-// bf16 / fp16 MFMA kernels (gfx950, wave64).  The arithmetic is laid out for d = e = 128.
-// Three instantiations of every kernel: M_ALIGNED (chunk length a multiple of 64), M_RAGGED
-// (one partial last block) and M_NARROW (rows of d, e < 128 features, multiples of 8, read
-// zero-extended to 128 and written back at their own width; any chunk length).
+// bf16 / fp16 MFMA kernels (gfx950, wave64).  The arithmetic is laid out for d = e = W, W = 128 or 64.
+// Three instantiations of every kernel and width: M_ALIGNED (chunk length a multiple of 64), M_RAGGED
+// (one partial last block) and M_NARROW (rows of d, e < W features, multiples of 8, read
+// zero-extended to W and written back at their own width; any chunk length).
 //
 // One device routine, `ws_body`, evaluates a causal (or anti-causal) decayed linear
 // attention over a segment of 64-token blocks given the state entering it:
@@ -11,7 +11,7 @@
 //   anti-causal  out_a = sum_{b>=a} l^(b-a) (x_a . y_b) z_b + l^(64-a) x_a St
 //                St   <- l^64 St + sum_b l^b      y_b^T z_b           (blocks descending)
 //
-// (a, b: token index inside the block; St is 128 x 128, rows = features of y,
+// (a, b: token index inside the block; St is W x W, rows = features of y,
 // columns = features of z.)  The four outputs of the operator are instances:
 //   O  : x=Q  y=K  z=V   causal       St = KV            lasp/lasp_fuse.py:104-124
 //   dQ : x=dO y=V  z=K   causal       St = KV^T          lasp/lasp_fuse.py:237-260
@@ -46,9 +46,7 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 typedef uint16_t elem16_t;  // raw bits of one bf16 or fp16 element
 
-constexpr int F = 128;      // feature size (d = e)
 constexpr int BLK = 64;     // tokens per block
-constexpr int LDN = 272;    // bytes per row of a token-major tile (256 + 16: rows shift 4 banks)
 constexpr int LDT = 128;    // bytes per row of a feature-major tile (64 tokens), XOR-swizzled
 constexpr int LDSC = 144;   // bytes per row of the score tile (128 + 16)
 constexpr float LOG2E = kLog2e;
@@ -126,22 +124,24 @@ struct LoaderRole {
   int G, j;    // feature group and half handled by this thread
   int rowq;    // X: row within a 16-row band; Y/Z: group of four rows
 };
-// X tile: 16 consecutive lanes fetch one 256-byte row
+// X tile: W / 8 consecutive lanes fetch one row of W features
+template <int W>
 __device__ __forceinline__ LoaderRole x_role(int tid) {
   LoaderRole r;
-  r.G = (tid >> 1) & 7;
+  r.G = (tid >> 1) & (W / 16 - 1);
   r.j = tid & 1;
-  r.rowq = tid >> 4;
+  r.rowq = tid / (W / 8);
   return r;
 }
 // Y / Z tiles (also stored transposed): lane bits are dealt so that any 16 consecutive
 // lanes cover 8 feature units x 2 row groups -- 16 distinct 8-byte slots of the
-// feature-major tile, i.e. conflict-free ds_write_b64
+// feature-major tile, i.e. conflict-free ds_write_b64.  A tile of W features takes 2 W threads.
+template <int W>
 __device__ __forceinline__ LoaderRole yz_role(int tid) {
   LoaderRole r;
   r.j = tid & 1;
-  r.G = ((tid >> 1) & 3) | (((tid >> 4) & 1) << 2);
-  r.rowq = ((tid >> 3) & 1) | ((tid >> 5) << 1);
+  r.G = W == 128 ? ((tid >> 1) & 3) | (((tid >> 4) & 1) << 2) : (tid >> 1) & 3;
+  r.rowq = ((tid >> 3) & 1) | ((W == 128 ? tid >> 5 : tid >> 4) << 1);
   return r;
 }
 
@@ -233,10 +233,12 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
 // ------------------------------------------------------------------------------
 // Every sweep kernel below is an instance of ws_body<E, REV, TRANS, SRC, MODE>.
 //
+// W.  The width the arithmetic is laid out for: 128, or 64 where neither d nor e is larger.
+//
 // MODE.  M_RAGGED: the chunk length is not a multiple of 64, so the last block of the last segment is
 // partial (rows past its end read as zeros, stores are masked, and the decay factors of that one block use
 // its true length).  M_NARROW: in addition X and Y rows hold `fa` features, Z and Out rows `fb`
-// (multiples of 8, at most 128), read zero-extended to 128 and written back at their own width; the upper
+// (multiples of 8, at most W), read zero-extended to W and written back at their own width; the upper
 // half of the feature steps and state tiles, and waves whose columns lie in the zero extension, are skipped
 // when they would only see zeros.  M_ALIGNED carries none of that bookkeeping; fa and fb are read in
 // M_NARROW only.
@@ -272,13 +274,27 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
 //   ---- barrier ----
 // O(t-1) waits in the X tile of the set that fill(t+1) overwrites after the first barrier.
 // Both groups run their own loop; each executes exactly 1 + 2 * nblk barriers.
+//
+// W = 64 keeps that split with a quarter of the state and half of every tile: 78 848 B of LDS and at most 128
+// registers, so two workgroups share a CU and fill each other's waits.  A feed wave then fetches either Y (waves
+// 0, 1) or Z (waves 2, 3), and a math wave owns one 32 x 32 tile of the output -- columns [32 (w & 1), + 32) of tokens
+// [32 (w >> 1), + 32) -- and the 64 x 32 state columns it needs (both token halves keep those: 8 products per block and
+// wave, against a reduction through LDS).  Rows of 64 features ran on the W = 128 kernels before, where two of the four
+// math waves own columns that do not exist and one workgroup holds the CU (forward + backward, b*h = 64, n = 4096: 210 us
+// against 118; b*h = 16, n = 65536: 692 against 390).
 constexpr int WS_THREADS = 512;
-constexpr int WS_XN = 0, WS_YN = BLK * LDN, WS_YT = 2 * BLK * LDN, WS_ZT = WS_YT + F * LDT;
-constexpr int WS_SET = WS_ZT + F * LDT;        // one block's tiles
-constexpr int WS_SC = 2 * WS_SET;              // the score tile
-constexpr int WS_LDS = WS_SC + BLK * LDSC;     // 144 384 B: one workgroup per CU
+template <int W>
+struct WsLds {
+  static constexpr int LDN = 2 * W + 16;  // bytes per row of a token-major tile (rows shift 4 banks)
+  static constexpr int XN = 0, YN = BLK * LDN, YT = 2 * BLK * LDN, ZT = YT + W * LDT;
+  static constexpr int SET = ZT + W * LDT;         // one block's tiles
+  static constexpr int SC = 2 * SET;               // the score tile
+  static constexpr int BYTES = SC + BLK * LDSC;    // W = 128: 144 384 B, one workgroup per CU; 64: 78 848 B, two
+};
+// workgroups of a sweep that share a CU, and with them the waves per SIMD the registers must leave room for
+constexpr int ws_waves_per_simd(int w) { return w == 64 ? 4 : 1; }
 
-template <class E, bool REV, bool TRANS, int SRC, int MODE>
+template <class E, bool REV, bool TRANS, int SRC, int MODE, int W>
 __device__ __forceinline__ void
 ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z,
         const float *__restrict__ S, const float *__restrict__ states, elem16_t *__restrict__ Out, const Geom &g,
@@ -286,10 +302,15 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
         float *__restrict__ carry_out = nullptr) {
   constexpr bool RAGGED = MODE != M_ALIGNED, NARROW = MODE == M_NARROW;
   constexpr bool LEAVES_STATE = SRC != SRC_SCANNED;  // the sweep's final state is the chunk's outgoing one
+  using L = WsLds<W>;
+  constexpr int NT = W / 32;           // 32-row tiles of a wave's state columns
+  constexpr int NI = W == 128 ? 2 : 1;  // 32-token halves of the output a math wave owns
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int w = w8 & 3;  // feed: score quadrant; math: column block
+  const int w = w8 & 3;                     // feed: score quadrant
+  const int wcol = W == 128 ? w : w & 1;    // math: column block
+  const int ih = W == 128 ? 0 : w >> 1;     // math: (first) token half
   const int c = lane & 31, hh = lane >> 5;
 
   const SegWork sw = seg_work(g, item);
@@ -331,9 +352,13 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   if (w8 < 4) {
     // ================================ feed waves ================================
     const int ftid = tid;  // 0..255
-    const LoaderRole xr = x_role(ftid), yr = yz_role(ftid);
-    const int chunk = ftid & 15, rowq = ftid >> 4;
-    const int xw = NARROW ? fa : F, zw = NARROW ? fb : F;  // row widths in elements
+    constexpr int XI = W / 32;           // X rows per thread
+    constexpr int XROWS = 2048 / W;      // X rows that the feed threads fetch at a time
+    constexpr bool SPLIT = W == 64;      // a thread fetches Y or Z, not both
+    const bool zfeed = SPLIT && w8 >= 2;
+    const LoaderRole xr = x_role<W>(ftid), yr = yz_role<W>(SPLIT ? ftid & 127 : ftid);
+    const int chunk = ftid & (W / 8 - 1), rowq = ftid / (W / 8);
+    const int xw = NARROW ? fa : W, zw = NARROW ? fb : W;  // row widths in elements
     const u32x2 *Xg = reinterpret_cast<const u32x2 *>(X + row0 * xw);
     const u32x2 *Yg = reinterpret_cast<const u32x2 *>(Y + row0 * xw);
     const u32x2 *Zg = reinterpret_cast<const u32x2 *>(Z + row0 * zw);
@@ -348,31 +373,32 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     }
     const int qI = w >> 1, qJ = w & 1;
     const bool q_active = REV ? !(qI == 1 && qJ == 0) : !(qI == 0 && qJ == 1);
-    const uint32_t x_off = lane_offset(xr, xr.rowq, xu), y_off = lane_offset(yr, 4 * yr.rowq, xu),
+    const int yu = zfeed ? zu : xu;      // SPLIT: of the tile that this wave fetches through ny
+    const uint32_t x_off = lane_offset(xr, xr.rowq, xu), y_off = lane_offset(yr, 4 * yr.rowq, yu),
                    z_off = lane_offset(yr, 4 * yr.rowq, zu);
     const PieceMask all = {true, true};
-    const PieceMask x_ok = piece_mask(xr, xu), y_ok = piece_mask(yr, xu), z_ok = piece_mask(yr, zu);
+    const PieceMask x_ok = piece_mask(xr, xu), y_ok = piece_mask(yr, yu), z_ok = piece_mask(yr, zu);
 
-    // the block in flight, two 8-byte pieces per row (see LoaderRole)
-    u32x4 nx[4], ny[4], nz[4];
+    // the block in flight, two 8-byte pieces per row (see LoaderRole); SPLIT: ny holds Y or Z
+    u32x4 nx[XI], ny[4], nz[4];
     // k: position in the run; walk blocks (k < runup) need no X tile
     auto issue_loads = [&](int k) __attribute__((always_inline)) {
       const int blk = first_blk + k * step;
       const int len = len_of(blk);  // rows past a partial block's end and pieces past a narrow row's width read as zeros
       const gmem_ptr xblk = uniform_ptr(reinterpret_cast<const char *>(Xg) + (int64_t)blk * BLK * xu * 8);
-      const gmem_ptr yblk = uniform_ptr(reinterpret_cast<const char *>(Yg) + (int64_t)blk * BLK * xu * 8);
+      const gmem_ptr yblk = uniform_ptr(reinterpret_cast<const char *>(zfeed ? Zg : Yg) + (int64_t)blk * BLK * yu * 8);
       const gmem_ptr zblk = uniform_ptr(reinterpret_cast<const char *>(Zg) + (int64_t)blk * BLK * zu * 8);
       if (SRC != SRC_WALK || k >= runup) {
 #pragma unroll
-        for (int it = 0; it < 4; ++it)
-          nx[it] = load_row_pieces(xblk, 16 * it * xu * 8, x_off, NARROW ? x_ok : all,
-                                   !RAGGED || xr.rowq + 16 * it < len);
+        for (int it = 0; it < XI; ++it)
+          nx[it] = load_row_pieces(xblk, XROWS * it * xu * 8, x_off, NARROW ? x_ok : all,
+                                   !RAGGED || xr.rowq + XROWS * it < len);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const bool row_ok = !RAGGED || 4 * yr.rowq + r < len;
-        ny[r] = load_row_pieces(yblk, r * xu * 8, y_off, NARROW ? y_ok : all, row_ok);
-        nz[r] = load_row_pieces(zblk, r * zu * 8, z_off, NARROW ? z_ok : all, row_ok);
+        ny[r] = load_row_pieces(yblk, r * yu * 8, y_off, NARROW ? y_ok : all, row_ok);
+        if (!SPLIT) nz[r] = load_row_pieces(zblk, r * zu * 8, z_off, NARROW ? z_ok : all, row_ok);
       }
     };
     // writes the block held in nx / ny / nz into a tile set: token-major X and Y, feature-major Y (scaled by the
@@ -380,11 +406,17 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     auto fill = [&](char *set, int k) __attribute__((always_inline)) {
       if (SRC != SRC_WALK || k >= runup) {  // a walk block is only multiplied into the state
 #pragma unroll
-        for (int it = 0; it < 4; ++it)
-          *reinterpret_cast<u32x4 *>(set + WS_XN + (xr.rowq + 16 * it) * LDN + (2 * xr.G + xr.j) * 16) = nx[it];
+        for (int it = 0; it < XI; ++it)
+          *reinterpret_cast<u32x4 *>(set + L::XN + (xr.rowq + XROWS * it) * L::LDN + (2 * xr.G + xr.j) * 16) = nx[it];
+        if (!zfeed) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          *reinterpret_cast<u32x4 *>(set + WS_YN + (4 * yr.rowq + r) * LDN + (2 * yr.G + yr.j) * 16) = ny[r];
+          for (int r = 0; r < 4; ++r)
+            *reinterpret_cast<u32x4 *>(set + L::YN + (4 * yr.rowq + r) * L::LDN + (2 * yr.G + yr.j) * 16) = ny[r];
+        }
+      }
+      if (zfeed) {
+        store_transposed<E, false>(set + L::ZT, ny, yr, kdec);
+        return;
       }
       const int len = len_of(first_blk + k * step);
       if (LEAVES_STATE && RAGGED && !REV && len != BLK) {
@@ -393,22 +425,22 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
         float kd[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) kd[r] = decay(sl, (float)max(len - (4 * yr.rowq + r), 0));
-        store_transposed<E, true>(set + WS_YT, ny, yr, kd);
+        store_transposed<E, true>(set + L::YT, ny, yr, kd);
       } else {
-        store_transposed<E, true>(set + WS_YT, ny, yr, kdec);
+        store_transposed<E, true>(set + L::YT, ny, yr, kdec);
       }
-      store_transposed<E, false>(set + WS_ZT, nz, yr, kdec);
+      if (!SPLIT) store_transposed<E, false>(set + L::ZT, nz, yr, kdec);
     };
     // the output tile staged in `set`'s X region -> global rows of block `blk`
     auto store_out = [&](const char *set, int blk) __attribute__((always_inline)) {
       const int64_t brow = (int64_t)blk * BLK;
       const int len = len_of(blk);
 #pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const int row = rowq + 16 * r4;
+      for (int r4 = 0; r4 < XI; ++r4) {
+        const int row = rowq + XROWS * r4;
         if (!RAGGED || (row < len && (!NARROW || chunk < ou)))
-          __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(set + WS_XN + row * LDN + chunk * 16),
-                                      &Og[(brow + row) * (NARROW ? ou : F / 8) + chunk]);
+          __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(set + L::XN + row * L::LDN + chunk * 16),
+                                      &Og[(brow + row) * (NARROW ? ou : W / 8) + chunk]);
       }
     };
     // this wave's quadrant of the transposed score tile: sc[4g+r] = y_b . x_a, b = 32qJ+8g+4hh+r, a = 32qI+c
@@ -417,10 +449,10 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       floatx16 sc;
 #pragma unroll
       for (int r = 0; r < 16; ++r) sc[r] = 0.f;
-      const char *xa = set + WS_XN + (32 * qI + c) * LDN + hh * 16;
-      const char *ya = set + WS_YN + (32 * qJ + c) * LDN + hh * 16;
+      const char *xa = set + L::XN + (32 * qI + c) * L::LDN + hh * 16;
+      const char *ya = set + L::YN + (32 * qJ + c) * L::LDN + hh * 16;
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) sc = E::mfma(lds16(ya + ks * 32), lds16(xa + ks * 32), sc);
+      for (int ks = 0; ks < W / 16; ++ks) sc = E::mfma(lds16(ya + ks * 32), lds16(xa + ks * 32), sc);
       const int a = 32 * qI + c;
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
@@ -434,7 +466,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
         u32x2 o;
         o.x = E::pack(m[0], m[1]);
         o.y = E::pack(m[2], m[3]);
-        *reinterpret_cast<u32x2 *>(smem + WS_SC + a * LDSC + (32 * qJ + 8 * gq + 4 * hh) * 2) = o;
+        *reinterpret_cast<u32x2 *>(smem + L::SC + a * LDSC + (32 * qJ + 8 * gq + 4 * hh) * 2) = o;
       }
     };
 
@@ -444,12 +476,12 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     __syncthreads();  // barrier 0: block 0 of the run visible
     int k = 0;
     for (; k < runup; ++k) {  // walk: the math waves multiply block k into the state meanwhile
-      fill(smem + ((k + 1) & 1) * WS_SET, k + 1);  // k + 1 < run: a sweep block follows the walk
+      fill(smem + ((k + 1) & 1) * L::SET, k + 1);  // k + 1 < run: a sweep block follows the walk
       if (k + 2 < run) issue_loads(k + 2);
       __syncthreads();  // walk barrier k
     }
     for (; k < run; ++k) {
-      char *cur = smem + (k & 1) * WS_SET, *nxt = smem + ((k + 1) & 1) * WS_SET;
+      char *cur = smem + (k & 1) * L::SET, *nxt = smem + ((k + 1) & 1) * L::SET;
       // the stores go first: by the time the fill below waits for its loads (loads and stores share one
       // counter, so that wait drains both) they have long left
       if (k > runup) store_out(nxt, first_blk + (k - 1) * step);
@@ -461,36 +493,36 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       }
       __syncthreads();  // second barrier: next block visible; output of this block staged
     }
-    store_out(smem + ((run - 1) & 1) * WS_SET, first_blk + (run - 1) * step);
+    store_out(smem + ((run - 1) & 1) * L::SET, first_blk + (run - 1) * step);
     return;
   }
 
   // ================================== math waves ==================================
-  float qdec[2];
+  float qdec[NI];
 #pragma unroll
-  for (int I = 0; I < 2; ++I) {
-    const int a = 32 * I + c;
+  for (int I = 0; I < NI; ++I) {
+    const int a = 32 * (ih + I) + c;
     qdec[I] = decay(sl, REV ? (float)(BLK - a) : (float)a);
   }
-  // state entering the segment: st[T][4g+r] = St[32T+8g+4hh+r][32w+c]
-  floatx16 st[4];
+  // state entering the segment: st[T][4g+r] = St[32T+8g+4hh+r][32 wcol + c]
+  floatx16 st[NT];
 #pragma unroll
-  for (int T = 0; T < 4; ++T)
+  for (int T = 0; T < NT; ++T)
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[T][r] = 0.f;
   // M_NARROW: a wave whose 32 columns all lie past the width of Z has nothing to compute (it still takes part in
-  // every barrier); the upper 64 features are skipped as a whole when the rows are no wider
-  const bool wave_active = !NARROW || 32 * w < fb;
-  const bool upper_half = !NARROW || fa > 64;
-  // st <- f * st + M, M being the 128 x 128 fp32 tile whose element (row, col) is src[row * ld + col], or for a
+  // every barrier); the upper half of the features is skipped as a whole when the rows are no wider
+  const bool wave_active = !NARROW || W == 64 || 32 * wcol < fb;  // (at W = 64 the skipping costs registers that two workgroups per CU do not have)
+  const bool upper_half = !NARROW || W == 64 || fa > W / 2;
+  // st <- f * st + M, M being the W x W fp32 tile whose element (row, col) is src[row * ld + col], or for a
   // transposed role src[col * ld + row]; `bounded`: src holds only fa x fb (transposed: fb x fa) elements
   auto add_state_ld = [&](const float *src, int ld, float f, bool bounded) __attribute__((always_inline)) {
     typedef const __attribute__((address_space(1))) float *gmem_f32;
     const uint32_t lane_off =
-        (uint32_t)(TRANS ? (32 * w + c) * ld + 4 * hh : 4 * hh * ld + 32 * w + c) * (uint32_t)sizeof(float);
-    const bool col_ok = !bounded || 32 * w + c < fb;
+        (uint32_t)(TRANS ? (32 * wcol + c) * ld + 4 * hh : 4 * hh * ld + 32 * wcol + c) * (uint32_t)sizeof(float);
+    const bool col_ok = !bounded || 32 * wcol + c < fb;
 #pragma unroll
-    for (int T = 0; T < 4; ++T)
+    for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
         const int band = 32 * T + 8 * gq;
@@ -504,10 +536,10 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
         }
       }
   };
-  // a state of the workspace (128 x 128, zero beyond fa x fb) / the chunk's incoming state (fa x fb, unpadded)
-  auto add_state = [&](const float *src, float f) __attribute__((always_inline)) { add_state_ld(src, F, f, false); };
+  // a state of the workspace (W x W, zero beyond fa x fb) / the chunk's incoming state (fa x fb, unpadded)
+  auto add_state = [&](const float *src, float f) __attribute__((always_inline)) { add_state_ld(src, W, f, false); };
   auto add_carry = [&]() __attribute__((always_inline)) {
-    add_state_ld(carry_in + (int64_t)sw.bh * fa * fb, NARROW ? (TRANS ? fa : fb) : F, 0.f, NARROW);
+    add_state_ld(carry_in + (int64_t)sw.bh * fa * fb, NARROW ? (TRANS ? fa : fb) : W, 0.f, NARROW);
   };
   if (SRC == SRC_WALK) {
     if (take_carry) add_carry();
@@ -521,18 +553,18 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       // enters it is the one entering its first piece in sweep order.
       const int sub = g.seg_len / g.pre_len;
       const int piece = REV ? min(sw.seg * sub + sub, g.pre_n) - 1 : sw.seg * sub;
-      const float *src = states + ((int64_t)sw.bh * g.pre_n + piece) * (F * F);
+      const float *src = states + ((int64_t)sw.bh * g.pre_n + piece) * (W * W);
       bool from_carry = false;
       if (state_dies_in_segment(S[sw.bh % g.h], g)) {
         const int nb = REV ? piece + 1 : piece - 1;
         if (nb < 0 || nb >= g.pre_n)
           from_carry = true;
         else
-          src = states + ((int64_t)sw.bh * g.pre_n + nb) * (F * F);
+          src = states + ((int64_t)sw.bh * g.pre_n + nb) * (W * W);
       }
       // (for such a head the scan kernel has parked the chunk's incoming state in the slot of the piece it
       // visits last, so that nothing reads `carry_in`'s memory once the outgoing state may have replaced it)
-      if (from_carry) src = states + ((int64_t)sw.bh * g.pre_n + (REV ? 0 : g.pre_n - 1)) * (F * F);
+      if (from_carry) src = states + ((int64_t)sw.bh * g.pre_n + (REV ? 0 : g.pre_n - 1)) * (W * W);
       if (!from_carry || carry_in != nullptr) add_state(src, 0.f);
     }
   } else {
@@ -550,154 +582,154 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     first = __builtin_amdgcn_readfirstlane(first);
     if (first == 0 && carry_in) add_carry();
     if (states) {
-      const float *base = states + (int64_t)sw.bh * g.n_seg * (F * F);
+      const float *base = states + (int64_t)sw.bh * g.n_seg * (W * W);
       const float full = decay(sl, (float)g.seg_len);
       const float last = decay(sl, (float)(g.n - (int64_t)(g.n_seg - 1) * g.seg_len));
       for (int i = first; i < n_before; ++i) {
         const int j = REV ? g.n_seg - 1 - i : i;
-        add_state(base + (int64_t)j * (F * F), j == g.n_seg - 1 ? last : full);
+        add_state(base + (int64_t)j * (W * W), j == g.n_seg - 1 ? last : full);
       }
     }
   }
   // St <- l^64 St + (scaled Y)^T Z from the feature-major tiles of `set`
   auto update_state = [&](const char *set, const u32x4 (&zf)[4], float bd) __attribute__((always_inline)) {
 #pragma unroll
-    for (int T = 0; T < 4; ++T)
+    for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int r = 0; r < 16; ++r) st[T][r] *= bd;
-    u32x4 yf[4][4];
+    u32x4 yf[4][NT];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int T = 0; T < 4; ++T)
-        if (T < 2 || upper_half) yf[u][T] = lds16(set + WS_YT + tr_off(32 * T + c, 2 * u + hh));
+      for (int T = 0; T < NT; ++T)
+        if (T < NT / 2 || upper_half) yf[u][T] = lds16(set + L::YT + tr_off(32 * T + c, 2 * u + hh));
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int T = 0; T < 4; ++T)
-        if (T < 2 || upper_half) st[T] = E::mfma(yf[u][T], zf[u], st[T]);  // state rows past the width of Y stay zero
+      for (int T = 0; T < NT; ++T)
+        if (T < NT / 2 || upper_half) st[T] = E::mfma(yf[u][T], zf[u], st[T]);  // state rows past the width of Y stay zero
   };
   __syncthreads();  // barrier 0
   for (int k = 0; k < runup; ++k) {  // walk
-    const char *set = smem + (k & 1) * WS_SET;
+    const char *set = smem + (k & 1) * L::SET;
     if (wave_active) {
       const int len = len_of(first_blk + k * step);
       u32x4 zf[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) zf[u] = lds16(set + WS_ZT + tr_off(32 * w + c, 2 * u + hh));
+      for (int u = 0; u < 4; ++u) zf[u] = lds16(set + L::ZT + tr_off(32 * wcol + c, 2 * u + hh));
       update_state(set, zf, RAGGED && len != BLK ? decay(sl, (float)len) : blockdec);
     }
     __syncthreads();  // walk barrier k
   }
   for (int it = 0; it < nblk; ++it) {
-    char *cur = smem + ((runup + it) & 1) * WS_SET;
+    char *cur = smem + ((runup + it) & 1) * L::SET;
     // A partial block is the chunk's last one.  Going forwards nothing after it uses the state (but the outgoing
     // state where the sweep leaves it); going backwards it comes first and the entering state sits `len` (not 64)
     // tokens ahead.
     const int len = len_of(blk0 + it * step);
-    float qd[2] = {qdec[0], qdec[1]};
+    float qd[NI];
+#pragma unroll
+    for (int I = 0; I < NI; ++I) qd[I] = qdec[I];
     float bd = blockdec;
     if (RAGGED && REV && len != BLK) {
-      qd[0] = decay(sl, (float)max(len - c, 0));
-      qd[1] = decay(sl, (float)max(len - 32 - c, 0));
+#pragma unroll
+      for (int I = 0; I < NI; ++I) qd[I] = decay(sl, (float)max(len - 32 * (ih + I) - c, 0));
       bd = decay(sl, (float)len);
     }
     if (LEAVES_STATE && RAGGED && !REV && len != BLK) bd = decay(sl, (float)len);
-    // state term, transposed: acc[I][4g+r] = sum_f St[f][32w+8g+4hh+r] x_a[f], a = 32I+c
-    floatx16 acc[2];
+    // state term, transposed: acc[I][4g+r] = sum_f St[f][32 wcol + 8g+4hh+r] x_a[f], a = 32 (ih + I) + c
+    floatx16 acc[NI];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      acc[0][r] = 0.f;
-      acc[1][r] = 0.f;
-    }
+    for (int I = 0; I < NI; ++I)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[I][r] = 0.f;
     if (wave_active) {
-      // all sixteen X fragments are requested before the first product (these waves have the registers for it)
-      const char *x0 = cur + WS_XN + c * LDN + hh * 16;
-      const char *x1 = x0 + 32 * LDN;
-      u32x4 xf[8][2];
+      // all X fragments are requested before the first product (these waves have the registers for it)
+      const char *x0 = cur + L::XN + (32 * ih + c) * L::LDN + hh * 16;
+      u32x4 xf[W / 16][NI];
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) {
-        if (ks >= 4 && !upper_half) continue;
-        xf[ks][0] = lds16(x0 + ks * 32);
-        xf[ks][1] = lds16(x1 + ks * 32);
+      for (int ks = 0; ks < W / 16; ++ks) {
+        if (ks >= W / 32 && !upper_half) continue;
+#pragma unroll
+        for (int I = 0; I < NI; ++I) xf[ks][I] = lds16(x0 + 32 * I * L::LDN + ks * 32);
       }
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) {
-        if (ks >= 4 && !upper_half) continue;
+      for (int ks = 0; ks < W / 16; ++ks) {
+        if (ks >= W / 32 && !upper_half) continue;
         const int T = ks >> 1, u = ks & 1;
         u32x4 a;
         a.x = E::pack(st[T][8 * u + 0], st[T][8 * u + 1]);
         a.y = E::pack(st[T][8 * u + 2], st[T][8 * u + 3]);
         a.z = E::pack(st[T][8 * u + 4], st[T][8 * u + 5]);
         a.w = E::pack(st[T][8 * u + 6], st[T][8 * u + 7]);
-        acc[0] = E::mfma(a, xf[ks][0], acc[0]);
-        acc[1] = E::mfma(a, xf[ks][1], acc[1]);
+#pragma unroll
+        for (int I = 0; I < NI; ++I) acc[I] = E::mfma(a, xf[ks][I], acc[I]);
       }
     }
 #pragma unroll
-    for (int I = 0; I < 2; ++I)
+    for (int I = 0; I < NI; ++I)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[I][r] *= qd[I];
     __syncthreads();  // barrier 2 it + 1: score tile complete
     if (wave_active) {
       u32x4 zf[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) zf[u] = lds16(cur + WS_ZT + tr_off(32 * w + c, 2 * u + hh));
-      // intra-block term: acc[I] += Z^T[32w.., tokens] * score[a][tokens]
+      for (int u = 0; u < 4; ++u) zf[u] = lds16(cur + L::ZT + tr_off(32 * wcol + c, 2 * u + hh));
+      // intra-block term: acc[I] += Z^T[32 wcol.., tokens] * score[a][tokens]
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int I = 0; I < 2; ++I) {
-          const bool needed = REV ? (I == 0 || u >= 2) : (I == 1 || u < 2);
+        for (int I = 0; I < NI; ++I) {
+          const bool needed = REV ? (ih + I == 0 || u >= 2) : (ih + I == 1 || u < 2);
           if (needed)
-            acc[I] = E::mfma(zf[u], lds16(smem + WS_SC + (32 * I + c) * LDSC + (16 * u + 8 * hh) * 2), acc[I]);
+            acc[I] = E::mfma(zf[u], lds16(smem + L::SC + (32 * (ih + I) + c) * LDSC + (16 * u + 8 * hh) * 2), acc[I]);
         }
       update_state(cur, zf, bd);
     }
     // stage the output tile (token-major) in the X region of this block
     if (wave_active)
 #pragma unroll
-    for (int I = 0; I < 2; ++I)
+    for (int I = 0; I < NI; ++I)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
         u32x2 o;
         o.x = E::pack(acc[I][4 * gq + 0], acc[I][4 * gq + 1]);
         o.y = E::pack(acc[I][4 * gq + 2], acc[I][4 * gq + 3]);
-        *reinterpret_cast<u32x2 *>(cur + WS_XN + (32 * I + c) * LDN + (32 * w + 8 * gq + 4 * hh) * 2) = o;
+        *reinterpret_cast<u32x2 *>(cur + L::XN + (32 * (ih + I) + c) * L::LDN + (32 * wcol + 8 * gq + 4 * hh) * 2) = o;
       }
     __syncthreads();  // barrier 2 it + 2
   }
   // the segment visited last leaves the chunk's outgoing state
-  if (SRC != SRC_SCANNED && !TRANS && carry_out != nullptr && sw.seg == (REV ? 0 : g.n_seg - 1)) {
+  if (SRC != SRC_SCANNED && !TRANS && carry_out != nullptr && sw.seg == (REV ? 0 : g.n_seg - 1) && ih == 0) {
     float *cp = carry_out + (int64_t)sw.bh * fa * fb;
-    const int col = 32 * w + c;
+    const int col = 32 * wcol + c;
 #pragma unroll
-    for (int T = 0; T < 4; ++T)
+    for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = 32 * T + 8 * (r >> 2) + 4 * hh + (r & 3);
-        if (!NARROW || (row < fa && col < fb)) cp[row * (NARROW ? fb : F) + col] = st[T][r];
+        if (!NARROW || (row < fa && col < fb)) cp[row * (NARROW ? fb : W) + col] = st[T][r];
       }
   }
 }
 
-template <class E, bool REV, bool TRANS, int SRC, int MODE>
-__global__ void __launch_bounds__(WS_THREADS, 1)
+template <class E, bool REV, bool TRANS, int SRC, int MODE, int W>
+__global__ void __launch_bounds__(WS_THREADS, ws_waves_per_simd(W))
 la_apply(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z,
             const float *__restrict__ S, const float *__restrict__ states, const float *__restrict__ carry_in,
             float *__restrict__ carry_out, elem16_t *__restrict__ Out, Geom g) {
   extern __shared__ __align__(16) char smem[];
   // SRC_COMBINE: later segments have more states to gather first, so they are started first
   const int item = SRC == SRC_COMBINE ? g.b * g.h * g.n_seg - 1 - (int)blockIdx.x : (int)blockIdx.x;
-  ws_body<E, REV, TRANS, SRC, MODE>(X, Y, Z, S, states, Out, g, g.d, g.e, item, smem, carry_in, carry_out);
+  ws_body<E, REV, TRANS, SRC, MODE, W>(X, Y, Z, S, states, Out, g, g.d, g.e, item, smem, carry_in, carry_out);
 }
 
 // A whole short chunk in one launch: every workgroup rebuilds the state entering its segment (SRC_WALK), so
 // there is no pre-pass, no scan and no workspace.  Workgroups are dealt to the 8 XCDs round-robin: all
 // segments of one (b, h) go to the same XCD, whose L2 then serves the repeated walks over that (b, h)'s K
 // and V; later segments, which walk over more blocks first, are started first.
-template <class E, int MODE>
-__global__ void __launch_bounds__(WS_THREADS, 1)
+template <class E, int MODE, int W>
+__global__ void __launch_bounds__(WS_THREADS, ws_waves_per_simd(W))
 la_fused_fwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const elem16_t *__restrict__ V,
                 const float *__restrict__ S, const float *__restrict__ kv_in, float *__restrict__ kv_out,
                 elem16_t *__restrict__ O, Geom g) {
@@ -706,12 +738,12 @@ la_fused_fwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
   const int bh = (slot / g.n_seg) * 8 + xcd;
   if (bh >= g.b * g.h) return;
   const int item = bh * g.n_seg + (g.n_seg - 1 - slot % g.n_seg);
-  ws_body<E, false, false, SRC_WALK, MODE>(Q, K, V, S, nullptr, O, g, g.d, g.e, item, smem, kv_in, kv_out);
+  ws_body<E, false, false, SRC_WALK, MODE, W>(Q, K, V, S, nullptr, O, g, g.d, g.e, item, smem, kv_in, kv_out);
 }
 
 // roles as in la_bwd3 (the dV role leaves dKV_out); all roles and segments of one (b, h) on one XCD
-template <class E, int MODE>
-__global__ void __launch_bounds__(WS_THREADS, 1)
+template <class E, int MODE, int W>
+__global__ void __launch_bounds__(WS_THREADS, ws_waves_per_simd(W))
 la_fused_bwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const elem16_t *__restrict__ V,
                 const elem16_t *__restrict__ DO, const float *__restrict__ S, const float *__restrict__ kv_in,
                 const float *__restrict__ dkv_in, float *__restrict__ dkv_out, elem16_t *__restrict__ DQ,
@@ -724,21 +756,21 @@ la_fused_bwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
   const int rem = slot % per_bh;
   const int role = rem % 3, k = rem / 3;  // k-th longest walk of its role
   if (role == 0)
-    ws_body<E, false, true, SRC_WALK, MODE>(DO, V, K, S, nullptr, DQ, g, g.e, g.d, bh * g.n_seg + g.n_seg - 1 - k, smem,
+    ws_body<E, false, true, SRC_WALK, MODE, W>(DO, V, K, S, nullptr, DQ, g, g.e, g.d, bh * g.n_seg + g.n_seg - 1 - k, smem,
                                             kv_in);
   else if (role == 1)
-    ws_body<E, true, false, SRC_WALK, MODE>(K, Q, DO, S, nullptr, DV, g, g.d, g.e, bh * g.n_seg + k, smem, dkv_in,
+    ws_body<E, true, false, SRC_WALK, MODE, W>(K, Q, DO, S, nullptr, DV, g, g.d, g.e, bh * g.n_seg + k, smem, dkv_in,
                                             dkv_out);
   else
-    ws_body<E, true, true, SRC_WALK, MODE>(V, DO, Q, S, nullptr, DK, g, g.e, g.d, bh * g.n_seg + k, smem, dkv_in);
+    ws_body<E, true, true, SRC_WALK, MODE, W>(V, DO, Q, S, nullptr, DK, g, g.e, g.d, bh * g.n_seg + k, smem, dkv_in);
 }
 
 // The three gradients in one launch.  Workgroups come in triples (dQ, dV, dK) that work on the same
 // (b*h, segment) and therefore read the same Q, K, V, dO blocks; the triple is spread over block indices 8
 // apart so that all three land on the same XCD (workgroups are dealt to the 8 XCDs round-robin) and share
 // its L2.
-template <class E, int SRC, int MODE>
-__global__ void __launch_bounds__(WS_THREADS, 1)
+template <class E, int SRC, int MODE, int W>
+__global__ void __launch_bounds__(WS_THREADS, ws_waves_per_simd(W))
 la_bwd3(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const elem16_t *__restrict__ V,
            const elem16_t *__restrict__ DO, const float *__restrict__ S, const float *__restrict__ kv_states,
            const float *__restrict__ dkv_states, const float *__restrict__ kv_in, const float *__restrict__ dkv_in,
@@ -751,11 +783,11 @@ la_bwd3(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const el
   const int item = n_items - 1 - (grp * 8 + (r & 7));
   if (item < 0) return;
   if (role == 0)
-    ws_body<E, false, true, SRC, MODE>(DO, V, K, S, kv_states, DQ, g, g.e, g.d, item, smem, kv_in);
+    ws_body<E, false, true, SRC, MODE, W>(DO, V, K, S, kv_states, DQ, g, g.e, g.d, item, smem, kv_in);
   else if (role == 1)
-    ws_body<E, true, false, SRC, MODE>(K, Q, DO, S, dkv_states, DV, g, g.d, g.e, item, smem, dkv_in, dkv_out);
+    ws_body<E, true, false, SRC, MODE, W>(K, Q, DO, S, dkv_states, DV, g, g.d, g.e, item, smem, dkv_in, dkv_out);
   else
-    ws_body<E, true, true, SRC, MODE>(V, DO, Q, S, dkv_states, DK, g, g.e, g.d, item, smem, dkv_in);
+    ws_body<E, true, true, SRC, MODE, W>(V, DO, Q, S, dkv_states, DK, g, g.e, g.d, item, smem, dkv_in);
 }
 
 // ------------------------------------------------------------------------------
@@ -775,15 +807,25 @@ la_bwd3(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const el
 // keeping D blocks in flight in registers (16 registers per block) on top of the two LDS
 // buffers; wave (wc, rh) owns rows [64 rh, 64 rh + 64) x columns [32 wc, 32 wc + 32) of the state
 // as two accumulator tiles.
+// W = 64: a step takes two blocks of the walk, i.e. the same bytes, and the four waves that fetch Z (and so have
+// nothing to scale) own a 32 x 32 tile of the state each.  The blocks are weighted and added one after the other, as at
+// W = 128, so that rows of 64 features give the bits that the same rows zero-extended to 128 give.
 //
 // Both tiles stay token-major in LDS, as they are in memory (16-byte copies, Y scaled by the decay
 // weights on the way); the products contract over tokens, so the MFMA operands are fetched with
 // the transposing LDS read.
 constexpr int STATE_THREADS = 512;
-constexpr int LDR = 320;  // bytes per token row (256 + 64: the four rows that one transposing read
-                          // touches per half-wave fall on disjoint banks)
-constexpr int STATE_TILE = BLK * LDR;
-constexpr int STATE_LDS = 2 * 2 * STATE_TILE;  // double-buffered {Y scaled, Z}: 80 KiB
+template <int W>
+struct StateLds {
+  // Bytes per token row.  The four rows x 64 bytes that one transposing read touches per half-wave fall on
+  // disjoint banks: W = 128 rows are 64 bytes longer than the data; W = 64 rows (two to a set of banks) swap their
+  // 64-byte halves in every other pair of rows (see row_swap).
+  static constexpr int LDR = W == 128 ? 320 : 128;
+  static constexpr int BPS = W == 128 ? 1 : 2;  // blocks per step
+  static constexpr int TILE = BPS * BLK * LDR;
+  static constexpr int BYTES = 2 * 2 * TILE;  // double-buffered {Y scaled, Z}: 80 KiB, W = 64: 64 KiB
+  static __device__ __forceinline__ int row_swap(int row) { return W == 128 ? 0 : ((row >> 1) & 1) << 6; }
+};
 // Blocks in flight per thread in registers (even).  Long walks gain from the deeper pipeline (b*h = 16,
 // n = 65536, 2048-token pieces: 46 us per launch against 49); on short ones the longer start-up costs more
 // than it gains (320-token segments: 13.1 us against 12.4).  The shallow form stays within 128 registers, so two
@@ -801,9 +843,10 @@ __device__ __forceinline__ u32x2 lds_tr8(const char *p) {
   return __builtin_bit_cast(u32x2, r);
 }
 // MFMA operand of lane (c, hh): feature f0 + c, tokens t0 + 8 hh .. + 7 (`lane_part` holds the lane's share
-// of the address, see la_seg_state)
-__device__ __forceinline__ u32x4 token_fragment(const char *tile, int lane_part, int f0, int t0) {
-  const char *p = tile + lane_part + t0 * LDR + f0 * 2;
+// of the address, see la_seg_state; rows LDR bytes apart)
+template <int LDR>
+__device__ __forceinline__ u32x4 token_fragment(const char *tile, int lane_part, int t0) {
+  const char *p = tile + lane_part + t0 * LDR;
   const u32x2 lo = lds_tr8(p), hi = lds_tr8(p + 4 * LDR);
   u32x4 r;
   r.x = lo.x;
@@ -813,21 +856,26 @@ __device__ __forceinline__ u32x4 token_fragment(const char *tile, int lane_part,
   return r;
 }
 
-template <class E, bool REV, int MODE, int D>
+template <class E, bool REV, int MODE, int W, int D>
 __global__ void __launch_bounds__(STATE_THREADS, 1)
 la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, const float *__restrict__ S,
              float *__restrict__ states, Geom g, int skip_seg, int sub) {
   constexpr bool RAGGED = MODE != M_ALIGNED, NARROW = MODE == M_NARROW;
+  using L = StateLds<W>;
+  constexpr int BPS = L::BPS;              // blocks per step
+  constexpr int NTILE = W == 128 ? 2 : 1;  // 32 x 32 tiles of the state per wave
+  constexpr int ROWS = 2048 / W;           // token rows that 256 threads fetch at a time
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform: keeps it in an SGPR
-  const int wc = w8 & 3, rh = w8 >> 2;                      // column block and row half of this wave's tiles
+  const int wc = W == 128 ? w8 & 3 : w8 & 1;                // column block ...
+  const int row0s = W == 128 ? 64 * (w8 >> 2) : 32 * ((w8 >> 1) & 1);  // ... and first row of this wave's tiles
   const bool zgrp = w8 >= 4;                                // this wave fetches Z (else Y)
   const int c = lane & 31, hh = lane >> 5;
-  // loader: 16 consecutive threads copy one row, the thread's 16 bytes are features 8 cq .. + 7 of rows
-  // rq, rq + 16, rq + 32, rq + 48
-  const int cq = tid & 15, rq = (tid & 255) >> 4;
+  // loader: W / 8 consecutive threads copy one row, the thread's 16 bytes are features 8 cq .. + 7 of rows
+  // rq + ROWS * {0, 1, 2, 3}
+  const int cq = tid & (W / 8 - 1), rq = (tid & 255) / (W / 8);
 
   // slow-decaying heads (the later ones in the usual slope schedules) have the most to read: first
   const int n_items = g.b * g.h * g.n_seg;
@@ -847,18 +895,18 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   }
   const float sl = slope * LOG2E;
   const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
-  const int yw = NARROW ? g.d : F, zw = NARROW ? g.e : F;  // row widths in elements
+  const int yw = NARROW ? g.d : W, zw = NARROW ? g.e : W;  // row widths in elements
   const int tw = zgrp ? zw : yw;                           // of the tile this thread fetches
   const char *Tg = reinterpret_cast<const char *>(zgrp ? Z + row0 * zw : Y + row0 * yw);
   const int row_bytes = tw * 2;
 
+  // row r of the thread's four: token row_of(r) of block half_of(r) of the step
+  auto half_of = [](int r) { return BPS == 1 ? 0 : r >> 1; };
+  auto row_of = [&](int r) __attribute__((always_inline)) { return rq + ROWS * (BPS == 1 ? r : r & 1); };
   const float blockdec = decay(sl, (float)BLK);
-  float kdec[4];
+  float kdec[4 / BPS];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int b = rq + 16 * r;
-    kdec[r] = decay(sl, REV ? (float)b : (float)(BLK - b));
-  }
+  for (int r = 0; r < 4 / BPS; ++r) kdec[r] = decay(sl, REV ? (float)row_of(r) : (float)(BLK - row_of(r)));
 
   // blocks lo..hi of the segment are processed (uniform across the workgroup)
   int lo = 0, hi = sw.nblk - 1;
@@ -880,9 +928,9 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   hi = __builtin_amdgcn_readfirstlane(hi);
   const int cnt = hi - lo + 1;
 
-  floatx16 st[2];
+  floatx16 st[NTILE];
 #pragma unroll
-  for (int T = 0; T < 2; ++T)
+  for (int T = 0; T < NTILE; ++T)
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[T][r] = 0.f;
 
@@ -891,16 +939,24 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   // segment end.
   const uint32_t t_off = (uint32_t)(rq * row_bytes + cq * 16);
   const bool col_ok = !NARROW || cq * 8 < tw;  // chunks past the row width read as zeros
+  const int first = REV ? hi : lo;
+  const int step = REV ? -1 : 1;
+  auto block_of = [&](int i) __attribute__((always_inline)) { return first + min(i, cnt - 1) * step; };
+  auto len_of = [&](int blk) __attribute__((always_inline)) { return RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK; };
   // every address is a workgroup-uniform block pointer plus one per-thread 32-bit offset
-  auto issue_loads = [&](u32x4 (&nt)[4], int blk) __attribute__((always_inline)) {
+  auto issue_loads = [&](u32x4 (&nt)[4], int i) __attribute__((always_inline)) {
     typedef const __attribute__((address_space(1))) u32x4 *gmem_u32x4;
-    const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
-    const gmem_ptr tblk = uniform_ptr(Tg + (int64_t)blk * BLK * row_bytes);
     const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const bool ok = col_ok && (!RAGGED || rq + 16 * r < len);
-      nt[r] = ok ? *reinterpret_cast<gmem_u32x4>(tblk + 16 * r * row_bytes + t_off) : zero;
+    for (int half = 0; half < BPS; ++half) {
+      const int blk = block_of(BPS * i + half), len = len_of(blk);
+      const gmem_ptr tblk = uniform_ptr(Tg + (int64_t)blk * BLK * row_bytes);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (half_of(r) != half) continue;
+        const bool ok = col_ok && (!RAGGED || row_of(r) < len);
+        nt[r] = ok ? *reinterpret_cast<gmem_u32x4>(tblk + (row_of(r) - rq) * row_bytes + t_off) : zero;
+      }
     }
   };
   auto scaled = [&](const u32x4 &q, float w) __attribute__((always_inline)) {
@@ -911,54 +967,63 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
     o.w = E::pack(elem_f32<E>(q, 6) * w, elem_f32<E>(q, 7) * w);
     return o;
   };
-  char *const my_rows = smem + (zgrp ? STATE_TILE : 0) + rq * LDR + cq * 16;
-  auto fill_lds = [&](int buf, const u32x4 (&nt)[4], int blk) __attribute__((always_inline)) {
-    const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
-    char *dst = my_rows + buf * (2 * STATE_TILE);
-    const bool partial = RAGGED && !REV && len != BLK;
+  char *const my_rows = smem + (zgrp ? L::TILE : 0) + rq * L::LDR + ((cq * 16) ^ L::row_swap(rq));
+  auto fill_lds = [&](int buf, const u32x4 (&nt)[4], int i) __attribute__((always_inline)) {
+    char *dst = my_rows + buf * (2 * L::TILE);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
+      const int len = len_of(block_of(BPS * i + half_of(r)));
+      const bool partial = RAGGED && !REV && len != BLK;
       u32x4 v = nt[r];
-      if (!zgrp) v = scaled(v, partial ? decay(sl, (float)max(len - (rq + 16 * r), 0)) : kdec[r]);
-      *reinterpret_cast<u32x4 *>(dst + 16 * r * LDR) = v;
+      if (!zgrp) v = scaled(v, partial ? decay(sl, (float)max(len - row_of(r), 0)) : kdec[BPS == 1 ? r : r & 1]);
+      *reinterpret_cast<u32x4 *>(dst + ROWS * r * L::LDR) = v;
     }
   };
   // M_NARROW: columns past the width of Z stay zero, as do rows past Y's
-  const bool wave_active = !NARROW || (32 * wc < g.e && (rh == 0 || g.d > 64));
+  const bool wave_active = (W == 128 || zgrp) && (!NARROW || (32 * wc < g.e && row0s < g.d));
   // the lane's share of a fragment address: token 8 hh + (lane % 16) / 4, feature 16 ((lane / 16) % 2) + 4 (lane % 4)
-  const int lane_part = (8 * hh + ((lane & 15) >> 2)) * LDR + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
-  auto accumulate = [&](int buf, int blk) __attribute__((always_inline)) {
-    const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
-    const float bd = RAGGED && len != BLK ? decay(sl, (float)len) : blockdec;
-    const char *yt = smem + buf * (2 * STATE_TILE);
-    const char *zt = yt + STATE_TILE;
+  // (rows 4 apart, and the rows of different fragments, share their row_swap)
+  const int lane_row = 8 * hh + ((lane & 15) >> 2), lane_feat = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  auto lane_part = [&](int f0) __attribute__((always_inline)) {
+    return lane_row * L::LDR + ((2 * (f0 + lane_feat)) ^ L::row_swap(lane_row));
+  };
+  const int z_part = lane_part(32 * wc);
+  int y_part[NTILE];
+#pragma unroll
+  for (int T = 0; T < NTILE; ++T) y_part[T] = lane_part(row0s + 32 * T);
+  auto accumulate = [&](int buf, int i) __attribute__((always_inline)) {
     if (wave_active) {
-      u32x4 zf[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) zf[u] = token_fragment(zt, lane_part, 32 * wc, 16 * u);
+      for (int half = 0; half < BPS; ++half) {
+        if (half > 0 && BPS * i + half >= cnt) break;  // an odd block at the end of the walk
+        const int len = len_of(block_of(BPS * i + half));
+        const float bd = RAGGED && len != BLK ? decay(sl, (float)len) : blockdec;
+        const char *yt = smem + buf * (2 * L::TILE) + half * (BLK * L::LDR);
+        const char *zt = yt + L::TILE;
+        u32x4 zf[4];
 #pragma unroll
-      for (int T = 0; T < 2; ++T) {
+        for (int u = 0; u < 4; ++u) zf[u] = token_fragment<L::LDR>(zt, z_part, 16 * u);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) st[T][r] *= bd;
+        for (int T = 0; T < NTILE; ++T) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          st[T] = E::mfma(token_fragment(yt, lane_part, 64 * rh + 32 * T, 16 * u), zf[u], st[T]);
+          for (int r = 0; r < 16; ++r) st[T][r] *= bd;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            st[T] = E::mfma(token_fragment<L::LDR>(yt, y_part[T], 16 * u), zf[u], st[T]);
+        }
       }
     }
   };
 
-  // Block i of the walk (0 <= i < cnt) travels through register set i mod D.  Loads and LDS fills
+  // Step i of the walk (block i, or blocks 2 i and 2 i + 1) travels through register set i mod D.  Loads and LDS fills
   // past the end of the walk are not skipped but repeat its last block (served by the cache, never
   // used): with the same number of loads in flight on every path, the wait before a fill covers
   // exactly the oldest register set.
-  const int first = REV ? hi : lo;
-  const int step = REV ? -1 : 1;
-  auto block_of = [&](int i) __attribute__((always_inline)) { return first + min(i, cnt - 1) * step; };
   u32x4 set[D][4];
 #pragma unroll
-  for (int k = 0; k < D; ++k) issue_loads(set[k], block_of(k));
-  fill_lds(0, set[0], block_of(0));
-  issue_loads(set[0], block_of(D));
+  for (int k = 0; k < D; ++k) issue_loads(set[k], k);
+  fill_lds(0, set[0], 0);
+  issue_loads(set[0], D);
   __syncthreads();
   // The walk leaves the loop from the middle of the unrolled body.  Were the exit test left to the loop
   // head, the compiler would have to assume that any of the D positions can precede the first one, could
@@ -967,13 +1032,13 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
     bool last = false;
 #pragma unroll
     for (int k = 0; k < D; ++k) {  // D is even: LDS buffer (i + k) & 1 == k & 1
-      accumulate(k & 1, block_of(i + k));
+      accumulate(k & 1, i + k);
       __builtin_amdgcn_sched_barrier(0);
-      fill_lds((k + 1) & 1, set[(k + 1) % D], block_of(i + k + 1));
+      fill_lds((k + 1) & 1, set[(k + 1) % D], i + k + 1);
       __builtin_amdgcn_sched_barrier(0);
-      issue_loads(set[(k + 1) % D], block_of(i + k + 1 + D));
+      issue_loads(set[(k + 1) % D], i + k + 1 + D);
       __syncthreads();
-      if (i + k + 1 >= cnt) {
+      if (BPS * (i + k + 1) >= cnt) {
         last = true;
         break;
       }
@@ -981,91 +1046,92 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
     if (last) break;
   }
 
+  if (W == 128 || zgrp)
   {
-    float *sp = states + ((int64_t)sw.bh * g.n_seg + sw.seg) * (F * F);
+    float *sp = states + ((int64_t)sw.bh * g.n_seg + sw.seg) * (W * W);
 #pragma unroll
-    for (int T = 0; T < 2; ++T)
+    for (int T = 0; T < NTILE; ++T)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        sp[(64 * rh + 32 * T + 8 * (r >> 2) + 4 * hh + (r & 3)) * F + 32 * wc + c] = st[T][r];
+        sp[(row0s + 32 * T + 8 * (r >> 2) + 4 * hh + (r & 3)) * W + 32 * wc + c] = st[T][r];
   }
 }
 
-template <class E, bool REV, bool TRANS, int SRC, int MODE>
+template <class E, bool REV, bool TRANS, int SRC, int MODE, int W>
 int launch_apply(const void *x, const void *y, const void *z, const float *s, const float *states,
                     const float *carry_in, float *carry_out, void *out, const Geom &g, hipStream_t st) {
-  int rc = grant_lds<la_apply<E, REV, TRANS, SRC, MODE>>(WS_LDS);
+  int rc = grant_lds<la_apply<E, REV, TRANS, SRC, MODE, W>>(WsLds<W>::BYTES);
   if (rc) return rc;
   const unsigned grid = (unsigned)((int64_t)g.b * g.h * g.n_seg);
   ProfScope prof(KC_APPLY, st);
-  la_apply<E, REV, TRANS, SRC, MODE><<<grid, WS_THREADS, WS_LDS, st>>>(
+  la_apply<E, REV, TRANS, SRC, MODE, W><<<grid, WS_THREADS, WsLds<W>::BYTES, st>>>(
       (const elem16_t *)x, (const elem16_t *)y, (const elem16_t *)z, s, states, carry_in, carry_out, (elem16_t *)out, g);
   return (int)hipGetLastError();
 }
 
-template <class E, int SRC, int MODE>
+template <class E, int SRC, int MODE, int W>
 int launch_bwd3(const BwdArgs &a, const float *kv_states, const float *dkv_states, const Geom &g,
                    hipStream_t st) {
-  int rc = grant_lds<la_bwd3<E, SRC, MODE>>(WS_LDS);
+  int rc = grant_lds<la_bwd3<E, SRC, MODE, W>>(WsLds<W>::BYTES);
   if (rc) return rc;
   const int64_t n_items = (int64_t)g.b * g.h * g.n_seg;
   const unsigned grid = (unsigned)(((n_items + 7) / 8) * 24);
   ProfScope prof(KC_BWD3, st);
-  la_bwd3<E, SRC, MODE><<<grid, WS_THREADS, WS_LDS, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
+  la_bwd3<E, SRC, MODE, W><<<grid, WS_THREADS, WsLds<W>::BYTES, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
                                                          (const elem16_t *)a.v, (const elem16_t *)a.d_o, a.s,
                                                          kv_states, dkv_states, a.kv_in, a.dkv_in, a.dkv_out,
                                                          (elem16_t *)a.dq, (elem16_t *)a.dk, (elem16_t *)a.dv, g);
   return (int)hipGetLastError();
 }
 
-template <class E, bool REV, int MODE, int D>
+template <class E, bool REV, int MODE, int W, int D>
 int launch_state_depth(const void *y, const void *z, const float *s, float *states, const Geom &g, int skip_seg,
                        int sub, hipStream_t st) {
-  int rc = grant_lds<la_seg_state<E, REV, MODE, D>>(STATE_LDS);
+  int rc = grant_lds<la_seg_state<E, REV, MODE, W, D>>(StateLds<W>::BYTES);
   if (rc) return rc;
   const unsigned grid = (unsigned)((int64_t)g.b * g.h * g.n_seg);
   ProfScope prof(KC_STATE, st);
-  la_seg_state<E, REV, MODE, D><<<grid, STATE_THREADS, STATE_LDS, st>>>((const elem16_t *)y, (const elem16_t *)z, s,
+  la_seg_state<E, REV, MODE, W, D><<<grid, STATE_THREADS, StateLds<W>::BYTES, st>>>((const elem16_t *)y, (const elem16_t *)z, s,
                                                                         states, g, skip_seg, sub);
   return (int)hipGetLastError();
 }
 
 // skip_seg: the segment whose own state nothing reads (-1: none); its workgroups leave at once.
 // sub: segments of `g` per sweep segment (1 unless the plan cut the sweep segments finer for the pre-pass).
-template <class E, bool REV, int MODE>
+template <class E, bool REV, int MODE, int W>
 int launch_state_skipping(const void *y, const void *z, const float *s, float *states, const Geom &g, int skip_seg,
                           hipStream_t st, int sub = 1) {
   return g.seg_len >= STATE_LONG_WALK
-             ? launch_state_depth<E, REV, MODE, STATE_DEPTH_LONG>(y, z, s, states, g, skip_seg, sub, st)
-             : launch_state_depth<E, REV, MODE, STATE_DEPTH_SHORT>(y, z, s, states, g, skip_seg, sub, st);
+             ? launch_state_depth<E, REV, MODE, W, STATE_DEPTH_LONG>(y, z, s, states, g, skip_seg, sub, st)
+             : launch_state_depth<E, REV, MODE, W, STATE_DEPTH_SHORT>(y, z, s, states, g, skip_seg, sub, st);
 }
 
 // carry_wanted: whether the scan that follows has to produce the outgoing carry; if not, the
 // segment it visits last (whose own state feeds nothing else) is skipped.
-template <class E, bool REV, int MODE>
+template <class E, bool REV, int MODE, int W>
 int launch_state(const void *y, const void *z, const float *s, float *states, const Geom &g,
                  bool carry_wanted, int sub, hipStream_t st) {
-  return launch_state_skipping<E, REV, MODE>(y, z, s, states, g, carry_wanted ? -1 : (REV ? 0 : g.n_seg - 1), st, sub);
+  return launch_state_skipping<E, REV, MODE, W>(y, z, s, states, g, carry_wanted ? -1 : (REV ? 0 : g.n_seg - 1), st, sub);
 }
 
-template <class E, int MODE>
+template <class E, int MODE, int W>
 int launch_fused_fwd(const FwdArgs &a, const Geom &g, hipStream_t st) {
-  int rc = grant_lds<la_fused_fwd<E, MODE>>(WS_LDS);
+  int rc = grant_lds<la_fused_fwd<E, MODE, W>>(WsLds<W>::BYTES);
   if (rc) return rc;
   const unsigned grid = (unsigned)((((int64_t)g.b * g.h + 7) / 8) * 8 * g.n_seg);  // whole groups of 8 (b, h)
   ProfScope prof(KC_FUSED, st);
-  la_fused_fwd<E, MODE><<<grid, WS_THREADS, WS_LDS, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
+  la_fused_fwd<E, MODE, W><<<grid, WS_THREADS, WsLds<W>::BYTES, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
                                                          (const elem16_t *)a.v, a.s, a.kv_in, a.kv_out,
                                                          (elem16_t *)a.o, g);
   return (int)hipGetLastError();
 }
 
-// The backward's three workgroups per segment should fit the chip in one round (one workgroup per CU), and
+// The backward's three workgroups per segment should fit the chip in one round (one workgroup per CU, two at W = 64), and
 // nothing ties its segments to the forward's: no states are handed over on this path.
 Geom fused_bwd_geom(const Geom &g) {
   Geom gb = g;
   const int64_t bh = (int64_t)g.b * g.h;
-  int64_t fit = 256 / (3 * bh);  // segments per (b, h) in one round
+  int64_t fit = (g.width == 64 ? 512 : 256) / (3 * bh);  // segments per (b, h) in one round
   if (fit < 1) fit = 1;
   if (fit < g.n_seg) {
     int64_t len = (g.n + fit - 1) / fit;
@@ -1076,14 +1142,14 @@ Geom fused_bwd_geom(const Geom &g) {
   return gb;
 }
 
-template <class E, int MODE>
+template <class E, int MODE, int W>
 int launch_fused_bwd(const BwdArgs &a, const Geom &g_fwd, hipStream_t st) {
-  int rc = grant_lds<la_fused_bwd<E, MODE>>(WS_LDS);
+  int rc = grant_lds<la_fused_bwd<E, MODE, W>>(WsLds<W>::BYTES);
   if (rc) return rc;
   const Geom g = fused_bwd_geom(g_fwd);
   const unsigned grid = (unsigned)((((int64_t)g.b * g.h + 7) / 8) * 8 * 3 * g.n_seg);
   ProfScope prof(KC_FUSED, st);
-  la_fused_bwd<E, MODE><<<grid, WS_THREADS, WS_LDS, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
+  la_fused_bwd<E, MODE, W><<<grid, WS_THREADS, WsLds<W>::BYTES, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
                                                          (const elem16_t *)a.v, (const elem16_t *)a.d_o, a.s,
                                                          a.kv_in, a.dkv_in, a.dkv_out, (elem16_t *)a.dq,
                                                          (elem16_t *)a.dk, (elem16_t *)a.dv, g);
@@ -1099,92 +1165,106 @@ Geom pre_pass_geom(const Geom &g) {
   return gp;
 }
 
-template <class E, int MODE>
+template <class E, int MODE, int W>
 int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
-  if (g.fused) return launch_fused_fwd<E, MODE>(a, g, st);
+  if (g.fused) return launch_fused_fwd<E, MODE, W>(a, g, st);
   int rc;
   if constexpr (MODE != M_NARROW) if (g.combine) {  // (the plan combines full-width heads only)
     // few segments: the pre-pass leaves every segment's own state (the last one's is never read), each
     // sweep workgroup gathers the ones before it, and the last segment's sweep ends with KV_out
     if (g.n_seg > 1 &&
-        (rc = launch_state_skipping<E, false, MODE>(a.k, a.v, a.s, a.seg_states, g, g.n_seg - 1, st)))
+        (rc = launch_state_skipping<E, false, MODE, W>(a.k, a.v, a.s, a.seg_states, g, g.n_seg - 1, st)))
       return rc;
-    return launch_apply<E, false, false, SRC_COMBINE, MODE>(a.q, a.k, a.v, a.s, g.n_seg > 1 ? a.seg_states : nullptr,
+    return launch_apply<E, false, false, SRC_COMBINE, MODE, W>(a.q, a.k, a.v, a.s, g.n_seg > 1 ? a.seg_states : nullptr,
                                                                a.kv_in, a.kv_out, a.o, g, st);
   }
   const bool need_states = g.n_seg > 1 || a.kv_in || a.kv_out;
   const Geom gp = pre_pass_geom(g);
   const int sub = g.seg_len / g.pre_len;  // pre-pass segments per sweep segment
   if (need_states) {
-    if ((rc = launch_state<E, false, MODE>(a.k, a.v, a.s, a.seg_states, gp, a.kv_out != nullptr, sub, st))) return rc;
+    if ((rc = launch_state<E, false, MODE, W>(a.k, a.v, a.s, a.seg_states, gp, a.kv_out != nullptr, sub, st))) return rc;
     if ((rc = launch_segment_scan(a.seg_states, a.kv_in, a.kv_out, a.s, gp, 0, st))) return rc;
   }
-  return launch_apply<E, false, false, SRC_SCANNED, MODE>(a.q, a.k, a.v, a.s, need_states ? a.seg_states : nullptr,
+  return launch_apply<E, false, false, SRC_SCANNED, MODE, W>(a.q, a.k, a.v, a.s, need_states ? a.seg_states : nullptr,
                                                              a.kv_in, nullptr, a.o, g, st);
 }
 
-template <class E, int MODE>
+template <class E, int MODE, int W>
 int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
-  if (g.fused) return launch_fused_bwd<E, MODE>(a, g, st);
+  if (g.fused) return launch_fused_bwd<E, MODE, W>(a, g, st);
   int rc;
   if constexpr (MODE != M_NARROW) if (g.combine) {
     const float *kv_states = a.kv_seg_states;
     if (!kv_states && g.n_seg > 1) {
-      if ((rc = launch_state_skipping<E, false, MODE>(a.k, a.v, a.s, a.ws_kv, g, g.n_seg - 1, st))) return rc;
+      if ((rc = launch_state_skipping<E, false, MODE, W>(a.k, a.v, a.s, a.ws_kv, g, g.n_seg - 1, st))) return rc;
       kv_states = a.ws_kv;
     }
-    if (g.n_seg > 1 && (rc = launch_state_skipping<E, true, MODE>(a.q, a.d_o, a.s, a.ws_dkv, g, 0, st))) return rc;
-    return launch_bwd3<E, SRC_COMBINE, MODE>(a, g.n_seg > 1 ? kv_states : nullptr,
+    if (g.n_seg > 1 && (rc = launch_state_skipping<E, true, MODE, W>(a.q, a.d_o, a.s, a.ws_dkv, g, 0, st))) return rc;
+    return launch_bwd3<E, SRC_COMBINE, MODE, W>(a, g.n_seg > 1 ? kv_states : nullptr,
                                                 g.n_seg > 1 ? a.ws_dkv : nullptr, g, st);
   }
   const Geom gp = pre_pass_geom(g);
   const int sub = g.seg_len / g.pre_len;  // pre-pass segments per sweep segment
   const float *kv_states = a.kv_seg_states;
   if (!kv_states && (g.n_seg > 1 || a.kv_in)) {
-    if ((rc = launch_state<E, false, MODE>(a.k, a.v, a.s, a.ws_kv, gp, false, sub, st))) return rc;
+    if ((rc = launch_state<E, false, MODE, W>(a.k, a.v, a.s, a.ws_kv, gp, false, sub, st))) return rc;
     if ((rc = launch_segment_scan(a.ws_kv, a.kv_in, nullptr, a.s, gp, 0, st))) return rc;
     kv_states = a.ws_kv;
   }
   const float *dkv_states = nullptr;
   if (g.n_seg > 1 || a.dkv_in || a.dkv_out) {
-    if ((rc = launch_state<E, true, MODE>(a.q, a.d_o, a.s, a.ws_dkv, gp, a.dkv_out != nullptr, sub, st))) return rc;
+    if ((rc = launch_state<E, true, MODE, W>(a.q, a.d_o, a.s, a.ws_dkv, gp, a.dkv_out != nullptr, sub, st))) return rc;
     if ((rc = launch_segment_scan(a.ws_dkv, a.dkv_in, a.dkv_out, a.s, gp, 1, st))) return rc;
     dkv_states = a.ws_dkv;
   }
-  return launch_bwd3<E, SRC_SCANNED, MODE>(a, kv_states, dkv_states, g, st);
+  return launch_bwd3<E, SRC_SCANNED, MODE, W>(a, kv_states, dkv_states, g, st);
 }
 
 
+// rows of g.sd = g.se features (64 or 128) run without the bookkeeping of narrower ones
 int mode_of(const Geom &g) {
-  if (g.d != F || g.e != F) return M_NARROW;
+  if (g.d != g.sd || g.e != g.se) return M_NARROW;
   return g.n % BLK != 0 ? M_RAGGED : M_ALIGNED;
 }
 
-template <class E>
+template <class E, int W>
 int fwd_m(const FwdArgs &a, const Geom &g, hipStream_t st) {
   switch (mode_of(g)) {
-    case M_ALIGNED: return fwd_e<E, M_ALIGNED>(a, g, st);
-    case M_RAGGED: return fwd_e<E, M_RAGGED>(a, g, st);
-    default: return fwd_e<E, M_NARROW>(a, g, st);
+    case M_ALIGNED: return fwd_e<E, M_ALIGNED, W>(a, g, st);
+    case M_RAGGED: return fwd_e<E, M_RAGGED, W>(a, g, st);
+    default: return fwd_e<E, M_NARROW, W>(a, g, st);
+  }
+}
+template <class E, int W>
+int bwd_m(const BwdArgs &a, const Geom &g, hipStream_t st) {
+  switch (mode_of(g)) {
+    case M_ALIGNED: return bwd_e<E, M_ALIGNED, W>(a, g, st);
+    case M_RAGGED: return bwd_e<E, M_RAGGED, W>(a, g, st);
+    default: return bwd_e<E, M_NARROW, W>(a, g, st);
   }
 }
 template <class E>
-int bwd_m(const BwdArgs &a, const Geom &g, hipStream_t st) {
-  switch (mode_of(g)) {
-    case M_ALIGNED: return bwd_e<E, M_ALIGNED>(a, g, st);
-    case M_RAGGED: return bwd_e<E, M_RAGGED>(a, g, st);
-    default: return bwd_e<E, M_NARROW>(a, g, st);
-  }
+int fwd_w(const FwdArgs &a, const Geom &g, hipStream_t st) {
+  return g.width == 64 ? fwd_m<E, 64>(a, g, st) : fwd_m<E, 128>(a, g, st);
+}
+template <class E>
+int bwd_w(const BwdArgs &a, const Geom &g, hipStream_t st) {
+  return g.width == 64 ? bwd_m<E, 64>(a, g, st) : bwd_m<E, 128>(a, g, st);
 }
 
 }  // namespace
 
+// This file is compiled once per element type: as it stands for bf16, and through lasp_mfma_f16.hip for fp16.
+#ifdef LASP_MFMA_F16
+int mfma_f16_fwd(const FwdArgs &a, const Geom &g, hipStream_t st) { return fwd_w<ElemF16>(a, g, st); }
+int mfma_f16_bwd(const BwdArgs &a, const Geom &g, hipStream_t st) { return bwd_w<ElemF16>(a, g, st); }
+#else
 int mfma_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
-  return dtype == LASP_DTYPE_F16 ? fwd_m<ElemF16>(a, g, st) : fwd_m<ElemBF16>(a, g, st);
+  return dtype == LASP_DTYPE_F16 ? mfma_f16_fwd(a, g, st) : fwd_w<ElemBF16>(a, g, st);
 }
-
 int mfma_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
-  return dtype == LASP_DTYPE_F16 ? bwd_m<ElemF16>(a, g, st) : bwd_m<ElemBF16>(a, g, st);
+  return dtype == LASP_DTYPE_F16 ? mfma_f16_bwd(a, g, st) : bwd_w<ElemBF16>(a, g, st);
 }
+#endif
 
 }  // namespace lasp
