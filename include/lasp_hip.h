@@ -13,6 +13,9 @@
  *     kv_in, kv_out, dkv_in, dkv_out : (b, h, d, e) float, may be NULL
  *     seg states   : float workspace of lasp_plan's state_bytes (one state per (b, h) and segment, or per
  *                    piece of a long segment; each d x e, or zero-extended to 128 x 128): opaque to the caller
+ * Widths: d, e <= 128.  With 16-bit elements and d, e multiples of 8, d may be up to 1024: such wide heads are swept in
+ * slices of 128 features of q and k (one state per slice in the workspace), and the parts of o and dv that slices
+ * after the first contribute are added to what is there, rounded to the element type once per slice.
  *
  * Alignment: q, k, v, o, do, dq, dk, dv start on a 16-byte boundary (the kernels
  * fetch rows with 8- and 16-byte loads and store them with 16-byte stores; rows of d or e
@@ -74,8 +77,8 @@ extern "C" {
 /* Which kernel family a shape/dtype is served by (lasp_kernel_path). */
 #define LASP_PATH_GENERIC 0 /* fp32-FMA kernels: any dtype, any n, d,e <= 128 */
 #define LASP_PATH_MFMA 1    /* MFMA kernels, any n (a ragged tail is masked): bf16 / fp16 with d and e
-                               multiples of 8 (rows narrower than 128 are read zero-extended), fp32 with
-                               d = e = 128 */
+                               multiples of 8 (rows narrower than the 64 or 128 features that a kernel works on are
+                               read zero-extended, d > 128 in slices), fp32 with d = e = 128 */
 #define LASP_PATH_MFMA_FUSED 2 /* short chunks of the 16-bit MFMA shapes called with seg_len = 0 (n <= 2048
                                and few enough segments that rebuilding a segment's incoming state from
                                the blocks before it -- at most 16 of them -- is cheaper than a pre-pass

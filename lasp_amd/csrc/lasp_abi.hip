@@ -53,8 +53,9 @@ ProfScope::~ProfScope() {
 
 namespace {
 
-constexpr int kMaxFeature = 128;     // d and e of one launch (the Python wrappers slice d, as
-                                     // lasp/lightning_attention.py:513-519 does)
+constexpr int kMaxFeature = 128;     // d and e of one sweep
+constexpr int kMaxSliced = 1024;     // d of a wide head, swept in slices of 128 features (as the wrapper of
+                                     // lasp/lightning_attention.py:513-519 does; 16-bit kernels only)
 constexpr int kSegQuantum = 64;      // segment lengths are multiples of this
 constexpr int64_t kTargetGroups = 512;  // workgroups wanted per launch (2 per CU on 256 CUs)
 constexpr int kMinSeg = 256;
@@ -66,14 +67,26 @@ constexpr int kPreMaxSeg = 2304;        // longest segment the pre-pass walks in
                                         // 2048 tokens and a little more, so that lengths just above 4096, 8192, ...
                                         // are still cut in 2, 4, ... and not in twice as many pieces
 
+// The 16-bit MFMA kernels work on 128 features, or 64 where neither d nor e is larger, and read narrower rows
+// zero-extended (wider ones in slices of 128); their 8-byte loads and 16-byte stores need every row to start on such
+// a boundary.
+bool mfma_eligible(int d, int e, int dtype) {
+  return (dtype == LASP_DTYPE_BF16 || dtype == LASP_DTYPE_F16) && d % 8 == 0 && e % 8 == 0;
+}
+int sweep_width(int d, int e) { return d <= 64 && e <= 64 ? 64 : kMaxFeature; }
+bool mfma_f32_eligible(int d, int e, int dtype) {
+  return dtype == LASP_DTYPE_F32 && d == kMaxFeature && e == kMaxFeature;
+}
+
 int check_shape(int b, int h, int64_t n, int d, int e, int dtype) {
   if (dtype != LASP_DTYPE_F32 && dtype != LASP_DTYPE_BF16 && dtype != LASP_DTYPE_F16) {
     set_error("unknown dtype code %d", dtype);
     return LASP_E_DTYPE;
   }
-  if (b <= 0 || h <= 0 || n <= 0 || d <= 0 || e <= 0 || d > kMaxFeature || e > kMaxFeature) {
-    set_error("unsupported shape b=%d h=%d n=%lld d=%d e=%d (need b,h,n >= 1 and 1 <= d,e <= %d)", b,
-              h, (long long)n, d, e, kMaxFeature);
+  const int max_d = mfma_eligible(d, e, dtype) ? kMaxSliced : kMaxFeature;
+  if (b <= 0 || h <= 0 || n <= 0 || d <= 0 || e <= 0 || d > max_d || e > kMaxFeature) {
+    set_error("unsupported shape b=%d h=%d n=%lld d=%d e=%d (need b,h,n >= 1 and 1 <= d,e <= %d, or d <= %d in 16 bits "
+              "with d and e multiples of 8)", b, h, (long long)n, d, e, kMaxFeature, kMaxSliced);
     return LASP_E_SHAPE;
   }
   if ((int64_t)b * h > (int64_t)1 << 24) {
@@ -135,16 +148,6 @@ int default_seg_len(int b, int h, int64_t n, bool narrow64) {
   if (balanced > kMinSeg && balanced > len && bh * ((n + balanced - 1) / balanced) <= kMinGroups) len = balanced;
   if (len > kMaxSeg) len = kMaxSeg;
   return (int)len;
-}
-
-// The 16-bit MFMA kernels work on 128 features, or 64 where neither d nor e is larger, and read narrower rows zero-extended; their
-// 8-byte loads and 16-byte stores need every row to start on such a boundary.
-bool mfma_eligible(int d, int e, int dtype) {
-  return (dtype == LASP_DTYPE_BF16 || dtype == LASP_DTYPE_F16) && d % 8 == 0 && e % 8 == 0;
-}
-int sweep_width(int d, int e) { return d <= 64 && e <= 64 ? 64 : kMaxFeature; }
-bool mfma_f32_eligible(int d, int e, int dtype) {
-  return dtype == LASP_DTYPE_F32 && d == kMaxFeature && e == kMaxFeature;
 }
 
 // Short chunks given to the library with the default plan run as ONE launch per direction: every
@@ -308,7 +311,9 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   g->b = b;
   g->h = h;
   g->n = n;
-  g->d = d;
+  g->d = d < kMaxFeature ? d : kMaxFeature;
+  g->dt = d;
+  g->add = 0;
   g->e = e;
   g->seg_len = seg_len;
   g->n_seg = (int)n_seg_final;
@@ -443,7 +448,8 @@ int static_scratch(float **out) {
 // (a state of the 64-wide kernels takes a quarter of its slot: every caller sizes the array for 128 x 128)
 size_t state_bytes_of(const Geom &g) {
   const size_t one = g.width == 64 ? (size_t)kMaxFeature * kMaxFeature : (size_t)g.sd * g.se;
-  return sizeof(float) * (size_t)g.b * g.h * g.pre_n * one;
+  const size_t slices = (g.dt + kMaxWidth - 1) / kMaxWidth;
+  return sizeof(float) * (size_t)g.b * g.h * g.pre_n * one * slices;
 }
 
 }  // namespace
@@ -550,7 +556,7 @@ static int chunk_fwd_impl(const char *me, const void *q, const void *k, const vo
                           const float *kv_in, float *kv_out, void *o, float *seg_states, const Geom &g,
                           int dtype, void *stream) {
   int rc;
-  if ((rc = check_alias(me, "kv", kv_in, kv_out, sizeof(float) * (size_t)g.b * g.h * g.d * g.e, g, false))) return rc;
+  if ((rc = check_alias(me, "kv", kv_in, kv_out, sizeof(float) * (size_t)g.b * g.h * g.dt * g.e, g, false))) return rc;
   if ((rc = check_aligned(me, "q", q, 16)) || (rc = check_aligned(me, "k", k, 16)) ||
       (rc = check_aligned(me, "v", v, 16)) || (rc = check_aligned(me, "o", o, 16)) ||
       (rc = check_aligned(me, "s", s, 4)) || (rc = check_aligned(me, "kv_in", kv_in, 4)) ||
@@ -560,7 +566,7 @@ static int chunk_fwd_impl(const char *me, const void *q, const void *k, const vo
   (void)hipGetLastError();  // an earlier, unrelated error of this thread is not this call's
   FwdArgs a{q, k, v, s, kv_in, kv_out, o, seg_states};
   hipStream_t st = (hipStream_t)stream;
-  rc = mfma_eligible(g.d, g.e, dtype)       ? mfma_fwd(a, g, dtype, st)
+  rc = mfma_eligible(g.dt, g.e, dtype)      ? mfma_fwd(a, g, dtype, st)
        : mfma_f32_eligible(g.d, g.e, dtype) ? mfma_f32_fwd(a, g, st)
                                             : generic_fwd(a, g, dtype, st);
   if (rc > 0) set_error("%s: HIP error %d: %s", me, rc, hipGetErrorString((hipError_t)rc));

@@ -58,6 +58,8 @@ struct Geom {
   int sd, se;   // rows and columns of one segment state as stored in the workspace: d x e for the
                 // generic kernels, 128 x 128 or 64 x 64 (zero beyond d, e) for the MFMA kernels
   int width;    // 16-bit MFMA kernels: the width they are laid out for, 128 or 64; else 0
+  int dt;       // features in a row of q and k: d, or more where the head is wide and d is the slice at hand
+  int add;      // the sweep adds its O (dV) to what a slice before it left there
   int fused;    // the chunk is served by the single-launch kernels, which use no workspace
   int combine;  // few segments: no scan launch, the sweep workgroups gather the segments' own states
   int bypass;   // the scan leaves out heads whose state dies within one segment (see state_dies_in_segment)
@@ -72,6 +74,7 @@ struct Geom {
 // bf16) before they multiply with it.
 constexpr float kSkipLog2 = 24.f;
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr int kMaxWidth = 128;  // features that one sweep works on
 
 // With g.bypass set, a head whose decay over the shortest segment of the pre-pass (the last one) is below
 // 2^-kSkipLog2 takes no part in the scan: whatever enters a segment has faded to nothing at its far

@@ -348,11 +348,14 @@ segment_scan_kernel(float *__restrict__ states, const float *carry_in, float *ca
   const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * W;
   const int64_t total = (int64_t)g.b * g.h * sde;
   if (idx >= total) return;
+  const int slice = blockIdx.y;  // of a wide head: 128 of its g.dt rows, states in an array of their own
+  const int d = min(g.d, g.dt - slice * kMaxWidth);
+  states += (int64_t)slice * total * g.n_seg;
   const int bh = (int)(idx / sde);
   const int64_t el = idx - (int64_t)bh * sde;
   const int row = (int)(el / g.se), col = (int)(el - (int64_t)row * g.se);
-  const bool in_carry = row < g.d && col < g.e;  // the padding of a stored state stays zero
-  const int64_t cidx = ((int64_t)bh * g.d + row) * g.e + col;
+  const bool in_carry = row < d && col < g.e;  // the padding of a stored state stays zero
+  const int64_t cidx = ((int64_t)bh * g.dt + slice * kMaxWidth + row) * g.e + col;
   const float s = S[bh % g.h];
   ScanVec<W> run;
 #pragma unroll
@@ -495,7 +498,7 @@ int launch_segment_scan(float *states, const float *carry_in, float *carry_out, 
   const int64_t total = (int64_t)g.b * g.h * g.sd * g.se;
   const bool wide = g.se % 4 == 0 && g.e % 4 == 0 && (uintptr_t)states % 16 == 0;
   const int64_t threads = wide ? total / 4 : total;
-  const unsigned grid = (unsigned)((threads + 255) / 256);
+  const dim3 grid((unsigned)((threads + 255) / 256), (unsigned)((g.dt + kMaxWidth - 1) / kMaxWidth));
   ProfScope prof(KC_SCAN, st);
   if (wide)
     segment_scan_kernel<4><<<grid, 256, 0, st>>>(states, carry_in, carry_out, s, g, reverse);

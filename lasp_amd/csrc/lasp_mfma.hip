@@ -240,8 +240,8 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
 // its true length).  M_NARROW: in addition X and Y rows hold `fa` features, Z and Out rows `fb`
 // (multiples of 8, at most W), read zero-extended to W and written back at their own width; the upper
 // half of the feature steps and state tiles, and waves whose columns lie in the zero extension, are skipped
-// when they would only see zeros.  M_ALIGNED carries none of that bookkeeping; fa and fb are read in
-// M_NARROW only.
+// when they would only see zeros.  The slices of a wide head (d > 128) run in this mode too, their rows being g.dt
+// features apart.  M_ALIGNED carries none of that bookkeeping; fa and fb are read in M_NARROW only.
 //
 // SRC says where the state entering the segment comes from.
 // SRC_SCANNED: `states` holds it, left there by the decayed scan over the segments' own states.
@@ -316,6 +316,9 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   const SegWork sw = seg_work(g, item);
   const float sl = S[sw.bh % g.h] * LOG2E;
   const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
+  // elements from row to row of X and Y, and of Z and Out: q, k and their gradients have rows of g.dt features, of which
+  // a slice of a wide head reads and writes fa (fb)
+  const int xp = NARROW ? (TRANS ? g.e : g.dt) : W, zp = NARROW ? (TRANS ? g.dt : g.e) : W;
   const int nblk = sw.nblk;
   const int step = REV ? -1 : 1;
   const int blk0 = REV ? nblk - 1 : 0;
@@ -358,13 +361,11 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     const bool zfeed = SPLIT && w8 >= 2;
     const LoaderRole xr = x_role<W>(ftid), yr = yz_role<W>(SPLIT ? ftid & 127 : ftid);
     const int chunk = ftid & (W / 8 - 1), rowq = ftid / (W / 8);
-    const int xw = NARROW ? fa : W, zw = NARROW ? fb : W;  // row widths in elements
-    const u32x2 *Xg = reinterpret_cast<const u32x2 *>(X + row0 * xw);
-    const u32x2 *Yg = reinterpret_cast<const u32x2 *>(Y + row0 * xw);
-    const u32x2 *Zg = reinterpret_cast<const u32x2 *>(Z + row0 * zw);
-    u32x4 *Og = reinterpret_cast<u32x4 *>(Out + row0 * zw);
-    const int xu = xw / 4, zu = zw / 4;  // 8-byte units per row
-    const int ou = zw / 8;               // 16-byte units per output row
+    const u32x2 *Xg = reinterpret_cast<const u32x2 *>(X + row0 * xp);
+    const u32x2 *Yg = reinterpret_cast<const u32x2 *>(Y + row0 * xp);
+    const u32x2 *Zg = reinterpret_cast<const u32x2 *>(Z + row0 * zp);
+    u32x4 *Og = reinterpret_cast<u32x4 *>(Out + row0 * zp);
+    const int xu = xp / 4, zu = zp / 4;  // 8-byte units from row to row
     float kdec[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -377,7 +378,8 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     const uint32_t x_off = lane_offset(xr, xr.rowq, xu), y_off = lane_offset(yr, 4 * yr.rowq, yu),
                    z_off = lane_offset(yr, 4 * yr.rowq, zu);
     const PieceMask all = {true, true};
-    const PieceMask x_ok = piece_mask(xr, xu), y_ok = piece_mask(yr, yu), z_ok = piece_mask(yr, zu);
+    const PieceMask x_ok = piece_mask(xr, fa / 4), y_ok = piece_mask(yr, (zfeed ? fb : fa) / 4),
+                    z_ok = piece_mask(yr, fb / 4);
 
     // the block in flight, two 8-byte pieces per row (see LoaderRole); SPLIT: ny holds Y or Z
     u32x4 nx[XI], ny[4], nz[4];
@@ -438,9 +440,9 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
 #pragma unroll
       for (int r4 = 0; r4 < XI; ++r4) {
         const int row = rowq + XROWS * r4;
-        if (!RAGGED || (row < len && (!NARROW || chunk < ou)))
+        if (!RAGGED || (row < len && (!NARROW || chunk < fb / 8)))
           __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(set + L::XN + row * L::LDN + chunk * 16),
-                                      &Og[(brow + row) * (NARROW ? ou : W / 8) + chunk]);
+                                      &Og[(brow + row) * (NARROW ? zp / 8 : W / 8) + chunk]);
       }
     };
     // this wave's quadrant of the transposed score tile: sc[4g+r] = y_b . x_a, b = 32qJ+8g+4hh+r, a = 32qI+c
@@ -513,6 +515,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   // M_NARROW: a wave whose 32 columns all lie past the width of Z has nothing to compute (it still takes part in
   // every barrier); the upper half of the features is skipped as a whole when the rows are no wider
   const bool wave_active = !NARROW || W == 64 || 32 * wcol < fb;  // (at W = 64 the skipping costs registers that two workgroups per CU do not have)
+  constexpr int PARTS = NARROW ? 2 : 1;  // M_NARROW takes the lower and the upper features one after the other
   const bool upper_half = !NARROW || W == 64 || fa > W / 2;
   // st <- f * st + M, M being the W x W fp32 tile whose element (row, col) is src[row * ld + col], or for a
   // transposed role src[col * ld + row]; `bounded`: src holds only fa x fb (transposed: fb x fa) elements
@@ -539,7 +542,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   // a state of the workspace (W x W, zero beyond fa x fb) / the chunk's incoming state (fa x fb, unpadded)
   auto add_state = [&](const float *src, float f) __attribute__((always_inline)) { add_state_ld(src, W, f, false); };
   auto add_carry = [&]() __attribute__((always_inline)) {
-    add_state_ld(carry_in + (int64_t)sw.bh * fa * fb, NARROW ? (TRANS ? fa : fb) : W, 0.f, NARROW);
+    add_state_ld(carry_in + (int64_t)sw.bh * g.dt * g.e, NARROW ? (TRANS ? fa : fb) : W, 0.f, NARROW);
   };
   if (SRC == SRC_WALK) {
     if (take_carry) add_carry();
@@ -597,18 +600,41 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int r = 0; r < 16; ++r) st[T][r] *= bd;
-    u32x4 yf[4][NT];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int part = 0; part < PARTS; ++part) {
+      if (part > 0 && !upper_half) break;  // state rows past the width of Y stay zero
+      constexpr int TP = NT / PARTS;
+      u32x4 yf[4][TP];
 #pragma unroll
-      for (int T = 0; T < NT; ++T)
-        if (T < NT / 2 || upper_half) yf[u][T] = lds16(set + L::YT + tr_off(32 * T + c, 2 * u + hh));
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+        for (int T = 0; T < TP; ++T) yf[u][T] = lds16(set + L::YT + tr_off(32 * (part * TP + T) + c, 2 * u + hh));
 #pragma unroll
-      for (int T = 0; T < NT; ++T)
-        if (T < NT / 2 || upper_half) st[T] = E::mfma(yf[u][T], zf[u], st[T]);  // state rows past the width of Y stay zero
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int T = 0; T < TP; ++T) st[part * TP + T] = E::mfma(yf[u][T], zf[u], st[part * TP + T]);
+    }
   };
+  // Slices of a wide head after the first add to what the slices before them left in Out (its rows are whole
+  // features of v, so only the non-transposed roles).  A block's old output is fetched while the block before it is
+  // computed; the lane holds the columns that its accumulators hold.
+  constexpr bool MAY_ADD = NARROW && !TRANS && W == 128;
+  const bool adds = MAY_ADD && g.add != 0;
+  u32x2 old[NI][4];
+  auto fetch_old = [&](int blk) __attribute__((always_inline)) {
+    const int len = len_of(blk);
+    const elem16_t *rows = Out + (row0 + (int64_t)blk * BLK) * zp + 32 * wcol + 4 * hh;
+    const u32x2 zero = {0u, 0u};
+#pragma unroll
+    for (int I = 0; I < NI; ++I)
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) {
+        const int row = 32 * (ih + I) + c;
+        const bool ok = row < len && 32 * wcol + 8 * gq + 4 * hh < fb;
+        old[I][gq] = ok ? *reinterpret_cast<const u32x2 *>(rows + (int64_t)row * zp + 8 * gq) : zero;
+      }
+  };
+  if (adds) fetch_old(blk0);
   __syncthreads();  // barrier 0
   for (int k = 0; k < runup; ++k) {  // walk
     const char *set = smem + (k & 1) * L::SET;
@@ -644,32 +670,42 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[I][r] = 0.f;
     if (wave_active) {
-      // all X fragments are requested before the first product (these waves have the registers for it)
+      // all X fragments (of a part) are requested before the first product (these waves have the registers for it)
       const char *x0 = cur + L::XN + (32 * ih + c) * L::LDN + hh * 16;
-      u32x4 xf[W / 16][NI];
 #pragma unroll
-      for (int ks = 0; ks < W / 16; ++ks) {
-        if (ks >= W / 32 && !upper_half) continue;
+      for (int part = 0; part < PARTS; ++part) {
+        if (part > 0 && !upper_half) break;
+        constexpr int KS = W / 16 / PARTS;
+        u32x4 xf[KS][NI];
 #pragma unroll
-        for (int I = 0; I < NI; ++I) xf[ks][I] = lds16(x0 + 32 * I * L::LDN + ks * 32);
-      }
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int ks = 0; ks < W / 16; ++ks) {
-        if (ks >= W / 32 && !upper_half) continue;
-        const int T = ks >> 1, u = ks & 1;
-        u32x4 a;
-        a.x = E::pack(st[T][8 * u + 0], st[T][8 * u + 1]);
-        a.y = E::pack(st[T][8 * u + 2], st[T][8 * u + 3]);
-        a.z = E::pack(st[T][8 * u + 4], st[T][8 * u + 5]);
-        a.w = E::pack(st[T][8 * u + 6], st[T][8 * u + 7]);
+          for (int I = 0; I < NI; ++I) xf[ks][I] = lds16(x0 + 32 * I * L::LDN + (part * KS + ks) * 32);
 #pragma unroll
-        for (int I = 0; I < NI; ++I) acc[I] = E::mfma(a, xf[ks][I], acc[I]);
+        for (int ks = 0; ks < KS; ++ks) {
+          const int T = (part * KS + ks) >> 1, u = ks & 1;
+          u32x4 a;
+          a.x = E::pack(st[T][8 * u + 0], st[T][8 * u + 1]);
+          a.y = E::pack(st[T][8 * u + 2], st[T][8 * u + 3]);
+          a.z = E::pack(st[T][8 * u + 4], st[T][8 * u + 5]);
+          a.w = E::pack(st[T][8 * u + 6], st[T][8 * u + 7]);
+#pragma unroll
+          for (int I = 0; I < NI; ++I) acc[I] = E::mfma(a, xf[ks][I], acc[I]);
+        }
       }
     }
 #pragma unroll
     for (int I = 0; I < NI; ++I)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[I][r] *= qd[I];
+    if (adds) {
+#pragma unroll
+      for (int I = 0; I < NI; ++I)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          acc[I][r] += E::widen((r & 2) ? old[I][r >> 2].y : old[I][r >> 2].x, r & 1);
+      if (it + 1 < nblk) fetch_old(blk0 + (it + 1) * step);
+    }
     __syncthreads();  // barrier 2 it + 1: score tile complete
     if (wave_active) {
       u32x4 zf[4];
@@ -701,7 +737,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   }
   // the segment visited last leaves the chunk's outgoing state
   if (SRC != SRC_SCANNED && !TRANS && carry_out != nullptr && sw.seg == (REV ? 0 : g.n_seg - 1) && ih == 0) {
-    float *cp = carry_out + (int64_t)sw.bh * fa * fb;
+    float *cp = carry_out + (int64_t)sw.bh * g.dt * g.e;
     const int col = 32 * wcol + c;
 #pragma unroll
     for (int T = 0; T < NT; ++T)
@@ -895,10 +931,14 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   }
   const float sl = slope * LOG2E;
   const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
-  const int yw = NARROW ? g.d : W, zw = NARROW ? g.e : W;  // row widths in elements
-  const int tw = zgrp ? zw : yw;                           // of the tile this thread fetches
-  const char *Tg = reinterpret_cast<const char *>(zgrp ? Z + row0 * zw : Y + row0 * yw);
-  const int row_bytes = tw * 2;
+  // the feature slice of a wide head (blockIdx.y; rows of Y are g.dt features apart) and its width
+  const int slice = NARROW && W == 128 ? (int)blockIdx.y : 0;
+  const int gd = NARROW ? min(W, g.dt - slice * W) : W;
+  states += (int64_t)slice * n_items * (W * W);
+  const int yp = NARROW ? g.dt : W, zp = NARROW ? g.e : W;  // elements from row to row
+  const int tw = NARROW ? (zgrp ? g.e : gd) : W;            // width of the tile this thread fetches
+  const char *Tg = reinterpret_cast<const char *>(zgrp ? Z + row0 * zp : Y + row0 * yp + slice * W);
+  const int row_bytes = (zgrp ? zp : yp) * 2;
 
   // row r of the thread's four: token row_of(r) of block half_of(r) of the step
   auto half_of = [](int r) { return BPS == 1 ? 0 : r >> 1; };
@@ -980,7 +1020,7 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
     }
   };
   // M_NARROW: columns past the width of Z stay zero, as do rows past Y's
-  const bool wave_active = (W == 128 || zgrp) && (!NARROW || (32 * wc < g.e && row0s < g.d));
+  const bool wave_active = (W == 128 || zgrp) && (!NARROW || (32 * wc < g.e && row0s < gd));
   // the lane's share of a fragment address: token 8 hh + (lane % 16) / 4, feature 16 ((lane / 16) % 2) + 4 (lane % 4)
   // (rows 4 apart, and the rows of different fragments, share their row_swap)
   const int lane_row = 8 * hh + ((lane & 15) >> 2), lane_feat = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
@@ -1084,6 +1124,8 @@ int launch_bwd3(const BwdArgs &a, const float *kv_states, const float *dkv_state
   return (int)hipGetLastError();
 }
 
+unsigned slices_of(const Geom &g) { return (unsigned)(g.dt + kMaxWidth - 1) / kMaxWidth; }
+
 template <class E, bool REV, int MODE, int W, int D>
 int launch_state_depth(const void *y, const void *z, const float *s, float *states, const Geom &g, int skip_seg,
                        int sub, hipStream_t st) {
@@ -1091,7 +1133,7 @@ int launch_state_depth(const void *y, const void *z, const float *s, float *stat
   if (rc) return rc;
   const unsigned grid = (unsigned)((int64_t)g.b * g.h * g.n_seg);
   ProfScope prof(KC_STATE, st);
-  la_seg_state<E, REV, MODE, W, D><<<grid, STATE_THREADS, StateLds<W>::BYTES, st>>>((const elem16_t *)y, (const elem16_t *)z, s,
+  la_seg_state<E, REV, MODE, W, D><<<dim3(grid, slices_of(g)), STATE_THREADS, StateLds<W>::BYTES, st>>>((const elem16_t *)y, (const elem16_t *)z, s,
                                                                         states, g, skip_seg, sub);
   return (int)hipGetLastError();
 }
@@ -1165,10 +1207,52 @@ Geom pre_pass_geom(const Geom &g) {
   return gp;
 }
 
+// A wide head (d > 128) is swept one slice of 128 features of q and k after the other, straight from and to their rows
+// (b*h = 8, n = 8192, d = 256, e = 128, forward + backward: 197 us, against 383 with slices copied out and summed outside):
+// the scores and the state terms are sums over features, so every slice after the first adds its part of O (dV) to
+// what is there, while dQ, dK and the states fall apart into slices.  The pre-pass and the scan take all slices in one launch.
+Geom slice_geom(const Geom &g, int i) {
+  Geom gs = g;
+  gs.d = g.dt - i * kMaxWidth < kMaxWidth ? g.dt - i * kMaxWidth : kMaxWidth;
+  gs.add = i > 0;
+  return gs;
+}
+const void *row_slice(const void *p, int i) { return (const elem16_t *)p + i * kMaxWidth; }
+void *row_slice(void *p, int i) { return (elem16_t *)p + i * kMaxWidth; }
+template <class T>  // of the chunk's d x e states
+T *carry_slice(T *p, const Geom &g, int i) { return p ? p + (int64_t)i * kMaxWidth * g.e : p; }
+template <class T>  // of the workspace
+T *state_slice(T *p, const Geom &g, int i) {
+  return p ? p + (int64_t)i * g.b * g.h * g.pre_n * kMaxWidth * kMaxWidth : p;
+}
+FwdArgs slice_args(const FwdArgs &a, const Geom &g, int i) {
+  FwdArgs r = a;
+  r.q = row_slice(a.q, i);
+  r.k = row_slice(a.k, i);
+  r.kv_in = carry_slice(a.kv_in, g, i);
+  r.kv_out = carry_slice(a.kv_out, g, i);
+  return r;
+}
+BwdArgs slice_args(const BwdArgs &a, const Geom &g, int i) {
+  BwdArgs r = a;
+  r.q = row_slice(a.q, i);
+  r.k = row_slice(a.k, i);
+  r.dq = row_slice(a.dq, i);
+  r.dk = row_slice(a.dk, i);
+  r.kv_in = carry_slice(a.kv_in, g, i);
+  r.dkv_in = carry_slice(a.dkv_in, g, i);
+  r.dkv_out = carry_slice(a.dkv_out, g, i);
+  return r;
+}
+
 template <class E, int MODE, int W>
 int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
-  if (g.fused) return launch_fused_fwd<E, MODE, W>(a, g, st);
-  int rc;
+  int rc = 0;
+  const int slices = (int)slices_of(g);
+  if (g.fused) {
+    for (int i = 0; i < slices && !rc; ++i) rc = launch_fused_fwd<E, MODE, W>(slice_args(a, g, i), slice_geom(g, i), st);
+    return rc;
+  }
   if constexpr (MODE != M_NARROW) if (g.combine) {  // (the plan combines full-width heads only)
     // few segments: the pre-pass leaves every segment's own state (the last one's is never read), each
     // sweep workgroup gathers the ones before it, and the last segment's sweep ends with KV_out
@@ -1185,14 +1269,23 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
     if ((rc = launch_state<E, false, MODE, W>(a.k, a.v, a.s, a.seg_states, gp, a.kv_out != nullptr, sub, st))) return rc;
     if ((rc = launch_segment_scan(a.seg_states, a.kv_in, a.kv_out, a.s, gp, 0, st))) return rc;
   }
-  return launch_apply<E, false, false, SRC_SCANNED, MODE, W>(a.q, a.k, a.v, a.s, need_states ? a.seg_states : nullptr,
-                                                             a.kv_in, nullptr, a.o, g, st);
+  for (int i = 0; i < slices && !rc; ++i) {
+    const FwdArgs as = slice_args(a, g, i);
+    rc = launch_apply<E, false, false, SRC_SCANNED, MODE, W>(
+        as.q, as.k, as.v, as.s, need_states ? state_slice(as.seg_states, g, i) : nullptr, as.kv_in, nullptr, as.o,
+        slice_geom(g, i), st);
+  }
+  return rc;
 }
 
 template <class E, int MODE, int W>
 int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
-  if (g.fused) return launch_fused_bwd<E, MODE, W>(a, g, st);
-  int rc;
+  int rc = 0;
+  const int slices = (int)slices_of(g);
+  if (g.fused) {
+    for (int i = 0; i < slices && !rc; ++i) rc = launch_fused_bwd<E, MODE, W>(slice_args(a, g, i), slice_geom(g, i), st);
+    return rc;
+  }
   if constexpr (MODE != M_NARROW) if (g.combine) {
     const float *kv_states = a.kv_seg_states;
     if (!kv_states && g.n_seg > 1) {
@@ -1217,13 +1310,16 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
     if ((rc = launch_segment_scan(a.ws_dkv, a.dkv_in, a.dkv_out, a.s, gp, 1, st))) return rc;
     dkv_states = a.ws_dkv;
   }
-  return launch_bwd3<E, SRC_SCANNED, MODE, W>(a, kv_states, dkv_states, g, st);
+  for (int i = 0; i < slices && !rc; ++i)
+    rc = launch_bwd3<E, SRC_SCANNED, MODE, W>(slice_args(a, g, i), state_slice(kv_states, g, i),
+                                              state_slice(dkv_states, g, i), slice_geom(g, i), st);
+  return rc;
 }
 
 
-// rows of g.sd = g.se features (64 or 128) run without the bookkeeping of narrower ones
+// rows of g.sd = g.se features (64 or 128) run without the bookkeeping of narrower ones and of slices
 int mode_of(const Geom &g) {
-  if (g.d != g.sd || g.e != g.se) return M_NARROW;
+  if (g.dt != g.sd || g.e != g.se) return M_NARROW;
   return g.n % BLK != 0 ? M_RAGGED : M_ALIGNED;
 }
 
