@@ -10,11 +10,16 @@
 // lane (c, hh) supplies A[c][k_hh] and B[k_hh][c], and leaves C[8g+4hh+r][c] in register
 // 4g+r.  Choosing (k_0, k_1) = (8g+r, 8g+4+r) makes register 4g+r of an accumulator tile
 // exactly the operand element the next product needs, so
-//   * the state tiles feed the state-term product straight from registers,
-//   * the masked 32x32 score tile feeds the intra-block product straight from registers
-//     (every wave computes the whole tile: no LDS round trip, no rounding),
-// and the LDS only holds the block's inputs: X and Y token-major, (w (.) Y)^T and Z^T
-// feature-major (XOR-swizzled 16-byte granules).  Blocks are 32 tokens.
+// the state tiles feed the state-term product straight from registers.  The LDS holds the block's inputs -- X and Y
+// token-major, (w (.) Y)^T and Z^T feature-major (XOR-swizzled 16-byte granules) -- and the masked 32 x 32 score tile,
+// of which each of the four waves computes one 16 x 16 quadrant (v_mfma_f32_16x16x4_f32).  Blocks are 32 tokens.
+//
+// What bounds it: the fp32 matrix rate.  A block costs a wave 160 products of 32x32x2 (64 state term, 64 state
+// update, 16 intra-block, and 16 products' time for its quadrant of the scores) = 10 240 cycles; with every wave
+// computing the whole score tile, as before, it was 208.  Two barriers a block: the X and Y tiles of the next block are
+// written while this one's second half runs, its transposed tiles while the next one's first half does, so no fill
+// stands between two barriers.  b*h = 24, n = 2048, forward + backward: 238 us against 275 (forward sweep 57 us against
+// 63, backward 131 against 149); b*h = 24, n = 16384: 1384 against 1555, 71 % of the time the fp32 products alone take.
 #include "lasp_common.h"
 
 namespace lasp {
@@ -32,7 +37,9 @@ constexpr int OFF_XN = 0;
 constexpr int OFF_YN = OFF_XN + BLK * LDN;
 constexpr int OFF_YT = OFF_YN + BLK * LDN;
 constexpr int OFF_ZT = OFF_YT + F * LDT;
-constexpr int APPLY_LDS = OFF_ZT + F * LDT;  // 66560 B: two workgroups per CU
+constexpr int LDSC = 144;                    // bytes per row of the score tile (128 + 16), row = token of X
+constexpr int OFF_SC = OFF_ZT + F * LDT;
+constexpr int APPLY_LDS = OFF_SC + BLK * LDSC;  // 71168 B: two workgroups per CU
 constexpr float LOG2E = 1.4426950408889634f;
 
 __device__ __forceinline__ float decay(float s_log2e, float x) {
@@ -41,6 +48,9 @@ __device__ __forceinline__ float decay(float s_log2e, float x) {
 __device__ __forceinline__ f32x4 lds16(const char *p) { return *reinterpret_cast<const f32x4 *>(p); }
 __device__ __forceinline__ floatx16 mfma(float a, float b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
 // byte offset of 16-byte granule g16 (4 tokens) of feature row f.  The XOR term is a bijection
@@ -154,26 +164,37 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       nz[r] = (!RAGGED || row < len) ? Zg[off + row * 32 + cq] : zero;
     }
   };
-  auto fill_lds = [&]() __attribute__((always_inline)) {
+  auto fill_rows = [&]() __attribute__((always_inline)) {  // X and Y as they are
 #pragma unroll
     for (int it = 0; it < 4; ++it)
       *reinterpret_cast<f32x4 *>(smem + OFF_XN + (rq + 8 * it) * LDN + cq * 16) = nx[it];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       *reinterpret_cast<f32x4 *>(smem + OFF_YN + (4 * rq + r) * LDN + cq * 16) = ny[r];
+  };
+  auto fill_transposed = [&]() __attribute__((always_inline)) {  // (w (.) Y)^T and Z^T
     store_transposed(smem + OFF_YT, ny, cq, rq, kdec);
     store_transposed(smem + OFF_ZT, nz, cq, rq, ones);
   };
+  // this wave's quadrant of the score tile: tokens b = 16 qb .. of Y, a = 16 qa .. of X
+  const int qb = w >> 1, qa = w & 1;
+  const bool q_active = REV ? !(qb == 0 && qa == 1) : !(qb == 1 && qa == 0);  // else wholly masked
+  const int q_lane = lane & 15, q_grp = lane >> 4;
 
   const int first = REV ? sw.nblk - 1 : 0;
   const int step = REV ? -1 : 1;
   issue_loads(first);
-  fill_lds();
+  fill_rows();
+  fill_transposed();
+  if (sw.nblk > 1) issue_loads(first + step);
   __syncthreads();
 
   for (int it = 0, blk = first; it < sw.nblk; ++it, blk += step) {
     const bool more = it + 1 < sw.nblk;
-    if (more) issue_loads(blk + step);
+    if (it > 0) {
+      fill_transposed();  // of this block; read after the first barrier
+      if (more) issue_loads(blk + step);
+    }
     const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
     float qd = qdec, bd = blockdec;
     if (RAGGED && REV && len != BLK) {
@@ -181,45 +202,57 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       bd = decay(sl, (float)len);
     }
 
-    // (1) sweep over the features: state term and score tile from the same X elements
-    //     acc[4g+r] = sum_f St[f][32w+8g+4hh+r] x_a[f]      (a = c)
-    //     sc[4g+r]  = y_b . x_a,  b = 8g+4hh+r
-    floatx16 acc, sc;
+    // (1) scores of the quadrant and state term
+    //     sc[r]     = y_b . x_a,                          b = 16 qb + 4 q_grp + r, a = 16 qa + q_lane
+    //     acc[4g+r] = sum_f St[f][32w+8g+4hh+r] x_a[f]    (a = c)
+    // (the scores contract features 16 m + 4 q_grp + r over q_grp, in that order on both sides)
+    floatx16 acc;
+    f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      acc[r] = 0.f;
-      sc[r] = 0.f;
-    }
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
     {
       const char *xp = smem + OFF_XN + c * LDN + hh * 16;
-      const char *yp = smem + OFF_YN + c * LDN + hh * 16;
+      const char *xq = smem + OFF_XN + (16 * qa + q_lane) * LDN + q_grp * 16;
+      const char *yq = smem + OFF_YN + (16 * qb + q_lane) * LDN + q_grp * 16;
 #pragma unroll
-      for (int m = 0; m < 16; ++m) {  // features 8m + 4hh + {0..3}
-        const f32x4 xf = lds16(xp + m * 32);
-        const f32x4 yf = lds16(yp + m * 32);
+      for (int m = 0; m < 8; ++m) {
+        const f32x4 ys = lds16(yq + m * 64), xs = lds16(xq + m * 64);
+        const f32x4 x0 = lds16(xp + m * 64), x1 = lds16(xp + m * 64 + 32);  // features 16m + 4hh + .., 16m + 8 + 4hh + ..
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          acc = mfma(st[m >> 2][4 * (m & 3) + r], xf[r], acc);
-          sc = mfma(yf[r], xf[r], sc);
+          acc = mfma(st[m >> 1][8 * (m & 1) + r], x0[r], acc);
+          if (q_active) sc = mfma16(ys[r], xs[r], sc);
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc = mfma(st[m >> 1][8 * (m & 1) + 4 + r], x1[r], acc);
       }
     }
     // (2) mask the scores, scale the state term
+    {
+      const int a = 16 * qa + q_lane, b0 = 16 * qb + 4 * q_grp;
+      f32x4 m;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int b = 8 * (r >> 2) + 4 * hh + (r & 3);
-      const int dist = REV ? b - c : c - b;
-      sc[r] = dist >= 0 ? sc[r] * decay(sl, (float)dist) : 0.f;
-      acc[r] *= qd;
+      for (int r = 0; r < 4; ++r) {
+        const int dist = REV ? b0 + r - a : a - b0 - r;
+        m[r] = dist >= 0 ? sc[r] * decay(sl, (float)dist) : 0.f;
+      }
+      *reinterpret_cast<f32x4 *>(smem + OFF_SC + a * LDSC + b0 * 4) = m;
     }
-    // (3) intra-block term and (4) state update share the Z^T elements
-    f32x4 zf[4];
 #pragma unroll
-    for (int gq = 0; gq < 4; ++gq) zf[gq] = lds16(smem + OFF_ZT + tr_off(32 * w + c, 2 * gq + hh));
+    for (int r = 0; r < 16; ++r) acc[r] *= qd;
+    __syncthreads();  // the score tile and the transposed tiles are complete; X and Y are no longer read
+    if (more) fill_rows();  // of the next block
+    // (3) intra-block term and (4) state update share the Z^T elements
+    f32x4 zf[4], sf[4];
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      zf[gq] = lds16(smem + OFF_ZT + tr_off(32 * w + c, 2 * gq + hh));
+      sf[gq] = lds16(smem + OFF_SC + c * LDSC + (8 * gq + 4 * hh) * 4);
+    }
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc = mfma(zf[gq][r], sc[4 * gq + r], acc);
+      for (int r = 0; r < 4; ++r) acc = mfma(zf[gq][r], sf[gq][r], acc);
 #pragma unroll
     for (int T = 0; T < 4; ++T) {
 #pragma unroll
@@ -244,11 +277,7 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
         *reinterpret_cast<f32x4 *>(orow + 8 * gq) = o;
       }
     }
-    if (more) {
-      __syncthreads();  // every wave is done reading this block's tiles
-      fill_lds();
-      __syncthreads();  // next block visible
-    }
+    if (more) __syncthreads();  // the next block's X and Y are complete; this block's transposed tiles are no longer read
   }
 }
 
