@@ -17,7 +17,7 @@ from __future__ import annotations
 
 import torch
 
-from . import _abi
+from . import _native
 from .utils import seq_parallel_manager as spm
 
 
@@ -32,6 +32,60 @@ def feature_slices(d: int):
     return [(lo, min(lo + width, d)) for lo in range(0, d, width)]
 
 
+class Exchange:
+    """Where a chunk sits in its chain: whom it receives states from and sends them to.
+
+    rebind: the outgoing state goes to a new tensor and the caller's KV / DKV buffer is left
+    holding the INCOMING state, which is what lasp_fuse_parallel's `KV = ...` rebinding does
+    (lasp/lasp_fuse_parallel.py:941-942,1099-1106); otherwise the buffer receives the outgoing
+    state in place (lasp/lasp_fuse.py:126-127,352-353).
+    tag: feature-slice index, keeps the loopback messages of different slices apart.
+    """
+
+    __slots__ = ("group", "rank", "world", "prev_rank", "next_rank", "rebind", "tag")
+
+    def __init__(self, rebind, tag=0):
+        self.group = spm.get_sequence_parallel_group()
+        self.rank = spm.get_sequence_parallel_rank()
+        self.world = spm.get_sequence_parallel_world_size()
+        self.prev_rank = spm.get_seq_parallel_send_rank()
+        self.next_rank = spm.get_seq_parallel_receive_rank()
+        self.rebind, self.tag = rebind, tag
+
+    def _outgoing(self, buffer, incoming, wanted):
+        if not self.rebind:
+            return buffer
+        if incoming is None:
+            buffer.zero_()
+        else:
+            buffer.copy_(incoming)
+        return torch.empty_like(buffer) if wanted else None  # the last rank's outgoing state goes nowhere
+
+    def before_forward(self, KV, barrier):
+        """(state entering the chunk or None, tensor for the state that leaves it or None)."""
+        if barrier and not isinstance(self.group, spm.LoopbackGroup):
+            torch.distributed.barrier()
+        kv_in = spm.state_take(KV, self.prev_rank, self.group, tag=self.tag) if self.rank > 0 else None
+        return kv_in, self._outgoing(KV, kv_in, self.rank < self.world - 1)
+
+    def after_forward(self, kv_out):
+        if self.rank < self.world - 1:
+            spm.state_send(kv_out, self.next_rank, self.group, tag=self.tag, give=self.rebind)
+
+
+def before_backward(x: Exchange, DKV):
+    """The same for the backward of the chunk, whose states travel the other way."""
+    dkv_in = None
+    if x.rank < x.world - 1:
+        dkv_in = spm.state_take(DKV, x.next_rank, x.group, dst=x.rank, tag=x.tag)
+    return dkv_in, x._outgoing(DKV, dkv_in, x.rank > 0)
+
+
+def after_backward(x: Exchange, dkv_out):
+    if x.rank > 0:
+        spm.state_send(dkv_out, x.prev_rank, x.group, src=x.rank, tag=x.tag, give=x.rebind)
+
+
 class ChunkFunction(torch.autograd.Function):
     """forward(q, k, v, s, KV, DKV, cache_states, barrier, rebind=False, tag=0) -> o
 
@@ -41,11 +95,7 @@ class ChunkFunction(torch.autograd.Function):
     lasp_fuse_parallel trade, lasp/lasp_fuse_parallel.py:1103) instead of
     recomputing them (lasp_fuse, whose backward re-runs the kv recurrence,
     lasp/lasp_fuse.py:237-260).
-    rebind: the outgoing state goes to a new tensor and the caller's KV / DKV buffer is left
-    holding the INCOMING state, which is what lasp_fuse_parallel's `KV = ...` rebinding does
-    (lasp/lasp_fuse_parallel.py:941-942,1099-1106); otherwise the buffer receives the outgoing
-    state in place (lasp/lasp_fuse.py:126-127,352-353).
-    tag: feature-slice index, keeps the loopback messages of different slices apart.
+    rebind, tag: see Exchange.
     """
 
     @staticmethod
@@ -53,36 +103,21 @@ class ChunkFunction(torch.autograd.Function):
         chained = KV is not None
         ctx.chained = chained
         if not chained:
-            o, states, seg_len = _abi.chunk_fwd(q, k, v, s)
+            o, states, seg_len = _native.chunk_fwd(q, k, v, s)
             ctx.save_for_backward(q, k, v, s, states if cache_states else None)
             ctx.seg_len = seg_len
             return o
 
-        group = spm.get_sequence_parallel_group()
-        rank = spm.get_sequence_parallel_rank()
-        world = spm.get_sequence_parallel_world_size()
-        prev_rank = spm.get_seq_parallel_send_rank()
-        next_rank = spm.get_seq_parallel_receive_rank()
-        if barrier and not isinstance(group, spm.LoopbackGroup):
-            torch.distributed.barrier()
-        kv_in = spm.state_take(KV, prev_rank, group, tag=tag) if rank > 0 else None
-        kv_out = KV
-        if rebind:  # the caller's buffer is left holding the incoming state
-            if kv_in is None:
-                KV.zero_()
-            else:
-                KV.copy_(kv_in)
-            kv_out = torch.empty_like(KV) if rank < world - 1 else None  # the last rank's KV_out goes nowhere
-        o, states, seg_len = _abi.chunk_fwd(q, k, v, s, kv_in=kv_in, kv_out=kv_out)
+        x = Exchange(rebind, tag)
+        kv_in, kv_out = x.before_forward(KV, barrier)
+        o, states, seg_len = _native.chunk_fwd(q, k, v, s, kv_in=kv_in, kv_out=kv_out)
         # DKV is a scratch buffer that later backward calls overwrite in place, so it is
         # kept by reference rather than as a version-checked saved tensor.
         ctx.save_for_backward(q, k, v, s, states if cache_states else None, kv_in)
         ctx.dkv_buffer = DKV
         ctx.seg_len = seg_len
-        if rank < world - 1:
-            spm.state_send(kv_out, next_rank, group, tag=tag, give=rebind)
-        ctx.group, ctx.rank, ctx.world, ctx.tag, ctx.rebind = group, rank, world, tag, rebind
-        ctx.prev_rank, ctx.next_rank = prev_rank, next_rank
+        ctx.exchange = x
+        x.after_forward(kv_out)
         return o
 
     @staticmethod
@@ -90,42 +125,38 @@ class ChunkFunction(torch.autograd.Function):
         none = (None,) * 7
         if not ctx.chained:
             q, k, v, s, states = ctx.saved_tensors
-            dq, dk, dv = _abi.chunk_bwd(q, k, v, s, do, kv_seg_states=states, seg_len=ctx.seg_len)
+            dq, dk, dv = _native.chunk_bwd(q, k, v, s, do, kv_seg_states=states, seg_len=ctx.seg_len)
             return (dq, dk, dv) + none
 
         q, k, v, s, states, kv_in = ctx.saved_tensors
-        DKV = ctx.dkv_buffer
-        dkv_in = None
-        if ctx.rank < ctx.world - 1:
-            dkv_in = spm.state_take(DKV, ctx.next_rank, ctx.group, dst=ctx.rank, tag=ctx.tag)
-        dkv_out = DKV
-        if ctx.rebind:
-            if dkv_in is None:
-                DKV.zero_()
-            else:
-                DKV.copy_(dkv_in)
-            dkv_out = torch.empty_like(DKV) if ctx.rank > 0 else None
-        dq, dk, dv = _abi.chunk_bwd(q, k, v, s, do, kv_in=kv_in, dkv_in=dkv_in, dkv_out=dkv_out,
+        dkv_in, dkv_out = before_backward(ctx.exchange, ctx.dkv_buffer)
+        dq, dk, dv = _native.chunk_bwd(q, k, v, s, do, kv_in=kv_in, dkv_in=dkv_in, dkv_out=dkv_out,
                                     kv_seg_states=states, seg_len=ctx.seg_len)
-        if ctx.rank > 0:
-            spm.state_send(dkv_out, ctx.prev_rank, ctx.group, src=ctx.rank, tag=ctx.tag, give=ctx.rebind)
+        after_backward(ctx.exchange, dkv_out)
         return (dq, dk, dv) + none
 
 
-def _sliced_in_kernels(q, v, KV, DKV) -> bool:
-    """Whether the library takes this wide head whole: its 16-bit kernels read the slices from q's and k's own rows."""
-    return (q.is_cuda and q.dtype in (torch.bfloat16, torch.float16) and q.shape[-1] <= 1024 and q.shape[-1] % 8 == 0
-            and v.shape[-1] <= 128 and v.shape[-1] % 8 == 0
-            and (KV is None or (KV.is_contiguous() and DKV.is_contiguous())))
+def native_chunk(q, k, v, s, KV, DKV, barrier, rebind=False):
+    """A chunk of a chain as ChunkFunction runs it (states kept for backward), through the native autograd node;
+    None where the extension does not take the call."""
+    if not q.is_cuda:
+        return None
+    ext = _native.ext()
+    if not ext.takes(q, k, v, s, KV, DKV):
+        return None
+    x = Exchange(rebind)
+    kv_in, kv_out = x.before_forward(KV, barrier)
+    o = ext.chunk(q, k, v, s, kv_in, kv_out, DKV, x)
+    x.after_forward(kv_out)
+    return o
 
 
 def run_sliced(q, k, v, ed, KV, DKV, cache_states, barrier, rebind=False):
-    """Applies ChunkFunction per feature slice of q/k and adds the outputs; 16-bit heads on the GPU in one call, whose
-    kernels slice and add (b*h = 8, n = 8192, d = 256: the copies, zero fills and additions of this loop were half of a
-    forward + backward)."""
+    """Applies ChunkFunction per feature slice of q/k and adds the outputs (the library slices 16-bit heads itself, see
+    native_chunk)."""
     d = q.shape[-1]
     parts = feature_slices(d)
-    if len(parts) == 1 or _sliced_in_kernels(q, v, KV, DKV):
+    if len(parts) == 1:
         return ChunkFunction.apply(q, k, v, ed, KV, DKV, cache_states, barrier, rebind, 0)
     out = None
     for tag, (lo, hi) in enumerate(parts):

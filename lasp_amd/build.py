@@ -1,10 +1,11 @@
-"""Builds lasp_amd/liblasp_hip.so for gfx950 with hipcc (cross-compiles without a GPU).
+"""Builds lasp_amd/liblasp_hip.so for gfx950 with hipcc (cross-compiles without a GPU) and lasp_amd/_lasp_torch.so.
 
     python -m lasp_amd.build
 """
 import os
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
@@ -12,6 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liblasp_hip.so")
+TORCH_LIB = os.path.join(HERE, "_lasp_torch.so")
 SOURCES = ["lasp_abi.hip", "lasp_generic.hip", "lasp_mfma.hip", "lasp_mfma_f16.hip", "lasp_mfma_f32.hip", "lasp_probe.hip"]
 
 HIPCC_FLAGS = [
@@ -47,7 +49,27 @@ def build(verbose: bool = True, extra_flags=()) -> str:
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.run(cmd, check=True)
+    build_torch_side(verbose)
     return LIB
+
+
+def build_torch_side(verbose: bool = True) -> str:
+    """Compiles lasp_torch.cpp, host code over the library's C ABI, against torch's headers."""
+    import torch
+
+    base = os.path.dirname(os.path.abspath(torch.__file__))
+    include = [os.path.join(base, "include"), os.path.join(base, "include", "torch", "csrc", "api", "include"),
+               os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"],
+               os.path.join(ROOT, "include")]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[x for path in include for x in ("-isystem", path)], os.path.join(CSRC, "lasp_torch.cpp"), "-o", TORCH_LIB,
+           "-L" + HERE, "-llasp_hip", "-L" + os.path.join(base, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10",
+           "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    return TORCH_LIB
 
 
 if __name__ == "__main__":

@@ -1,0 +1,321 @@
+// The PyTorch side of the library in native code: argument checks, allocations and autograd of the operators' usual
+// case, above the C ABI of include/lasp_hip.h.
+//
+// A call on a short sequence is bound by the host: the kernels of a forward + backward over 256 tokens on 8 heads take
+// 23 us, while the Python path around them (ctypes with twenty arguments, a torch.autograd.Function in Python,
+// whose backward also has to take the interpreter lock on autograd's thread) took 49-108 us.  Here a forward is one
+// C++ call (5.7 us with its launch, against about 22) that leaves one autograd node behind, and a backward never enters
+// the interpreter (but for the state exchange of a sequence-parallel chain, which is Python).  Forward + backward, before
+// and now: b*h = 8, n = 256: 101 and 53 us, of which some 35 are autograd's own handover to its device thread; b*h = 96,
+// n = 512: 108 and 52 us (the kernels); eight chained chunks of 2048 tokens at b*h = 24: 762 and 674 us.
+//
+// "Usual case": contiguity aside, what the kernels take as it is -- device tensors of one type, fp32 with
+// d = e = 128 or 16 bits with widths that are multiples of 8, float32 slopes on the same device.  Everything else (padding, other
+// types, errors to report) stays with lasp_amd/_abi.py and lasp_amd/_chain.py: the functions below return None for it.
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/extension.h>
+
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include "lasp_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+// ---- errors ------------------------------------------------------------------------------------------------
+PyObject *g_error = nullptr;  // lasp_amd._abi.LaspError
+
+// A library error as the Python exception LaspError, from whatever thread autograd runs this on.
+[[noreturn]] void raise_lasp(int rc, const char *what) {
+  const std::string msg = std::string(what) + " failed (code " + std::to_string(rc) + "): " + lasp_last_error();
+  pybind11::gil_scoped_acquire gil;
+  PyErr_SetString(g_error ? g_error : PyExc_RuntimeError, msg.c_str());
+  python_error err;
+  err.persist();
+  throw err;
+}
+
+// ---- shapes ------------------------------------------------------------------------------------------------
+struct Shape {
+  int b, h, d, e, dtype;
+  int64_t n;
+};
+
+int dtype_code(const Tensor &t) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return LASP_DTYPE_F32;
+    case at::kBFloat16: return LASP_DTYPE_BF16;
+    case at::kHalf: return LASP_DTYPE_F16;
+    default: return -1;
+  }
+}
+
+// The usual case, see above; fills `sh`.
+bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Shape &sh) {
+  if (!q.is_cuda() || q.dim() != 4 || v.dim() != 4 || k.sizes() != q.sizes() || q.numel() == 0 || v.numel() == 0) return false;
+  if (k.device() != q.device() || v.device() != q.device() || s.device() != q.device()) return false;
+  if (k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type()) return false;
+  for (int i = 0; i < 3; ++i)
+    if (v.size(i) != q.size(i)) return false;
+  if (q.size(0) > INT32_MAX || q.size(1) > INT32_MAX || s.scalar_type() != at::kFloat || s.numel() != q.size(1) || !s.is_contiguous())
+    return false;
+  sh.dtype = dtype_code(q);
+  const int64_t d = q.size(3), e = v.size(3);
+  if (sh.dtype == LASP_DTYPE_F32 ? d != 128 || e != 128 : sh.dtype < 0 || d % 8 || e % 8 || d > 1024 || e > 128) return false;
+  sh.b = (int)q.size(0);
+  sh.h = (int)q.size(1);
+  sh.n = q.size(2);
+  sh.d = (int)d;
+  sh.e = (int)e;
+  return true;
+}
+
+bool state_ok(const Tensor &t, const Shape &sh, const Tensor &q) {
+  return !t.defined() || (t.scalar_type() == at::kFloat && t.device() == q.device() && t.is_contiguous() && t.dim() == 4 &&
+                          t.size(0) == sh.b && t.size(1) == sh.h && t.size(2) == sh.d && t.size(3) == sh.e);
+}
+
+void *data(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+// ---- the two calls -----------------------------------------------------------------------------------------
+struct Plan {
+  int seg_len = 0, n_seg = 1;
+  size_t bytes = 0;
+  bool fused = false;  // one launch, no workspace, no states; seg_len stays 0 so that the backward chooses alike
+};
+Plan plan_of(const Shape &sh, int seg_len) {
+  Plan p;
+  if (seg_len == 0) {
+    const int path = lasp_kernel_path(sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype);
+    if (path < 0) raise_lasp(path, "lasp_kernel_path");
+    if (path == LASP_PATH_MFMA_FUSED) {
+      p.fused = true;
+      return p;
+    }
+  }
+  const int rc = lasp_plan(sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, seg_len, &p.seg_len, &p.n_seg, &p.bytes);
+  if (rc) raise_lasp(rc, "lasp_plan");
+  return p;
+}
+
+// `in`, or a copy where `out` is the same memory and this shape's kernels cannot update a state in place
+Tensor private_incoming(const Tensor &in, const Tensor &out, const Shape &sh, int seg_len, bool backward) {
+  if (!in.defined() || !out.defined() || in.data_ptr() != out.data_ptr()) return in;
+  return lasp_inplace_ok(sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, seg_len, backward) == 1 ? in : in.clone();
+}
+
+Tensor floats(size_t bytes, const Tensor &like) {
+  return at::empty({(int64_t)(bytes / sizeof(float))}, like.options().dtype(at::kFloat));
+}
+
+struct Forward {
+  Tensor o, states;
+  int seg_len = 0;
+};
+// q, k, v contiguous
+Forward run_forward(const Shape &sh, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Tensor kv_in,
+                    const Tensor &kv_out, int seg_len) {
+  const Plan p = plan_of(sh, seg_len);
+  kv_in = private_incoming(kv_in, kv_out, sh, p.seg_len, false);
+  Forward f;
+  f.seg_len = p.seg_len;
+  f.o = at::empty(v.sizes(), v.options());
+  if (!p.fused && (p.n_seg > 1 || kv_in.defined() || kv_out.defined())) f.states = floats(p.bytes, q);
+  const int rc = lasp_chunk_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), (const float *)data(kv_in),
+                                (float *)data(kv_out), f.o.data_ptr(), (float *)data(f.states), sh.b, sh.h, sh.n, sh.d, sh.e,
+                                sh.dtype, p.seg_len, c10::hip::getCurrentHIPStream(q.device().index()).stream());
+  if (rc) raise_lasp(rc, "lasp_chunk_fwd");
+  return f;
+}
+
+struct Backward {
+  Tensor dq, dk, dv;
+};
+// q, k, v, d_o contiguous; `states` undefined: rebuilt
+Backward run_backward(const Shape &sh, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &d_o,
+                      const Tensor &kv_in, Tensor dkv_in, const Tensor &dkv_out, const Tensor &states, int seg_len) {
+  const Plan p = plan_of(sh, seg_len);
+  dkv_in = private_incoming(dkv_in, dkv_out, sh, p.seg_len, true);
+  Backward r;
+  r.dq = at::empty(q.sizes(), q.options());
+  r.dk = at::empty(q.sizes(), q.options());
+  r.dv = at::empty(v.sizes(), v.options());
+  const bool need_dkv = !p.fused && (p.n_seg > 1 || dkv_in.defined() || dkv_out.defined());
+  const bool need_kv = !p.fused && !states.defined() && (p.n_seg > 1 || kv_in.defined());
+  const size_t bytes = p.bytes * ((need_dkv ? 1 : 0) + (need_kv ? 1 : 0));
+  Tensor ws;
+  if (bytes) ws = floats(bytes, q);
+  const int rc = lasp_chunk_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), d_o.data_ptr(),
+                                (const float *)data(kv_in), (const float *)data(dkv_in), r.dq.data_ptr(), r.dk.data_ptr(),
+                                r.dv.data_ptr(), (float *)data(dkv_out), p.fused ? nullptr : (const float *)data(states),
+                                (float *)data(ws), bytes, sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, p.seg_len,
+                                c10::hip::getCurrentHIPStream(q.device().index()).stream());
+  if (rc) raise_lasp(rc, "lasp_chunk_bwd");
+  return r;
+}
+
+// ---- autograd ----------------------------------------------------------------------------------------------
+// Python side of a chain's backward: before(exchange, DKV) -> (dkv_in or None, dkv_out or None) receives the state from
+// the next rank, after(exchange, dkv_out) sends the one that this chunk leaves.
+PyObject *g_before = nullptr, *g_after = nullptr;
+
+struct PyRef {  // a Python object held by a node, which any thread may drop
+  PyObject *p = nullptr;
+  ~PyRef() {
+    if (p && Py_IsInitialized()) {
+      pybind11::gil_scoped_acquire gil;
+      Py_DECREF(p);
+    }
+  }
+};
+
+struct ChunkNode : public torch::autograd::Node {
+  Shape sh;
+  int seg_len = 0;
+  SavedVariable q, k, v, s, states, kv_in;
+  Tensor dkv_buffer;  // the caller's DKV: later backward calls overwrite it, so it is kept by reference
+  PyRef exchange;     // set in a chain
+
+  std::string name() const override { return "LaspChunkBackward"; }
+
+  void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (SavedVariable *x : {&q, &k, &v, &s, &states, &kv_in}) x->reset_data();
+  }
+
+  variable_list apply(variable_list &&grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
+    if (!grads[0].defined()) return variable_list(4);
+    const Tensor q_ = q.unpack().contiguous(), k_ = k.unpack().contiguous(), v_ = v.unpack().contiguous(), s_ = s.unpack();
+    const Tensor states_ = states.unpack(), kv_in_ = kv_in.unpack();
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    c10::OptionalDeviceGuard guard(q_.device());
+    Tensor dkv_in, dkv_out;
+    if (exchange.p) call_python([&] {
+      pybind11::object r = pybind11::reinterpret_borrow<pybind11::object>(g_before)(
+          pybind11::reinterpret_borrow<pybind11::object>(exchange.p), dkv_buffer);
+      auto pair = r.cast<std::pair<std::optional<Tensor>, std::optional<Tensor>>>();
+      if (pair.first) dkv_in = *pair.first;
+      if (pair.second) dkv_out = *pair.second;
+    });
+    Backward r = run_backward(sh, q_, k_, v_, s_, grads[0].contiguous(), kv_in_, dkv_in, dkv_out, states_, seg_len);
+    if (exchange.p) call_python([&] {
+      pybind11::reinterpret_borrow<pybind11::object>(g_after)(pybind11::reinterpret_borrow<pybind11::object>(exchange.p),
+                                                              dkv_out.defined() ? std::optional<Tensor>(dkv_out) : std::nullopt);
+    });
+    variable_list out(4);
+    out[0] = std::move(r.dq);
+    out[1] = std::move(r.dk);
+    out[2] = std::move(r.dv);
+    return out;
+  }
+
+  template <class F>
+  static void call_python(F &&f) {
+    pybind11::gil_scoped_acquire gil;
+    try {
+      f();
+    } catch (pybind11::error_already_set &e) {
+      e.restore();
+      python_error err;
+      err.persist();
+      throw err;
+    }
+  }
+};
+
+std::optional<Tensor> operator_call(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &kv_in,
+                                    const Tensor &kv_out, const Tensor &dkv_buffer, PyObject *exchange) {
+  Shape sh;
+  if (!regular(q, k, v, s, sh)) return std::nullopt;
+  const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() || s.requires_grad());
+  c10::OptionalDeviceGuard guard(q.device());
+  Forward f;
+  {
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, kv_in, kv_out, 0);
+  }
+  if (grad) {
+    std::shared_ptr<ChunkNode> node(new ChunkNode(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(q, k, v, s));
+    node->sh = sh;
+    node->seg_len = f.seg_len;
+    node->q = SavedVariable(q, false);
+    node->k = SavedVariable(k, false);
+    node->v = SavedVariable(v, false);
+    node->s = SavedVariable(s, false);
+    if (f.states.defined()) node->states = SavedVariable(f.states, false);
+    if (kv_in.defined()) node->kv_in = SavedVariable(kv_in, false);
+    node->dkv_buffer = dkv_buffer;
+    if (exchange) {
+      Py_INCREF(exchange);
+      node->exchange.p = exchange;
+    }
+    torch::autograd::set_history(f.o, node);
+  }
+  return f.o;
+}
+
+Tensor or_none(const std::optional<Tensor> &t) { return t ? *t : Tensor(); }
+
+}  // namespace
+
+PYBIND11_MODULE(_lasp_torch, m) {
+  namespace py = pybind11;
+  m.def("bind", [](py::object error, py::object before, py::object after) {
+    g_error = error.release().ptr();
+    g_before = before.release().ptr();
+    g_after = after.release().ptr();
+  });
+  // the stateless operator
+  m.def("attention", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s) {
+    return operator_call(q, k, v, s, Tensor(), Tensor(), Tensor(), nullptr);
+  });
+  // whether a chain's chunk is a usual case (asked before its incoming state is received)
+  m.def("takes", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &KV, const Tensor &DKV) {
+    Shape sh;
+    return regular(q, k, v, s, sh) && state_ok(KV, sh, q) && state_ok(DKV, sh, q);
+  });
+  // a chunk of a chain
+  m.def("chunk", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
+                    const std::optional<Tensor> &kv_out, const Tensor &dkv_buffer, py::object exchange) {
+    return operator_call(q, k, v, s, or_none(kv_in), or_none(kv_out), dkv_buffer, exchange.ptr());
+  });
+  // _abi.chunk_fwd / chunk_bwd
+  m.def("chunk_fwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
+                        const std::optional<Tensor> &kv_out, int seg_len) -> py::object {
+    Shape sh;
+    const Tensor in = or_none(kv_in), out = or_none(kv_out);
+    if (!regular(q, k, v, s, sh) || !state_ok(in, sh, q) || !state_ok(out, sh, q)) return py::none();
+    c10::OptionalDeviceGuard guard(q.device());
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    Forward f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, in, out, seg_len);
+    return py::make_tuple(f.o, f.states.defined() ? std::optional<Tensor>(f.states) : std::nullopt, f.seg_len);
+  });
+  m.def("chunk_bwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &d_o,
+                        const std::optional<Tensor> &kv_in, const std::optional<Tensor> &dkv_in,
+                        const std::optional<Tensor> &dkv_out, const std::optional<Tensor> &states, int seg_len) -> py::object {
+    Shape sh;
+    const Tensor in = or_none(kv_in), din = or_none(dkv_in), dout = or_none(dkv_out), st = or_none(states);
+    if (!regular(q, k, v, s, sh) || !state_ok(in, sh, q) || !state_ok(din, sh, q) || !state_ok(dout, sh, q) ||
+        d_o.device() != q.device() || d_o.scalar_type() != q.scalar_type() || d_o.sizes() != v.sizes())
+      return py::none();
+    if (st.defined()) {  // what chunk_fwd returned for this shape
+      const Plan p = plan_of(sh, seg_len);
+      if (!p.fused && (st.scalar_type() != at::kFloat || st.device() != q.device() || !st.is_contiguous() ||
+                       (size_t)st.numel() * sizeof(float) != p.bytes))
+        return py::none();
+    }
+    c10::OptionalDeviceGuard guard(q.device());
+    at::AutoDispatchBelowADInplaceOrView below_autograd;
+    Backward r = run_backward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, d_o.contiguous(), in, din, dout, st, seg_len);
+    return py::make_tuple(r.dq, r.dk, r.dv);
+  });
+}

@@ -5,8 +5,8 @@ torch), KV and DKV tensors instead of allocating them per call (lasp/lasp_cache.
 the decays are derived from the slopes inside the kernels, so `array` is accepted and ignored."""
 import torch
 
-from . import _abi
-from ._chain import ChunkFunction, run_sliced
+from . import _native
+from ._chain import ChunkFunction, native_chunk, run_sliced
 
 __all__ = ["LaspCache", "lasp_cache_", "lasp_cache"]
 
@@ -19,7 +19,7 @@ def lasp_forward(q, k, v, s):
     buffer holds, :104-106; the state is returned as computed here.)"""
     b, h, _, d = q.shape
     kv = torch.empty((b, h, d, v.shape[-1]), dtype=torch.float32, device=q.device)
-    o, _, _ = _abi.chunk_fwd(q, k, v, s, kv_in=None, kv_out=kv)
+    o, _, _ = _native.chunk_fwd(q, k, v, s, kv_in=None, kv_out=kv)
     return o, kv.to(q.dtype)
 
 
@@ -27,7 +27,7 @@ def lasp_backward(q, k, v, s, do):
     """Launch shim with the signature of lasp/lasp_cache.py:468-536: (dq, dk, dv, None, dkv)."""
     b, h, _, d = q.shape
     dkv = torch.empty((b, h, d, v.shape[-1]), dtype=torch.float32, device=q.device)
-    dq, dk, dv = _abi.chunk_bwd(q, k, v, s, do, dkv_out=dkv)
+    dq, dk, dv = _native.chunk_bwd(q, k, v, s, do, dkv_out=dkv)
     return dq, dk, dv, None, dkv.to(q.dtype)
 
 
@@ -51,6 +51,9 @@ lasp_cache_ = LaspCache.apply
 
 
 def lasp_cache(q, k, v, ed, array, KV, DKV):
+    o = native_chunk(q, k, v, ed, KV, DKV, False, True)
+    if o is not None:
+        return o
     if q.shape[-1] <= 128:
         return lasp_cache_(q, k, v, ed, array, KV, DKV)
     return run_sliced(q, k, v, ed, KV, DKV, True, False, True)

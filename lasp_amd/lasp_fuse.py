@@ -6,8 +6,8 @@ leaves the state entering each segment in a workspace anyway, so the operator ke
 recompute, as they have no place to keep it."""
 import torch
 
-from . import _abi
-from ._chain import ChunkFunction, run_sliced
+from . import _native
+from ._chain import ChunkFunction, native_chunk, run_sliced
 
 __all__ = ["LaspFuse", "lasp_fuse_", "lasp_fuse"]
 
@@ -18,7 +18,7 @@ def lasp_forward(q, k, v, s, KV):
     Returns o for one chunk.  KV, float32 (b, h, d, e), holds the incoming state and
     is overwritten with the outgoing one, as the reference kernel does (:126-127).
     """
-    o, _, _ = _abi.chunk_fwd(q, k, v, s, kv_in=KV, kv_out=KV)
+    o, _, _ = _native.chunk_fwd(q, k, v, s, kv_in=KV, kv_out=KV)
     return o
 
 
@@ -28,7 +28,7 @@ def lasp_backward(q, k, v, s, do, KV, DKV):
     KV is the state that entered the forward (the copy saved at :496); DKV holds the
     incoming dKV and is overwritten with the outgoing one.  Returns (dq, dk, dv).
     """
-    return _abi.chunk_bwd(q, k, v, s, do, kv_in=KV, dkv_in=DKV, dkv_out=DKV)
+    return _native.chunk_bwd(q, k, v, s, do, kv_in=KV, dkv_in=DKV, dkv_out=DKV)
 
 
 class LaspFuse(torch.autograd.Function):
@@ -48,6 +48,9 @@ lasp_fuse_ = LaspFuse.apply
 
 def lasp_fuse(q, k, v, ed, KV, DKV):
     """KV, DKV: float32 (b, h, d, e) scratch owned by the caller; KV is left holding KV_out."""
+    o = native_chunk(q, k, v, ed, KV, DKV, False)
+    if o is not None:
+        return o
     if q.shape[-1] <= 128:
         return lasp_fuse_(q, k, v, ed, KV, DKV)
     return run_sliced(q, k, v, ed, KV, DKV, True, False)

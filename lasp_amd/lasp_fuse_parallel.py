@@ -2,8 +2,8 @@
 parallel and the per-segment states are kept for backward (lasp/lasp_fuse_parallel.py)."""
 import torch
 
-from . import _abi
-from ._chain import ChunkFunction, run_sliced
+from . import _native
+from ._chain import ChunkFunction, native_chunk, run_sliced
 
 __all__ = ["LaspFuseParallel", "lasp_fuse_parallel_", "lasp_fuse_parallel"]
 
@@ -17,7 +17,7 @@ def lasp_forward(q, k, v, s, KV, BLOCK=128, CBLOCK=64):
     are accepted for signature compatibility; the segment length is the library's.
     """
     KV_out = torch.empty_like(KV)
-    o, kv, _ = _abi.chunk_fwd(q, k, v, s, kv_in=KV, kv_out=KV_out)
+    o, kv, _ = _native.chunk_fwd(q, k, v, s, kv_in=KV, kv_out=KV_out)
     return o, kv, KV_out
 
 
@@ -29,7 +29,7 @@ def lasp_backward(q, k, v, s, do, kv, KV, DKV, BLOCK=128, CBLOCK=64):
     new tensor (:1067-1070).
     """
     DKV_out = torch.empty_like(DKV)
-    dq, dk, dv = _abi.chunk_bwd(q, k, v, s, do, kv_in=KV, dkv_in=DKV, dkv_out=DKV_out, kv_seg_states=kv)
+    dq, dk, dv = _native.chunk_bwd(q, k, v, s, do, kv_in=KV, dkv_in=DKV, dkv_out=DKV_out, kv_seg_states=kv)
     return dq, dk, dv, DKV_out
 
 
@@ -49,6 +49,9 @@ lasp_fuse_parallel_ = LaspFuseParallel.apply
 
 
 def lasp_fuse_parallel(q, k, v, ed, KV, DKV):
+    o = native_chunk(q, k, v, ed, KV, DKV, True, True)
+    if o is not None:
+        return o
     if q.shape[-1] <= 128:
         return lasp_fuse_parallel_(q, k, v, ed, KV, DKV)
     return run_sliced(q, k, v, ed, KV, DKV, True, True, True)

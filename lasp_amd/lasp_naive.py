@@ -6,8 +6,8 @@ runs the fused kernels, and the module-level launch shims keep the reference's s
 the chunk WITHOUT incoming state and hand back the chunk's own state contribution."""
 import torch
 
-from . import _abi
-from ._chain import ChunkFunction, run_sliced
+from . import _native
+from ._chain import ChunkFunction, native_chunk, run_sliced
 
 __all__ = ["LaspNaive", "lasp_naive_", "lasp_naive"]
 
@@ -20,7 +20,7 @@ def lasp_forward(q, k, v, s, kv):
     sum_j l^(n-j) k_j^T v_j, which the caller combines as KV <- l^n KV + kv (:565)."""
     kv32 = kv if kv.dtype == torch.float32 and kv.is_contiguous() else torch.empty(kv.shape, dtype=torch.float32,
                                                                                    device=kv.device)
-    o, _, _ = _abi.chunk_fwd(q, k, v, s, kv_in=None, kv_out=kv32)
+    o, _, _ = _native.chunk_fwd(q, k, v, s, kv_in=None, kv_out=kv32)
     if kv32 is not kv:
         kv.copy_(kv32)
     return o
@@ -33,7 +33,7 @@ def lasp_backward(q, k, v, s, do):
     (:489), which the caller combines as DKV <- l^n DKV + dkv (:614)."""
     b, h, _, d = q.shape
     dkv = torch.empty((b, h, d, v.shape[-1]), dtype=torch.float32, device=q.device)
-    dq, dk, dv = _abi.chunk_bwd(q, k, v, s, do, dkv_out=dkv)
+    dq, dk, dv = _native.chunk_bwd(q, k, v, s, do, dkv_out=dkv)
     return dq, dk, dv, None, dkv.to(q.dtype)
 
 
@@ -61,6 +61,11 @@ lasp_naive_ = LaspNaive.apply
 
 
 def lasp_naive(q, k, v, ed):
+    if q.is_cuda:
+        KV, DKV = _state_buffers(q, v)
+        o = native_chunk(q, k, v, ed, KV, DKV, False)
+        if o is not None:
+            return o
     if q.shape[-1] <= 128:
         return lasp_naive_(q, k, v, ed)
     KV, DKV = _state_buffers(q, v)

@@ -1,6 +1,7 @@
 """Single-device causal decayed linear attention (lasp/lightning_attention.py)."""
 import torch
 
+from . import _native
 from ._chain import ChunkFunction, run_sliced
 
 __all__ = ["LightningAttention", "lightning_attn_", "lightning_attn"]
@@ -29,7 +30,10 @@ lightning_attn_ = LightningAttention.apply
 
 def lightning_attn(q, k, v, ed):
     """q, k (b, h, n, d); v (b, h, n, e); ed: h slopes.  Returns (b, h, n, e) in q.dtype."""
-    d = q.shape[-1]
-    if d <= 128:
+    if q.is_cuda:
+        o = _native.ext().attention(q, k, v, ed)
+        if o is not None:
+            return o
+    if q.shape[-1] <= 128:
         return lightning_attn_(q, k, v, ed)
     return run_sliced(q, k, v, ed, None, None, True, False)

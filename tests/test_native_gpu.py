@@ -1,0 +1,96 @@
+"""The native autograd node (lasp_amd/csrc/lasp_torch.cpp) against the Python autograd Function over the same kernels: the
+same bits, graphs that can be kept or not, and the calls that it leaves to the Python path."""
+import pytest
+import torch
+
+import lasp_amd
+from lasp_amd._chain import ChunkFunction
+
+pytestmark = pytest.mark.gpu
+
+
+def _leaves(dev, b, h, n, d, e, dtype, seed=0):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    mk = lambda w: (torch.randn(b, h, n, w, generator=g, device=dev) / w ** 0.5).to(dtype)
+    return [mk(w).requires_grad_(True) for w in (d, d, e)], mk(e)
+
+
+@pytest.mark.parametrize("b,h,n,d,e,dtype", [(1, 2, 1, 128, 128, torch.bfloat16), (2, 3, 300, 64, 40, torch.float16),
+                                             (1, 4, 4096, 128, 128, torch.bfloat16), (1, 2, 777, 128, 128, torch.float32),
+                                             (1, 2, 500, 256, 128, torch.bfloat16)])
+def test_native_node_gives_the_bits_of_the_python_function(gpu_device, b, h, n, d, e, dtype):
+    (q, k, v), do = _leaves(gpu_device, b, h, n, d, e, dtype)
+    s = lasp_amd.build_slope_tensor(h).to(gpu_device)
+    o = lasp_amd.lightning_attn(q, k, v, s)
+    assert "LaspChunk" in o.grad_fn.name()
+    native = torch.autograd.grad(o, (q, k, v), do, retain_graph=True)
+    again = torch.autograd.grad(o, (q, k, v), do)
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(o, (q, k, v), do)
+    op = ChunkFunction.apply(q, k, v, s, None, None, True, False)
+    python = torch.autograd.grad(op, (q, k, v), do)
+    assert torch.equal(o, op)
+    for a, b_, c in zip(native, again, python):
+        assert torch.equal(a, c) and torch.equal(b_, c)
+    with torch.no_grad():
+        assert lasp_amd.lightning_attn(q, k, v, s).grad_fn is None
+
+
+def test_calls_that_stay_with_the_python_path(gpu_device):
+    """Non-contiguous inputs and expanded gradients run natively; slopes on the host and widths that need padding do not:
+    all give the values of the plain call."""
+    (q, k, v), do = _leaves(gpu_device, 1, 2, 200, 128, 128, torch.bfloat16)
+    s = lasp_amd.build_slope_tensor(2).to(gpu_device)
+    want = lasp_amd.lightning_attn(q, k, v, s)
+    strided = lasp_amd.lightning_attn(q.transpose(1, 2).contiguous().transpose(1, 2), k, v, s)
+    assert torch.equal(strided, want)
+    assert torch.equal(lasp_amd.lightning_attn(q, k, v, s.cpu()), want)
+    gs = torch.autograd.grad(want.float().sum(), (q, k, v))
+    gd = torch.autograd.grad(lasp_amd.lightning_attn(q, k, v, s), (q, k, v), torch.ones_like(want))
+    assert all(torch.equal(a, b) for a, b in zip(gs, gd))
+    (q, k, v), _ = _leaves(gpu_device, 1, 2, 100, 60, 36, torch.bfloat16)
+    assert lasp_amd.lightning_attn(q, k, v, s).shape == v.shape
+
+
+@pytest.mark.parametrize("name,rebind", [("lasp_fuse", False), ("lasp_fuse_parallel", True)])
+def test_native_chain_gives_the_bits_of_the_python_function(gpu_device, name, rebind):
+    results = []
+    s = lasp_amd.build_slope_tensor(4).to(gpu_device)
+    for native in (True, False):
+        lasp_amd.destroy_parallel_groups()
+        lasp_amd.initialize_lasp(1, 3)
+        try:
+            KV = torch.empty(1, 4, 128, 128, device=gpu_device)
+            DKV = torch.empty_like(KV)
+            outs, leaves, dos = [], [], []
+            for c in range(3):
+                lasp_amd.set_sequence_parallel_rank(c)
+                (q, k, v), do = _leaves(gpu_device, 1, 4, 1100, 128, 128, torch.bfloat16, seed=c)
+                if native:
+                    outs.append(getattr(lasp_amd, name)(q, k, v, s, KV, DKV))
+                else:
+                    outs.append(ChunkFunction.apply(q, k, v, s, KV, DKV, True, False, rebind))
+                dos.append(do)
+                leaves += [q, k, v]
+            assert ("LaspChunk" in outs[0].grad_fn.name()) == native
+            torch.autograd.backward(outs, dos)
+            assert not lasp_amd.loopback_pending()
+            results.append([*outs, *[t.grad for t in leaves], KV, DKV])
+        finally:
+            lasp_amd.destroy_parallel_groups()
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+def test_a_receive_without_a_sender_raises_from_the_backward(gpu_device):
+    """An error of the state exchange on autograd's thread arrives as the Python exception it is."""
+    lasp_amd.destroy_parallel_groups()
+    lasp_amd.initialize_lasp(1, 2)
+    try:
+        (q, k, v), do = _leaves(gpu_device, 1, 2, 64, 128, 128, torch.bfloat16)
+        KV = torch.empty(1, 2, 128, 128, device=gpu_device)
+        lasp_amd.set_sequence_parallel_rank(0)
+        o = lasp_amd.lasp_fuse(q, k, v, lasp_amd.build_slope_tensor(2).to(gpu_device), KV, torch.empty_like(KV))
+        with pytest.raises(RuntimeError, match="loopback recv"):
+            o.backward(do)
+    finally:
+        lasp_amd.destroy_parallel_groups()
