@@ -11,11 +11,15 @@
 //
 // "Usual case": contiguity aside, what the kernels take as it is -- device tensors of one type, fp32 with
 // d = e = 128 or 16 bits with widths that are multiples of 8, float32 slopes on the same device.  Everything else (padding, other
-// types, errors to report) stays with lasp_amd/_abi.py and lasp_amd/_chain.py: the functions below return None for it.
+// types, errors to report; tensor subclasses, function transforms, tracing and forward-mode differentiation, which a
+// node built here would not be seen by) stays with lasp_amd/_abi.py and lasp_amd/_chain.py: the functions below return
+// None for it.
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
@@ -57,8 +61,13 @@ int dtype_code(const Tensor &t) {
   }
 }
 
+// A tensor whose operations others follow through the dispatcher or a tangent: only the Python autograd Function is seen
+// by them (and refuses what it has no rule for).
+bool followed(const Tensor &t) { return at::isTensorSubclassLike(t) || t._fw_grad(0).defined(); }
+
 // The usual case, see above; fills `sh`.
 bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Shape &sh) {
+  if (torch::jit::tracer::isTracing() || followed(q) || followed(k) || followed(v) || followed(s)) return false;
   if (!q.is_cuda() || q.dim() != 4 || v.dim() != 4 || k.sizes() != q.sizes() || q.numel() == 0 || v.numel() == 0) return false;
   if (k.device() != q.device() || v.device() != q.device() || s.device() != q.device()) return false;
   if (k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type()) return false;
@@ -192,11 +201,12 @@ struct ChunkNode : public torch::autograd::Node {
 
   variable_list apply(variable_list &&grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
-    if (!grads[0].defined()) return variable_list(4);
     const Tensor q_ = q.unpack().contiguous(), k_ = k.unpack().contiguous(), v_ = v.unpack().contiguous(), s_ = s.unpack();
     const Tensor states_ = states.unpack(), kv_in_ = kv_in.unpack();
     at::AutoDispatchBelowADInplaceOrView below_autograd;
     c10::OptionalDeviceGuard guard(q_.device());
+    // no gradient for the output is one of zeros: a chunk of a chain still has its neighbours' states to pass on
+    const Tensor d_o = grads[0].defined() ? grads[0].contiguous() : at::zeros(v_.sizes(), v_.options());
     Tensor dkv_in, dkv_out;
     if (exchange.p) call_python([&] {
       pybind11::object r = pybind11::reinterpret_borrow<pybind11::object>(g_before)(
@@ -205,7 +215,7 @@ struct ChunkNode : public torch::autograd::Node {
       if (pair.first) dkv_in = *pair.first;
       if (pair.second) dkv_out = *pair.second;
     });
-    Backward r = run_backward(sh, q_, k_, v_, s_, grads[0].contiguous(), kv_in_, dkv_in, dkv_out, states_, seg_len);
+    Backward r = run_backward(sh, q_, k_, v_, s_, d_o, kv_in_, dkv_in, dkv_out, states_, seg_len);
     if (exchange.p) call_python([&] {
       pybind11::reinterpret_borrow<pybind11::object>(g_after)(pybind11::reinterpret_borrow<pybind11::object>(exchange.p),
                                                               dkv_out.defined() ? std::optional<Tensor>(dkv_out) : std::nullopt);

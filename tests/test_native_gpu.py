@@ -94,3 +94,59 @@ def test_a_receive_without_a_sender_raises_from_the_backward(gpu_device):
             o.backward(do)
     finally:
         lasp_amd.destroy_parallel_groups()
+
+
+class _NoGradient(torch.autograd.Function):
+    """x -> x whose backward has no gradient to give."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+def test_an_output_without_a_gradient_counts_as_one_of_zeros(gpu_device):
+    """Also in a chain, where the chunk still passes its neighbours' states on."""
+    (q, k, v), do = _leaves(gpu_device, 1, 2, 100, 128, 128, torch.bfloat16)
+    s = lasp_amd.build_slope_tensor(2).to(gpu_device)
+    _NoGradient.apply(lasp_amd.lightning_attn(q, k, v, s)).backward(do)
+    assert all(torch.equal(t.grad, torch.zeros_like(t)) for t in (q, k, v))
+    lasp_amd.destroy_parallel_groups()
+    lasp_amd.initialize_lasp(1, 2)
+    try:
+        grads = []
+        for silent in (True, False):
+            KV = torch.empty(1, 2, 128, 128, device=gpu_device)
+            DKV = torch.empty_like(KV)
+            outs, leaves, dos = [], [], []
+            for c in range(2):
+                lasp_amd.set_sequence_parallel_rank(c)
+                (q, k, v), do = _leaves(gpu_device, 1, 2, 100, 128, 128, torch.bfloat16, seed=c)
+                o = lasp_amd.lasp_fuse(q, k, v, s, KV, DKV)
+                outs.append(_NoGradient.apply(o) if silent and c == 1 else o)
+                dos.append(do if c == 0 else torch.zeros_like(do))
+                leaves += [q, k, v]
+            torch.autograd.backward(outs, dos)
+            assert not lasp_amd.loopback_pending()
+            grads.append([t.grad for t in leaves])
+        assert all(torch.equal(a, b) for a, b in zip(*grads))
+    finally:
+        lasp_amd.destroy_parallel_groups()
+
+
+def test_transforms_see_the_operator(gpu_device):
+    """Forward-mode differentiation and vmap, for which the operator has no rule, are refused; a traced call replays."""
+    (q, k, v), do = _leaves(gpu_device, 1, 2, 70, 128, 128, torch.bfloat16)
+    s = lasp_amd.build_slope_tensor(2).to(gpu_device)
+    import torch.autograd.forward_ad as fwad
+
+    with fwad.dual_level(), pytest.raises(RuntimeError):
+        lasp_amd.lightning_attn(fwad.make_dual(q.detach(), do), k, v, s)
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda x: lasp_amd.lightning_attn(x, k.detach(), v.detach(), s))(q.detach()[None])
+    traced = torch.jit.trace(lasp_amd.lightning_attn, (q, k, v, s), check_trace=False)
+    q2 = torch.randn_like(q)
+    assert torch.equal(traced(q2, k, v, s), lasp_amd.lightning_attn(q2, k, v, s))
