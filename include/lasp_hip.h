@@ -146,6 +146,16 @@ int lasp_chunk_fwd(const void *q, const void *k, const void *v, const float *s,
                    void *stream);
 
 /*
+ * A few tokens under their states, as a serving loop's step has them: lasp_chunk_fwd for n <= LASP_STEP_TOKENS, d <= 128
+ * and e a multiple of 4, any element type, in one launch that holds the states in registers.  No workspace, and no segment
+ * states left for a backward; kv_out may be the same buffer as kv_in.  Any other shape returns LASP_E_SHAPE.  (On
+ * LASP_PATH_MFMA_FUSED lasp_chunk_fwd runs the same kernel for such shapes.)
+ */
+#define LASP_STEP_TOKENS 4
+int lasp_step_fwd(const void *q, const void *k, const void *v, const float *s, const float *kv_in, float *kv_out,
+                  void *o, int b, int h, int64_t n, int d, int e, int dtype, void *stream);
+
+/*
  * lasp_chunk_fwd without a workspace argument.  No counterpart in the reference: it is
  * for callers that cannot allocate device memory around the call (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same computation and

@@ -28,10 +28,11 @@ def ext():
     return _ext
 
 
-def chunk_fwd(q, k, v, s, kv_in=None, kv_out=None):
-    """`_abi.chunk_fwd` under the default plan, natively where the extension takes the call."""
+def chunk_fwd(q, k, v, s, kv_in=None, kv_out=None, keep=True):
+    """`_abi.chunk_fwd` under the default plan, natively where the extension takes the call.  keep=False: the caller has
+    no use for the segment states, and None may be returned in their place."""
     if q.is_cuda:
-        done = ext().chunk_fwd(q, k, v, s, kv_in, kv_out, 0)
+        done = ext().chunk_fwd(q, k, v, s, kv_in, kv_out, 0, keep)
         if done is not None:
             return done
     return _abi.chunk_fwd(q, k, v, s, kv_in=kv_in, kv_out=kv_out)

@@ -14,7 +14,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "liblasp_hip.so")
 TORCH_LIB = os.path.join(HERE, "_lasp_torch.so")
-SOURCES = ["lasp_abi.hip", "lasp_generic.hip", "lasp_mfma.hip", "lasp_mfma_f16.hip", "lasp_mfma_f32.hip", "lasp_probe.hip"]
+SOURCES = ["lasp_abi.hip", "lasp_generic.hip", "lasp_mfma.hip", "lasp_mfma_f16.hip", "lasp_mfma_f32.hip", "lasp_probe.hip", "lasp_step.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -566,7 +566,9 @@ static int chunk_fwd_impl(const char *me, const void *q, const void *k, const vo
   (void)hipGetLastError();  // an earlier, unrelated error of this thread is not this call's
   FwdArgs a{q, k, v, s, kv_in, kv_out, o, seg_states};
   hipStream_t st = (hipStream_t)stream;
-  rc = mfma_eligible(g.dt, g.e, dtype)      ? mfma_fwd(a, g, dtype, st)
+  // (where a single launch leaves no segment states behind anyway, a few tokens take their own kernel)
+  rc = step_eligible(g) && (g.fused || !seg_states) ? step_fwd(a, g, dtype, st)
+       : mfma_eligible(g.dt, g.e, dtype)    ? mfma_fwd(a, g, dtype, st)
        : mfma_f32_eligible(g.d, g.e, dtype) ? mfma_f32_fwd(a, g, st)
                                             : generic_fwd(a, g, dtype, st);
   if (rc > 0) set_error("%s: HIP error %d: %s", me, rc, hipGetErrorString((hipError_t)rc));
@@ -589,6 +591,23 @@ int lasp_chunk_fwd(const void *q, const void *k, const void *v, const float *s, 
     return LASP_E_WORKSPACE;
   }
   return chunk_fwd_impl("lasp_chunk_fwd", q, k, v, s, kv_in, kv_out, o, seg_states, g, dtype, stream);
+}
+
+int lasp_step_fwd(const void *q, const void *k, const void *v, const float *s, const float *kv_in, float *kv_out, void *o,
+                  int b, int h, int64_t n, int d, int e, int dtype, void *stream) {
+  Geom g;
+  int rc = make_geom(b, h, n, d, e, dtype, 0, &g);
+  if (rc) return rc;
+  if (!step_eligible(g)) {
+    set_error("lasp_step_fwd: n=%lld d=%d e=%d (need n <= %d, d <= %d and e a multiple of 4)", (long long)n, d, e,
+              LASP_STEP_TOKENS, kMaxFeature);
+    return LASP_E_SHAPE;
+  }
+  if (!q || !k || !v || !s || !o) {
+    set_error("lasp_step_fwd: q, k, v, s and o must not be NULL");
+    return LASP_E_NULL;
+  }
+  return chunk_fwd_impl("lasp_step_fwd", q, k, v, s, kv_in, kv_out, o, nullptr, g, dtype, stream);
 }
 
 int lasp_chunk_fwd_static(const void *q, const void *k, const void *v, const float *s, const float *kv_in,

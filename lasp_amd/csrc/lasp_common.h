@@ -117,6 +117,10 @@ int mfma_f16_bwd(const BwdArgs &a, const Geom &g, hipStream_t st);
 int mfma_f32_fwd(const FwdArgs &a, const Geom &g, hipStream_t st);
 int mfma_f32_bwd(const BwdArgs &a, const Geom &g, hipStream_t st);
 
+// A few tokens under their states in one launch, without a workspace (n <= LASP_STEP_TOKENS).
+bool step_eligible(const Geom &g);
+int step_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st);
+
 // The decayed scan over segment states is shared by both kernel families.
 //   forward  (reverse = 0): states[seg] <- state entering segment seg from the
 //             left (segment 0: carry_in or 0); carry_out <- state after the chunk

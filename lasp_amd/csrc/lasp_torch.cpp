@@ -65,8 +65,11 @@ int dtype_code(const Tensor &t) {
 // by them (and refuses what it has no rule for).
 bool followed(const Tensor &t) { return at::isTensorSubclassLike(t) || t._fw_grad(0).defined(); }
 
-// The usual case, see above; fills `sh`.
-bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Shape &sh) {
+// What the library takes as a few tokens under their states, of any type and without a workspace.
+bool is_step(int64_t n, int64_t d, int64_t e) { return n <= LASP_STEP_TOKENS && d <= 128 && e <= 128 && e % 4 == 0; }
+
+// The usual case, see above; fills `sh`.  `keep`: the segment states are kept for a backward.
+bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Shape &sh, bool keep = true) {
   if (torch::jit::tracer::isTracing() || followed(q) || followed(k) || followed(v) || followed(s)) return false;
   if (!q.is_cuda() || q.dim() != 4 || v.dim() != 4 || k.sizes() != q.sizes() || q.numel() == 0 || v.numel() == 0) return false;
   if (k.device() != q.device() || v.device() != q.device() || s.device() != q.device()) return false;
@@ -77,7 +80,8 @@ bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s,
     return false;
   sh.dtype = dtype_code(q);
   const int64_t d = q.size(3), e = v.size(3);
-  if (sh.dtype == LASP_DTYPE_F32 ? d != 128 || e != 128 : sh.dtype < 0 || d % 8 || e % 8 || d > 1024 || e > 128) return false;
+  if (keep || sh.dtype < 0 || !is_step(q.size(2), d, e))
+    if (sh.dtype == LASP_DTYPE_F32 ? d != 128 || e != 128 : sh.dtype < 0 || d % 8 || e % 8 || d > 1024 || e > 128) return false;
   sh.b = (int)q.size(0);
   sh.h = (int)q.size(1);
   sh.n = q.size(2);
@@ -130,16 +134,23 @@ struct Forward {
 };
 // q, k, v contiguous
 Forward run_forward(const Shape &sh, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Tensor kv_in,
-                    const Tensor &kv_out, int seg_len) {
+                    const Tensor &kv_out, int seg_len, bool keep = true) {
+  const auto stream = [&] { return c10::hip::getCurrentHIPStream(q.device().index()).stream(); };
+  Forward f;
+  f.o = at::empty(v.sizes(), v.options());
+  if (!keep && seg_len == 0 && is_step(sh.n, sh.d, sh.e)) {
+    const int rc = lasp_step_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), (const float *)data(kv_in),
+                                 (float *)data(kv_out), f.o.data_ptr(), sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, stream());
+    if (rc) raise_lasp(rc, "lasp_step_fwd");
+    return f;
+  }
   const Plan p = plan_of(sh, seg_len);
   kv_in = private_incoming(kv_in, kv_out, sh, p.seg_len, false);
-  Forward f;
   f.seg_len = p.seg_len;
-  f.o = at::empty(v.sizes(), v.options());
   if (!p.fused && (p.n_seg > 1 || kv_in.defined() || kv_out.defined())) f.states = floats(p.bytes, q);
   const int rc = lasp_chunk_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), (const float *)data(kv_in),
                                 (float *)data(kv_out), f.o.data_ptr(), (float *)data(f.states), sh.b, sh.h, sh.n, sh.d, sh.e,
-                                sh.dtype, p.seg_len, c10::hip::getCurrentHIPStream(q.device().index()).stream());
+                                sh.dtype, p.seg_len, stream());
   if (rc) raise_lasp(rc, "lasp_chunk_fwd");
   return f;
 }
@@ -250,7 +261,7 @@ std::optional<Tensor> operator_call(const Tensor &q, const Tensor &k, const Tens
   Forward f;
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, kv_in, kv_out, 0);
+    f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, kv_in, kv_out, 0, grad);
   }
   if (grad) {
     std::shared_ptr<ChunkNode> node(new ChunkNode(), torch::autograd::deleteNode);
@@ -300,13 +311,13 @@ PYBIND11_MODULE(_lasp_torch, m) {
   });
   // _abi.chunk_fwd / chunk_bwd
   m.def("chunk_fwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
-                        const std::optional<Tensor> &kv_out, int seg_len) -> py::object {
+                        const std::optional<Tensor> &kv_out, int seg_len, bool keep) -> py::object {
     Shape sh;
     const Tensor in = or_none(kv_in), out = or_none(kv_out);
-    if (!regular(q, k, v, s, sh) || !state_ok(in, sh, q) || !state_ok(out, sh, q)) return py::none();
+    if (!regular(q, k, v, s, sh, keep) || !state_ok(in, sh, q) || !state_ok(out, sh, q)) return py::none();
     c10::OptionalDeviceGuard guard(q.device());
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    Forward f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, in, out, seg_len);
+    Forward f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, in, out, seg_len, keep);
     return py::make_tuple(f.o, f.states.defined() ? std::optional<Tensor>(f.states) : std::nullopt, f.seg_len);
   });
   m.def("chunk_bwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &d_o,

@@ -18,7 +18,7 @@ def lasp_forward(q, k, v, s, KV):
     Returns o for one chunk.  KV, float32 (b, h, d, e), holds the incoming state and
     is overwritten with the outgoing one, as the reference kernel does (:126-127).
     """
-    o, _, _ = _native.chunk_fwd(q, k, v, s, kv_in=KV, kv_out=KV)
+    o, _, _ = _native.chunk_fwd(q, k, v, s, kv_in=KV, kv_out=KV, keep=False)
     return o
 
 
