@@ -200,6 +200,22 @@ int lasp_chunk_bwd(const void *q, const void *k, const void *v, const float *s,
                    int dtype, int seg_len, void *stream);
 
 /*
+ * lasp_chunk_fwd / lasp_chunk_bwd that leave the outgoing state in two places: kv_out (dkv_out), which must then be
+ * wanted, and kv_twin (dkv_twin), a buffer of the same size that overlaps neither state of the call.  For a caller that
+ * keeps the state and hands a copy to the next chunk; NULL is the plain call.
+ */
+int lasp_chunk_fwd_twin(const void *q, const void *k, const void *v, const float *s,
+                        const float *kv_in, float *kv_out, float *kv_twin, void *o, float *seg_states,
+                        int b, int h, int64_t n, int d, int e, int dtype, int seg_len,
+                        void *stream);
+int lasp_chunk_bwd_twin(const void *q, const void *k, const void *v, const float *s,
+                        const void *d_o, const float *kv_in, const float *dkv_in,
+                        void *dq, void *dk, void *dv, float *dkv_out, float *dkv_twin,
+                        const float *kv_seg_states, float *workspace,
+                        size_t workspace_bytes, int b, int h, int64_t n, int d, int e,
+                        int dtype, int seg_len, void *stream);
+
+/*
  * Measurement hook (no counterpart in the reference, which times nothing).
  * Between lasp_profile_begin and lasp_profile_end every kernel the library
  * launches is bracketed by two hipEvents on its launch stream (at most

@@ -68,9 +68,17 @@ class Exchange:
         kv_in = spm.state_take(KV, self.prev_rank, self.group, tag=self.tag) if self.rank > 0 else None
         return kv_in, self._outgoing(KV, kv_in, self.rank < self.world - 1)
 
-    def after_forward(self, kv_out):
+    def twin(self, buffer, outgoing):
+        """A tensor for a second copy of the outgoing state, or None: where the caller keeps `outgoing` in its buffer and
+        the loopback would park a copy of it, the kernels write that copy beside the original."""
+        if outgoing is not buffer or not isinstance(self.group, spm.LoopbackGroup):
+            return None
+        return torch.empty_like(buffer)
+
+    def after_forward(self, kv_out, twin=None):
         if self.rank < self.world - 1:
-            spm.state_send(kv_out, self.next_rank, self.group, tag=self.tag, give=self.rebind)
+            spm.state_send(kv_out if twin is None else twin, self.next_rank, self.group, tag=self.tag,
+                           give=self.rebind or twin is not None)
 
 
 def before_backward(x: Exchange, DKV):
@@ -81,9 +89,16 @@ def before_backward(x: Exchange, DKV):
     return dkv_in, x._outgoing(DKV, dkv_in, x.rank > 0)
 
 
-def after_backward(x: Exchange, dkv_out):
+def after_backward(x: Exchange, dkv_out, twin=None):
     if x.rank > 0:
-        spm.state_send(dkv_out, x.prev_rank, x.group, src=x.rank, tag=x.tag, give=x.rebind)
+        spm.state_send(dkv_out if twin is None else twin, x.prev_rank, x.group, src=x.rank, tag=x.tag,
+                       give=x.rebind or twin is not None)
+
+
+def before_native_backward(x: Exchange, DKV):
+    """before_backward for the native node: the outgoing state's twin comes third (see Exchange.twin)."""
+    dkv_in, dkv_out = before_backward(x, DKV)
+    return dkv_in, dkv_out, x.twin(DKV, dkv_out) if x.rank > 0 else None
 
 
 class ChunkFunction(torch.autograd.Function):
@@ -146,8 +161,9 @@ def native_chunk(q, k, v, s, KV, DKV, barrier, rebind=False):
         return None
     x = Exchange(rebind)
     kv_in, kv_out = x.before_forward(KV, barrier)
-    o = ext.chunk(q, k, v, s, kv_in, kv_out, DKV, x)
-    x.after_forward(kv_out)
+    twin = x.twin(KV, kv_out) if x.rank < x.world - 1 else None
+    o = ext.chunk(q, k, v, s, kv_in, kv_out, twin, DKV, x)
+    x.after_forward(kv_out, twin)
     return o
 
 

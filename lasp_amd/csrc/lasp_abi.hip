@@ -339,6 +339,7 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
     if (pre <= kPreMaxSeg) g->pre_len = pre;
   }
   g->pre_n = (int)((n + g->pre_len - 1) / g->pre_len);
+  g->twin = nullptr;
   const bool padded_states = mfma_eligible(d, e, dtype) || mfma_f32_eligible(d, e, dtype);
   g->sd = mfma_eligible(d, e, dtype) ? width : padded_states ? kMaxFeature : d;
   g->se = mfma_eligible(d, e, dtype) ? width : padded_states ? kMaxFeature : e;
@@ -405,6 +406,25 @@ int check_alias(const char *call, const char *what, const float *in, const float
     return LASP_E_ALIAS;
   }
   return 0;
+}
+
+// A second place for the outgoing state: shares no byte with the states of the call.
+int check_twin(const char *call, const char *what, const float *in, const float *out, const float *twin, size_t bytes) {
+  if (!twin) return 0;
+  if (!out) {
+    set_error("%s: %s_twin without %s_out", call, what, what);
+    return LASP_E_NULL;
+  }
+  const uintptr_t t = (uintptr_t)twin;
+  for (const float *p : {in, out}) {
+    const uintptr_t a = (uintptr_t)p;
+    if (p && t < a + bytes && a < t + bytes) {
+      set_error("%s: %s_twin = %p overlaps %s_%s = %p", call, what, (const void *)twin, what, p == out ? "out" : "in",
+                (const void *)p);
+      return LASP_E_ALIAS;
+    }
+  }
+  return check_aligned(call, what, twin, 4);
 }
 
 // ---- segment-state scratch owned by the library (lasp_chunk_fwd_static) ------------------------
@@ -578,6 +598,12 @@ static int chunk_fwd_impl(const char *me, const void *q, const void *k, const vo
 int lasp_chunk_fwd(const void *q, const void *k, const void *v, const float *s, const float *kv_in,
                    float *kv_out, void *o, float *seg_states, int b, int h, int64_t n, int d, int e,
                    int dtype, int seg_len, void *stream) {
+  return lasp_chunk_fwd_twin(q, k, v, s, kv_in, kv_out, nullptr, o, seg_states, b, h, n, d, e, dtype, seg_len, stream);
+}
+
+int lasp_chunk_fwd_twin(const void *q, const void *k, const void *v, const float *s, const float *kv_in,
+                        float *kv_out, float *kv_twin, void *o, float *seg_states, int b, int h, int64_t n, int d, int e,
+                        int dtype, int seg_len, void *stream) {
   Geom g;
   int rc = make_geom(b, h, n, d, e, dtype, seg_len, &g);
   if (rc) return rc;
@@ -590,6 +616,8 @@ int lasp_chunk_fwd(const void *q, const void *k, const void *v, const float *s, 
               state_bytes_of(g), g.n_seg, (kv_in || kv_out) ? " with KV in/out" : "");
     return LASP_E_WORKSPACE;
   }
+  if ((rc = check_twin("lasp_chunk_fwd", "kv", kv_in, kv_out, kv_twin, sizeof(float) * (size_t)b * h * d * e))) return rc;
+  g.twin = kv_twin;
   return chunk_fwd_impl("lasp_chunk_fwd", q, k, v, s, kv_in, kv_out, o, seg_states, g, dtype, stream);
 }
 
@@ -638,6 +666,15 @@ int lasp_chunk_bwd(const void *q, const void *k, const void *v, const float *s, 
                    float *dkv_out, const float *kv_seg_states, float *workspace,
                    size_t workspace_bytes, int b, int h, int64_t n, int d, int e, int dtype,
                    int seg_len, void *stream) {
+  return lasp_chunk_bwd_twin(q, k, v, s, d_o, kv_in, dkv_in, dq, dk, dv, dkv_out, nullptr, kv_seg_states, workspace,
+                             workspace_bytes, b, h, n, d, e, dtype, seg_len, stream);
+}
+
+int lasp_chunk_bwd_twin(const void *q, const void *k, const void *v, const float *s, const void *d_o,
+                        const float *kv_in, const float *dkv_in, void *dq, void *dk, void *dv,
+                        float *dkv_out, float *dkv_twin, const float *kv_seg_states, float *workspace,
+                        size_t workspace_bytes, int b, int h, int64_t n, int d, int e, int dtype,
+                        int seg_len, void *stream) {
   Geom g;
   int rc = make_geom(b, h, n, d, e, dtype, seg_len, &g);
   if (rc) return rc;
@@ -656,6 +693,8 @@ int lasp_chunk_bwd(const void *q, const void *k, const void *v, const float *s, 
   }
   const char *me = "lasp_chunk_bwd";
   if ((rc = check_alias(me, "dkv", dkv_in, dkv_out, sizeof(float) * (size_t)b * h * d * e, g, true))) return rc;
+  if ((rc = check_twin(me, "dkv", dkv_in, dkv_out, dkv_twin, sizeof(float) * (size_t)b * h * d * e))) return rc;
+  g.twin = dkv_twin;
   if ((rc = check_aligned(me, "q", q, 16)) || (rc = check_aligned(me, "k", k, 16)) ||
       (rc = check_aligned(me, "v", v, 16)) || (rc = check_aligned(me, "do", d_o, 16)) ||
       (rc = check_aligned(me, "dq", dq, 16)) || (rc = check_aligned(me, "dk", dk, 16)) ||

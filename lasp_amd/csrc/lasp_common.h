@@ -66,6 +66,9 @@ struct Geom {
   int pre_len;  // tokens per segment of the pre-pass and the scan: seg_len, or seg_len / 2^k where long sweep
                 // segments are cut finer for the pre-pass (16-bit scan path only)
   int pre_n;    // ceil(n / pre_len): states per (b, h) in the workspace
+  float *twin;  // where an outgoing state is written a second time (NULL: nowhere): the copy that a caller keeping the state
+                // would hand on.  A copy of its own is a launch of 3.6 us for 24 states (4.6 for 16 beside long sweeps)
+                // and its host call; eight chained chunks of 2048 tokens, b*h = 24: 675 us, 651 without them
 };
 
 // Decay weights below 2^-kSkipLog2 are treated as zero by the 16-bit MFMA kernels.  A state is an fp32 sum

@@ -374,7 +374,11 @@ segment_scan_kernel(float *__restrict__ states, const float *carry_in, float *ca
       b.load(p + (int64_t)end * sde);
       const float f = end == g.n_seg - 1 ? tail : full;
 #pragma unroll
-      for (int w = 0; w < W; ++w) carry_out[cidx + w] = fmaf(f, a.v[w], b.v[w]);
+      for (int w = 0; w < W; ++w) {
+        const float out = fmaf(f, a.v[w], b.v[w]);
+        carry_out[cidx + w] = out;
+        if (g.twin) g.twin[cidx + w] = out;
+      }
     }
     // The incoming carry (read above, before the outgoing one was written: the two may be the same memory)
     // moves into the slot of the segment visited last, whose own state nothing reads from here on; the sweep
@@ -416,7 +420,10 @@ segment_scan_kernel(float *__restrict__ states, const float *carry_in, float *ca
   }
   if (carry_out && in_carry) {
 #pragma unroll
-    for (int w = 0; w < W; ++w) carry_out[cidx + w] = run.v[w];
+    for (int w = 0; w < W; ++w) {
+      carry_out[cidx + w] = run.v[w];
+      if (g.twin) g.twin[cidx + w] = run.v[w];
+    }
   }
 }
 

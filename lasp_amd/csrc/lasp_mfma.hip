@@ -737,14 +737,17 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   }
   // the segment visited last leaves the chunk's outgoing state
   if (SRC != SRC_SCANNED && !TRANS && carry_out != nullptr && sw.seg == (REV ? 0 : g.n_seg - 1) && ih == 0) {
-    float *cp = carry_out + (int64_t)sw.bh * g.dt * g.e;
+    float *cp = carry_out + (int64_t)sw.bh * g.dt * g.e, *tp = g.twin ? g.twin + (int64_t)sw.bh * g.dt * g.e : nullptr;
     const int col = 32 * wcol + c;
 #pragma unroll
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = 32 * T + 8 * (r >> 2) + 4 * hh + (r & 3);
-        if (!NARROW || (row < fa && col < fb)) cp[row * (NARROW ? fb : W) + col] = st[T][r];
+        if (!NARROW || (row < fa && col < fb)) {
+          cp[row * (NARROW ? fb : W) + col] = st[T][r];
+          if (tp) tp[row * (NARROW ? fb : W) + col] = st[T][r];
+        }
       }
   }
 }
@@ -1215,6 +1218,7 @@ Geom slice_geom(const Geom &g, int i) {
   Geom gs = g;
   gs.d = g.dt - i * kMaxWidth < kMaxWidth ? g.dt - i * kMaxWidth : kMaxWidth;
   gs.add = i > 0;
+  if (g.twin) gs.twin = g.twin + (int64_t)i * kMaxWidth * g.e;
   return gs;
 }
 const void *row_slice(const void *p, int i) { return (const elem16_t *)p + i * kMaxWidth; }

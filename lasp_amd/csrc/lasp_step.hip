@@ -95,7 +95,10 @@ la_step(const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ 
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int r = rg + RG * i;
-      if (r < d) *reinterpret_cast<f32x4u *>(kv_out + base + (int64_t)r * e) = st[i];
+      if (r < d) {
+        *reinterpret_cast<f32x4u *>(kv_out + base + (int64_t)r * e) = st[i];
+        if (g.twin) *reinterpret_cast<f32x4u *>(g.twin + base + (int64_t)r * e) = st[i];
+      }
     }
   }
   __syncthreads();

@@ -134,11 +134,11 @@ struct Forward {
 };
 // q, k, v contiguous
 Forward run_forward(const Shape &sh, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Tensor kv_in,
-                    const Tensor &kv_out, int seg_len, bool keep = true) {
+                    const Tensor &kv_out, const Tensor &kv_twin, int seg_len, bool keep = true) {
   const auto stream = [&] { return c10::hip::getCurrentHIPStream(q.device().index()).stream(); };
   Forward f;
   f.o = at::empty(v.sizes(), v.options());
-  if (!keep && seg_len == 0 && is_step(sh.n, sh.d, sh.e)) {
+  if (!keep && seg_len == 0 && !kv_twin.defined() && is_step(sh.n, sh.d, sh.e)) {
     const int rc = lasp_step_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), (const float *)data(kv_in),
                                  (float *)data(kv_out), f.o.data_ptr(), sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, stream());
     if (rc) raise_lasp(rc, "lasp_step_fwd");
@@ -148,9 +148,9 @@ Forward run_forward(const Shape &sh, const Tensor &q, const Tensor &k, const Ten
   kv_in = private_incoming(kv_in, kv_out, sh, p.seg_len, false);
   f.seg_len = p.seg_len;
   if (!p.fused && (p.n_seg > 1 || kv_in.defined() || kv_out.defined())) f.states = floats(p.bytes, q);
-  const int rc = lasp_chunk_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), (const float *)data(kv_in),
-                                (float *)data(kv_out), f.o.data_ptr(), (float *)data(f.states), sh.b, sh.h, sh.n, sh.d, sh.e,
-                                sh.dtype, p.seg_len, stream());
+  const int rc = lasp_chunk_fwd_twin(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(),
+                                     (const float *)data(kv_in), (float *)data(kv_out), (float *)data(kv_twin), f.o.data_ptr(),
+                                     (float *)data(f.states), sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, p.seg_len, stream());
   if (rc) raise_lasp(rc, "lasp_chunk_fwd");
   return f;
 }
@@ -160,7 +160,7 @@ struct Backward {
 };
 // q, k, v, d_o contiguous; `states` undefined: rebuilt
 Backward run_backward(const Shape &sh, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &d_o,
-                      const Tensor &kv_in, Tensor dkv_in, const Tensor &dkv_out, const Tensor &states, int seg_len) {
+                      const Tensor &kv_in, Tensor dkv_in, const Tensor &dkv_out, const Tensor &dkv_twin, const Tensor &states, int seg_len) {
   const Plan p = plan_of(sh, seg_len);
   dkv_in = private_incoming(dkv_in, dkv_out, sh, p.seg_len, true);
   Backward r;
@@ -172,18 +172,18 @@ Backward run_backward(const Shape &sh, const Tensor &q, const Tensor &k, const T
   const size_t bytes = p.bytes * ((need_dkv ? 1 : 0) + (need_kv ? 1 : 0));
   Tensor ws;
   if (bytes) ws = floats(bytes, q);
-  const int rc = lasp_chunk_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), d_o.data_ptr(),
+  const int rc = lasp_chunk_bwd_twin(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), d_o.data_ptr(),
                                 (const float *)data(kv_in), (const float *)data(dkv_in), r.dq.data_ptr(), r.dk.data_ptr(),
-                                r.dv.data_ptr(), (float *)data(dkv_out), p.fused ? nullptr : (const float *)data(states),
-                                (float *)data(ws), bytes, sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, p.seg_len,
-                                c10::hip::getCurrentHIPStream(q.device().index()).stream());
+                                r.dv.data_ptr(), (float *)data(dkv_out), (float *)data(dkv_twin),
+                                p.fused ? nullptr : (const float *)data(states), (float *)data(ws), bytes, sh.b, sh.h, sh.n,
+                                sh.d, sh.e, sh.dtype, p.seg_len, c10::hip::getCurrentHIPStream(q.device().index()).stream());
   if (rc) raise_lasp(rc, "lasp_chunk_bwd");
   return r;
 }
 
 // ---- autograd ----------------------------------------------------------------------------------------------
-// Python side of a chain's backward: before(exchange, DKV) -> (dkv_in or None, dkv_out or None) receives the state from
-// the next rank, after(exchange, dkv_out) sends the one that this chunk leaves.
+// Python side of a chain's backward: before(exchange, DKV) -> (dkv_in, dkv_out, dkv_twin), each may be None, receives the
+// state from the next rank; after(exchange, dkv_out, dkv_twin) sends the one that this chunk leaves.
 PyObject *g_before = nullptr, *g_after = nullptr;
 
 struct PyRef {  // a Python object held by a node, which any thread may drop
@@ -218,18 +218,20 @@ struct ChunkNode : public torch::autograd::Node {
     c10::OptionalDeviceGuard guard(q_.device());
     // no gradient for the output is one of zeros: a chunk of a chain still has its neighbours' states to pass on
     const Tensor d_o = grads[0].defined() ? grads[0].contiguous() : at::zeros(v_.sizes(), v_.options());
-    Tensor dkv_in, dkv_out;
+    Tensor dkv_in, dkv_out, dkv_twin;
     if (exchange.p) call_python([&] {
       pybind11::object r = pybind11::reinterpret_borrow<pybind11::object>(g_before)(
           pybind11::reinterpret_borrow<pybind11::object>(exchange.p), dkv_buffer);
-      auto pair = r.cast<std::pair<std::optional<Tensor>, std::optional<Tensor>>>();
-      if (pair.first) dkv_in = *pair.first;
-      if (pair.second) dkv_out = *pair.second;
+      auto states = r.cast<std::tuple<std::optional<Tensor>, std::optional<Tensor>, std::optional<Tensor>>>();
+      dkv_in = std::get<0>(states).value_or(Tensor());
+      dkv_out = std::get<1>(states).value_or(Tensor());
+      dkv_twin = std::get<2>(states).value_or(Tensor());
     });
-    Backward r = run_backward(sh, q_, k_, v_, s_, d_o, kv_in_, dkv_in, dkv_out, states_, seg_len);
+    Backward r = run_backward(sh, q_, k_, v_, s_, d_o, kv_in_, dkv_in, dkv_out, dkv_twin, states_, seg_len);
     if (exchange.p) call_python([&] {
+      const auto or_nothing = [](const Tensor &t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
       pybind11::reinterpret_borrow<pybind11::object>(g_after)(pybind11::reinterpret_borrow<pybind11::object>(exchange.p),
-                                                              dkv_out.defined() ? std::optional<Tensor>(dkv_out) : std::nullopt);
+                                                              or_nothing(dkv_out), or_nothing(dkv_twin));
     });
     variable_list out(4);
     out[0] = std::move(r.dq);
@@ -253,7 +255,7 @@ struct ChunkNode : public torch::autograd::Node {
 };
 
 std::optional<Tensor> operator_call(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &kv_in,
-                                    const Tensor &kv_out, const Tensor &dkv_buffer, PyObject *exchange) {
+                                    const Tensor &kv_out, const Tensor &kv_twin, const Tensor &dkv_buffer, PyObject *exchange) {
   Shape sh;
   if (!regular(q, k, v, s, sh)) return std::nullopt;
   const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() || s.requires_grad());
@@ -261,7 +263,7 @@ std::optional<Tensor> operator_call(const Tensor &q, const Tensor &k, const Tens
   Forward f;
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, kv_in, kv_out, 0, grad);
+    f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, kv_in, kv_out, kv_twin, 0, grad);
   }
   if (grad) {
     std::shared_ptr<ChunkNode> node(new ChunkNode(), torch::autograd::deleteNode);
@@ -297,7 +299,7 @@ PYBIND11_MODULE(_lasp_torch, m) {
   });
   // the stateless operator
   m.def("attention", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s) {
-    return operator_call(q, k, v, s, Tensor(), Tensor(), Tensor(), nullptr);
+    return operator_call(q, k, v, s, Tensor(), Tensor(), Tensor(), Tensor(), nullptr);
   });
   // whether a chain's chunk is a usual case (asked before its incoming state is received)
   m.def("takes", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &KV, const Tensor &DKV) {
@@ -306,8 +308,9 @@ PYBIND11_MODULE(_lasp_torch, m) {
   });
   // a chunk of a chain
   m.def("chunk", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
-                    const std::optional<Tensor> &kv_out, const Tensor &dkv_buffer, py::object exchange) {
-    return operator_call(q, k, v, s, or_none(kv_in), or_none(kv_out), dkv_buffer, exchange.ptr());
+                    const std::optional<Tensor> &kv_out, const std::optional<Tensor> &kv_twin, const Tensor &dkv_buffer,
+                    py::object exchange) {
+    return operator_call(q, k, v, s, or_none(kv_in), or_none(kv_out), or_none(kv_twin), dkv_buffer, exchange.ptr());
   });
   // _abi.chunk_fwd / chunk_bwd
   m.def("chunk_fwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
@@ -317,7 +320,7 @@ PYBIND11_MODULE(_lasp_torch, m) {
     if (!regular(q, k, v, s, sh, keep) || !state_ok(in, sh, q) || !state_ok(out, sh, q)) return py::none();
     c10::OptionalDeviceGuard guard(q.device());
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    Forward f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, in, out, seg_len, keep);
+    Forward f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, in, out, Tensor(), seg_len, keep);
     return py::make_tuple(f.o, f.states.defined() ? std::optional<Tensor>(f.states) : std::nullopt, f.seg_len);
   });
   m.def("chunk_bwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &d_o,
@@ -336,7 +339,7 @@ PYBIND11_MODULE(_lasp_torch, m) {
     }
     c10::OptionalDeviceGuard guard(q.device());
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    Backward r = run_backward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, d_o.contiguous(), in, din, dout, st, seg_len);
+    Backward r = run_backward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, d_o.contiguous(), in, din, dout, Tensor(), st, seg_len);
     return py::make_tuple(r.dq, r.dk, r.dv);
   });
 }

@@ -54,18 +54,30 @@ def test_calls_that_stay_with_the_python_path(gpu_device):
 
 @pytest.mark.parametrize("name,rebind", [("lasp_fuse", False), ("lasp_fuse_parallel", True)])
 def test_native_chain_gives_the_bits_of_the_python_function(gpu_device, name, rebind):
+    _compare_chains(gpu_device, name, rebind, 1100, 128, 128, torch.bfloat16)
+
+
+@pytest.mark.parametrize("n,d,e,dtype", [(3, 128, 128, torch.bfloat16), (200, 128, 128, torch.float16), (200, 64, 40, torch.bfloat16),
+                                         (4096, 128, 128, torch.bfloat16), (2500, 64, 64, torch.bfloat16),
+                                         (300, 128, 128, torch.float32)])
+def test_chain_on_every_kind_of_kernel_that_leaves_a_state(gpu_device, n, d, e, dtype):
+    """The copy of the outgoing state that the kernels write for the next rank, against the one that the Python path makes."""
+    _compare_chains(gpu_device, "lasp_fuse", False, n, d, e, dtype)
+
+
+def _compare_chains(gpu_device, name, rebind, n, d, e, dtype):
     results = []
     s = lasp_amd.build_slope_tensor(4).to(gpu_device)
     for native in (True, False):
         lasp_amd.destroy_parallel_groups()
         lasp_amd.initialize_lasp(1, 3)
         try:
-            KV = torch.empty(1, 4, 128, 128, device=gpu_device)
+            KV = torch.empty(1, 4, d, e, device=gpu_device)
             DKV = torch.empty_like(KV)
             outs, leaves, dos = [], [], []
             for c in range(3):
                 lasp_amd.set_sequence_parallel_rank(c)
-                (q, k, v), do = _leaves(gpu_device, 1, 4, 1100, 128, 128, torch.bfloat16, seed=c)
+                (q, k, v), do = _leaves(gpu_device, 1, 4, n, d, e, dtype, seed=c)
                 if native:
                     outs.append(getattr(lasp_amd, name)(q, k, v, s, KV, DKV))
                 else:
