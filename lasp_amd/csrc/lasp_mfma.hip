@@ -99,6 +99,10 @@ __device__ __forceinline__ gmem_ptr uniform_ptr(const char *p) {
   return (gmem_ptr)(((uint64_t)hi << 32) | lo);
 }
 
+// Left to itself the scheduler puts every LDS read right before the product that uses it, to save registers that these
+// kernels have to spare; each product then waits for a whole LDS round trip.  Nothing is moved across this line, so the reads
+// above it are in flight together.
+__device__ __forceinline__ void reads_first() { __builtin_amdgcn_sched_barrier(0); }
 __device__ __forceinline__ u32x4 lds16(const char *p) { return *reinterpret_cast<const u32x4 *>(p); }
 
 // element x (0..7) of a 16-byte group of 16-bit elements, widened to fp32
@@ -178,19 +182,21 @@ __device__ __forceinline__ void store_transposed(char *tile, const u32x4 (&rows)
   }
 }
 
-// A thread's two 8-byte pieces of the row that starts `row_bytes` (uniform across the workgroup) past
-// the block pointer `tile` (scalar, see uniform_ptr), at the thread's own byte offset `lane_off` (32 bits,
-// loop-invariant); a piece that lies beyond the row width, or the whole row, reads as zeros.
-struct PieceMask {
-  bool lo, hi;
-};
-__device__ __forceinline__ u32x4 load_row_pieces(gmem_ptr tile, int row_bytes, uint32_t lane_off, PieceMask ok,
-                                                 bool row_ok) {
-  typedef const __attribute__((address_space(1))) u32x2 *gmem_u32x2;
-  gmem_ptr p = tile + row_bytes;
-  const u32x2 zero = {0u, 0u};
-  const u32x2 lo = (row_ok && ok.lo) ? *reinterpret_cast<gmem_u32x2>(p + lane_off) : zero;
-  const u32x2 hi = (row_ok && ok.hi) ? *reinterpret_cast<gmem_u32x2>(p + lane_off + 16) : zero;
+// A block of token rows as a buffer that ends with them: a lane that addresses past the end -- a row that a partial block
+// does not have, a piece beyond a narrow row's width, a block beyond the walk's end -- reads zeros and stores nothing, with no
+// branch around the access.  (Branches would cost more than themselves: where the number of accesses in flight depends on
+// the path, a wait for the oldest of them has to wait for all, the stores and the loads just issued among them.)
+// Offsets are 32-bit and per lane; none is larger than 2 kOutside.
+constexpr uint32_t kOutside = 0x40000000u;
+typedef __amdgpu_buffer_rsrc_t rows_t;
+__device__ __forceinline__ rows_t rows_of(const void *p, int bytes) {
+  const gmem_ptr u = uniform_ptr(reinterpret_cast<const char *>(p));
+  return __builtin_amdgcn_make_buffer_rsrc((void *)(const char *)u, 0, bytes, 0x00020000);
+}
+// A thread's two 8-byte pieces of a row: 16 bytes apart, the second `hi_step` after the first
+__device__ __forceinline__ u32x4 load_row_pieces(rows_t rows, uint32_t lane_off, uint32_t hi_step) {
+  const u32x2 lo = __builtin_amdgcn_raw_buffer_load_b64(rows, (int)lane_off, 0, 0);
+  const u32x2 hi = __builtin_amdgcn_raw_buffer_load_b64(rows, (int)(lane_off + hi_step), 0, 0);
   u32x4 r;
   r.x = lo.x;
   r.y = lo.y;
@@ -198,15 +204,13 @@ __device__ __forceinline__ u32x4 load_row_pieces(gmem_ptr tile, int row_bytes, u
   r.w = hi.y;
   return r;
 }
-// thread-own part of the address: `row` rows down, then the thread's first piece
-__device__ __forceinline__ uint32_t lane_offset(const LoaderRole &role, int row, int units) {
-  return (uint32_t)((row * units + 4 * role.G + role.j) * 8);
+// where the thread's first piece lies in a block, `row` rows down (rows of `units` 8-byte units, of which `width` are read),
+// and how far its second piece is from it
+__device__ __forceinline__ uint32_t lane_offset(const LoaderRole &role, int row, int units, int width) {
+  return 4 * role.G + role.j < width ? (uint32_t)((row * units + 4 * role.G + role.j) * 8) : kOutside;
 }
-__device__ __forceinline__ PieceMask piece_mask(const LoaderRole &role, int units) {
-  PieceMask m;
-  m.lo = 4 * role.G + role.j < units;
-  m.hi = 4 * role.G + 2 + role.j < units;
-  return m;
+__device__ __forceinline__ uint32_t second_piece(const LoaderRole &role, int width) {
+  return 4 * role.G + 2 + role.j < width ? 16u : kOutside;
 }
 
 struct SegWork {
@@ -267,12 +271,21 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
 //     state term, intra-block term, state update, output staging.
 // The tiles are double-buffered (two sets of X, Y token-major and Y^T, Z^T feature-major, 144 384 B
 // with the score tile), and a block takes two barriers:
-//     feed: store O(t-1), score(t)    | math: state term(t)
+//     feed: store O(t-1), score(t),   | math: state term(t), state update(t)
+//           fill Y, Z(t+1),           |
+//           issue loads Y, Z(t+2)     |
 //   ---- barrier ----
-//     feed: fill(t+1),                | math: intra(t) from the score tile, state update(t), stage O(t) into
-//           issue loads(t+2)          |       the X tile of block t (no longer read)
+//     feed: fill X(t+1),              | math: intra(t) from the score tile, stage O(t) into the X tile of block t
+//           issue loads X(t+2)        |       (no longer read)
 //   ---- barrier ----
-// O(t-1) waits in the X tile of the set that fill(t+1) overwrites after the first barrier.
+// O(t-1) waits in the X tile of the set that the fill of X(t+1) overwrites after the first barrier; the set's other tiles
+// were last read before the second barrier of block t-1.
+// What bounds a block: with long chunks HBM; otherwise the LDS, which moves some 330 KB per block (every math wave reads
+// all of X and Y^T), and the round trips that nothing covers.  Against a form that updated the state after the first barrier,
+// filled all tiles there and read LDS operand by operand (forward + backward): b*h = 16, n = 65536: 773 us against 815;
+// b*h = 36, n = 5003: 170 against 184; d = e = 64, b*h = 64, n = 4096: 107 against 112; forward with a state, b*h = 16,
+// n = 2000: 25.3 against 26.2.  Half of that comes from loads and stores without branches (see rows_of): in the ragged
+// form each of the 24 loads of a block had been one of its own, and every fill waited for everything in flight.
 // Both groups run their own loop; each executes exactly 1 + 2 * nblk barriers.
 //
 // W = 64 keeps that split with a quarter of the state and half of every tile: 78 848 B of LDS and at most 128
@@ -314,7 +327,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   const int c = lane & 31, hh = lane >> 5;
 
   const SegWork sw = seg_work(g, item);
-  const float sl = S[sw.bh % g.h] * LOG2E;
+  const int head = sw.bh % g.h;
   const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
   // elements from row to row of X and Y, and of Z and Out: q, k and their gradients have rows of g.dt features, of which
   // a slice of a wide head reads and writes fa (fb)
@@ -322,7 +335,6 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   const int nblk = sw.nblk;
   const int step = REV ? -1 : 1;
   const int blk0 = REV ? nblk - 1 : 0;
-  const float blockdec = decay(sl, (float)BLK);
 
   // SRC_WALK: the state entering the segment is rebuilt by walking `runup` blocks outside it first (before it,
   // or after it going backwards), as far as the head's decay reaches, from the chunk's incoming state if the
@@ -342,6 +354,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   if (SRC == SRC_WALK) {
     const int avail = REV ? total_blk - (seg_blk0 + nblk) : seg_blk0;
     int reach = avail;
+    const float sl = S[head] * LOG2E;
     if (sl > 0.f) {
       const float x = SKIP_LOG2 / (sl * (float)BLK);  // blocks over which a weight falls to 2^-SKIP_LOG2
       if (x < (float)avail) reach = (int)x + 1;
@@ -361,60 +374,74 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     const bool zfeed = SPLIT && w8 >= 2;
     const LoaderRole xr = x_role<W>(ftid), yr = yz_role<W>(SPLIT ? ftid & 127 : ftid);
     const int chunk = ftid & (W / 8 - 1), rowq = ftid / (W / 8);
-    const u32x2 *Xg = reinterpret_cast<const u32x2 *>(X + row0 * xp);
-    const u32x2 *Yg = reinterpret_cast<const u32x2 *>(Y + row0 * xp);
-    const u32x2 *Zg = reinterpret_cast<const u32x2 *>(Z + row0 * zp);
-    u32x4 *Og = reinterpret_cast<u32x4 *>(Out + row0 * zp);
     const int xu = xp / 4, zu = zp / 4;  // 8-byte units from row to row
+    const int qI = w >> 1, qJ = w & 1;
+    const bool q_active = REV ? !(qI == 1 && qJ == 0) : !(qI == 0 && qJ == 1);
+    const int yu = zfeed ? zu : xu;      // SPLIT: of the tile that this wave fetches through ny
+    const int xw = NARROW ? fa / 4 : W / 4, zw = NARROW ? fb / 4 : W / 4, yw = zfeed ? zw : xw;  // 8-byte units read of a row
+    uint32_t x_off[XI], y_off[4], z_off[4];
+#pragma unroll
+    for (int it = 0; it < XI; ++it) x_off[it] = lane_offset(xr, xr.rowq + XROWS * it, xu, xw);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      y_off[r] = lane_offset(yr, 4 * yr.rowq + r, yu, yw);
+      z_off[r] = lane_offset(yr, 4 * yr.rowq + r, zu, zw);
+    }
+    const uint32_t x_hi = NARROW ? second_piece(xr, xw) : 16, y_hi = NARROW ? second_piece(yr, yw) : 16,
+                   z_hi = NARROW ? second_piece(yr, zw) : 16;
+    const elem16_t *Xg = X + row0 * xp, *Yg = zfeed ? Z + row0 * zp : Y + row0 * xp, *Zg = Z + row0 * zp;
+    elem16_t *Og = Out + row0 * zp;
+
+    // the block in flight, two 8-byte pieces per row (see LoaderRole); SPLIT: ny holds Y or Z
+    u32x4 nx[XI], ny[4], nz[4];
+    // block k of the run as a buffer; none of its rows where it is not `wanted`
+    auto rows = [&](const elem16_t *base, int k, int units, bool wanted) __attribute__((always_inline)) {
+      const int blk = first_blk + k * step;
+      return rows_of(base + (int64_t)blk * BLK * units * 4, wanted ? len_of(blk) * units * 8 : 0);
+    };
+    // Always the same number of loads (see rows_of); walk blocks (k < runup) need no X tile
+    auto issue_x = [&](int k) __attribute__((always_inline)) {
+      const rows_t x = rows(Xg, k, xu, k < run && (SRC != SRC_WALK || k >= runup));
+#pragma unroll
+      for (int it = 0; it < XI; ++it) nx[it] = load_row_pieces(x, x_off[it], x_hi);
+    };
+    auto issue_yz = [&](int k) __attribute__((always_inline)) {
+      const rows_t y = rows(Yg, k, yu, k < run), z = rows(Zg, k, zu, k < run);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        ny[r] = load_row_pieces(y, y_off[r], y_hi);
+        if (!SPLIT) nz[r] = load_row_pieces(z, z_off[r], z_hi);
+      }
+    };
+    // The slope comes as a lane's load in front of the first block's: as a scalar one, whose waits know no order, it would
+    // have to arrive before the first of these loads could leave.
+    int lane_head = head;
+    asm volatile("" : "+v"(lane_head));
+    const float slope = S[lane_head];
+    issue_yz(0);
+    issue_x(0);
+    __builtin_amdgcn_sched_barrier(0);
+    const float sl = slope * LOG2E;
     float kdec[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int b = 4 * yr.rowq + r;
       kdec[r] = decay(sl, REV ? (float)b : (float)(BLK - b));
     }
-    const int qI = w >> 1, qJ = w & 1;
-    const bool q_active = REV ? !(qI == 1 && qJ == 0) : !(qI == 0 && qJ == 1);
-    const int yu = zfeed ? zu : xu;      // SPLIT: of the tile that this wave fetches through ny
-    const uint32_t x_off = lane_offset(xr, xr.rowq, xu), y_off = lane_offset(yr, 4 * yr.rowq, yu),
-                   z_off = lane_offset(yr, 4 * yr.rowq, zu);
-    const PieceMask all = {true, true};
-    const PieceMask x_ok = piece_mask(xr, fa / 4), y_ok = piece_mask(yr, (zfeed ? fb : fa) / 4),
-                    z_ok = piece_mask(yr, fb / 4);
-
-    // the block in flight, two 8-byte pieces per row (see LoaderRole); SPLIT: ny holds Y or Z
-    u32x4 nx[XI], ny[4], nz[4];
-    // k: position in the run; walk blocks (k < runup) need no X tile
-    auto issue_loads = [&](int k) __attribute__((always_inline)) {
-      const int blk = first_blk + k * step;
-      const int len = len_of(blk);  // rows past a partial block's end and pieces past a narrow row's width read as zeros
-      const gmem_ptr xblk = uniform_ptr(reinterpret_cast<const char *>(Xg) + (int64_t)blk * BLK * xu * 8);
-      const gmem_ptr yblk = uniform_ptr(reinterpret_cast<const char *>(zfeed ? Zg : Yg) + (int64_t)blk * BLK * yu * 8);
-      const gmem_ptr zblk = uniform_ptr(reinterpret_cast<const char *>(Zg) + (int64_t)blk * BLK * zu * 8);
-      if (SRC != SRC_WALK || k >= runup) {
-#pragma unroll
-        for (int it = 0; it < XI; ++it)
-          nx[it] = load_row_pieces(xblk, XROWS * it * xu * 8, x_off, NARROW ? x_ok : all,
-                                   !RAGGED || xr.rowq + XROWS * it < len);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const bool row_ok = !RAGGED || 4 * yr.rowq + r < len;
-        ny[r] = load_row_pieces(yblk, r * yu * 8, y_off, NARROW ? y_ok : all, row_ok);
-        if (!SPLIT) nz[r] = load_row_pieces(zblk, r * zu * 8, z_off, NARROW ? z_ok : all, row_ok);
-      }
-    };
-    // writes the block held in nx / ny / nz into a tile set: token-major X and Y, feature-major Y (scaled by the
-    // key decay) and Z
-    auto fill = [&](char *set, int k) __attribute__((always_inline)) {
+    // writes the block held in nx / ny / nz into a tile set: token-major X ...
+    auto fill_x = [&](char *set, int k) __attribute__((always_inline)) {
       if (SRC != SRC_WALK || k >= runup) {  // a walk block is only multiplied into the state
 #pragma unroll
         for (int it = 0; it < XI; ++it)
           *reinterpret_cast<u32x4 *>(set + L::XN + (xr.rowq + XROWS * it) * L::LDN + (2 * xr.G + xr.j) * 16) = nx[it];
-        if (!zfeed) {
+      }
+    };
+    // ... token-major Y, and feature-major Y (scaled by the key decay) and Z
+    auto fill_yz = [&](char *set, int k) __attribute__((always_inline)) {
+      if ((SRC != SRC_WALK || k >= runup) && !zfeed) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            *reinterpret_cast<u32x4 *>(set + L::YN + (4 * yr.rowq + r) * L::LDN + (2 * yr.G + yr.j) * 16) = ny[r];
-        }
+        for (int r = 0; r < 4; ++r)
+          *reinterpret_cast<u32x4 *>(set + L::YN + (4 * yr.rowq + r) * L::LDN + (2 * yr.G + yr.j) * 16) = ny[r];
       }
       if (zfeed) {
         store_transposed<E, false>(set + L::ZT, ny, yr, kdec);
@@ -433,17 +460,18 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       }
       if (!SPLIT) store_transposed<E, false>(set + L::ZT, nz, yr, kdec);
     };
-    // the output tile staged in `set`'s X region -> global rows of block `blk`
-    auto store_out = [&](const char *set, int blk) __attribute__((always_inline)) {
-      const int64_t brow = (int64_t)blk * BLK;
-      const int len = len_of(blk);
+    // the output tile staged in `set`'s X region -> global rows of block k of the run
+    uint32_t o_off[XI];
 #pragma unroll
-      for (int r4 = 0; r4 < XI; ++r4) {
-        const int row = rowq + XROWS * r4;
-        if (!RAGGED || (row < len && (!NARROW || chunk < fb / 8)))
-          __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(set + L::XN + row * L::LDN + chunk * 16),
-                                      &Og[(brow + row) * (NARROW ? zp / 8 : W / 8) + chunk]);
-      }
+    for (int r4 = 0; r4 < XI; ++r4)
+      o_off[r4] = !NARROW || chunk < fb / 8 ? (uint32_t)(((rowq + XROWS * r4) * zu * 8) + chunk * 16) : kOutside;
+    auto store_out = [&](const char *set, int k, bool wanted) __attribute__((always_inline)) {
+      const rows_t out = rows(Og, k, zu, wanted);
+#pragma unroll
+      for (int r4 = 0; r4 < XI; ++r4)
+        __builtin_amdgcn_raw_buffer_store_b128(
+            *reinterpret_cast<const u32x4 *>(set + L::XN + (rowq + XROWS * r4) * L::LDN + chunk * 16), out, (int)o_off[r4], 0,
+            2 /* non-temporal */);
     };
     // this wave's quadrant of the transposed score tile: sc[4g+r] = y_b . x_a, b = 32qJ+8g+4hh+r, a = 32qI+c
     auto score = [&](const char *set) __attribute__((always_inline)) {
@@ -453,8 +481,15 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       for (int r = 0; r < 16; ++r) sc[r] = 0.f;
       const char *xa = set + L::XN + (32 * qI + c) * L::LDN + hh * 16;
       const char *ya = set + L::YN + (32 * qJ + c) * L::LDN + hh * 16;
+      u32x4 yf[W / 16], xf[W / 16];
 #pragma unroll
-      for (int ks = 0; ks < W / 16; ++ks) sc = E::mfma(lds16(ya + ks * 32), lds16(xa + ks * 32), sc);
+      for (int ks = 0; ks < W / 16; ++ks) {
+        yf[ks] = lds16(ya + ks * 32);
+        xf[ks] = lds16(xa + ks * 32);
+      }
+      reads_first();
+#pragma unroll
+      for (int ks = 0; ks < W / 16; ++ks) sc = E::mfma(yf[ks], xf[ks], sc);
       const int a = 32 * qI + c;
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
@@ -472,34 +507,40 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       }
     };
 
-    issue_loads(0);
-    fill(smem, 0);
-    if (run > 1) issue_loads(1);
+    fill_yz(smem, 0);
+    issue_yz(1);
+    fill_x(smem, 0);
+    issue_x(1);
     __syncthreads();  // barrier 0: block 0 of the run visible
     int k = 0;
     for (; k < runup; ++k) {  // walk: the math waves multiply block k into the state meanwhile
-      fill(smem + ((k + 1) & 1) * L::SET, k + 1);  // k + 1 < run: a sweep block follows the walk
-      if (k + 2 < run) issue_loads(k + 2);
+      char *nxt = smem + ((k + 1) & 1) * L::SET;  // k + 1 < run: a sweep block follows the walk
+      fill_yz(nxt, k + 1);
+      issue_yz(k + 2);
+      fill_x(nxt, k + 1);
+      issue_x(k + 2);
       __syncthreads();  // walk barrier k
     }
     for (; k < run; ++k) {
       char *cur = smem + (k & 1) * L::SET, *nxt = smem + ((k + 1) & 1) * L::SET;
-      // the stores go first: by the time the fill below waits for its loads (loads and stores share one
-      // counter, so that wait drains both) they have long left
-      if (k > runup) store_out(nxt, first_blk + (k - 1) * step);
+      // per block: 4 stores, 16 loads of Y and Z, 8 of X, in this order, so the waits of the fills leave what was issued
+      // after their own loads in flight
+      store_out(nxt, k - 1, k > runup);
       score(cur);
-      __syncthreads();  // first barrier of a sweep block: score tile complete; X / Y of `cur` and the output staged in `nxt` no longer read
-      if (k + 1 < run) {
-        fill(nxt, k + 1);
-        if (k + 2 < run) issue_loads(k + 2);
-      }
+      if (k + 1 < run) fill_yz(nxt, k + 1);
+      issue_yz(k + 2);
+      __syncthreads();  // first barrier of a sweep block: score tile complete; `cur` and the output staged in `nxt` no longer read
+      if (k + 1 < run) fill_x(nxt, k + 1);
+      issue_x(k + 2);
       __syncthreads();  // second barrier: next block visible; output of this block staged
     }
-    store_out(smem + ((run - 1) & 1) * L::SET, first_blk + (run - 1) * step);
+    store_out(smem + ((run - 1) & 1) * L::SET, run - 1, true);
     return;
   }
 
   // ================================== math waves ==================================
+  const float sl = S[head] * LOG2E;
+  const float blockdec = decay(sl, (float)BLK);
   float qdec[NI];
 #pragma unroll
   for (int I = 0; I < NI; ++I) {
@@ -558,7 +599,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       const int piece = REV ? min(sw.seg * sub + sub, g.pre_n) - 1 : sw.seg * sub;
       const float *src = states + ((int64_t)sw.bh * g.pre_n + piece) * (W * W);
       bool from_carry = false;
-      if (state_dies_in_segment(S[sw.bh % g.h], g)) {
+      if (state_dies_in_segment(S[head], g)) {
         const int nb = REV ? piece + 1 : piece - 1;
         if (nb < 0 || nb >= g.pre_n)
           from_carry = true;
@@ -609,6 +650,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int T = 0; T < TP; ++T) yf[u][T] = lds16(set + L::YT + tr_off(32 * (part * TP + T) + c, 2 * u + hh));
+      reads_first();
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -681,6 +723,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
           for (int I = 0; I < NI; ++I) xf[ks][I] = lds16(x0 + 32 * I * L::LDN + (part * KS + ks) * 32);
+        reads_first();
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
           const int T = (part * KS + ks) >> 1, u = ks & 1;
@@ -706,21 +749,28 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
           acc[I][r] += E::widen((r & 2) ? old[I][r >> 2].y : old[I][r >> 2].x, r & 1);
       if (it + 1 < nblk) fetch_old(blk0 + (it + 1) * step);
     }
-    __syncthreads();  // barrier 2 it + 1: score tile complete
+    u32x4 zf[4];
     if (wave_active) {
-      u32x4 zf[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) zf[u] = lds16(cur + L::ZT + tr_off(32 * wcol + c, 2 * u + hh));
+      update_state(cur, zf, bd);
+    }
+    __syncthreads();  // barrier 2 it + 1: score tile complete
+    if (wave_active) {
       // intra-block term: acc[I] += Z^T[32 wcol.., tokens] * score[a][tokens]
+      u32x4 sf[4][NI];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int I = 0; I < NI; ++I) sf[u][I] = lds16(smem + L::SC + (32 * (ih + I) + c) * LDSC + (16 * u + 8 * hh) * 2);
+      reads_first();
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int I = 0; I < NI; ++I) {
           const bool needed = REV ? (ih + I == 0 || u >= 2) : (ih + I == 1 || u < 2);
-          if (needed)
-            acc[I] = E::mfma(zf[u], lds16(smem + L::SC + (32 * (ih + I) + c) * LDSC + (16 * u + 8 * hh) * 2), acc[I]);
+          if (needed) acc[I] = E::mfma(zf[u], sf[u][I], acc[I]);
         }
-      update_state(cur, zf, bd);
     }
     // stage the output tile (token-major) in the X region of this block
     if (wave_active)
@@ -940,7 +990,7 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   states += (int64_t)slice * n_items * (W * W);
   const int yp = NARROW ? g.dt : W, zp = NARROW ? g.e : W;  // elements from row to row
   const int tw = NARROW ? (zgrp ? g.e : gd) : W;            // width of the tile this thread fetches
-  const char *Tg = reinterpret_cast<const char *>(zgrp ? Z + row0 * zp : Y + row0 * yp + slice * W);
+  const elem16_t *Tg = zgrp ? Z + row0 * zp : Y + row0 * yp + slice * W;
   const int row_bytes = (zgrp ? zp : yp) * 2;
 
   // row r of the thread's four: token row_of(r) of block half_of(r) of the step
@@ -980,26 +1030,22 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   // A partial block (the end of a ragged chunk) reads its missing rows as zeros; going
   // forwards it is the last block, and its tokens sit `len - b` (not 64 - b) before the
   // segment end.
-  const uint32_t t_off = (uint32_t)(rq * row_bytes + cq * 16);
-  const bool col_ok = !NARROW || cq * 8 < tw;  // chunks past the row width read as zeros
+  // the thread's four rows (see row_of); chunks past the row width read as zeros
+  uint32_t t_off[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) t_off[r] = !NARROW || cq * 8 < tw ? (uint32_t)(row_of(r) * row_bytes + cq * 16) : kOutside;
   const int first = REV ? hi : lo;
   const int step = REV ? -1 : 1;
   auto block_of = [&](int i) __attribute__((always_inline)) { return first + min(i, cnt - 1) * step; };
   auto len_of = [&](int blk) __attribute__((always_inline)) { return RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK; };
-  // every address is a workgroup-uniform block pointer plus one per-thread 32-bit offset
   auto issue_loads = [&](u32x4 (&nt)[4], int i) __attribute__((always_inline)) {
-    typedef const __attribute__((address_space(1))) u32x4 *gmem_u32x4;
-    const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int half = 0; half < BPS; ++half) {
       const int blk = block_of(BPS * i + half), len = len_of(blk);
-      const gmem_ptr tblk = uniform_ptr(Tg + (int64_t)blk * BLK * row_bytes);
+      const rows_t rows = rows_of(Tg + (int64_t)blk * BLK * (row_bytes / 2), len * row_bytes);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (half_of(r) != half) continue;
-        const bool ok = col_ok && (!RAGGED || row_of(r) < len);
-        nt[r] = ok ? *reinterpret_cast<gmem_u32x4>(tblk + (row_of(r) - rq) * row_bytes + t_off) : zero;
-      }
+      for (int r = 0; r < 4; ++r)
+        if (half_of(r) == half) nt[r] = __builtin_amdgcn_raw_buffer_load_b128(rows, (int)t_off[r], 0, 0);
     }
   };
   auto scaled = [&](const u32x4 &q, float w) __attribute__((always_inline)) {
