@@ -20,6 +20,8 @@
 // written while this one's second half runs, its transposed tiles while the next one's first half does, so no fill
 // stands between two barriers.  b*h = 24, n = 2048, forward + backward: 238 us against 275 (forward sweep 57 us against
 // 63, backward 131 against 149); b*h = 24, n = 16384: 1384 against 1555, 71 % of the time the fp32 products alone take.
+// Operands are read one step of products ahead, and nothing in a block branches (a masked quadrant of the scores, rows that
+// a partial block lacks): 231 us against 238 at b*h = 24, n = 2048.
 #include "lasp_common.h"
 
 namespace lasp {
@@ -27,6 +29,7 @@ namespace {
 
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int F = 128;
 constexpr int BLK = 32;
@@ -59,6 +62,22 @@ __device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
 __device__ __forceinline__ int tr_off(int f, int g16) {
   const int sw = ((f & 3) ^ ((f >> 3) & 3)) | (f & 4);
   return f * LDT + (((g16 ^ sw) & 7) << 4);
+}
+
+// Nothing is moved across this line: the reads above it are in flight while the products below run.  (The scheduler by itself
+// reads an operand right before the product that needs it.)
+__device__ __forceinline__ void reads_first() { __builtin_amdgcn_sched_barrier(0); }
+
+// A block of token rows as a buffer that ends with them: rows that a partial block does not have read as zeros and are not
+// stored, without a branch per access (after which a wait for the oldest access would have to wait for all of them).
+typedef __amdgpu_buffer_rsrc_t rows_t;
+__device__ __forceinline__ rows_t rows_of(const float *p, int count) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);  // the same for every lane
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc((void *)(((uint64_t)hi << 32) | lo), 0, count * F * 4, 0x00020000);
+}
+__device__ __forceinline__ f32x4 load16(rows_t rows, int off) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, off, 0, 0));
 }
 
 struct SegWork {
@@ -112,10 +131,6 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
   const SegWork sw = seg_work(g, item);
   const float sl = S[sw.bh % g.h] * LOG2E;
   const int64_t base = ((int64_t)sw.bh * g.n + sw.tok0) * F;
-  const f32x4 *Xg = reinterpret_cast<const f32x4 *>(X + base);
-  const f32x4 *Yg = reinterpret_cast<const f32x4 *>(Y + base);
-  const f32x4 *Zg = reinterpret_cast<const f32x4 *>(Z + base);
-  float *Og = Out + base;
 
   // ---- constants (all exponents <= 0)
   const float blockdec = decay(sl, (float)BLK);
@@ -148,20 +163,16 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
   }
 
   f32x4 nx[4], ny[4], nz[4];
+  auto len_of = [&](int blk) __attribute__((always_inline)) { return RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK; };
   auto issue_loads = [&](int blk) __attribute__((always_inline)) {
-    const int64_t off = (int64_t)blk * (BLK * F / 4);  // 16-byte units, 32 per row
-    const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const int64_t off = base + (int64_t)blk * (BLK * F);
+    const rows_t x = rows_of(X + off, len_of(blk)), y = rows_of(Y + off, len_of(blk)), z = rows_of(Z + off, len_of(blk));
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int row = rq + 8 * it;
-      nx[it] = (!RAGGED || row < len) ? Xg[off + row * 32 + cq] : zero;
-    }
+    for (int it = 0; it < 4; ++it) nx[it] = load16(x, (rq + 8 * it) * (F * 4) + cq * 16);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = 4 * rq + r;
-      ny[r] = (!RAGGED || row < len) ? Yg[off + row * 32 + cq] : zero;
-      nz[r] = (!RAGGED || row < len) ? Zg[off + row * 32 + cq] : zero;
+      ny[r] = load16(y, (4 * rq + r) * (F * 4) + cq * 16);
+      nz[r] = load16(z, (4 * rq + r) * (F * 4) + cq * 16);
     }
   };
   auto fill_rows = [&]() __attribute__((always_inline)) {  // X and Y as they are
@@ -178,7 +189,6 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
   };
   // this wave's quadrant of the score tile: tokens b = 16 qb .. of Y, a = 16 qa .. of X
   const int qb = w >> 1, qa = w & 1;
-  const bool q_active = REV ? !(qb == 0 && qa == 1) : !(qb == 1 && qa == 0);  // else wholly masked
   const int q_lane = lane & 15, q_grp = lane >> 4;
 
   const int first = REV ? sw.nblk - 1 : 0;
@@ -195,7 +205,7 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       fill_transposed();  // of this block; read after the first barrier
       if (more) issue_loads(blk + step);
     }
-    const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
+    const int len = len_of(blk);
     float qd = qdec, bd = blockdec;
     if (RAGGED && REV && len != BLK) {
       qd = decay(sl, (float)max(len - c, 0));
@@ -214,17 +224,27 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       const char *xp = smem + OFF_XN + c * LDN + hh * 16;
       const char *xq = smem + OFF_XN + (16 * qa + q_lane) * LDN + q_grp * 16;
       const char *yq = smem + OFF_YN + (16 * qb + q_lane) * LDN + q_grp * 16;
+      f32x4 ys[2], xs[2], x0[2], x1[2];
+      auto fetch = [&](int m) __attribute__((always_inline)) {  // features 16m + 4hh + .., 16m + 8 + 4hh + .. of X
+        x0[m & 1] = lds16(xp + m * 64);
+        x1[m & 1] = lds16(xp + m * 64 + 32);
+        ys[m & 1] = lds16(yq + m * 64);
+        xs[m & 1] = lds16(xq + m * 64);
+      };
+      fetch(0);
 #pragma unroll
       for (int m = 0; m < 8; ++m) {
-        const f32x4 ys = lds16(yq + m * 64), xs = lds16(xq + m * 64);
-        const f32x4 x0 = lds16(xp + m * 64), x1 = lds16(xp + m * 64 + 32);  // features 16m + 4hh + .., 16m + 8 + 4hh + ..
+        if (m < 7) fetch(m + 1);
+        reads_first();
+        // (the wave whose quadrant is wholly masked computes it as well: it would only wait for the others)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          acc = mfma(st[m >> 1][8 * (m & 1) + r], x0[r], acc);
-          if (q_active) sc = mfma16(ys[r], xs[r], sc);
+          acc = mfma(st[m >> 1][8 * (m & 1) + r], x0[m & 1][r], acc);
+          sc = mfma16(ys[m & 1][r], xs[m & 1][r], sc);
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc = mfma(st[m >> 1][8 * (m & 1) + 4 + r], x1[r], acc);
+        for (int r = 0; r < 4; ++r) acc = mfma(st[m >> 1][8 * (m & 1) + 4 + r], x1[m & 1][r], acc);
+        reads_first();
       }
     }
     // (2) mask the scores, scale the state term
@@ -249,33 +269,39 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       zf[gq] = lds16(smem + OFF_ZT + tr_off(32 * w + c, 2 * gq + hh));
       sf[gq] = lds16(smem + OFF_SC + c * LDSC + (8 * gq + 4 * hh) * 4);
     }
+    f32x4 yt[2][4];
+    auto fetch_y = [&](int T) __attribute__((always_inline)) {
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) yt[T & 1][gq] = lds16(smem + OFF_YT + tr_off(32 * T + c, 2 * gq + hh));
+    };
+    fetch_y(0);
+    reads_first();
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc = mfma(zf[gq][r], sf[gq][r], acc);
 #pragma unroll
     for (int T = 0; T < 4; ++T) {
+      if (T < 3) fetch_y(T + 1);
+      reads_first();
 #pragma unroll
       for (int r = 0; r < 16; ++r) st[T][r] *= bd;
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        const f32x4 yt = lds16(smem + OFF_YT + tr_off(32 * T + c, 2 * gq + hh));
+      for (int gq = 0; gq < 4; ++gq)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) st[T] = mfma(yt[r], zf[gq][r], st[T]);
-      }
+        for (int r = 0; r < 4; ++r) st[T] = mfma(yt[T & 1][gq][r], zf[gq][r], st[T]);
+      reads_first();
     }
     // (5) output: lane (c, hh) holds, for token c, four consecutive columns per g
-    if (!RAGGED || c < len) {
-      float *orow = Og + ((int64_t)blk * BLK + c) * F + 32 * w + 4 * hh;
+    const rows_t out = rows_of(Out + base + (int64_t)blk * (BLK * F), len);
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        f32x4 o;
-        o.x = acc[4 * gq + 0];
-        o.y = acc[4 * gq + 1];
-        o.z = acc[4 * gq + 2];
-        o.w = acc[4 * gq + 3];
-        *reinterpret_cast<f32x4 *>(orow + 8 * gq) = o;
-      }
+    for (int gq = 0; gq < 4; ++gq) {
+      f32x4 o;
+      o.x = acc[4 * gq + 0];
+      o.y = acc[4 * gq + 1];
+      o.z = acc[4 * gq + 2];
+      o.w = acc[4 * gq + 3];
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), out, c * (F * 4) + (32 * w + 4 * hh + 8 * gq) * 4, 0, 0);
     }
     if (more) __syncthreads();  // the next block's X and Y are complete; this block's transposed tiles are no longer read
   }
@@ -327,8 +353,6 @@ la32_seg_state(const float *__restrict__ Y, const float *__restrict__ Z, const f
   if (sw.seg == skip_seg) return;
   const float sl = S[sw.bh % g.h] * LOG2E;
   const int64_t base = ((int64_t)sw.bh * g.n + sw.tok0) * F;
-  const f32x4 *Yg = reinterpret_cast<const f32x4 *>(Y + base);
-  const f32x4 *Zg = reinterpret_cast<const f32x4 *>(Z + base);
 
   const float blockdec = decay(sl, (float)BLK);
   float kdec[4], ones[4];
@@ -346,14 +370,13 @@ la32_seg_state(const float *__restrict__ Y, const float *__restrict__ Z, const f
 
   f32x4 ny[4], nz[4];
   auto issue_loads = [&](int blk) __attribute__((always_inline)) {
-    const int64_t off = (int64_t)blk * (BLK * F / 4);
+    const int64_t off = base + (int64_t)blk * (BLK * F);
     const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const rows_t y = rows_of(Y + off, len), z = rows_of(Z + off, len);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = 4 * rq + r;
-      ny[r] = (!RAGGED || row < len) ? Yg[off + row * 32 + cq] : zero;
-      nz[r] = (!RAGGED || row < len) ? Zg[off + row * 32 + cq] : zero;
+      ny[r] = load16(y, (4 * rq + r) * (F * 4) + cq * 16);
+      nz[r] = load16(z, (4 * rq + r) * (F * 4) + cq * 16);
     }
   };
   // going forwards a partial block is the last one: its tokens sit `len - b` before the segment end
@@ -385,16 +408,23 @@ la32_seg_state(const float *__restrict__ Y, const float *__restrict__ Z, const f
     f32x4 zf[4];
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) zf[gq] = lds16(ztile + tr_off(32 * w + c, 2 * gq + hh));
+    f32x4 yt[2][4];
+    auto fetch_y = [&](int T) __attribute__((always_inline)) {
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) yt[T & 1][gq] = lds16(ytile + tr_off(32 * T + c, 2 * gq + hh));
+    };
+    fetch_y(0);
 #pragma unroll
     for (int T = 0; T < 4; ++T) {
+      if (T < 3) fetch_y(T + 1);
+      reads_first();
 #pragma unroll
       for (int r = 0; r < 16; ++r) st[T][r] *= bd;
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        const f32x4 yt = lds16(ytile + tr_off(32 * T + c, 2 * gq + hh));
+      for (int gq = 0; gq < 4; ++gq)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) st[T] = mfma(yt[r], zf[gq][r], st[T]);
-      }
+        for (int r = 0; r < 4; ++r) st[T] = mfma(yt[T & 1][gq][r], zf[gq][r], st[T]);
+      reads_first();
     }
     if (more) fill_lds((it + 1) & 1, blk + step);
     __syncthreads();
