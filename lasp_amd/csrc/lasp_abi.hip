@@ -340,6 +340,8 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   }
   g->pre_n = (int)((n + g->pre_len - 1) / g->pre_len);
   g->twin = nullptr;
+  g->by_seg = divisor_of((uint32_t)g->n_seg);
+  g->by_h = divisor_of((uint32_t)h);
   const bool padded_states = mfma_eligible(d, e, dtype) || mfma_f32_eligible(d, e, dtype);
   g->sd = mfma_eligible(d, e, dtype) ? width : padded_states ? kMaxFeature : d;
   g->se = mfma_eligible(d, e, dtype) ? width : padded_states ? kMaxFeature : e;

@@ -222,8 +222,7 @@ struct SegWork {
 // `item` enumerates (b*h, segment) pairs
 __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
   SegWork r;
-  // the division runs on the vector unit; its (uniform) result goes back to a scalar register
-  r.bh = __builtin_amdgcn_readfirstlane(item / g.n_seg);
+  r.bh = quotient(item, g.by_seg);
   r.seg = item - r.bh * g.n_seg;
   r.tok0 = (int64_t)r.seg * g.seg_len;
   int64_t t1 = r.tok0 + g.seg_len;
@@ -327,7 +326,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   const int c = lane & 31, hh = lane >> 5;
 
   const SegWork sw = seg_work(g, item);
-  const int head = sw.bh % g.h;
+  const int head = sw.bh - quotient(sw.bh, g.by_h) * g.h;
   const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
   // elements from row to row of X and Y, and of Z and Out: q, k and their gradients have rows of g.dt features, of which
   // a slice of a wide head reads and writes fa (fb)
@@ -558,9 +557,10 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   const bool wave_active = !NARROW || W == 64 || 32 * wcol < fb;  // (at W = 64 the skipping costs registers that two workgroups per CU do not have)
   constexpr int PARTS = NARROW ? 2 : 1;  // M_NARROW takes the lower and the upper features one after the other
   const bool upper_half = !NARROW || W == 64 || fa > W / 2;
-  // st <- f * st + M, M being the W x W fp32 tile whose element (row, col) is src[row * ld + col], or for a
+  // st <- f * st + M (`fresh`: st <- M, which leaves the loads in flight until a product needs them: the feed waves go on
+  // with the first block meanwhile), M being the W x W fp32 tile whose element (row, col) is src[row * ld + col], or for a
   // transposed role src[col * ld + row]; `bounded`: src holds only fa x fb (transposed: fb x fa) elements
-  auto add_state_ld = [&](const float *src, int ld, float f, bool bounded) __attribute__((always_inline)) {
+  auto add_state_ld = [&](const float *src, int ld, float f, bool bounded, bool fresh) __attribute__((always_inline)) {
     typedef const __attribute__((address_space(1))) float *gmem_f32;
     const uint32_t lane_off =
         (uint32_t)(TRANS ? (32 * wcol + c) * ld + 4 * hh : 4 * hh * ld + 32 * wcol + c) * (uint32_t)sizeof(float);
@@ -576,14 +576,16 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
           const bool ok = col_ok && (!bounded || band + 4 * hh + r < fa);
           const float own =
               ok ? *reinterpret_cast<gmem_f32>(bp + lane_off + (uint32_t)(TRANS ? r : r * ld) * sizeof(float)) : 0.f;
-          st[T][4 * gq + r] = fmaf(f, st[T][4 * gq + r], own);
+          st[T][4 * gq + r] = fresh ? own : fmaf(f, st[T][4 * gq + r], own);
         }
       }
   };
   // a state of the workspace (W x W, zero beyond fa x fb) / the chunk's incoming state (fa x fb, unpadded)
-  auto add_state = [&](const float *src, float f) __attribute__((always_inline)) { add_state_ld(src, W, f, false); };
+  auto add_state = [&](const float *src, float f, bool fresh = false) __attribute__((always_inline)) {
+    add_state_ld(src, W, f, false, fresh);
+  };
   auto add_carry = [&]() __attribute__((always_inline)) {
-    add_state_ld(carry_in + (int64_t)sw.bh * g.dt * g.e, NARROW ? (TRANS ? fa : fb) : W, 0.f, NARROW);
+    add_state_ld(carry_in + (int64_t)sw.bh * g.dt * g.e, NARROW ? (TRANS ? fa : fb) : W, 0.f, NARROW, true);
   };
   if (SRC == SRC_WALK) {
     if (take_carry) add_carry();
@@ -609,7 +611,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       // (for such a head the scan kernel has parked the chunk's incoming state in the slot of the piece it
       // visits last, so that nothing reads `carry_in`'s memory once the outgoing state may have replaced it)
       if (from_carry) src = states + ((int64_t)sw.bh * g.pre_n + (REV ? 0 : g.pre_n - 1)) * (W * W);
-      if (!from_carry || carry_in != nullptr) add_state(src, 0.f);
+      if (!from_carry || carry_in != nullptr) add_state(src, 0.f, true);
     }
   } else {
     // `states` holds the segments' OWN states.  The scan's recurrence, St <- l^len_j St + own_j over the
@@ -824,9 +826,9 @@ la_fused_fwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
                 elem16_t *__restrict__ O, Geom g) {
   extern __shared__ __align__(16) char smem[];
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int bh = (slot / g.n_seg) * 8 + xcd;
+  const int group = quotient(slot, g.by_seg), bh = group * 8 + xcd;
   if (bh >= g.b * g.h) return;
-  const int item = bh * g.n_seg + (g.n_seg - 1 - slot % g.n_seg);
+  const int item = bh * g.n_seg + (g.n_seg - 1 - (slot - group * g.n_seg));
   ws_body<E, false, false, SRC_WALK, MODE, W>(Q, K, V, S, nullptr, O, g, g.d, g.e, item, smem, kv_in, kv_out);
 }
 
@@ -839,11 +841,10 @@ la_fused_bwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
                 elem16_t *__restrict__ DK, elem16_t *__restrict__ DV, Geom g) {
   extern __shared__ __align__(16) char smem[];
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int per_bh = 3 * g.n_seg;
-  const int bh = (slot / per_bh) * 8 + xcd;
+  const int triple = slot / 3, role = slot - 3 * triple;
+  const int group = quotient(triple, g.by_seg), bh = group * 8 + xcd;
   if (bh >= g.b * g.h) return;
-  const int rem = slot % per_bh;
-  const int role = rem % 3, k = rem / 3;  // k-th longest walk of its role
+  const int k = triple - group * g.n_seg;  // k-th longest walk of its role
   if (role == 0)
     ws_body<E, false, true, SRC_WALK, MODE, W>(DO, V, K, S, nullptr, DQ, g, g.e, g.d, bh * g.n_seg + g.n_seg - 1 - k, smem,
                                             kv_in);
@@ -970,7 +971,7 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   const int n_items = g.b * g.h * g.n_seg;
   const SegWork sw = seg_work(g, n_items - 1 - (int)blockIdx.x);
   if (sw.seg == skip_seg) return;  // the scan's final segment feeds only the outgoing carry
-  const float slope = S[sw.bh % g.h];
+  const float slope = S[sw.bh - quotient(sw.bh, g.by_h) * g.h];
   // Where sweep segments span `sub` > 1 of these segments, a head that takes no part in the scan
   // (state_dies_in_segment) has readers for one state in `sub` only: a sweep reads the own state of the piece
   // next to its segment -- the last piece of the segment before it, or going backwards the first piece of the
@@ -1229,6 +1230,7 @@ Geom fused_bwd_geom(const Geom &g) {
     len = ((len + BLK - 1) / BLK) * BLK;
     gb.seg_len = (int)len;
     gb.n_seg = (int)((g.n + len - 1) / len);
+    gb.by_seg = divisor_of((uint32_t)gb.n_seg);
   }
   return gb;
 }
@@ -1253,6 +1255,7 @@ Geom pre_pass_geom(const Geom &g) {
   Geom gp = g;
   gp.seg_len = g.pre_len;
   gp.n_seg = g.pre_n;
+  gp.by_seg = divisor_of((uint32_t)gp.n_seg);
   return gp;
 }
 
