@@ -343,20 +343,20 @@ struct ScanVec {
 template <int W>
 __global__ void __launch_bounds__(256)
 segment_scan_kernel(float *__restrict__ states, const float *carry_in, float *carry_out,
-                    const float *__restrict__ S, Geom g, int reverse) {
-  const int64_t sde = (int64_t)g.sd * g.se;
-  const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * W;
+                    const float *__restrict__ S, Geom g, int reverse, Divisor by_per, Divisor by_se) {
+  // `per` workgroups to a state (the 64-bit divisions of a flat index had taken a tenth of a short launch)
+  const int sde = g.sd * g.se, per = (sde + 256 * W - 1) / (256 * W);
+  const int bh = quotient(blockIdx.x, by_per);
+  const int el = ((blockIdx.x - bh * per) * 256 + threadIdx.x) * W;
+  if (el >= sde) return;
   const int64_t total = (int64_t)g.b * g.h * sde;
-  if (idx >= total) return;
   const int slice = blockIdx.y;  // of a wide head: 128 of its g.dt rows, states in an array of their own
   const int d = min(g.d, g.dt - slice * kMaxWidth);
   states += (int64_t)slice * total * g.n_seg;
-  const int bh = (int)(idx / sde);
-  const int64_t el = idx - (int64_t)bh * sde;
-  const int row = (int)(el / g.se), col = (int)(el - (int64_t)row * g.se);
+  const int row = quotient(el, by_se), col = el - row * g.se;
   const bool in_carry = row < d && col < g.e;  // the padding of a stored state stays zero
   const int64_t cidx = ((int64_t)bh * g.dt + slice * kMaxWidth + row) * g.e + col;
-  const float s = S[bh % g.h];
+  const float s = S[bh - quotient(bh, g.by_h) * g.h];
   ScanVec<W> run;
 #pragma unroll
   for (int w = 0; w < W; ++w) run.v[w] = (carry_in && in_carry) ? carry_in[cidx + w] : 0.f;
@@ -502,15 +502,15 @@ int bwd_t(const BwdArgs &a, const Geom &g, hipStream_t st) {
 
 int launch_segment_scan(float *states, const float *carry_in, float *carry_out, const float *s,
                         const Geom &g, int reverse, hipStream_t st) {
-  const int64_t total = (int64_t)g.b * g.h * g.sd * g.se;
   const bool wide = g.se % 4 == 0 && g.e % 4 == 0 && (uintptr_t)states % 16 == 0;
-  const int64_t threads = wide ? total / 4 : total;
-  const dim3 grid((unsigned)((threads + 255) / 256), (unsigned)((g.dt + kMaxWidth - 1) / kMaxWidth));
+  const unsigned per_group = wide ? 1024 : 256, per = (unsigned)(g.sd * g.se + per_group - 1) / per_group;
+  const dim3 grid((unsigned)(g.b * g.h) * per, (unsigned)((g.dt + kMaxWidth - 1) / kMaxWidth));
+  const Divisor by_per = divisor_of(per), by_se = divisor_of((uint32_t)g.se);
   ProfScope prof(KC_SCAN, st);
   if (wide)
-    segment_scan_kernel<4><<<grid, 256, 0, st>>>(states, carry_in, carry_out, s, g, reverse);
+    segment_scan_kernel<4><<<grid, 256, 0, st>>>(states, carry_in, carry_out, s, g, reverse, by_per, by_se);
   else
-    segment_scan_kernel<1><<<grid, 256, 0, st>>>(states, carry_in, carry_out, s, g, reverse);
+    segment_scan_kernel<1><<<grid, 256, 0, st>>>(states, carry_in, carry_out, s, g, reverse, by_per, by_se);
   return (int)hipGetLastError();
 }
 

@@ -921,6 +921,9 @@ struct StateLds {
 // than it gains (320-token segments: 13.1 us against 12.4).  The shallow form stays within 128 registers, so two
 // workgroups share a CU; the deep one runs one per CU (squeezed into 128 registers it spills and measured slower).
 constexpr int STATE_DEPTH_LONG = 4, STATE_DEPTH_SHORT = 2;
+// Tokens per segment up to which every block is read, whatever the decay (forward with a state, b*h = 16, n = 2000, with the
+// scan's shorter start-up: 24.1 us against 24.7; eight chained chunks of 2048 tokens, b*h = 24: 624 against 631).
+constexpr int STATE_WHOLE = 512;
 constexpr int STATE_LONG_WALK = 1024;  // tokens per segment from which the deeper pipeline is used
 
 typedef short v4i16 __attribute__((ext_vector_type(4)));
@@ -971,7 +974,14 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   const int n_items = g.b * g.h * g.n_seg;
   const SegWork sw = seg_work(g, n_items - 1 - (int)blockIdx.x);
   if (sw.seg == skip_seg) return;  // the scan's final segment feeds only the outgoing carry
-  const float slope = S[sw.bh - quotient(sw.bh, g.by_h) * g.h];
+  // Short segments are walked whole: the few blocks that a fast-decaying head could leave out delay nobody, while the slope,
+  // which says which, would have to arrive before the first load can leave.
+  const bool whole = g.seg_len <= STATE_WHOLE;
+  const int head = sw.bh - quotient(sw.bh, g.by_h) * g.h;
+  int lane_head = head;
+  asm volatile("" : "+v"(lane_head));  // (a lane's load, waited for in order; see ws_body)
+  const float lane_slope = S[lane_head];
+  const float slope = whole ? 0.f : S[head];  // of the decisions which blocks to read
   // Where sweep segments span `sub` > 1 of these segments, a head that takes no part in the scan
   // (state_dies_in_segment) has readers for one state in `sub` only: a sweep reads the own state of the piece
   // next to its segment -- the last piece of the segment before it, or going backwards the first piece of the
@@ -983,7 +993,6 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
     if (skip_seg < 0) read = read || (REV ? p <= 1 : p >= g.n_seg - 2);
     if (!read) return;
   }
-  const float sl = slope * LOG2E;
   const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
   // the feature slice of a wide head (blockIdx.y; rows of Y are g.dt features apart) and its width
   const int slice = NARROW && W == 128 ? (int)blockIdx.y : 0;
@@ -997,15 +1006,13 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   // row r of the thread's four: token row_of(r) of block half_of(r) of the step
   auto half_of = [](int r) { return BPS == 1 ? 0 : r >> 1; };
   auto row_of = [&](int r) __attribute__((always_inline)) { return rq + ROWS * (BPS == 1 ? r : r & 1); };
-  const float blockdec = decay(sl, (float)BLK);
-  float kdec[4 / BPS];
-#pragma unroll
-  for (int r = 0; r < 4 / BPS; ++r) kdec[r] = decay(sl, REV ? (float)row_of(r) : (float)(BLK - row_of(r)));
+  u32x4 set[D][4];  // blocks in flight
+  float sl, blockdec, kdec[4 / BPS];  // (set once the first loads are on their way)
 
   // blocks lo..hi of the segment are processed (uniform across the workgroup)
   int lo = 0, hi = sw.nblk - 1;
-  if (sl > 0.f) {
-    const float keep = SKIP_LOG2 / sl;  // tokens whose weight is at least 2^-SKIP_LOG2
+  if (slope > 0.f) {
+    const float keep = SKIP_LOG2 / (slope * LOG2E);  // tokens whose weight is at least 2^-SKIP_LOG2
     if (!REV) {
       // the last token of block t lies (tokens - 64 t - 63) tokens before the segment end
       const float x = ((float)((sw.nblk - 1) * BLK + sw.tail) - 63.f - keep) * (1.f / BLK);
@@ -1109,9 +1116,13 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   // past the end of the walk are not skipped but repeat its last block (served by the cache, never
   // used): with the same number of loads in flight on every path, the wait before a fill covers
   // exactly the oldest register set.
-  u32x4 set[D][4];
 #pragma unroll
   for (int k = 0; k < D; ++k) issue_loads(set[k], k);
+  __builtin_amdgcn_sched_barrier(0);
+  sl = lane_slope * LOG2E;
+  blockdec = decay(sl, (float)BLK);
+#pragma unroll
+  for (int r = 0; r < 4 / BPS; ++r) kdec[r] = decay(sl, REV ? (float)row_of(r) : (float)(BLK - row_of(r)));
   fill_lds(0, set[0], 0);
   issue_loads(set[0], D);
   __syncthreads();
