@@ -832,17 +832,31 @@ la_fused_fwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
   ws_body<E, false, false, SRC_WALK, MODE, W>(Q, K, V, S, nullptr, O, g, g.d, g.e, item, smem, kv_in, kv_out);
 }
 
+// The (b, h) from bh0 on are cut into segments of their own (n_seg of seg_len tokens): see launch_fused_bwd.
+struct Fine {
+  int bh0, seg_len, n_seg;
+  Divisor by_seg;
+};
+
 // roles as in la_bwd3 (the dV role leaves dKV_out); all roles and segments of one (b, h) on one XCD
 template <class E, int MODE, int W>
 __global__ void __launch_bounds__(WS_THREADS, ws_waves_per_simd(W))
 la_fused_bwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const elem16_t *__restrict__ V,
                 const elem16_t *__restrict__ DO, const float *__restrict__ S, const float *__restrict__ kv_in,
                 const float *__restrict__ dkv_in, float *__restrict__ dkv_out, elem16_t *__restrict__ DQ,
-                elem16_t *__restrict__ DK, elem16_t *__restrict__ DV, Geom g) {
+                elem16_t *__restrict__ DK, elem16_t *__restrict__ DV, Geom g, Fine fine) {
   extern __shared__ __align__(16) char smem[];
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int before = 3 * fine.bh0 * g.n_seg;  // workgroups of the (b, h) before bh0, a multiple of 8
+  const bool cut = (int)blockIdx.x >= before;
+  if (cut) {
+    g.seg_len = fine.seg_len;
+    g.n_seg = fine.n_seg;
+    g.by_seg = fine.by_seg;
+  }
+  const int local = (int)blockIdx.x - (cut ? before : 0);
+  const int xcd = local & 7, slot = local >> 3;
   const int triple = slot / 3, role = slot - 3 * triple;
-  const int group = quotient(triple, g.by_seg), bh = group * 8 + xcd;
+  const int group = quotient(triple, g.by_seg), bh = (cut ? fine.bh0 : 0) + group * 8 + xcd;
   if (bh >= g.b * g.h) return;
   const int k = triple - group * g.n_seg;  // k-th longest walk of its role
   if (role == 0)
@@ -1246,17 +1260,41 @@ Geom fused_bwd_geom(const Geom &g) {
   return gb;
 }
 
+// Where whole chunks fill more than one round of the chip, the workgroups of the last, partly filled round would take as
+// long as a full one.  Their (b, h) are cut into as many segments as fill it instead: walks over the blocks before a segment
+// cost less than half of sweeping them.  Backward kernel, d = e = 128, bf16, before and now: n = 512, b*h = 88: 37.8 and
+// 28.5 us, 96: 38.9 and 33.4, 120 (two segments only): 39.2 and 37.7, 172: 58.5 and 51.6; n = 1024, b*h = 96: 71.3 and 56.1, 120:
+// 73.6 and 74.4; d = e = 64, b*h = 192, n = 1024: 53.7 and 50.0.
+Fine fused_bwd_tail(const Geom &g) {
+  const int64_t bh = (int64_t)g.b * g.h, slots = g.width == 64 ? 512 : 256;
+  Fine f = {(int)((bh + 7) / 8 * 8), g.seg_len, g.n_seg, g.by_seg};  // nothing is cut
+  if (g.n_seg > 1 || 3 * bh <= slots) return f;
+  const int64_t bh0 = 3 * bh / slots * slots / 24 * 8;  // whole rounds of whole groups of 8
+  const int64_t rest = (bh - bh0 + 7) / 8 * 8, room = slots + (3 * bh / slots * slots - 3 * bh0);
+  const int64_t nblk = (g.n + BLK - 1) / BLK;
+  int64_t n_seg = rest > 0 ? room / (3 * rest) : 1;
+  if (n_seg > nblk) n_seg = nblk;
+  if (n_seg < 2) return f;
+  f.bh0 = (int)bh0;
+  f.seg_len = (int)((nblk + n_seg - 1) / n_seg) * BLK;
+  f.n_seg = (int)((g.n + f.seg_len - 1) / f.seg_len);
+  f.by_seg = divisor_of((uint32_t)f.n_seg);
+  return f;
+}
+
 template <class E, int MODE, int W>
 int launch_fused_bwd(const BwdArgs &a, const Geom &g_fwd, hipStream_t st) {
   int rc = grant_lds<la_fused_bwd<E, MODE, W>>(WsLds<W>::BYTES);
   if (rc) return rc;
   const Geom g = fused_bwd_geom(g_fwd);
-  const unsigned grid = (unsigned)((((int64_t)g.b * g.h + 7) / 8) * 8 * 3 * g.n_seg);
+  const Fine fine = fused_bwd_tail(g);
+  const int64_t tail8 = ((int64_t)g.b * g.h - fine.bh0 + 7) / 8 * 8;
+  const unsigned grid = (unsigned)(3 * ((int64_t)fine.bh0 * g.n_seg + tail8 * fine.n_seg));
   ProfScope prof(KC_FUSED, st);
   la_fused_bwd<E, MODE, W><<<grid, WS_THREADS, WsLds<W>::BYTES, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
                                                          (const elem16_t *)a.v, (const elem16_t *)a.d_o, a.s,
                                                          a.kv_in, a.dkv_in, a.dkv_out, (elem16_t *)a.dq,
-                                                         (elem16_t *)a.dk, (elem16_t *)a.dv, g);
+                                                         (elem16_t *)a.dk, (elem16_t *)a.dv, g, fine);
   return (int)hipGetLastError();
 }
 

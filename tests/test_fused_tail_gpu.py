@@ -1,0 +1,33 @@
+"""Short chunks whose (b, h) fill more than one round of the chip in the backward: the (b, h) of the last, partly filled round
+are cut into segments, the others run whole.  Every (b, h) against the oracle in 64 bits."""
+import pytest
+import torch
+
+import lasp_amd
+from oracle import lasp_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# one rounding of an input-sized operand per product and one of the result: 2^-9 (bf16), 2^-12 (fp16), a few of them
+REL = {torch.bfloat16: 1.2e-2, torch.float16: 1.6e-3}
+
+
+@pytest.mark.parametrize("b,h,n,d,e,dtype", [
+    (8, 12, 512, 128, 128, torch.float16),   # 80 whole, 16 in 4 segments
+    (1, 86, 300, 128, 128, torch.bfloat16),  # one group of 8 (two of them missing) in segments of one block, the last partial
+    (5, 24, 130, 128, 128, torch.bfloat16),  # 40 in 2 segments, the second with one block of 2 tokens
+    (4, 43, 128, 96, 40, torch.bfloat16),    # two whole rounds, narrow rows
+    (2, 90, 200, 64, 64, torch.bfloat16),    # the 64-wide kernels: 512 workgroups to a round
+])
+def test_every_head_of_a_cut_last_round(gpu_device, b, h, n, d, e, dtype):
+    g = torch.Generator().manual_seed(b * h + n)
+    mk = lambda w: (torch.randn(b, h, n, w, generator=g) / w ** 0.5).to(dtype)
+    q, k, v, do = mk(d), mk(d), mk(e), mk(e)
+    s = torch.rand(h, 1, 1, generator=g) * 0.1  # walks of every length, and none that is always short
+    ref = O.ref_chunked(q, k, v, s, do, dtype=torch.float64)
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in (q, k, v)]
+    lasp_amd.lightning_attn(*leaves, s.to(gpu_device)).backward(do.to(gpu_device))
+    for t, name in zip(leaves, ("dq", "dk", "dv")):
+        diff, want = t.grad.double().cpu() - ref[name], ref[name]
+        rel = diff.flatten(2).norm(dim=2) / want.flatten(2).norm(dim=2)
+        assert float(rel.max()) < REL[dtype], (name, float(rel.max()), int(rel.argmax()))
