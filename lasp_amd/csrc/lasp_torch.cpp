@@ -25,6 +25,8 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <sstream>
+
 #include "lasp_hip.h"
 
 namespace {
@@ -36,14 +38,16 @@ using torch::autograd::variable_list;
 // ---- errors ------------------------------------------------------------------------------------------------
 PyObject *g_error = nullptr;  // lasp_amd._abi.LaspError
 
-// A library error as the Python exception LaspError, from whatever thread autograd runs this on.
-[[noreturn]] void raise_lasp(int rc, const char *what) {
-  const std::string msg = std::string(what) + " failed (code " + std::to_string(rc) + "): " + lasp_last_error();
+// The Python exception LaspError, from whatever thread autograd runs this on.
+[[noreturn]] void raise_lasp(const std::string &msg) {
   pybind11::gil_scoped_acquire gil;
   PyErr_SetString(g_error ? g_error : PyExc_RuntimeError, msg.c_str());
   python_error err;
   err.persist();
   throw err;
+}
+[[noreturn]] void raise_lasp(int rc, const char *what) {
+  raise_lasp(std::string(what) + " failed (code " + std::to_string(rc) + "): " + lasp_last_error());
 }
 
 // ---- shapes ------------------------------------------------------------------------------------------------
@@ -93,6 +97,16 @@ bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s,
 bool state_ok(const Tensor &t, const Shape &sh, const Tensor &q) {
   return !t.defined() || (t.scalar_type() == at::kFloat && t.device() == q.device() && t.is_contiguous() && t.dim() == 4 &&
                           t.size(0) == sh.b && t.size(1) == sh.h && t.size(2) == sh.d && t.size(3) == sh.e);
+}
+
+// A state that comes out of the exchange is whatever another chunk of the chain left there: the kernels may read (b, h, d, e)
+// floats only where there are as many.
+void check_state(const char *name, const Tensor &t, const Shape &sh, const Tensor &q) {
+  if (state_ok(t, sh, q)) return;
+  std::ostringstream msg;
+  msg << name << " must be a contiguous float32 tensor of shape (" << sh.b << ", " << sh.h << ", " << sh.d << ", " << sh.e
+      << ") on " << q.device() << ", got " << t.scalar_type() << " " << t.sizes() << " on " << t.device();
+  raise_lasp(msg.str());
 }
 
 void *data(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
@@ -227,6 +241,9 @@ struct ChunkNode : public torch::autograd::Node {
       dkv_out = std::get<1>(states).value_or(Tensor());
       dkv_twin = std::get<2>(states).value_or(Tensor());
     });
+    check_state("dkv_in", dkv_in, sh, q_);
+    check_state("dkv_out", dkv_out, sh, q_);
+    check_state("dkv_twin", dkv_twin, sh, q_);
     Backward r = run_backward(sh, q_, k_, v_, s_, d_o, kv_in_, dkv_in, dkv_out, dkv_twin, states_, seg_len);
     if (exchange.p) call_python([&] {
       const auto or_nothing = [](const Tensor &t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
@@ -258,6 +275,9 @@ std::optional<Tensor> operator_call(const Tensor &q, const Tensor &k, const Tens
                                     const Tensor &kv_out, const Tensor &kv_twin, const Tensor &dkv_buffer, PyObject *exchange) {
   Shape sh;
   if (!regular(q, k, v, s, sh)) return std::nullopt;
+  check_state("kv_in", kv_in, sh, q);
+  check_state("kv_out", kv_out, sh, q);
+  check_state("kv_twin", kv_twin, sh, q);
   const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() || s.requires_grad());
   c10::OptionalDeviceGuard guard(q.device());
   Forward f;

@@ -108,6 +108,35 @@ def test_a_receive_without_a_sender_raises_from_the_backward(gpu_device):
         lasp_amd.destroy_parallel_groups()
 
 
+def test_a_state_of_another_shape_is_refused(gpu_device):
+    """A received state is read as (b, h, d, e) floats: one that another chunk left with fewer raises, in both directions."""
+    from lasp_amd._abi import LaspError
+    from lasp_amd.utils import seq_parallel_manager as spm
+
+    s = lasp_amd.build_slope_tensor(2).to(gpu_device)
+    zeros = lambda *shape, **k: torch.zeros(*shape, device=gpu_device, **k)
+    for received in (zeros(1, 2, 64, 128), zeros(1, 2, 128, 128, dtype=torch.bfloat16), zeros(1, 2, 128, 256)[..., ::2],
+                     torch.zeros(1, 2, 128, 128)):
+        lasp_amd.destroy_parallel_groups()
+        lasp_amd.initialize_lasp(1, 2)
+        try:
+            (q, k, v), do = _leaves(gpu_device, 1, 2, 200, 128, 128, torch.bfloat16)
+            KV = torch.empty(1, 2, 128, 128, device=gpu_device)
+            DKV = torch.empty_like(KV)
+            lasp_amd.set_sequence_parallel_rank(0)
+            o = lasp_amd.lasp_fuse(q, k, v, s, KV, DKV)
+            spm.state_send(received, 0, spm.get_sequence_parallel_group(), src=1, give=True)
+            with pytest.raises(LaspError, match="dkv_in must be"):
+                o.backward(do)
+            lasp_amd.set_sequence_parallel_rank(1)
+            spm.state_recv(torch.empty_like(KV), 0, spm.get_sequence_parallel_group())  # the one that the call above left
+            spm.state_send(received, 1, spm.get_sequence_parallel_group(), src=0, give=True)
+            with pytest.raises(LaspError, match="kv_in must be"):
+                lasp_amd.lasp_fuse(q, k, v, s, KV, DKV)
+        finally:
+            lasp_amd.destroy_parallel_groups()
+
+
 class _NoGradient(torch.autograd.Function):
     """x -> x whose backward has no gradient to give."""
 
