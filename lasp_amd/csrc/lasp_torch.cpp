@@ -321,10 +321,11 @@ PYBIND11_MODULE(_lasp_torch, m) {
   m.def("attention", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s) {
     return operator_call(q, k, v, s, Tensor(), Tensor(), Tensor(), Tensor(), nullptr);
   });
-  // whether a chain's chunk is a usual case (asked before its incoming state is received)
-  m.def("takes", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &KV, const Tensor &DKV) {
+  // whether a chain's chunk is a usual case (asked before its incoming state is received); one without a KV or DKV buffer is not
+  m.def("takes", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &KV,
+                    const std::optional<Tensor> &DKV) {
     Shape sh;
-    return regular(q, k, v, s, sh) && state_ok(KV, sh, q) && state_ok(DKV, sh, q);
+    return KV && DKV && regular(q, k, v, s, sh) && state_ok(*KV, sh, q) && state_ok(*DKV, sh, q);
   });
   // a chunk of a chain
   m.def("chunk", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,

@@ -137,6 +137,25 @@ def test_a_state_of_another_shape_is_refused(gpu_device):
             lasp_amd.destroy_parallel_groups()
 
 
+@pytest.mark.parametrize("name", ["lasp_fuse", "lasp_fuse_parallel"])
+def test_calls_without_state_buffers(gpu_device, name):
+    """Without a DKV a forward still runs, and the backward of a group of one; without either the call is the stateless one."""
+    op = getattr(lasp_amd, name)
+    (q, k, v), do = _leaves(gpu_device, 1, 2, 200, 128, 128, torch.bfloat16)
+    s = lasp_amd.build_slope_tensor(2).to(gpu_device)
+    o = lasp_amd.lightning_attn(q, k, v, s)
+    want = torch.autograd.grad(o, (q, k, v), do)
+    lasp_amd.destroy_parallel_groups()
+    KV = torch.empty(1, 2, 128, 128, device=gpu_device)
+    with torch.no_grad():
+        assert torch.equal(op(q, k, v, s, KV, None), o)
+    stateless = op(q, k, v, s, None, None)
+    assert torch.equal(stateless, o)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(stateless, (q, k, v), do), want))
+    if name == "lasp_fuse":
+        assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(op(q, k, v, s, KV, None), (q, k, v), do), want))
+
+
 class _NoGradient(torch.autograd.Function):
     """x -> x whose backward has no gradient to give."""
 
