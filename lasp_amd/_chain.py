@@ -160,10 +160,12 @@ def native_chunk(q, k, v, s, KV, DKV, barrier, rebind=False):
     if not ext.takes(q, k, v, s, KV, DKV):
         return None
     x = Exchange(rebind)
-    kv_in, kv_out = x.before_forward(KV, barrier)
-    twin = x.twin(KV, kv_out) if x.rank < x.world - 1 else None
+    with torch.no_grad():  # as in a Function's forward: the buffers take no part in the graph, whatever they require
+        kv_in, kv_out = x.before_forward(KV, barrier)
+        twin = x.twin(KV, kv_out) if x.rank < x.world - 1 else None
     o = ext.chunk(q, k, v, s, kv_in, kv_out, twin, DKV, x)
-    x.after_forward(kv_out, twin)
+    with torch.no_grad():
+        x.after_forward(kv_out, twin)
     return o
 
 

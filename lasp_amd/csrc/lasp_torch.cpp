@@ -228,7 +228,6 @@ struct ChunkNode : public torch::autograd::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     const Tensor q_ = q.unpack().contiguous(), k_ = k.unpack().contiguous(), v_ = v.unpack().contiguous(), s_ = s.unpack();
     const Tensor states_ = states.unpack(), kv_in_ = kv_in.unpack();
-    at::AutoDispatchBelowADInplaceOrView below_autograd;
     c10::OptionalDeviceGuard guard(q_.device());
     // no gradient for the output is one of zeros: a chunk of a chain still has its neighbours' states to pass on
     const Tensor d_o = grads[0].defined() ? grads[0].contiguous() : at::zeros(v_.sizes(), v_.options());
@@ -244,7 +243,11 @@ struct ChunkNode : public torch::autograd::Node {
     check_state("dkv_in", dkv_in, sh, q_);
     check_state("dkv_out", dkv_out, sh, q_);
     check_state("dkv_twin", dkv_twin, sh, q_);
-    Backward r = run_backward(sh, q_, k_, v_, s_, d_o, kv_in_, dkv_in, dkv_out, dkv_twin, states_, seg_len);
+    Backward r;
+    {
+      at::AutoDispatchBelowADInplaceOrView below_autograd;  // (not around the exchange, whose writes to DKV count as versions)
+      r = run_backward(sh, q_, k_, v_, s_, d_o, kv_in_, dkv_in, dkv_out, dkv_twin, states_, seg_len);
+    }
     if (exchange.p) call_python([&] {
       const auto or_nothing = [](const Tensor &t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
       pybind11::reinterpret_borrow<pybind11::object>(g_after)(pybind11::reinterpret_borrow<pybind11::object>(exchange.p),

@@ -156,6 +156,30 @@ def test_calls_without_state_buffers(gpu_device, name):
         assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(op(q, k, v, s, KV, None), (q, k, v), do), want))
 
 
+@pytest.mark.parametrize("name", ["lasp_fuse", "lasp_fuse_parallel", "lasp_cache"])
+def test_state_buffers_that_require_a_gradient(gpu_device, name):
+    """They are scratch: they may be leaves that require a gradient, receive none, and their in-place changes are counted."""
+    op = getattr(lasp_amd, name)
+    s = lasp_amd.build_slope_tensor(2).to(gpu_device)
+    lasp_amd.destroy_parallel_groups()
+    lasp_amd.initialize_lasp(1, 2)
+    try:
+        outs, dos = [], []
+        KV, DKV = [torch.zeros(1, 2, 128, 128, device=gpu_device, requires_grad=True) for _ in range(2)]
+        for c in range(2):
+            lasp_amd.set_sequence_parallel_rank(c)
+            (q, k, v), do = _leaves(gpu_device, 1, 2, 100, 128, 128, torch.bfloat16, seed=c)
+            outs.append(op(q, k, v, s, *(() if name != "lasp_cache" else (None,)), KV, DKV))
+            assert "LaspChunk" in outs[-1].grad_fn.name()
+            dos.append(do)
+        assert name == "lasp_fuse" or KV._version == 2
+        torch.autograd.backward(outs, dos)
+        assert name == "lasp_fuse" or DKV._version == 2
+        assert KV.grad is None and DKV.grad is None
+    finally:
+        lasp_amd.destroy_parallel_groups()
+
+
 class _NoGradient(torch.autograd.Function):
     """x -> x whose backward has no gradient to give."""
 
