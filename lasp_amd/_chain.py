@@ -95,6 +95,12 @@ def after_backward(x: Exchange, dkv_out, twin=None):
                        give=x.rebind or twin is not None)
 
 
+@torch.no_grad()
+def after_native_forward(x: Exchange, kv_out, twin=None):
+    """Exchange.after_forward, called by the extension between the kernels of a chunk and the saving of its tensors."""
+    x.after_forward(kv_out, twin)
+
+
 def before_native_backward(x: Exchange, DKV):
     """before_backward for the native node: the outgoing state's twin comes third (see Exchange.twin)."""
     dkv_in, dkv_out = before_backward(x, DKV)
@@ -163,10 +169,7 @@ def native_chunk(q, k, v, s, KV, DKV, barrier, rebind=False):
     with torch.no_grad():  # as in a Function's forward: the buffers take no part in the graph, whatever they require
         kv_in, kv_out = x.before_forward(KV, barrier)
         twin = x.twin(KV, kv_out) if x.rank < x.world - 1 else None
-    o = ext.chunk(q, k, v, s, kv_in, kv_out, twin, DKV, x)
-    with torch.no_grad():
-        x.after_forward(kv_out, twin)
-    return o
+    return ext.chunk(q, k, v, s, kv_in, kv_out, twin, DKV, x)
 
 
 def run_sliced(q, k, v, ed, KV, DKV, cache_states, barrier, rebind=False):

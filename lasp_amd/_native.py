@@ -23,7 +23,7 @@ def ext():
         _abi.load()
         from . import _chain, _lasp_torch
 
-        _lasp_torch.bind(_abi.LaspError, _chain.before_native_backward, _chain.after_backward)
+        _lasp_torch.bind(_abi.LaspError, _chain.before_native_backward, _chain.after_backward, _chain.after_native_forward)
         _ext = _lasp_torch
     return _ext
 

@@ -199,6 +199,23 @@ Backward run_backward(const Shape &sh, const Tensor &q, const Tensor &k, const T
 // Python side of a chain's backward: before(exchange, DKV) -> (dkv_in, dkv_out, dkv_twin), each may be None, receives the
 // state from the next rank; after(exchange, dkv_out, dkv_twin) sends the one that this chunk leaves.
 PyObject *g_before = nullptr, *g_after = nullptr;
+// sent(exchange, kv_out, kv_twin): sends the state that the forward of a chunk leaves.
+PyObject *g_sent = nullptr;
+
+template <class F>
+void call_python(F &&f) {
+  pybind11::gil_scoped_acquire gil;
+  try {
+    f();
+  } catch (pybind11::error_already_set &e) {
+    e.restore();
+    python_error err;
+    err.persist();
+    throw err;
+  }
+}
+pybind11::object borrowed(PyObject *p) { return pybind11::reinterpret_borrow<pybind11::object>(p); }
+std::optional<Tensor> or_nothing(const Tensor &t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
 
 struct PyRef {  // a Python object held by a node, which any thread may drop
   PyObject *p = nullptr;
@@ -233,9 +250,8 @@ struct ChunkNode : public torch::autograd::Node {
     const Tensor d_o = grads[0].defined() ? grads[0].contiguous() : at::zeros(v_.sizes(), v_.options());
     Tensor dkv_in, dkv_out, dkv_twin;
     if (exchange.p) call_python([&] {
-      pybind11::object r = pybind11::reinterpret_borrow<pybind11::object>(g_before)(
-          pybind11::reinterpret_borrow<pybind11::object>(exchange.p), dkv_buffer);
-      auto states = r.cast<std::tuple<std::optional<Tensor>, std::optional<Tensor>, std::optional<Tensor>>>();
+      auto states = borrowed(g_before)(borrowed(exchange.p), dkv_buffer)
+                        .cast<std::tuple<std::optional<Tensor>, std::optional<Tensor>, std::optional<Tensor>>>();
       dkv_in = std::get<0>(states).value_or(Tensor());
       dkv_out = std::get<1>(states).value_or(Tensor());
       dkv_twin = std::get<2>(states).value_or(Tensor());
@@ -248,29 +264,12 @@ struct ChunkNode : public torch::autograd::Node {
       at::AutoDispatchBelowADInplaceOrView below_autograd;  // (not around the exchange, whose writes to DKV count as versions)
       r = run_backward(sh, q_, k_, v_, s_, d_o, kv_in_, dkv_in, dkv_out, dkv_twin, states_, seg_len);
     }
-    if (exchange.p) call_python([&] {
-      const auto or_nothing = [](const Tensor &t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
-      pybind11::reinterpret_borrow<pybind11::object>(g_after)(pybind11::reinterpret_borrow<pybind11::object>(exchange.p),
-                                                              or_nothing(dkv_out), or_nothing(dkv_twin));
-    });
+    if (exchange.p) call_python([&] { borrowed(g_after)(borrowed(exchange.p), or_nothing(dkv_out), or_nothing(dkv_twin)); });
     variable_list out(4);
     out[0] = std::move(r.dq);
     out[1] = std::move(r.dk);
     out[2] = std::move(r.dv);
     return out;
-  }
-
-  template <class F>
-  static void call_python(F &&f) {
-    pybind11::gil_scoped_acquire gil;
-    try {
-      f();
-    } catch (pybind11::error_already_set &e) {
-      e.restore();
-      python_error err;
-      err.persist();
-      throw err;
-    }
   }
 };
 
@@ -288,6 +287,9 @@ std::optional<Tensor> operator_call(const Tensor &q, const Tensor &k, const Tens
     at::AutoDispatchBelowADInplaceOrView below_autograd;
     f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, kv_in, kv_out, kv_twin, 0, grad);
   }
+  // Before any tensor is saved: a hook on one may end a recomputed forward there (torch.utils.checkpoint does), and the next
+  // rank, which recomputes too, waits for this state.
+  if (exchange) call_python([&] { borrowed(g_sent)(borrowed(exchange), or_nothing(kv_out), or_nothing(kv_twin)); });
   if (grad) {
     std::shared_ptr<ChunkNode> node(new ChunkNode(), torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(q, k, v, s));
@@ -315,10 +317,11 @@ Tensor or_none(const std::optional<Tensor> &t) { return t ? *t : Tensor(); }
 
 PYBIND11_MODULE(_lasp_torch, m) {
   namespace py = pybind11;
-  m.def("bind", [](py::object error, py::object before, py::object after) {
+  m.def("bind", [](py::object error, py::object before, py::object after, py::object sent) {
     g_error = error.release().ptr();
     g_before = before.release().ptr();
     g_after = after.release().ptr();
+    g_sent = sent.release().ptr();
   });
   // the stateless operator
   m.def("attention", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s) {

@@ -180,6 +180,53 @@ def test_state_buffers_that_require_a_gradient(gpu_device, name):
         lasp_amd.destroy_parallel_groups()
 
 
+@pytest.mark.parametrize("name", ["lasp_fuse", "lasp_fuse_parallel"])
+def test_a_checkpointed_chunk_sends_its_state_again(gpu_device, name, monkeypatch):
+    """torch.utils.checkpoint ends a recomputed forward from a hook on its last saved tensor.  The chunk has sent its state by
+    then, as the Python Function has: the next rank, which recomputes too, waits for it."""
+    from lasp_amd.utils import seq_parallel_manager as spm
+    from torch.utils.checkpoint import checkpoint
+
+    sent = []
+    state_send = spm.state_send
+    monkeypatch.setattr(spm, "state_send", lambda t, dst, *a, **k: (sent.append(dst), state_send(t, dst, *a, **k)))
+    s = lasp_amd.build_slope_tensor(2).to(gpu_device)
+    op = getattr(lasp_amd, name)
+    python = lambda q, k, v, s, KV, DKV: ChunkFunction.apply(q, k, v, s, KV, DKV, True, False, name != "lasp_fuse")
+    results = []
+    for call, checkpointed in ((op, False), (op, True), (python, True)):
+        lasp_amd.destroy_parallel_groups()
+        lasp_amd.initialize_lasp(1, 2)
+        del sent[:]
+        try:
+            (q, k, v), do = _leaves(gpu_device, 1, 2, 300, 128, 128, torch.bfloat16)
+            KV = torch.zeros(1, 2, 128, 128, device=gpu_device)
+            DKV = torch.zeros_like(KV)
+            run = lambda q, k, v: call(q, k, v, s, KV, DKV)
+            lasp_amd.set_sequence_parallel_rank(0)
+            o = checkpoint(run, q, k, v, use_reentrant=False) if checkpointed else run(q, k, v)
+            spm.state_send(torch.ones_like(KV), 0, spm.get_sequence_parallel_group(), src=1)
+            o.backward(do)
+            assert sent == ([1, 0, 1] if checkpointed else [1, 0])
+            results.append([o, q.grad, k.grad, v.grad])
+        finally:
+            lasp_amd.destroy_parallel_groups()
+    for r in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(results[0], r))
+
+
+def test_saved_tensor_hooks_see_what_the_node_keeps(gpu_device):
+    """Offloaded to the host and back, the node's tensors give the same gradients."""
+    (q, k, v), do = _leaves(gpu_device, 1, 2, 3000, 128, 128, torch.bfloat16)
+    s = lasp_amd.build_slope_tensor(2).to(gpu_device)
+    want = torch.autograd.grad(lasp_amd.lightning_attn(q, k, v, s), (q, k, v), do)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.cpu())[1], lambda t: t.to(gpu_device)):
+        o = lasp_amd.lightning_attn(q, k, v, s)
+    assert len(packed) == 5  # q, k, v, s and the segment states
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, (q, k, v), do), want))
+
+
 class _NoGradient(torch.autograd.Function):
     """x -> x whose backward has no gradient to give."""
 
