@@ -17,8 +17,6 @@
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
-#include <torch/csrc/autograd/functions/utils.h>
-#include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
@@ -26,13 +24,14 @@
 #include <c10/hip/HIPStream.h>
 
 #include <sstream>
+#include <unordered_map>
 
 #include "lasp_hip.h"
 
 namespace {
 
 using at::Tensor;
-using torch::autograd::SavedVariable;
+using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
 // ---- errors ------------------------------------------------------------------------------------------------
@@ -65,6 +64,17 @@ int dtype_code(const Tensor &t) {
   }
 }
 
+Shape shape_of(const Tensor &q, const Tensor &v) {
+  Shape sh;
+  sh.b = (int)q.size(0);
+  sh.h = (int)q.size(1);
+  sh.n = q.size(2);
+  sh.d = (int)q.size(3);
+  sh.e = (int)v.size(3);
+  sh.dtype = dtype_code(q);
+  return sh;
+}
+
 // A tensor whose operations others follow through the dispatcher or a tangent: only the Python autograd Function is seen
 // by them (and refuses what it has no rule for).
 bool followed(const Tensor &t) { return at::isTensorSubclassLike(t) || t._fw_grad(0).defined(); }
@@ -82,15 +92,11 @@ bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s,
     if (v.size(i) != q.size(i)) return false;
   if (q.size(0) > INT32_MAX || q.size(1) > INT32_MAX || s.scalar_type() != at::kFloat || s.numel() != q.size(1) || !s.is_contiguous())
     return false;
-  sh.dtype = dtype_code(q);
+  const int dtype = dtype_code(q);
   const int64_t d = q.size(3), e = v.size(3);
-  if (keep || sh.dtype < 0 || !is_step(q.size(2), d, e))
-    if (sh.dtype == LASP_DTYPE_F32 ? d != 128 || e != 128 : sh.dtype < 0 || d % 8 || e % 8 || d > 1024 || e > 128) return false;
-  sh.b = (int)q.size(0);
-  sh.h = (int)q.size(1);
-  sh.n = q.size(2);
-  sh.d = (int)d;
-  sh.e = (int)e;
+  if (keep || dtype < 0 || !is_step(q.size(2), d, e))
+    if (dtype == LASP_DTYPE_F32 ? d != 128 || e != 128 : dtype < 0 || d % 8 || e % 8 || d > 1024 || e > 128) return false;
+  sh = shape_of(q, v);
   return true;
 }
 
@@ -217,98 +223,128 @@ void call_python(F &&f) {
 pybind11::object borrowed(PyObject *p) { return pybind11::reinterpret_borrow<pybind11::object>(p); }
 std::optional<Tensor> or_nothing(const Tensor &t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
 
-struct PyRef {  // a Python object held by a node, which any thread may drop
-  PyObject *p = nullptr;
-  ~PyRef() {
-    if (p && Py_IsInitialized()) {
+// A Python object as a tensor: one int64, under which `handles` (guarded by the interpreter lock) holds a reference for as long
+// as the tensor's memory lives.  Unlike the object, a tensor may be among the things that an autograd context carries through
+// compiled autograd.
+std::unordered_map<int64_t, PyObject *> &handles() {
+  static auto *table = new std::unordered_map<int64_t, PyObject *>();
+  return *table;
+}
+Tensor handle_of(PyObject *object) {
+  static int64_t last = 0;
+  pybind11::gil_scoped_acquire gil;
+  auto *id = new int64_t(++last);
+  Py_INCREF(object);
+  handles()[*id] = object;
+  const auto drop = [](void *p) {  // on any thread
+    auto *id = static_cast<int64_t *>(p);
+    if (Py_IsInitialized()) {
       pybind11::gil_scoped_acquire gil;
-      Py_DECREF(p);
+      const auto held = handles().find(*id);
+      PyObject *object = held->second;
+      handles().erase(held);
+      Py_DECREF(object);
     }
-  }
+    delete id;
+  };
+  return at::from_blob(id, {1}, drop, at::TensorOptions().dtype(at::kLong));
+}
+pybind11::object object_of(const Tensor &handle) {  // under the interpreter lock
+  const auto held = handles().find(*handle.data_ptr<int64_t>());
+  if (held == handles().end()) raise_lasp("the exchange of this chunk is gone");
+  return borrowed(held->second);
+}
+
+// What a chunk of a chain brings along beside the inputs that take part in the graph (all empty without a chain).
+struct Chain {
+  Tensor kv_in, kv_out, kv_twin;
+  Tensor dkv_buffer;  // the caller's DKV: later backward calls overwrite it, so it is kept by reference, not as a saved tensor
+  PyObject *exchange = nullptr;
 };
 
-struct ChunkNode : public torch::autograd::Node {
-  Shape sh;
-  int seg_len = 0;
-  SavedVariable q, k, v, s, states, kv_in;
-  Tensor dkv_buffer;  // the caller's DKV: later backward calls overwrite it, so it is kept by reference
-  PyRef exchange;     // set in a chain
-
-  std::string name() const override { return "LaspChunkBackward"; }
-
-  void release_variables() override {
-    std::lock_guard<std::mutex> lock(mutex_);
-    for (SavedVariable *x : {&q, &k, &v, &s, &states, &kv_in}) x->reset_data();
-  }
-
-  variable_list apply(variable_list &&grads) override {
-    std::lock_guard<std::mutex> lock(mutex_);
-    const Tensor q_ = q.unpack().contiguous(), k_ = k.unpack().contiguous(), v_ = v.unpack().contiguous(), s_ = s.unpack();
-    const Tensor states_ = states.unpack(), kv_in_ = kv_in.unpack();
-    c10::OptionalDeviceGuard guard(q_.device());
-    // no gradient for the output is one of zeros: a chunk of a chain still has its neighbours' states to pass on
-    const Tensor d_o = grads[0].defined() ? grads[0].contiguous() : at::zeros(v_.sizes(), v_.options());
-    Tensor dkv_in, dkv_out, dkv_twin;
-    if (exchange.p) call_python([&] {
-      auto states = borrowed(g_before)(borrowed(exchange.p), dkv_buffer)
-                        .cast<std::tuple<std::optional<Tensor>, std::optional<Tensor>, std::optional<Tensor>>>();
-      dkv_in = std::get<0>(states).value_or(Tensor());
-      dkv_out = std::get<1>(states).value_or(Tensor());
-      dkv_twin = std::get<2>(states).value_or(Tensor());
-    });
-    check_state("dkv_in", dkv_in, sh, q_);
-    check_state("dkv_out", dkv_out, sh, q_);
-    check_state("dkv_twin", dkv_twin, sh, q_);
-    Backward r;
-    {
-      at::AutoDispatchBelowADInplaceOrView below_autograd;  // (not around the exchange, whose writes to DKV count as versions)
-      r = run_backward(sh, q_, k_, v_, s_, d_o, kv_in_, dkv_in, dkv_out, dkv_twin, states_, seg_len);
-    }
-    if (exchange.p) call_python([&] { borrowed(g_after)(borrowed(exchange.p), or_nothing(dkv_out), or_nothing(dkv_twin)); });
-    variable_list out(4);
-    out[0] = std::move(r.dq);
-    out[1] = std::move(r.dk);
-    out[2] = std::move(r.dv);
-    return out;
-  }
-};
-
-std::optional<Tensor> operator_call(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &kv_in,
-                                    const Tensor &kv_out, const Tensor &kv_twin, const Tensor &dkv_buffer, PyObject *exchange) {
-  Shape sh;
-  if (!regular(q, k, v, s, sh)) return std::nullopt;
-  check_state("kv_in", kv_in, sh, q);
-  check_state("kv_out", kv_out, sh, q);
-  check_state("kv_twin", kv_twin, sh, q);
-  const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() || s.requires_grad());
-  c10::OptionalDeviceGuard guard(q.device());
+Forward forward_call(const Shape &sh, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Chain &chain,
+                     bool keep) {
   Forward f;
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
-    f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, kv_in, kv_out, kv_twin, 0, grad);
+    f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, chain.kv_in, chain.kv_out, chain.kv_twin, 0, keep);
   }
   // Before any tensor is saved: a hook on one may end a recomputed forward there (torch.utils.checkpoint does), and the next
   // rank, which recomputes too, waits for this state.
-  if (exchange) call_python([&] { borrowed(g_sent)(borrowed(exchange), or_nothing(kv_out), or_nothing(kv_twin)); });
-  if (grad) {
-    std::shared_ptr<ChunkNode> node(new ChunkNode(), torch::autograd::deleteNode);
-    node->set_next_edges(torch::autograd::collect_next_edges(q, k, v, s));
-    node->sh = sh;
-    node->seg_len = f.seg_len;
-    node->q = SavedVariable(q, false);
-    node->k = SavedVariable(k, false);
-    node->v = SavedVariable(v, false);
-    node->s = SavedVariable(s, false);
-    if (f.states.defined()) node->states = SavedVariable(f.states, false);
-    if (kv_in.defined()) node->kv_in = SavedVariable(kv_in, false);
-    node->dkv_buffer = dkv_buffer;
-    if (exchange) {
-      Py_INCREF(exchange);
-      node->exchange.p = exchange;
+  if (chain.exchange) call_python([&] { borrowed(g_sent)(borrowed(chain.exchange), or_nothing(chain.kv_out), or_nothing(chain.kv_twin)); });
+  return f;
+}
+
+// The operator for autograd.  Compiled autograd calls `backward` as it is: it is left at is_traceable = false.
+struct LaspChunk : public torch::autograd::Function<LaspChunk> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Shape &sh,
+                        const Chain &chain) {
+    const Forward f = forward_call(sh, q, k, v, s, chain, true);
+    variable_list saved{q, k, v, s};
+    if (f.states.defined()) saved.push_back(f.states);
+    if (chain.kv_in.defined()) saved.push_back(chain.kv_in);
+    ctx->save_for_backward(std::move(saved));
+    // (a list, whose numbers compiled autograd takes as constants of the call; a short chunk without a state has none to keep)
+    if (f.seg_len != 0 || f.states.defined() || chain.kv_in.defined())
+      ctx->saved_data["call"] = c10::List<int64_t>({f.seg_len, f.states.defined(), chain.kv_in.defined()});
+    if (chain.exchange) {
+      ctx->saved_data["dkv_buffer"] = chain.dkv_buffer;
+      ctx->saved_data["exchange"] = handle_of(chain.exchange);
     }
-    torch::autograd::set_history(f.o, node);
+    return f.o;
   }
-  return f.o;
+
+  // (no gradient for the output arrives as one of zeros: a chunk of a chain still has its neighbours' states to pass on)
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor q = saved[0].contiguous(), k = saved[1].contiguous(), v = saved[2].contiguous(), s = saved[3];
+    Tensor states, kv_in;
+    int seg_len = 0;
+    auto &data = ctx->saved_data;
+    const auto call = data.empty() ? data.end() : data.find("call"), in_chain = data.empty() ? data.end() : data.find("exchange");
+    if (call != data.end()) {
+      const c10::List<int64_t> numbers = call->second.toIntList();
+      seg_len = (int)numbers[0];
+      if (numbers[1]) states = saved[4];
+      if (numbers[2]) kv_in = saved.back();
+    }
+    const Tensor d_o = grads[0].contiguous();
+    const Shape sh = shape_of(q, v);
+    c10::OptionalDeviceGuard guard(q.device());
+    Tensor dkv_in, dkv_out, dkv_twin, exchange;
+    if (in_chain != data.end()) {
+      exchange = in_chain->second.toTensor();
+      const Tensor dkv_buffer = data.at("dkv_buffer").toTensor();
+      call_python([&] {
+        auto states = borrowed(g_before)(object_of(exchange), dkv_buffer)
+                          .cast<std::tuple<std::optional<Tensor>, std::optional<Tensor>, std::optional<Tensor>>>();
+        dkv_in = std::get<0>(states).value_or(Tensor());
+        dkv_out = std::get<1>(states).value_or(Tensor());
+        dkv_twin = std::get<2>(states).value_or(Tensor());
+      });
+    }
+    check_state("dkv_in", dkv_in, sh, q);
+    check_state("dkv_out", dkv_out, sh, q);
+    check_state("dkv_twin", dkv_twin, sh, q);
+    Backward r;
+    {
+      at::AutoDispatchBelowADInplaceOrView below_autograd;  // (not around the exchange, whose writes to DKV count as versions)
+      r = run_backward(sh, q, k, v, s, d_o, kv_in, dkv_in, dkv_out, dkv_twin, states, seg_len);
+    }
+    if (exchange.defined()) call_python([&] { borrowed(g_after)(object_of(exchange), or_nothing(dkv_out), or_nothing(dkv_twin)); });
+    return {r.dq, r.dk, r.dv, Tensor(), Tensor(), Tensor()};
+  }
+};
+
+std::optional<Tensor> operator_call(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Chain &chain) {
+  Shape sh;
+  if (!regular(q, k, v, s, sh)) return std::nullopt;
+  check_state("kv_in", chain.kv_in, sh, q);
+  check_state("kv_out", chain.kv_out, sh, q);
+  check_state("kv_twin", chain.kv_twin, sh, q);
+  const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() || s.requires_grad());
+  c10::OptionalDeviceGuard guard(q.device());
+  return grad ? LaspChunk::apply(q, k, v, s, sh, chain) : forward_call(sh, q, k, v, s, chain, false).o;
 }
 
 Tensor or_none(const std::optional<Tensor> &t) { return t ? *t : Tensor(); }
@@ -325,7 +361,7 @@ PYBIND11_MODULE(_lasp_torch, m) {
   });
   // the stateless operator
   m.def("attention", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s) {
-    return operator_call(q, k, v, s, Tensor(), Tensor(), Tensor(), Tensor(), nullptr);
+    return operator_call(q, k, v, s, Chain());
   });
   // whether a chain's chunk is a usual case (asked before its incoming state is received); one without a KV or DKV buffer is not
   m.def("takes", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &KV,
@@ -337,7 +373,7 @@ PYBIND11_MODULE(_lasp_torch, m) {
   m.def("chunk", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
                     const std::optional<Tensor> &kv_out, const std::optional<Tensor> &kv_twin, const Tensor &dkv_buffer,
                     py::object exchange) {
-    return operator_call(q, k, v, s, or_none(kv_in), or_none(kv_out), or_none(kv_twin), dkv_buffer, exchange.ptr());
+    return operator_call(q, k, v, s, {or_none(kv_in), or_none(kv_out), or_none(kv_twin), dkv_buffer, exchange.ptr()});
   });
   // _abi.chunk_fwd / chunk_bwd
   m.def("chunk_fwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,

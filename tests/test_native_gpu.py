@@ -227,6 +227,40 @@ def test_saved_tensor_hooks_see_what_the_node_keeps(gpu_device):
     assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, (q, k, v), do), want))
 
 
+@pytest.mark.parametrize("name", ["lightning_attn", "lasp_fuse", "lasp_fuse_parallel"])
+def test_compiled_autograd_runs_the_backward(gpu_device, name):
+    """The node has the rules that compiled autograd asks for; a second run of the same shapes is served by what it compiled."""
+    from torch._dynamo import compiled_autograd
+
+    s = lasp_amd.build_slope_tensor(2).to(gpu_device)
+    chunks = 1 if name == "lightning_attn" else 2
+    results = []
+    for how in ("eager", "compiled", "compiled"):
+        lasp_amd.destroy_parallel_groups()
+        lasp_amd.initialize_lasp(1, chunks)
+        try:
+            outs, dos, leaves = [], [], []
+            KV = torch.zeros(1, 2, 128, 128, device=gpu_device)
+            DKV = torch.zeros_like(KV)
+            for c in range(chunks):
+                lasp_amd.set_sequence_parallel_rank(c)
+                (q, k, v), do = _leaves(gpu_device, 1, 2, 2500, 128, 128, torch.bfloat16, seed=c)
+                outs.append(getattr(lasp_amd, name)(q, k, v, s, *(() if chunks == 1 else (KV, DKV))))
+                dos.append(do)
+                leaves += [q, k, v]
+            if how == "eager":
+                torch.autograd.backward(outs, dos)
+            else:
+                with compiled_autograd._enable(torch.compile(backend="eager")):
+                    torch.autograd.backward(outs, dos)
+            assert not lasp_amd.loopback_pending()
+            results.append([*outs, *[t.grad for t in leaves], KV, DKV])
+        finally:
+            lasp_amd.destroy_parallel_groups()
+    for r in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(results[0], r))
+
+
 class _NoGradient(torch.autograd.Function):
     """x -> x whose backward has no gradient to give."""
 
