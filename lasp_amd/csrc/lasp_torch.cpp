@@ -359,10 +359,14 @@ PYBIND11_MODULE(_lasp_torch, m) {
     g_after = after.release().ptr();
     g_sent = sent.release().ptr();
   });
+  // The interpreter lock is free while these run, as it is during a ctypes call: an allocation may wait for the driver, and a
+  // launch for room in its queue.
+  using unlocked = py::call_guard<py::gil_scoped_release>;
   // the stateless operator
-  m.def("attention", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s) {
-    return operator_call(q, k, v, s, Chain());
-  });
+  m.def(
+      "attention",
+      [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s) { return operator_call(q, k, v, s, Chain()); },
+      unlocked());
   // whether a chain's chunk is a usual case (asked before its incoming state is received); one without a KV or DKV buffer is not
   m.def("takes", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &KV,
                     const std::optional<Tensor> &DKV) {
@@ -370,39 +374,48 @@ PYBIND11_MODULE(_lasp_torch, m) {
     return KV && DKV && regular(q, k, v, s, sh) && state_ok(*KV, sh, q) && state_ok(*DKV, sh, q);
   });
   // a chunk of a chain
-  m.def("chunk", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
-                    const std::optional<Tensor> &kv_out, const std::optional<Tensor> &kv_twin, const Tensor &dkv_buffer,
-                    py::object exchange) {
-    return operator_call(q, k, v, s, {or_none(kv_in), or_none(kv_out), or_none(kv_twin), dkv_buffer, exchange.ptr()});
-  });
+  m.def(
+      "chunk",
+      [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
+         const std::optional<Tensor> &kv_out, const std::optional<Tensor> &kv_twin, const Tensor &dkv_buffer,
+         const py::handle &exchange) {
+        return operator_call(q, k, v, s, {or_none(kv_in), or_none(kv_out), or_none(kv_twin), dkv_buffer, exchange.ptr()});
+      },
+      unlocked());
   // _abi.chunk_fwd / chunk_bwd
-  m.def("chunk_fwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
-                        const std::optional<Tensor> &kv_out, int seg_len, bool keep) -> py::object {
-    Shape sh;
-    const Tensor in = or_none(kv_in), out = or_none(kv_out);
-    if (!regular(q, k, v, s, sh, keep) || !state_ok(in, sh, q) || !state_ok(out, sh, q)) return py::none();
-    c10::OptionalDeviceGuard guard(q.device());
-    at::AutoDispatchBelowADInplaceOrView below_autograd;
-    Forward f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, in, out, Tensor(), seg_len, keep);
-    return py::make_tuple(f.o, f.states.defined() ? std::optional<Tensor>(f.states) : std::nullopt, f.seg_len);
-  });
-  m.def("chunk_bwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &d_o,
-                        const std::optional<Tensor> &kv_in, const std::optional<Tensor> &dkv_in,
-                        const std::optional<Tensor> &dkv_out, const std::optional<Tensor> &states, int seg_len) -> py::object {
-    Shape sh;
-    const Tensor in = or_none(kv_in), din = or_none(dkv_in), dout = or_none(dkv_out), st = or_none(states);
-    if (!regular(q, k, v, s, sh) || !state_ok(in, sh, q) || !state_ok(din, sh, q) || !state_ok(dout, sh, q) ||
-        d_o.device() != q.device() || d_o.scalar_type() != q.scalar_type() || d_o.sizes() != v.sizes())
-      return py::none();
-    if (st.defined()) {  // what chunk_fwd returned for this shape
-      const Plan p = plan_of(sh, seg_len);
-      if (!p.fused && (st.scalar_type() != at::kFloat || st.device() != q.device() || !st.is_contiguous() ||
-                       (size_t)st.numel() * sizeof(float) != p.bytes))
-        return py::none();
-    }
-    c10::OptionalDeviceGuard guard(q.device());
-    at::AutoDispatchBelowADInplaceOrView below_autograd;
-    Backward r = run_backward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, d_o.contiguous(), in, din, dout, Tensor(), st, seg_len);
-    return py::make_tuple(r.dq, r.dk, r.dv);
-  });
+  m.def(
+      "chunk_fwd",
+      [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const std::optional<Tensor> &kv_in,
+         const std::optional<Tensor> &kv_out, int seg_len, bool keep) -> std::optional<std::tuple<Tensor, std::optional<Tensor>, int>> {
+        Shape sh;
+        const Tensor in = or_none(kv_in), out = or_none(kv_out);
+        if (!regular(q, k, v, s, sh, keep) || !state_ok(in, sh, q) || !state_ok(out, sh, q)) return std::nullopt;
+        c10::OptionalDeviceGuard guard(q.device());
+        at::AutoDispatchBelowADInplaceOrView below_autograd;
+        Forward f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, in, out, Tensor(), seg_len, keep);
+        return std::make_tuple(f.o, or_nothing(f.states), f.seg_len);
+      },
+      unlocked());
+  m.def(
+      "chunk_bwd",
+      [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &d_o, const std::optional<Tensor> &kv_in,
+         const std::optional<Tensor> &dkv_in, const std::optional<Tensor> &dkv_out, const std::optional<Tensor> &states,
+         int seg_len) -> std::optional<std::tuple<Tensor, Tensor, Tensor>> {
+        Shape sh;
+        const Tensor in = or_none(kv_in), din = or_none(dkv_in), dout = or_none(dkv_out), st = or_none(states);
+        if (!regular(q, k, v, s, sh) || !state_ok(in, sh, q) || !state_ok(din, sh, q) || !state_ok(dout, sh, q) ||
+            d_o.device() != q.device() || d_o.scalar_type() != q.scalar_type() || d_o.sizes() != v.sizes())
+          return std::nullopt;
+        if (st.defined()) {  // what chunk_fwd returned for this shape
+          const Plan p = plan_of(sh, seg_len);
+          if (!p.fused && (st.scalar_type() != at::kFloat || st.device() != q.device() || !st.is_contiguous() ||
+                           (size_t)st.numel() * sizeof(float) != p.bytes))
+            return std::nullopt;
+        }
+        c10::OptionalDeviceGuard guard(q.device());
+        at::AutoDispatchBelowADInplaceOrView below_autograd;
+        Backward r = run_backward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, d_o.contiguous(), in, din, dout, Tensor(), st, seg_len);
+        return std::make_tuple(r.dq, r.dk, r.dv);
+      },
+      unlocked());
 }

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import lasp_amd
+from lasp_amd import _native
 from lasp_amd._chain import ChunkFunction
 
 pytestmark = pytest.mark.gpu
@@ -259,6 +260,54 @@ def test_compiled_autograd_runs_the_backward(gpu_device, name):
             lasp_amd.destroy_parallel_groups()
     for r in results[1:]:
         assert all(torch.equal(a, b) for a, b in zip(results[0], r))
+
+
+def test_the_interpreter_lock_is_free_during_a_call(gpu_device):
+    """Another thread gets to run while a call allocates and launches.  The lock is not taken from a thread that keeps it here
+    (the switch interval is longer than the test), so a tick inside a call means that the call had let go of it."""
+    import sys
+    import threading
+    import time
+
+    (q, k, v), do = _leaves(gpu_device, 1, 16, 65536, 128, 128, torch.bfloat16)
+    q, k, v = q.detach(), k.detach(), v.detach()
+    s = lasp_amd.build_slope_tensor(16).to(gpu_device)
+    ext = _native.ext()
+    calls = {
+        "attention": lambda: ext.attention(q, k, v, s),
+        "chunk_fwd": lambda: ext.chunk_fwd(q, k, v, s, None, None, 0, True),
+        "chunk_bwd": lambda: ext.chunk_bwd(q, k, v, s, do, None, None, None, None, 0),
+    }
+    ticks, done = [], threading.Event()
+
+    def tick():
+        while not done.is_set():
+            ticks.append(time.perf_counter_ns())
+            time.sleep(0)
+
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(600.0)
+    other = threading.Thread(target=tick)
+    other.start()
+    try:
+        for name, call in calls.items():
+            seen = False
+            for _ in range(20):
+                torch.cuda.synchronize()
+                torch.cuda.empty_cache()  # the call has to ask the driver for its outputs
+                begin = time.perf_counter_ns()
+                out = call()
+                end = time.perf_counter_ns()
+                assert out is not None
+                del out
+                seen = any(begin < t < end for t in ticks[-100000:])
+                if seen:
+                    break
+            assert seen, name
+    finally:
+        done.set()
+        sys.setswitchinterval(interval)
+        other.join()
 
 
 class _NoGradient(torch.autograd.Function):
