@@ -1261,16 +1261,20 @@ Geom fused_bwd_geom(const Geom &g) {
 }
 
 // Where whole chunks fill more than one round of the chip, the workgroups of the last, partly filled round would take as
-// long as a full one.  Their (b, h) are cut into as many segments as fill it instead: walks over the blocks before a segment
-// cost less than half of sweeping them.  Backward kernel, d = e = 128, bf16, before and now: n = 512, b*h = 88: 37.8 and
-// 28.5 us, 96: 38.9 and 33.4, 120 (two segments only): 39.2 and 37.7, 172: 58.5 and 51.6; n = 1024, b*h = 96: 71.3 and 56.1, 120:
-// 73.6 and 74.4; d = e = 64, b*h = 192, n = 1024: 53.7 and 50.0.
+// long as a full one.  Their (b, h) are cut into as many segments as fill the places that are left: walks over the blocks before
+// a segment cost less than half of sweeping them.  Backward kernel, bf16, uncut and cut.  d = e = 128: n = 512, b*h = 88: 35.4 and
+// 25.2 us, 96: 35.3 and 28.9, 120 (two segments only): 35.8 and 33.0, 172: 53.0 and 43.9; n = 1024, b*h = 96: 67.8 and 51.6, 120:
+// 70.8 and 69.6; never slower over b*h = 88 ... 512, n = 64 ... 1536.  d = e = 64: the places count one workgroup per CU, not
+// two: a last round of at most 256 has the CUs to itself and runs at up to twice the pace of a full one, which is all that cutting
+// it further can win (n = 1024: b*h = 171 uncut 50.2, cut for one per CU 38.5, for two 40.6; 200: 52.6, 50.4 and 51.1; 216, left
+// uncut with one per CU: 53.8 and 57.1; 240: 58.3 and 63.9).
 Fine fused_bwd_tail(const Geom &g) {
   const int64_t bh = (int64_t)g.b * g.h, slots = g.width == 64 ? 512 : 256;
   Fine f = {(int)((bh + 7) / 8 * 8), g.seg_len, g.n_seg, g.by_seg};  // nothing is cut
   if (g.n_seg > 1 || 3 * bh <= slots) return f;
-  const int64_t bh0 = 3 * bh / slots * slots / 24 * 8;  // whole rounds of whole groups of 8
-  const int64_t rest = (bh - bh0 + 7) / 8 * 8, room = slots + (3 * bh / slots * slots - 3 * bh0);
+  const int64_t whole = 3 * bh / slots * slots;  // workgroups in whole rounds
+  const int64_t bh0 = whole / 24 * 8;            // whole groups of 8
+  const int64_t rest = (bh - bh0 + 7) / 8 * 8, room = 256 + (g.width == 64 ? 0 : whole - 3 * bh0);
   const int64_t nblk = (g.n + BLK - 1) / BLK;
   int64_t n_seg = rest > 0 ? room / (3 * rest) : 1;
   if (n_seg > nblk) n_seg = nblk;

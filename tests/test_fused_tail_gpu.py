@@ -1,9 +1,12 @@
 """Short chunks whose (b, h) fill more than one round of the chip in the backward: the (b, h) of the last, partly filled round
 are cut into segments, the others run whole.  Every (b, h) against the oracle in 64 bits."""
+import statistics
+
 import pytest
 import torch
 
 import lasp_amd
+from lasp_amd import _native
 from oracle import lasp_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -17,7 +20,9 @@ REL = {torch.bfloat16: 1.2e-2, torch.float16: 1.6e-3}
     (1, 86, 300, 128, 128, torch.bfloat16),  # one group of 8 (two of them missing) in segments of one block, the last partial
     (5, 24, 130, 128, 128, torch.bfloat16),  # 40 in 2 segments, the second with one block of 2 tokens
     (4, 43, 128, 96, 40, torch.bfloat16),    # two whole rounds, narrow rows
-    (2, 90, 200, 64, 64, torch.bfloat16),    # the 64-wide kernels: 512 workgroups to a round
+    (2, 90, 200, 64, 64, torch.bfloat16),    # the 64-wide kernels: 512 workgroups to a round, 256 to the cut one
+    (8, 26, 200, 64, 64, torch.float16),     # 168 whole, 40 in 2 segments: the most that are cut
+    (8, 27, 200, 64, 64, torch.float16),     # 48 more than whole rounds: not cut
 ])
 def test_every_head_of_a_cut_last_round(gpu_device, b, h, n, d, e, dtype):
     g = torch.Generator().manual_seed(b * h + n)
@@ -31,3 +36,25 @@ def test_every_head_of_a_cut_last_round(gpu_device, b, h, n, d, e, dtype):
         diff, want = t.grad.double().cpu() - ref[name], ref[name]
         rel = diff.flatten(2).norm(dim=2) / want.flatten(2).norm(dim=2)
         assert float(rel.max()) < REL[dtype], (name, float(rel.max()), int(rel.argmax()))
+
+
+def test_a_last_round_is_cut_only_where_that_pays(gpu_device):
+    """64-wide heads, two workgroups to a CU: a last round that leaves the CUs half empty runs at twice the pace of a full one,
+    so cutting it to fill them cost more than it won, and 240 (b, h) took longer than 256."""
+    def calls(bh):
+        q, k, v, do = [torch.randn(1, bh, 1536, 64, device=gpu_device).to(torch.bfloat16) / 8 for _ in range(4)]
+        s = lasp_amd.build_slope_tensor(bh).to(gpu_device)
+        return lambda: _native.chunk_bwd(q, k, v, s, do)
+
+    runs, times = {bh: calls(bh) for bh in (240, 256)}, {240: [], 256: []}
+    for _ in range(15):
+        for bh, run in runs.items():
+            run()
+            start, stop = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            start.record()
+            for _ in range(8):
+                run()
+            stop.record()
+            stop.synchronize()
+            times[bh].append(start.elapsed_time(stop))
+    assert statistics.median(times[240]) < statistics.median(times[256])
