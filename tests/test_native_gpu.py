@@ -1,10 +1,12 @@
-"""The native autograd node (lasp_amd/csrc/lasp_torch.cpp) against the Python autograd Function over the same kernels: the
-same bits, graphs that can be kept or not, and the calls that it leaves to the Python path."""
+"""The native autograd node (lasp_amd/csrc/lasp_torch.cpp) against the Python autograd Function, which reaches the same kernels
+over ctypes: the same bits, graphs that can be kept or not, and the calls that it leaves to the Python path."""
+import contextlib
+
 import pytest
 import torch
 
 import lasp_amd
-from lasp_amd import _native
+from lasp_amd import _abi, _native
 from lasp_amd._chain import ChunkFunction
 
 pytestmark = pytest.mark.gpu
@@ -14,6 +16,19 @@ def _leaves(dev, b, h, n, d, e, dtype, seed=0):
     g = torch.Generator(device=dev).manual_seed(seed)
     mk = lambda w: (torch.randn(b, h, n, w, generator=g, device=dev) / w ** 0.5).to(dtype)
     return [mk(w).requires_grad_(True) for w in (d, d, e)], mk(e)
+
+
+@contextlib.contextmanager
+def _over_ctypes():
+    """ChunkFunction's calls (of the forward and, on autograd's thread, of the backward) go to `_abi` and not to the extension,
+    whose plans, workspaces and argument order are what is compared."""
+    calls = []
+    abi_call = lambda name: lambda *args, **kw: (calls.append(name), getattr(_abi, name)(*args, **kw))[1]
+    with pytest.MonkeyPatch.context() as patch:
+        patch.setattr(_native, "chunk_fwd", abi_call("chunk_fwd"))
+        patch.setattr(_native, "chunk_bwd", abi_call("chunk_bwd"))
+        yield
+    assert set(calls) == {"chunk_fwd", "chunk_bwd"}
 
 
 @pytest.mark.parametrize("b,h,n,d,e,dtype", [(1, 2, 1, 128, 128, torch.bfloat16), (2, 3, 300, 64, 40, torch.float16),
@@ -28,8 +43,9 @@ def test_native_node_gives_the_bits_of_the_python_function(gpu_device, b, h, n, 
     again = torch.autograd.grad(o, (q, k, v), do)
     with pytest.raises(RuntimeError, match="second time"):
         torch.autograd.grad(o, (q, k, v), do)
-    op = ChunkFunction.apply(q, k, v, s, None, None, True, False)
-    python = torch.autograd.grad(op, (q, k, v), do)
+    with _over_ctypes():
+        op = ChunkFunction.apply(q, k, v, s, None, None, True, False)
+        python = torch.autograd.grad(op, (q, k, v), do)
     assert torch.equal(o, op)
     for a, b_, c in zip(native, again, python):
         assert torch.equal(a, c) and torch.equal(b_, c)
@@ -72,7 +88,10 @@ def _compare_chains(gpu_device, name, rebind, n, d, e, dtype):
     for native in (True, False):
         lasp_amd.destroy_parallel_groups()
         lasp_amd.initialize_lasp(1, 3)
-        try:
+        with contextlib.ExitStack() as stack:
+            stack.callback(lasp_amd.destroy_parallel_groups)
+            if not native:
+                stack.enter_context(_over_ctypes())
             KV = torch.empty(1, 4, d, e, device=gpu_device)
             DKV = torch.empty_like(KV)
             outs, leaves, dos = [], [], []
@@ -89,8 +108,6 @@ def _compare_chains(gpu_device, name, rebind, n, d, e, dtype):
             torch.autograd.backward(outs, dos)
             assert not lasp_amd.loopback_pending()
             results.append([*outs, *[t.grad for t in leaves], KV, DKV])
-        finally:
-            lasp_amd.destroy_parallel_groups()
     assert all(torch.equal(a, b) for a, b in zip(*results))
 
 
@@ -256,8 +273,6 @@ def test_compiled_autograd_runs_the_backward(gpu_device, name):
                     torch.autograd.backward(outs, dos)
             assert not lasp_amd.loopback_pending()
             results.append([*outs, *[t.grad for t in leaves], KV, DKV])
-        finally:
-            lasp_amd.destroy_parallel_groups()
     for r in results[1:]:
         assert all(torch.equal(a, b) for a, b in zip(results[0], r))
 
