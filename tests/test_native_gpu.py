@@ -273,6 +273,8 @@ def test_compiled_autograd_runs_the_backward(gpu_device, name):
                     torch.autograd.backward(outs, dos)
             assert not lasp_amd.loopback_pending()
             results.append([*outs, *[t.grad for t in leaves], KV, DKV])
+        finally:
+            lasp_amd.destroy_parallel_groups()
     for r in results[1:]:
         assert all(torch.equal(a, b) for a, b in zip(results[0], r))
 
