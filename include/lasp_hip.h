@@ -12,7 +12,7 @@
  *     s            : h floats          per-head decay slope, >= 0
  *     kv_in, kv_out, dkv_in, dkv_out : (b, h, d, e) float, may be NULL
  *     seg states   : float workspace of lasp_plan's state_bytes (one state per (b, h) and segment, or per
- *                    piece of a long segment; each d x e, or zero-extended to 128 x 128): opaque to the caller
+ *                    piece of a long segment; each d x e, or zero-extended to 64 x 64 or 128 x 128): opaque to the caller
  * Widths: d, e <= 128.  With 16-bit elements and d, e multiples of 8, d may be up to 1024: such wide heads are swept in
  * slices of 128 features of q and k (one state per slice in the workspace), and the parts of o and dv that slices
  * after the first contribute are added to what is there, rounded to the element type once per slice.
@@ -101,8 +101,9 @@ const char *lasp_last_error(void);
  * positive multiple of 64, to the calls below); n_seg = ceil(n / seg_len) and
  * the byte size of ONE segment-state array are written through the pointers
  * (either may be NULL).  The array is opaque: the MFMA kernels keep every state
- * zero-extended to 128 x 128 floats, the generic ones as d x e.  Replaces the BLOCK/NUM_BLOCK choice of
- * lasp/lasp_fuse_parallel.py:1080-1085 and the `kv` buffer shape of :876.
+ * zero-extended to 128 x 128 floats, the generic ones as d x e.  (In 16 bits with d, e <= 64 they are kept as
+ * 64 x 64, one behind the other; state_bytes counts 128 x 128 each all the same.)  Replaces the BLOCK/NUM_BLOCK
+ * choice of lasp/lasp_fuse_parallel.py:1080-1085 and the `kv` buffer shape of :876.
  */
 int lasp_plan(int b, int h, int64_t n, int d, int e, int dtype, int seg_len_or_0,
               int *seg_len, int *n_seg, size_t *state_bytes);
@@ -163,8 +164,8 @@ int lasp_step_fwd(const void *q, const void *k, const void *v, const float *s, c
  * LASP_STATIC_SCRATCH_BYTES that is part of the library's code object (each GPU the
  * library runs on holds its own copy until the process ends).  The call allocates and
  * frees nothing, on the host or the device.
- * Limit: b * h * n_seg states of 64 KiB (128 x 128 floats; d x e floats on the generic
- * path) must fit, i.e. at most 512 states on the MFMA path -- the headline shape
+ * Limit: b * h * n_seg states of 64 KiB (128 x 128 floats, also where they are kept as 64 x 64; d x e
+ * floats on the generic path) must fit, i.e. at most 512 states on the MFMA path -- the headline shape
  * b=1 h=16 n=65536 with the default seg_len just fits; a larger call returns
  * LASP_E_WORKSPACE (a longer seg_len lowers n_seg).
  * The first call on a device looks the scratch's device address up (hipGetSymbolAddress, which

@@ -247,7 +247,7 @@ def _chunk_fwd_exact(q, k, v, s, kv_in=None, kv_out=None, seg_len: int = 0):
         states = None
         if not fused and (n_seg > 1 or kv_in is not None or kv_out is not None):
             # the library decides how many states it keeps (one per segment, or per piece of a long segment)
-            # and how each is stored (d x e, or zero-extended to 128 x 128): the array is opaque here
+            # and how each is stored (d x e, or zero-extended to 64 x 64 or 128 x 128): the array is opaque here
             states = torch.empty((state_bytes // 4,), dtype=torch.float32, device=dev)
         rc = lib.lasp_chunk_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr(), _ptr(kv_in), _ptr(kv_out),
                                 o.data_ptr(), _ptr(states), b, h, n, d, e, DTYPE_CODE[q.dtype], seg_len,

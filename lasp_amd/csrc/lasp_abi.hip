@@ -467,7 +467,8 @@ int static_scratch(float **out) {
   return 0;
 }
 
-// (a state of the 64-wide kernels takes a quarter of its slot: every caller sizes the array for 128 x 128)
+// The size that lasp_plan has always stated for 16-bit shapes: the 64-wide kernels index their states by 64 x 64 and leave
+// three quarters of the array unused.  What fits the library's scratch array goes by the same size.
 size_t state_bytes_of(const Geom &g) {
   const size_t one = g.width == 64 ? (size_t)kMaxFeature * kMaxFeature : (size_t)g.sd * g.se;
   const size_t slices = (g.dt + kMaxWidth - 1) / kMaxWidth;

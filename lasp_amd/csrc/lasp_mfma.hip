@@ -896,8 +896,8 @@ la_bwd3(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const el
 
 // ------------------------------------------------------------------------------
 // A segment's own state:  causal  sum_b l^(L-b) y_b^T z_b ;  anti-causal  sum_b l^b y_b^T z_b
-// (b from the segment start, L its length), written token-free as 128 x 128 fp32.  Y rows hold
-// g.d features and Z rows g.e (M_NARROW; 128 otherwise).
+// (b from the segment start, L its length), written token-free as W x W fp32 (W = 64 or 128).  Y rows hold
+// g.d features and Z rows g.e (M_NARROW; W otherwise).
 //
 // Blocks whose every token carries a weight below 2^-SKIP_LOG2 are neither read nor multiplied:
 // with slope s a token that lies x tokens from the segment's far end weighs exp(-s x), so a
