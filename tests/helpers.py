@@ -37,3 +37,27 @@ def check(got: dict, ref: dict, tol: float, names=NAMES, what=""):
     bad = {k_: v_ for k_, v_ in errs.items() if not (v_ <= tol)}
     assert not bad, f"{what}: worst (b,h) slice over {tol}: {bad} (per-head: {errs}; whole tensor: {whole})"
     return errs
+
+
+def in_place_bits(inp, s, seg):
+    """Outputs of a forward and two backwards (the forward's states, rebuilt ones) whose states are updated in place, each
+    with that of separate buffers.  Where the library does not take a shape in place in a direction, that one is left out."""
+    from lasp_amd import _abi
+
+    shape = (*inp["q"].shape, inp["v"].shape[-1], inp["q"].dtype)
+    takes = {backward: _abi.inplace_ok(*shape, seg, backward) for backward in (False, True)}
+    assert takes[False]
+
+    def run(in_place):
+        buffers = lambda x, backward: (x, x if in_place and takes[backward] else torch.empty_like(x))
+        kv, kv_out = buffers(inp["kv"].clone(), False)
+        o, states, seg_len = _abi._chunk_fwd_exact(inp["q"], inp["k"], inp["v"], s, kv_in=kv, kv_out=kv_out, seg_len=seg)
+        got = [o, kv_out]
+        for kept in (states, None):
+            dkv, dkv_out = buffers(inp["dkv"].clone(), True)
+            got += _abi._chunk_bwd_exact(inp["q"], inp["k"], inp["v"], s, inp["do"], kv_in=inp["kv"], dkv_in=dkv,
+                                         dkv_out=dkv_out, kv_seg_states=kept, seg_len=seg_len)
+            got.append(dkv_out)
+        return got
+
+    return list(zip(run(True), run(False)))

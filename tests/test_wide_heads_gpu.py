@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import lasp_amd
-from helpers import check, make_inputs, oracle
+from helpers import check, in_place_bits, make_inputs, oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -27,6 +27,16 @@ def test_feature_slices(gpu_device, n, seg, d, e, dtype):
         got = dict(o=o, kv_out=kvo, dq=dq, dk=dk, dv=dv, dkv_out=dkvo)
         # the bound of every 16-bit parity test; O and dV are rounded once more per slice (2^-9 each)
         check(got, ref, 2e-2, what=f"n={n} seg={seg} d={d} e={e} {dtype} kept={kept is not None}")
+
+
+@pytest.mark.parametrize("d", [192, 256])
+@pytest.mark.parametrize("n,seg", [(500, 64), (1152, 128), (65, 0)])
+def test_states_updated_in_place(gpu_device, n, seg, d):
+    """Every slice parks the incoming state of a head outside the scan (slope 0.4: gone within 64 tokens) in its own part of
+    the workspace, and reads it in a sweep that starts after all slices' outgoing states have replaced the incoming ones."""
+    inp = make_inputs(1, 3, n, d, 128, torch.bfloat16, seed=n + d, scale=0.3, state=True, state_std=1.0, device=gpu_device)
+    for i, (a, r) in enumerate(in_place_bits(inp, torch.tensor([0.4, 0.02, 0.0], device=gpu_device), seg)):
+        assert torch.equal(a, r), i
 
 
 def test_wide_operator_chain(gpu_device):

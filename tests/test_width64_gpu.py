@@ -3,7 +3,7 @@ segment of 64 or 192 tokens ends in half a step), rows narrower than 64, ragged 
 import pytest
 import torch
 
-from helpers import check, make_inputs, oracle
+from helpers import check, in_place_bits, make_inputs, oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -27,3 +27,13 @@ def test_rows_of_up_to_64_features(gpu_device, n, seg, d, e, dtype):
         got = dict(o=o, kv_out=kvo, dq=dq, dk=dk, dv=dv, dkv_out=dkvo)
         # the bound of every 16-bit parity test: roundings of 2^-9 in inputs, decayed keys, scores and states
         check(got, ref, 2e-2, what=f"n={n} seg={seg} d={d} e={e} {dtype} kept={kept is not None}")
+
+
+@pytest.mark.parametrize("d,e", [(64, 64), (56, 24)])
+@pytest.mark.parametrize("n,seg", [(500, 64), (1152, 128), (65, 0)])
+def test_states_updated_in_place(gpu_device, n, seg, d, e):
+    """Two waves hold each column block of the state that a single workgroup reads and replaces; heads outside the scan
+    (slope 0.4) find the incoming state in the workspace."""
+    inp = make_inputs(2, 3, n, d, e, torch.bfloat16, seed=n + d, state=True, state_std=1.0, device=gpu_device)
+    for i, (a, r) in enumerate(in_place_bits(inp, torch.tensor([0.4, 0.02, 0.0], device=gpu_device), seg)):
+        assert torch.equal(a, r), i
