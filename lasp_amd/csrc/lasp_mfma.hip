@@ -936,7 +936,9 @@ struct StateLds {
 // workgroups share a CU; the deep one runs one per CU (squeezed into 128 registers it spills and measured slower).
 constexpr int STATE_DEPTH_LONG = 4, STATE_DEPTH_SHORT = 2;
 // Tokens per segment up to which every block is read, whatever the decay (forward with a state, b*h = 16, n = 2000, with the
-// scan's shorter start-up: 24.1 us against 24.7; eight chained chunks of 2048 tokens, b*h = 24: 624 against 631).
+// scan's shorter start-up: 24.1 us against 24.7; eight chained chunks of 2048 tokens, b*h = 24: 624 against 631).  Not where a wide
+// head's slices run side by side: several workgroups per CU wait for one another's bytes, not for a slope (b*h = 8, n = 8192,
+// d = 256, forward + backward: 186.3 us against 188.6 with every block read).
 constexpr int STATE_WHOLE = 512;
 constexpr int STATE_LONG_WALK = 1024;  // tokens per segment from which the deeper pipeline is used
 
@@ -990,7 +992,7 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   if (sw.seg == skip_seg) return;  // the scan's final segment feeds only the outgoing carry
   // Short segments are walked whole: the few blocks that a fast-decaying head could leave out delay nobody, while the slope,
   // which says which, would have to arrive before the first load can leave.
-  const bool whole = g.seg_len <= STATE_WHOLE;
+  const bool whole = g.seg_len <= STATE_WHOLE && (!NARROW || g.dt <= W);
   const int head = sw.bh - quotient(sw.bh, g.by_h) * g.h;
   int lane_head = head;
   asm volatile("" : "+v"(lane_head));  // (a lane's load, waited for in order; see ws_body)
