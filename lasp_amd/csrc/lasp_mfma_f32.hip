@@ -3,66 +3,150 @@
 // attention over a segment given the state entering it, and the four outputs of the
 // operator are instances of it (O: x=Q y=K z=V; dQ: x=dO y=V z=K with the state transposed;
 // dV: x=K y=Q z=dO anti-causal; dK: x=V y=dO z=Q anti-causal, state transposed) -- but with
-// full-precision arithmetic throughout (v_mfma_f32_32x32x2_f32), for inputs whose tolerance
-// (1e-3) rules out 16-bit operands.
+// full-precision arithmetic, for inputs whose tolerance (1e-3) rules out 16-bit operands.
 //
-// v_mfma_f32_32x32x2_f32 contracts over two indices per instruction, one per lane half:
-// lane (c, hh) supplies A[c][k_hh] and B[k_hh][c], and leaves C[8g+4hh+r][c] in register
-// 4g+r.  Choosing (k_0, k_1) = (8g+r, 8g+4+r) makes register 4g+r of an accumulator tile
-// exactly the operand element the next product needs, so
-// the state tiles feed the state-term product straight from registers.  The LDS holds the block's inputs -- X and Y
-// token-major, (w (.) Y)^T and Z^T feature-major (XOR-swizzled 16-byte granules) -- and the masked 32 x 32 score tile,
-// of which each of the four waves computes one 16 x 16 quadrant (v_mfma_f32_16x16x4_f32).  Blocks are 32 tokens.
+// The matrix unit multiplies fp32 at a sixteenth of its bf16 rate, so every operand is split into three bf16 numbers,
+// x = h + m + l: h is x cut off after 8 bits, m what is left rounded to 8 bits, l the rest, and |x - h - m - l| <= 2^-25 |x|, no
+// more than fp32 itself rounds x by.  A product is the six of the nine partial products that reach 2^-24 of the whole, the small
+// ones first, in the unit's fp32 accumulators; m l and l m, left out, are of either sign and 2^-25 of a term as a rule (2^-23 at
+// most).  Sums of a few wide products round less often than sums of many narrow ones: the errors against 64 bits (2-norms) are
+// 0.71 - 0.83 of those with v_mfma_f32_32x32x2_f32, used before (n = 64 ... 7168, with and without states, 2.3e-7 against 2.9e-7
+// at b*h = 24, n = 2048).  All finite numbers are taken; an infinite one makes NaN of what it takes part in, where the fp32
+// instruction could leave an infinity.
 //
-// What bounds it: the fp32 matrix rate.  A block costs a wave 160 products of 32x32x2 (64 state term, 64 state
-// update, 16 intra-block, and 16 products' time for its quadrant of the scores) = 10 240 cycles; with every wave
-// computing the whole score tile, as before, it was 208.  Two barriers a block: the X and Y tiles of the next block are
-// written while this one's second half runs, its transposed tiles while the next one's first half does, so no fill
-// stands between two barriers.  b*h = 24, n = 2048, forward + backward: 238 us against 275 (forward sweep 57 us against
-// 63, backward 131 against 149); b*h = 24, n = 16384: 1384 against 1555, 71 % of the time the fp32 products alone take.
-// Operands are read one step of products ahead, and nothing in a block branches (a masked quadrant of the scores, rows that
-// a partial block lacks): 231 us against 238 at b*h = 24, n = 2048.
+// The state tiles feed the state-term product straight from registers (see the order of features below), each split anew for
+// every block.  The LDS holds the X and Y rows of a block, split, and the masked 32 x 32 score tile, split, of which each of the
+// four waves computes one 16 x 16 quadrant (v_mfma_f32_16x16x32_bf16); a wave's 32 columns of Z, which no other wave
+// needs, come from memory in operand order.  The scaled Y^T of the state update is not made: its operands are read from the Y
+// rows with the transposing LDS read, and the decay goes to Z instead.  Blocks are 32 tokens.
+//
+// What bounds it: a wave and block take 132 matrix instructions (3840 cycles of its SIMD's matrix unit) and some 870 others on
+// the vector unit, two thirds of them for splitting; one of those costs about 4 cycles of issue and a matrix instruction 11, so
+// that a block cannot take less than 4900 cycles.  It takes 8100 (two workgroups per CU, n = 16384).  The splitting stands between
+// the matrix instructions, one by one: 9200 with each operand split in one go.  Against v_mfma_f32_32x32x2_f32 (10 240
+// cycles of matrix unit per block), forward + backward: b*h = 24, n = 2048: 170 - 180 us against 231; n = 16384: 1034
+// against 1384.
 #include "lasp_common.h"
 
 namespace lasp {
 namespace {
 
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 
 constexpr int F = 128;
 constexpr int BLK = 32;
 constexpr int NTHR = 256;
-constexpr int LDN = 528;   // bytes per token-major row (512 + 16: consecutive rows shift 4 banks)
-constexpr int LDT = 128;   // bytes per feature-major row (32 tokens)
-constexpr int OFF_XN = 0;
-constexpr int OFF_YN = OFF_XN + BLK * LDN;
-constexpr int OFF_YT = OFF_YN + BLK * LDN;
-constexpr int OFF_ZT = OFF_YT + F * LDT;
-constexpr int LDSC = 144;                    // bytes per row of the score tile (128 + 16), row = token of X
-constexpr int OFF_SC = OFF_ZT + F * LDT;
-constexpr int APPLY_LDS = OFF_SC + BLK * LDSC;  // 71168 B: two workgroups per CU
+constexpr int ROW = 2 * F;           // bytes per row of one part of a tile (128 bf16)
+constexpr int PART = BLK * ROW;      // h, m and l of a tile lie PART bytes apart
+constexpr int TILE = 3 * PART;
+constexpr int SC_ROW = 2 * BLK;      // the score tile: a row per token of X, 32 tokens of Y
+constexpr int SC_PART = BLK * SC_ROW;
+constexpr int OFF_X = 0, OFF_Y = TILE, OFF_SC = 2 * TILE;
+constexpr int OFF_W = OFF_SC + 3 * SC_PART;  // the decay between each token of a block and the state that the block leaves
+constexpr int OFF_Z = OFF_W + BLK * 4;        // each wave's columns of Z, parked
+constexpr int APPLY_LDS = OFF_Z + BLK * F * 4;  // 71 808 B: two workgroups per CU
 constexpr float LOG2E = 1.4426950408889634f;
 
 __device__ __forceinline__ float decay(float s_log2e, float x) {
   return __builtin_amdgcn_exp2f(-s_log2e * x);
 }
-__device__ __forceinline__ f32x4 lds16(const char *p) { return *reinterpret_cast<const f32x4 *>(p); }
-__device__ __forceinline__ floatx16 mfma(float a, float b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+// of arguments that are the same for every lane, in a scalar register
+__device__ __forceinline__ float uniform_decay(float s_log2e, float x) {
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(decay(s_log2e, x))));
 }
-__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+__device__ __forceinline__ u32x4 lds16(const char *p) { return *reinterpret_cast<const u32x4 *>(p); }
+
+// Eight numbers as three bf16 parts each
+struct Split {
+  u32x4 h, m, l;
+};
+__device__ __forceinline__ uint32_t pack(float lo, float hi) {
+  float2_t v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+}
+__device__ __forceinline__ float high_half(uint32_t x) { return __uint_as_float(x & 0xffff0000u); }
+// h is cut off, not rounded, which would turn the largest finite numbers into infinities
+__device__ __forceinline__ void split2(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l) {
+  const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+  h = __builtin_amdgcn_perm(y, x, 0x07060302);  // their upper halves
+  a -= high_half(x);
+  b -= high_half(y);
+  m = pack(a, b);
+  a -= __uint_as_float(m << 16);
+  b -= high_half(m);
+  l = pack(a, b);
+}
+// numbers 2 i and 2 i + 1 of eight, here and not where they are used
+__device__ __forceinline__ void split_pair(Split &s, int i, float a, float b) {
+  uint32_t h, m, l;
+  split2(a, b, h, m, l);
+  asm volatile("" : "+v"(h), "+v"(m), "+v"(l));
+  s.h[i] = h;
+  s.m[i] = m;
+  s.l[i] = l;
+}
+__device__ __forceinline__ floatx16 mfma(u32x4 a, u32x4 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ floatx4 mfma(u32x4 a, u32x4 b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+// c + a b.  A product of 32 x 32 x 16 keeps the matrix unit busy for 32 cycles, in which the wave that issued it can issue eight
+// instructions to the vector unit; the scheduler would have all six products wait for all of the next operand's splitting and
+// the splitting for the products.  work(i) goes behind product i and stays there.
+template <class C, class Work>
+__device__ __forceinline__ C product(const Split &a, const Split &b, C c, Work &&work) {
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    const u32x4 x = i == 0 ? a.l : i == 2 || i == 3 ? a.m : a.h, y = i == 1 ? b.l : i == 2 || i == 4 ? b.m : b.h;
+    c = mfma(x, y, c);
+    work(i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  return c;
 }
 
-// byte offset of 16-byte granule g16 (4 tokens) of feature row f.  The XOR term is a bijection
-// both of f bits 0-2 (rows read by 8 consecutive lanes) and of f bits 2-4 (rows written by 8
-// consecutive loader lanes), so 16-byte reads and writes are bank-conflict free.
-__device__ __forceinline__ int tr_off(int f, int g16) {
-  const int sw = ((f & 3) ^ ((f >> 3) & 3)) | (f & 4);
-  return f * LDT + (((g16 ^ sw) & 7) << 4);
+// Rows of the X and Y tiles.  A 16-byte unit holds eight features: of each group of 16, unit 0 has features 0-3 and 8-11, unit 1
+// features 4-7 and 12-15, which is the order in which lane half hh = 0, 1 of an accumulator tile holds rows (8 g + 4 hh + r in
+// register 4 g + r), so that an accumulator tile is multiplied against rows without a shuffle.  Unit u of row r lies at unit
+// u ^ swizzle(r): eight consecutive rows read at one unit, and the four rows x 64 bytes that half a wave reads transposed,
+// fall on disjoint banks.
+__device__ __forceinline__ int swizzle(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+// 16 bytes at `off` of a tile's three parts
+__device__ __forceinline__ Split parts(const char *tile, int off, int part) {
+  return {lds16(tile + off), lds16(tile + off + part), lds16(tile + off + 2 * part)};
 }
+typedef short v4i16 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4i16 *lds_v4i16;
+// The transposing 8-byte read works in groups of 16 lanes: lane i of a group receives, as element j, element (i % 4) of what
+// lane (4 j + i / 4) of the group addressed.  With lane s addressing token T + s / 4, features f + 4 (s % 4) .. + 3, lane i ends
+// up with feature f + i of tokens T .. T + 3; two such reads are eight tokens.
+__device__ __forceinline__ u32x4 transposed(const char *lo, const char *hi) {
+  const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(lo)));
+  const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(hi)));
+  return {a.x, a.y, b.x, b.y};
+}
+// Operand of lane (c, hh) over tokens: features 32 T + c of tokens 16 u + 8 hh .. + 7 of a tile
+struct TokenReader {
+  int lo, hi;  // the lane's offsets in the first 32 features and 16 tokens
+  __device__ __forceinline__ explicit TokenReader(int lane) {
+    const int s = lane & 15, ch = (lane >> 4) & 1, hh = lane >> 5, p = s & 3;
+    const int row = 8 * hh + (s >> 2), unit = 2 * ch + (p & 1);
+    lo = row * ROW + ((unit ^ swizzle(row)) << 4) + ((p >> 1) << 3);
+    hi = (row + 4) * ROW + ((unit ^ swizzle(row + 4)) << 4) + ((p >> 1) << 3);
+  }
+  __device__ __forceinline__ Split read(const char *tile, int T, int u) const {
+    const char *a = tile + (lo ^ (T << 6)) + 16 * u * ROW, *b = tile + (hi ^ (T << 6)) + 16 * u * ROW;
+    return {transposed(a, b), transposed(a + PART, b + PART), transposed(a + 2 * PART, b + 2 * PART)};
+  }
+};
 
 // Nothing is moved across this line: the reads above it are in flight while the products below run.  (The scheduler by itself
 // reads an operand right before the product that needs it.)
@@ -88,7 +172,7 @@ struct SegWork {
 };
 __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
   SegWork r;
-  r.bh = item / g.n_seg;
+  r.bh = quotient(item, g.by_seg);
   r.seg = item - r.bh * g.n_seg;
   r.tok0 = (int64_t)r.seg * g.seg_len;
   int64_t t1 = r.tok0 + g.seg_len;
@@ -99,19 +183,45 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
   return r;
 }
 
-// four rows (tokens 4*rq .. +3) x four features (4*cq .. +3), written feature-major:
-// one 16-byte store per feature, holding the four tokens scaled by w[r]
-__device__ __forceinline__ void store_transposed(char *tile, const f32x4 (&rows)[4], int cq, int rq,
-                                                 const float (&w)[4]) {
-#pragma unroll
-  for (int x = 0; x < 4; ++x) {
-    f32x4 out;
-    out.x = rows[0][x] * w[0];
-    out.y = rows[1][x] * w[1];
-    out.z = rows[2][x] * w[2];
-    out.w = rows[3][x] * w[3];
-    *reinterpret_cast<f32x4 *>(tile + tr_off(4 * cq + x, rq)) = out;
+// The X (or Y) rows of a block: thread (cq, rq) holds features 4 cq .. + 3 of rows rq + 8 it
+struct Loader {
+  int from, to;  // the thread's place in a block of rows and in a tile
+  __device__ __forceinline__ explicit Loader(int tid) {
+    const int cq = tid & 31, rq = tid >> 5, p = cq & 3;
+    from = rq * (F * 4) + cq * 16;
+    to = rq * ROW + (((2 * (cq >> 2) + (p & 1)) ^ swizzle(rq)) << 4) + ((p >> 1) << 3);
   }
+  __device__ __forceinline__ void load(rows_t rows, f32x4 (&n)[4]) const {
+#pragma unroll
+    for (int it = 0; it < 4; ++it) n[it] = load16(rows, from + it * (8 * F * 4));
+  }
+  // half `k & 1` of row k >> 1, into `row`; the second half writes the row
+  __device__ __forceinline__ void fill_half(char *tile, const f32x4 (&n)[4], int k, u32x2 (&row)[3]) const {
+    const int it = k >> 1, half = k & 1;
+    uint32_t h, m, l;
+    if (half == 0)
+      split2(n[it].x, n[it].y, h, m, l);
+    else
+      split2(n[it].z, n[it].w, h, m, l);
+    row[0][half] = h;
+    row[1][half] = m;
+    row[2][half] = l;
+    if (half == 0) return;
+    char *at = tile + (to ^ ((it & 1) << 5)) + it * (8 * ROW);  // (eight rows on, bit 1 of the swizzle flips)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x2 *>(at + i * PART) = row[i];
+  }
+  __device__ __forceinline__ void fill(char *tile, const f32x4 (&n)[4]) const {
+    u32x2 row[3];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) fill_half(tile, n, k, row);
+  }
+};
+// A wave's own 32 columns of Z come straight from memory: lane (c, hh) holds tokens 16 u + 8 hh + j of column c in z[8 u + j]
+__device__ __forceinline__ void load_columns(rows_t rows, int lane_off, float (&z)[16]) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    z[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, lane_off + (16 * (i >> 3) + (i & 7)) * (F * 4), 0, 0));
 }
 
 // RAGGED: the chunk length is not a multiple of 32, so the last block of the last segment is
@@ -119,29 +229,58 @@ __device__ __forceinline__ void store_transposed(char *tile, const f32x4 (&rows)
 // comes first -- the entering state sits `len` tokens ahead instead of 32).
 template <bool REV, bool TRANS, bool RAGGED>
 __device__ __forceinline__ void
-apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float *__restrict__ Z,
+sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float *__restrict__ Z,
            const float *__restrict__ S, const float *__restrict__ states, float *__restrict__ Out,
            const Geom &g, int item, char *smem) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform: keeps it in an SGPR
   const int c = lane & 31, hh = lane >> 5;
-  const int cq = tid & 31, rq = tid >> 5;  // loader: 16-byte column, row (X) / group of four rows (Y, Z)
 
   const SegWork sw = seg_work(g, item);
-  const float sl = S[sw.bh % g.h] * LOG2E;
   const int64_t base = ((int64_t)sw.bh * g.n + sw.tok0) * F;
+  const Loader loader(tid);
+  const TokenReader tokens(lane);
+  const int z_off = 8 * hh * (F * 4) + (32 * w + c) * 4;
 
+  f32x4 nx[4], ny[4];
+  float z[16];
+  auto len_of = [&](int blk) __attribute__((always_inline)) { return RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK; };
+  auto rows = [&](const float *p, int blk) __attribute__((always_inline)) {
+    return rows_of(p + base + (int64_t)blk * (BLK * F), len_of(blk));
+  };
+  // the block after this one, or none of its rows where there is none: as many accesses in flight on every path
+  auto next_rows = [&](const float *p, bool more, int blk) __attribute__((always_inline)) {
+    return rows_of(p + base + (int64_t)blk * (BLK * F), more ? len_of(blk) : 0);
+  };
+  const int first = REV ? sw.nblk - 1 : 0;
+  const int step = REV ? -1 : 1;
+  loader.load(rows(X, first), nx);
+  loader.load(rows(Y, first), ny);
+  load_columns(rows(Z, first), z_off, z);
+
+  const float sl = S[sw.bh - quotient(sw.bh, g.by_h) * g.h] * LOG2E;
   // ---- constants (all exponents <= 0)
-  const float blockdec = decay(sl, (float)BLK);
+  const float blockdec = uniform_decay(sl, (float)BLK);
   const float qdec = decay(sl, REV ? (float)(BLK - c) : (float)c);
-  float kdec[4], ones[4];
+  if (tid < BLK) *reinterpret_cast<float *>(smem + OFF_W + 4 * tid) = decay(sl, REV ? (float)tid : (float)(BLK - tid));
+  // this wave's quadrant of the score tile: tokens b = 16 qb .. of Y, a = 16 qa .. of X
+  const int qb = w >> 1, qa = w & 1;
+  const bool q_active = REV ? !(qb == 0 && qa == 1) : !(qb == 1 && qa == 0);
+  const int q_lane = lane & 15, q_grp = lane >> 4;
+  const int xq = (16 * qa + q_lane) * ROW + ((q_grp ^ swizzle(16 * qa + q_lane)) << 4);
+  const int yq = (16 * qb + q_lane) * ROW + ((q_grp ^ swizzle(16 * qb + q_lane)) << 4);
+  float qmask[4];  // decay between the tokens of a score
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int b = 4 * rq + r;
-    kdec[r] = decay(sl, REV ? (float)b : (float)(BLK - b));
-    ones[r] = 1.f;
+    const int dist = (16 * qa + q_lane - 16 * qb - 4 * q_grp - r) * (REV ? -1 : 1);
+    qmask[r] = dist >= 0 ? decay(sl, (float)dist) : 0.f;
   }
+  // rows of 64 bytes; unit u of row a lies at u ^ ((a >> 2) & 3)
+  const int sc_at = (16 * qa + q_lane) * SC_ROW + (((2 * qb + (q_grp >> 1)) ^ ((q_lane >> 2) & 3)) << 4) + ((q_grp & 1) << 3);
+  const int sc_from = c * SC_ROW + ((hh ^ ((c >> 2) & 3)) << 4);
+  char *const z_park = smem + OFF_Z + w * 4096 + lane * 16;
+  const int x_from = c * ROW + ((hh ^ swizzle(c)) << 4);
 
   // ---- state entering the segment: st[T][4g+r] = St[32T+8g+4hh+r][32w+c]
   floatx16 st[4];
@@ -161,137 +300,127 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
 #pragma unroll
       for (int r = 0; r < 16; ++r) st[T][r] = 0.f;
   }
-
-  f32x4 nx[4], ny[4], nz[4];
-  auto len_of = [&](int blk) __attribute__((always_inline)) { return RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK; };
-  auto issue_loads = [&](int blk) __attribute__((always_inline)) {
-    const int64_t off = base + (int64_t)blk * (BLK * F);
-    const rows_t x = rows_of(X + off, len_of(blk)), y = rows_of(Y + off, len_of(blk)), z = rows_of(Z + off, len_of(blk));
-#pragma unroll
-    for (int it = 0; it < 4; ++it) nx[it] = load16(x, (rq + 8 * it) * (F * 4) + cq * 16);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      ny[r] = load16(y, (4 * rq + r) * (F * 4) + cq * 16);
-      nz[r] = load16(z, (4 * rq + r) * (F * 4) + cq * 16);
-    }
-  };
-  auto fill_rows = [&]() __attribute__((always_inline)) {  // X and Y as they are
-#pragma unroll
-    for (int it = 0; it < 4; ++it)
-      *reinterpret_cast<f32x4 *>(smem + OFF_XN + (rq + 8 * it) * LDN + cq * 16) = nx[it];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      *reinterpret_cast<f32x4 *>(smem + OFF_YN + (4 * rq + r) * LDN + cq * 16) = ny[r];
-  };
-  auto fill_transposed = [&]() __attribute__((always_inline)) {  // (w (.) Y)^T and Z^T
-    store_transposed(smem + OFF_YT, ny, cq, rq, kdec);
-    store_transposed(smem + OFF_ZT, nz, cq, rq, ones);
-  };
-  // this wave's quadrant of the score tile: tokens b = 16 qb .. of Y, a = 16 qa .. of X
-  const int qb = w >> 1, qa = w & 1;
-  const int q_lane = lane & 15, q_grp = lane >> 4;
-
-  const int first = REV ? sw.nblk - 1 : 0;
-  const int step = REV ? -1 : 1;
-  issue_loads(first);
-  fill_rows();
-  fill_transposed();
-  if (sw.nblk > 1) issue_loads(first + step);
+  loader.fill(smem + OFF_X, nx);
+  loader.fill(smem + OFF_Y, ny);
   __syncthreads();
 
   for (int it = 0, blk = first; it < sw.nblk; ++it, blk += step) {
     const bool more = it + 1 < sw.nblk;
-    if (it > 0) {
-      fill_transposed();  // of this block; read after the first barrier
-      if (more) issue_loads(blk + step);
-    }
     const int len = len_of(blk);
     float qd = qdec, bd = blockdec;
     if (RAGGED && REV && len != BLK) {
       qd = decay(sl, (float)max(len - c, 0));
-      bd = decay(sl, (float)len);
+      bd = uniform_decay(sl, (float)len);
     }
 
-    // (1) scores of the quadrant and state term
-    //     sc[r]     = y_b . x_a,                          b = 16 qb + 4 q_grp + r, a = 16 qa + q_lane
-    //     acc[4g+r] = sum_f St[f][32w+8g+4hh+r] x_a[f]    (a = c)
-    // (the scores contract features 16 m + 4 q_grp + r over q_grp, in that order on both sides)
+    // Z as the state update takes it, between the products of the scores
+    Split zs[2];
+    f32x4 wz[4];  // (kept in LDS: registers are short here)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wz[i] = *reinterpret_cast<const f32x4 *>(smem + OFF_W + (16 * (i >> 1) + 8 * hh + 4 * (i & 1)) * 4);
+    auto scale_z = [&](int i) __attribute__((always_inline)) {  // pair i of 8
+      const f32x4 &v = wz[i >> 1];
+      const float w0 = (i & 1) ? v.z : v.x, w1 = (i & 1) ? v.w : v.y;
+      split_pair(zs[i >> 2], i & 3, z[2 * i] * w0, z[2 * i + 1] * w1);
+    };
+    // (1) scores of the quadrant, masked: sc[r] = y_b . x_a, b = 16 qb + 4 q_grp + r, a = 16 qa + q_lane
+    Split xf[2], yf[2];
+    {
+      floatx4 sc = {0.f, 0.f, 0.f, 0.f};
+      Split ys[2], xs[2];
+      xs[0] = parts(smem + OFF_X, xq, PART);
+      ys[0] = parts(smem + OFF_Y, yq, PART);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        if (m < 3) {
+          xs[(m + 1) & 1] = parts(smem + OFF_X, xq ^ ((m + 1) << 6), PART);
+          ys[(m + 1) & 1] = parts(smem + OFF_Y, yq ^ ((m + 1) << 6), PART);
+        } else {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) xf[u] = parts(smem + OFF_X, x_from ^ (u << 5), PART);
+        }
+        reads_first();
+        sc = product(ys[m & 1], xs[m & 1], sc, [&](int i) __attribute__((always_inline)) {
+          if (i % 3 == 0) scale_z(2 * m + i / 3);
+        });
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) yf[u] = tokens.read(smem + OFF_Y, 0, u);
+      // z is wanted once more, for the intra-block term; until then it gives its registers away
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4 *>(z_park + 1024 * i) = f32x4{z[4 * i], z[4 * i + 1], z[4 * i + 2], z[4 * i + 3]};
+      reads_first();
+      u32x2 h, m, l;
+      uint32_t a, b, d;
+      split2(sc[0] * qmask[0], sc[1] * qmask[1], a, b, d);
+      h.x = a, m.x = b, l.x = d;
+      split2(sc[2] * qmask[2], sc[3] * qmask[3], a, b, d);
+      h.y = a, m.y = b, l.y = d;
+      char *at = smem + OFF_SC + sc_at;
+      *reinterpret_cast<u32x2 *>(at) = h;
+      *reinterpret_cast<u32x2 *>(at + SC_PART) = m;
+      *reinterpret_cast<u32x2 *>(at + 2 * SC_PART) = l;
+    }
+    // (2) state term, acc[4g+r] = sum_f St[f][32w+8g+4hh+r] x_a[f] (a = c), and (3) the state update, 32 features at a time
     floatx16 acc;
-    f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    {
-      const char *xp = smem + OFF_XN + c * LDN + hh * 16;
-      const char *xq = smem + OFF_XN + (16 * qa + q_lane) * LDN + q_grp * 16;
-      const char *yq = smem + OFF_YN + (16 * qb + q_lane) * LDN + q_grp * 16;
-      f32x4 ys[2], xs[2], x0[2], x1[2];
-      auto fetch = [&](int m) __attribute__((always_inline)) {  // features 16m + 4hh + .., 16m + 8 + 4hh + .. of X
-        x0[m & 1] = lds16(xp + m * 64);
-        x1[m & 1] = lds16(xp + m * 64 + 32);
-        ys[m & 1] = lds16(yq + m * 64);
-        xs[m & 1] = lds16(xq + m * 64);
-      };
-      fetch(0);
+    loader.load(next_rows(X, more, blk + step), nx);
+    Split a0, a1, zu[2];
+    f32x4 zp[4];
 #pragma unroll
-      for (int m = 0; m < 8; ++m) {
-        if (m < 7) fetch(m + 1);
-        reads_first();
-        // (the wave whose quadrant is wholly masked computes it as well: it would only wait for the others)
+    for (int i = 0; i < 4; ++i) split_pair(a0, i, st[0][2 * i], st[0][2 * i + 1]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          acc = mfma(st[m >> 1][8 * (m & 1) + r], x0[m & 1][r], acc);
-          sc = mfma16(ys[m & 1][r], xs[m & 1][r], sc);
-        }
+    for (int T = 0; T < 4; ++T) {
+      acc = product(a0, xf[0], acc, [&](int i) __attribute__((always_inline)) {
+        if (i < 4) split_pair(a1, i, st[T][8 + 2 * i], st[T][9 + 2 * i]);
+      });
+      acc = product(a1, xf[1], acc, [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc = mfma(st[m >> 1][8 * (m & 1) + 4 + r], x1[m & 1][r], acc);
+        for (int r = 3 * i; r < 3 * i + 3 && r < 16; ++r) st[T][r] *= bd;
+      });
+      if (T < 3) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) xf[u] = parts(smem + OFF_X, x_from ^ ((2 * T + 2 + u) << 5), PART);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) zp[i] = *reinterpret_cast<const f32x4 *>(z_park + 1024 * i);
+      }
+      reads_first();
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        st[T] = product(yf[u], zs[u], st[T], [&](int i) __attribute__((always_inline)) {
+          if (T < 3) {
+            if (u == 0 && i < 4) split_pair(a0, i, st[T + 1][2 * i], st[T + 1][2 * i + 1]);
+          } else if (i < 4) {
+            const f32x4 &v = zp[2 * u + (i >> 1)];
+            split_pair(zu[u], i, (i & 1) ? v.z : v.x, (i & 1) ? v.w : v.y);
+          }
+        });
+        if (T < 3) yf[u] = tokens.read(smem + OFF_Y, T + 1, u);
         reads_first();
       }
-    }
-    // (2) mask the scores, scale the state term
-    {
-      const int a = 16 * qa + q_lane, b0 = 16 * qb + 4 * q_grp;
-      f32x4 m;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int dist = REV ? b0 + r - a : a - b0 - r;
-        m[r] = dist >= 0 ? sc[r] * decay(sl, (float)dist) : 0.f;
-      }
-      *reinterpret_cast<f32x4 *>(smem + OFF_SC + a * LDSC + b0 * 4) = m;
+      if (T == 1) loader.load(next_rows(Y, more, blk + step), ny);
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] *= qd;
-    __syncthreads();  // the score tile and the transposed tiles are complete; X and Y are no longer read
-    if (more) fill_rows();  // of the next block
-    // (3) intra-block term and (4) state update share the Z^T elements
-    f32x4 zf[4], sf[4];
+    __syncthreads();  // the score tile is complete; X and Y are no longer read
+    // (4) intra-block term
+    {
+      Split sf[2];
 #pragma unroll
-    for (int gq = 0; gq < 4; ++gq) {
-      zf[gq] = lds16(smem + OFF_ZT + tr_off(32 * w + c, 2 * gq + hh));
-      sf[gq] = lds16(smem + OFF_SC + c * LDSC + (8 * gq + 4 * hh) * 4);
-    }
-    f32x4 yt[2][4];
-    auto fetch_y = [&](int T) __attribute__((always_inline)) {
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) yt[T & 1][gq] = lds16(smem + OFF_YT + tr_off(32 * T + c, 2 * gq + hh));
-    };
-    fetch_y(0);
-    reads_first();
-#pragma unroll
-    for (int gq = 0; gq < 4; ++gq)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc = mfma(zf[gq][r], sf[gq][r], acc);
-#pragma unroll
-    for (int T = 0; T < 4; ++T) {
-      if (T < 3) fetch_y(T + 1);
+      for (int u = 0; u < 2; ++u) sf[u] = parts(smem + OFF_SC, sc_from ^ (u << 5), SC_PART);
+      load_columns(next_rows(Z, more, blk + step), z_off, z);
       reads_first();
+      u32x2 row[3];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) st[T][r] *= bd;
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) st[T] = mfma(yt[T & 1][gq][r], zf[gq][r], st[T]);
-      reads_first();
+      for (int u = 0; u < 2; ++u)
+        acc = product(zu[u], sf[u], acc, [&](int i) __attribute__((always_inline)) {  // and the next block's X
+          if (6 * u + i < 8) loader.fill_half(smem + OFF_X, nx, 6 * u + i, row);
+        });
     }
+    loader.fill(smem + OFF_Y, ny);
     // (5) output: lane (c, hh) holds, for token c, four consecutive columns per g
     const rows_t out = rows_of(Out + base + (int64_t)blk * (BLK * F), len);
 #pragma unroll
@@ -303,7 +432,7 @@ apply_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       o.w = acc[4 * gq + 3];
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), out, c * (F * 4) + (32 * w + 4 * hh + 8 * gq) * 4, 0, 0);
     }
-    if (more) __syncthreads();  // the next block's X and Y are complete; this block's transposed tiles are no longer read
+    if (more) __syncthreads();  // the next block's X and Y are complete; the score tile is no longer read
   }
 }
 
@@ -312,7 +441,7 @@ __global__ void __launch_bounds__(NTHR, 2)
 la32_apply(const float *__restrict__ X, const float *__restrict__ Y, const float *__restrict__ Z,
            const float *__restrict__ S, const float *__restrict__ states, float *__restrict__ Out, Geom g) {
   extern __shared__ __align__(16) char smem[];
-  apply_body<REV, TRANS, RAGGED>(X, Y, Z, S, states, Out, g, (int)blockIdx.x, smem);
+  sweep_body<REV, TRANS, RAGGED>(X, Y, Z, S, states, Out, g, (int)blockIdx.x, smem);
 }
 
 // dQ, dV and dK in one launch; the three workgroups of a (b*h, segment) sit 8 block indices
@@ -330,11 +459,11 @@ la32_bwd3(const float *__restrict__ Q, const float *__restrict__ K, const float 
   const int item = n_items - 1 - (grp * 8 + (r & 7));
   if (item < 0) return;
   if (role == 0)
-    apply_body<false, true, RAGGED>(DO, V, K, S, kv_states, DQ, g, item, smem);
+    sweep_body<false, true, RAGGED>(DO, V, K, S, kv_states, DQ, g, item, smem);
   else if (role == 1)
-    apply_body<true, false, RAGGED>(K, Q, DO, S, dkv_states, DV, g, item, smem);
+    sweep_body<true, false, RAGGED>(K, Q, DO, S, dkv_states, DV, g, item, smem);
   else
-    apply_body<true, true, RAGGED>(V, DO, Q, S, dkv_states, DK, g, item, smem);
+    sweep_body<true, true, RAGGED>(V, DO, Q, S, dkv_states, DK, g, item, smem);
 }
 
 // a segment's own state: causal sum_b l^(L-b) y_b^T z_b ; anti-causal sum_b l^b y_b^T z_b
@@ -342,91 +471,76 @@ template <bool REV, bool RAGGED>
 __global__ void __launch_bounds__(NTHR, 2)
 la32_seg_state(const float *__restrict__ Y, const float *__restrict__ Z, const float *__restrict__ S,
                float *__restrict__ states, Geom g, int skip_seg) {
-  __shared__ __align__(16) char smem[2][2 * F * LDT];  // double-buffered {(w (.) Y)^T, Z^T}
+  __shared__ __align__(256) char smem[2][TILE];  // double-buffered Y
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform: keeps it in an SGPR
   const int c = lane & 31, hh = lane >> 5;
-  const int cq = tid & 31, rq = tid >> 5;
 
   const SegWork sw = seg_work(g, (int)blockIdx.x);
   if (sw.seg == skip_seg) return;
-  const float sl = S[sw.bh % g.h] * LOG2E;
   const int64_t base = ((int64_t)sw.bh * g.n + sw.tok0) * F;
+  const Loader loader(tid);
+  const TokenReader tokens(lane);
+  const int z_off = 8 * hh * (F * 4) + (32 * w + c) * 4;
+  auto len_of = [&](int blk) __attribute__((always_inline)) { return RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK; };
+  auto rows = [&](const float *p, int blk) __attribute__((always_inline)) {
+    return rows_of(p + base + (int64_t)blk * (BLK * F), len_of(blk));
+  };
+  f32x4 ny[4];
+  float z[16];
+  const int first = REV ? sw.nblk - 1 : 0;
+  const int step = REV ? -1 : 1;
+  loader.load(rows(Y, first), ny);
+  load_columns(rows(Z, first), z_off, z);
 
-  const float blockdec = decay(sl, (float)BLK);
-  float kdec[4], ones[4];
+  const float sl = S[sw.bh - quotient(sw.bh, g.by_h) * g.h] * LOG2E;
+  const float blockdec = uniform_decay(sl, (float)BLK);
+  float zdec[16];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int b = 4 * rq + r;
-    kdec[r] = decay(sl, REV ? (float)b : (float)(BLK - b));
-    ones[r] = 1.f;
+  for (int i = 0; i < 16; ++i) {
+    const int b = 16 * (i >> 3) + 8 * hh + (i & 7);
+    zdec[i] = decay(sl, REV ? (float)b : (float)(BLK - b));
   }
   floatx16 st[4];
 #pragma unroll
   for (int T = 0; T < 4; ++T)
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[T][r] = 0.f;
-
-  f32x4 ny[4], nz[4];
-  auto issue_loads = [&](int blk) __attribute__((always_inline)) {
-    const int64_t off = base + (int64_t)blk * (BLK * F);
-    const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
-    const rows_t y = rows_of(Y + off, len), z = rows_of(Z + off, len);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      ny[r] = load16(y, (4 * rq + r) * (F * 4) + cq * 16);
-      nz[r] = load16(z, (4 * rq + r) * (F * 4) + cq * 16);
-    }
-  };
-  // going forwards a partial block is the last one: its tokens sit `len - b` before the segment end
-  auto fill_lds = [&](int buf, int blk) __attribute__((always_inline)) {
-    const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
-    if (RAGGED && !REV && len != BLK) {
-      float kd[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) kd[r] = decay(sl, (float)max(len - (4 * rq + r), 0));
-      store_transposed(smem[buf], ny, cq, rq, kd);
-    } else {
-      store_transposed(smem[buf], ny, cq, rq, kdec);
-    }
-    store_transposed(smem[buf] + F * LDT, nz, cq, rq, ones);
-  };
-
-  const int first = REV ? sw.nblk - 1 : 0;
-  const int step = REV ? -1 : 1;
-  issue_loads(first);
-  fill_lds(0, first);
+  loader.fill(smem[0], ny);
   __syncthreads();
   for (int it = 0, blk = first; it < sw.nblk; ++it, blk += step) {
     const bool more = it + 1 < sw.nblk;
-    if (more) issue_loads(blk + step);
-    const int len = RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK;
-    const float bd = RAGGED && len != BLK ? decay(sl, (float)len) : blockdec;
-    const char *ytile = smem[it & 1];
-    const char *ztile = ytile + F * LDT;
-    f32x4 zf[4];
+    if (more) loader.load(rows(Y, blk + step), ny);
+    const int len = len_of(blk);
+    const float bd = RAGGED && len != BLK ? uniform_decay(sl, (float)len) : blockdec;
+    if (RAGGED && !REV && len != BLK)  // going forwards a partial block is the last one: its tokens sit `len - b` before the segment's end
 #pragma unroll
-    for (int gq = 0; gq < 4; ++gq) zf[gq] = lds16(ztile + tr_off(32 * w + c, 2 * gq + hh));
-    f32x4 yt[2][4];
-    auto fetch_y = [&](int T) __attribute__((always_inline)) {
+      for (int i = 0; i < 16; ++i) zdec[i] = decay(sl, (float)max(len - 16 * (i >> 3) - 8 * hh - (i & 7), 0));
+    const char *tile = smem[it & 1];
+    Split yf[2][2], zs[2];
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) yt[T & 1][gq] = lds16(ytile + tr_off(32 * T + c, 2 * gq + hh));
-    };
-    fetch_y(0);
+    for (int u = 0; u < 2; ++u) yf[0][u] = tokens.read(tile, 0, u);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) split_pair(zs[i >> 2], i & 3, z[2 * i] * zdec[2 * i], z[2 * i + 1] * zdec[2 * i + 1]);
+    if (more) load_columns(rows(Z, blk + step), z_off, z);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st[0][r] *= bd;
 #pragma unroll
     for (int T = 0; T < 4; ++T) {
-      if (T < 3) fetch_y(T + 1);
+      if (T < 3)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) yf[(T + 1) & 1][u] = tokens.read(tile, T + 1, u);
       reads_first();
 #pragma unroll
-      for (int r = 0; r < 16; ++r) st[T][r] *= bd;
+      for (int u = 0; u < 2; ++u)
+        st[T] = product(yf[T & 1][u], zs[u], st[T], [&](int i) __attribute__((always_inline)) {
+          if (T < 3 && u == 0)
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) st[T] = mfma(yt[T & 1][gq][r], zf[gq][r], st[T]);
-      reads_first();
+            for (int r = 3 * i; r < 3 * i + 3 && r < 16; ++r) st[T + 1][r] *= bd;
+        });
     }
-    if (more) fill_lds((it + 1) & 1, blk + step);
+    if (more) loader.fill(smem[(it + 1) & 1], ny);
     __syncthreads();
   }
   float *sp = states + ((int64_t)sw.bh * g.n_seg + sw.seg) * (F * F);
