@@ -217,6 +217,22 @@ int lasp_chunk_bwd_twin(const void *q, const void *k, const void *v, const float
                         int dtype, int seg_len, void *stream);
 
 /*
+ * The same calls on the fp32 MFMA kernels for float32 rows narrower than 128 features (d and e multiples of 4, at most
+ * 128), which lasp_chunk_fwd / lasp_chunk_bwd leave to the generic kernels.  Plan, workspaces, states, aliasing and errors
+ * are those of lasp_chunk_*; the forward's seg_states go to this backward.
+ */
+int lasp_narrow_fwd(const void *q, const void *k, const void *v, const float *s,
+                    const float *kv_in, float *kv_out, float *kv_twin, void *o, float *seg_states,
+                    int b, int h, int64_t n, int d, int e, int dtype, int seg_len,
+                    void *stream);
+int lasp_narrow_bwd(const void *q, const void *k, const void *v, const float *s,
+                    const void *d_o, const float *kv_in, const float *dkv_in,
+                    void *dq, void *dk, void *dv, float *dkv_out, float *dkv_twin,
+                    const float *kv_seg_states, float *workspace,
+                    size_t workspace_bytes, int b, int h, int64_t n, int d, int e,
+                    int dtype, int seg_len, void *stream);
+
+/*
  * Measurement hook (no counterpart in the reference, which times nothing).
  * Between lasp_profile_begin and lasp_profile_end every kernel the library
  * launches is bracketed by two hipEvents on its launch stream (at most

@@ -64,6 +64,10 @@ def load() -> ctypes.CDLL:
     lib.lasp_chunk_fwd_static.argtypes = [_c_void_p] * 7 + [_c_int, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_void_p]
     lib.lasp_chunk_bwd.restype = _c_int
     lib.lasp_chunk_bwd.argtypes = [_c_void_p] * 13 + [_c_size, _c_int, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_void_p]
+    lib.lasp_narrow_fwd.restype = _c_int
+    lib.lasp_narrow_fwd.argtypes = [_c_void_p] * 9 + [_c_int, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_void_p]
+    lib.lasp_narrow_bwd.restype = _c_int
+    lib.lasp_narrow_bwd.argtypes = [_c_void_p] * 14 + [_c_size, _c_int, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_void_p]
     lib.lasp_profile_begin.restype = _c_int
     lib.lasp_profile_begin.argtypes = [_c_int]
     lib.lasp_profile_end.restype = _c_int
@@ -222,12 +226,12 @@ class _on_device:
         return False
 
 
-def _chunk_fwd_exact(q, k, v, s, kv_in=None, kv_out=None, seg_len: int = 0):
+def _chunk_fwd_exact(q, k, v, s, kv_in=None, kv_out=None, seg_len: int = 0, narrow: bool = False):
     """Enqueues the forward of one chunk.  Returns (o, seg_states, seg_len).
 
     seg_states is the float32 array of states entering each segment, sized by
     lasp_plan (None when the call needed none); pass it to chunk_bwd to skip the
-    recompute.
+    recompute.  narrow: through lasp_narrow_fwd.
     """
     lib = load()
     dev = _check_dev(q, k, v, kv_in, kv_out)
@@ -249,9 +253,10 @@ def _chunk_fwd_exact(q, k, v, s, kv_in=None, kv_out=None, seg_len: int = 0):
             # the library decides how many states it keeps (one per segment, or per piece of a long segment)
             # and how each is stored (d x e, or zero-extended to 64 x 64 or 128 x 128): the array is opaque here
             states = torch.empty((state_bytes // 4,), dtype=torch.float32, device=dev)
-        rc = lib.lasp_chunk_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr(), _ptr(kv_in), _ptr(kv_out),
-                                o.data_ptr(), _ptr(states), b, h, n, d, e, DTYPE_CODE[q.dtype], seg_len,
-                                _raw_stream(dev))
+        outgoing = (_ptr(kv_out), None) if narrow else (_ptr(kv_out),)  # (no second place for the state)
+        rc = (lib.lasp_narrow_fwd if narrow else lib.lasp_chunk_fwd)(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr(), _ptr(kv_in), *outgoing, o.data_ptr(), _ptr(states),
+            b, h, n, d, e, DTYPE_CODE[q.dtype], seg_len, _raw_stream(dev))
     if rc:
         _raise(rc, "lasp_chunk_fwd")
     return o, states, seg_len
@@ -287,8 +292,9 @@ def chunk_fwd_static(q, k, v, s, o, kv_in=None, kv_out=None, seg_len: int = 0) -
         _raise(rc, "lasp_chunk_fwd_static")
 
 
-def _chunk_bwd_exact(q, k, v, s, do, kv_in=None, dkv_in=None, dkv_out=None, kv_seg_states=None, seg_len: int = 0):
-    """Enqueues the backward of one chunk.  Returns (dq, dk, dv)."""
+def _chunk_bwd_exact(q, k, v, s, do, kv_in=None, dkv_in=None, dkv_out=None, kv_seg_states=None, seg_len: int = 0,
+                     narrow: bool = False):
+    """Enqueues the backward of one chunk.  Returns (dq, dk, dv).  narrow: through lasp_narrow_bwd."""
     lib = load()
     dev = _check_dev(q, k, v, do, kv_in, dkv_in, dkv_out, kv_seg_states)
     b, h, n, d, e = _shapes(q, k, v)
@@ -320,10 +326,11 @@ def _chunk_bwd_exact(q, k, v, s, do, kv_in=None, dkv_in=None, dkv_out=None, kv_s
         need_kv = not fused and kv_seg_states is None and (n_seg > 1 or kv_in is not None)
         n_arrays = int(need_dkv) + int(need_kv)
         ws = torch.empty((n_arrays * state_bytes // 4,), dtype=torch.float32, device=dev) if n_arrays else None
-        rc = lib.lasp_chunk_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr(), do.data_ptr(), _ptr(kv_in),
-                                _ptr(dkv_in), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), _ptr(dkv_out),
-                                _ptr(kv_seg_states), _ptr(ws), n_arrays * state_bytes, b, h, n, d, e,
-                                DTYPE_CODE[q.dtype], seg_len, _raw_stream(dev))
+        outgoing = (_ptr(dkv_out), None) if narrow else (_ptr(dkv_out),)
+        rc = (lib.lasp_narrow_bwd if narrow else lib.lasp_chunk_bwd)(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), s.data_ptr(), do.data_ptr(), _ptr(kv_in), _ptr(dkv_in),
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *outgoing, _ptr(kv_seg_states), _ptr(ws), n_arrays * state_bytes,
+            b, h, n, d, e, DTYPE_CODE[q.dtype], seg_len, _raw_stream(dev))
     if rc:
         _raise(rc, "lasp_chunk_bwd")
     return dq, dk, dv
@@ -332,7 +339,7 @@ def _chunk_bwd_exact(q, k, v, s, do, kv_in=None, dkv_in=None, dkv_out=None, kv_s
 # ---------------------------------------------------------------------------------------
 # Narrow heads on the MFMA kernels.  The 16-bit MFMA kernels read rows of d, e <= 128 features
 # zero-extended when d and e are multiples of 8 (the reference's own test uses e = 64,
-# tests/test.py:95); the fp32 MFMA kernels take d = e = 128 only.  Any other narrow shape is
+# tests/test.py:95), the fp32 ones when they are multiples of 4 (lasp_narrow_*).  Any other narrow shape is
 # zero-padded to 128 here: zero feature columns add nothing to q.k, to the outputs or to the
 # states, so the results are exact, and the call runs an order of magnitude faster than on
 # the generic fp32-FMA kernels.  Everything else goes to the library unchanged.
@@ -343,7 +350,13 @@ def _pad_to_mfma(q, v) -> bool:
     d, e = q.shape[3], v.shape[3]
     if q.dtype not in DTYPE_CODE or d > _MFMA_F or e > _MFMA_F or (d == _MFMA_F and e == _MFMA_F):
         return False
-    return q.dtype == torch.float32 or d % 8 != 0 or e % 8 != 0
+    multiple = 4 if q.dtype == torch.float32 else 8
+    return d % multiple != 0 or e % multiple != 0 or (q.dtype == torch.float32 and min(d, e) == 0)
+
+
+def _narrow_rows(q, v) -> bool:
+    """float32 rows that the MFMA kernels read as they are, but not through lasp_chunk_* (which has the generic kernels for them)."""
+    return q.dtype == torch.float32 and not (q.shape[3] == _MFMA_F and v.shape[3] == _MFMA_F) and max(q.shape[3], v.shape[3]) <= _MFMA_F
 
 
 def _pad_last(t, size):
@@ -361,7 +374,8 @@ def _pad_state(t, d, e):
 def chunk_fwd(q, k, v, s, kv_in=None, kv_out=None, seg_len: int = 0):
     """Forward of one chunk: (o, seg_states, seg_len).  See _chunk_fwd_exact; narrow heads are padded."""
     if q.dim() != 4 or v.dim() != 4 or not _pad_to_mfma(q, v):
-        return _chunk_fwd_exact(q, k, v, s, kv_in, kv_out, seg_len)
+        narrow = q.dim() == 4 and v.dim() == 4 and _narrow_rows(q, v)
+        return _chunk_fwd_exact(q, k, v, s, kv_in, kv_out, seg_len, narrow)
     b, h, n, d, e = _shapes(q, k, v)
     _check_state("kv_in", kv_in, b, h, d, e)
     _check_state("kv_out", kv_out, b, h, d, e)
@@ -377,7 +391,8 @@ def chunk_bwd(q, k, v, s, do, kv_in=None, dkv_in=None, dkv_out=None, kv_seg_stat
     """Backward of one chunk: (dq, dk, dv).  See _chunk_bwd_exact; narrow heads are padded
     (kv_seg_states must then be what chunk_fwd returned for the same call)."""
     if q.dim() != 4 or v.dim() != 4 or not _pad_to_mfma(q, v):
-        return _chunk_bwd_exact(q, k, v, s, do, kv_in, dkv_in, dkv_out, kv_seg_states, seg_len)
+        narrow = q.dim() == 4 and v.dim() == 4 and _narrow_rows(q, v)
+        return _chunk_bwd_exact(q, k, v, s, do, kv_in, dkv_in, dkv_out, kv_seg_states, seg_len, narrow)
     b, h, n, d, e = _shapes(q, k, v)
     _check_state("kv_in", kv_in, b, h, d, e)
     _check_state("dkv_in", dkv_in, b, h, d, e)

@@ -78,6 +78,9 @@ bool mfma_f32_eligible(int d, int e, int dtype) {
   return dtype == LASP_DTYPE_F32 && d == kMaxFeature && e == kMaxFeature;
 }
 
+// The same kernels on narrower fp32 rows (lasp_narrow_fwd, lasp_narrow_bwd), fetched and stored 16 bytes at a time
+bool narrow_eligible(int d, int e, int dtype) { return dtype == LASP_DTYPE_F32 && d % 4 == 0 && e % 4 == 0; }
+
 int check_shape(int b, int h, int64_t n, int d, int e, int dtype) {
   if (dtype != LASP_DTYPE_F32 && dtype != LASP_DTYPE_BF16 && dtype != LASP_DTYPE_F16) {
     set_error("unknown dtype code %d", dtype);
@@ -577,7 +580,7 @@ int lasp_inplace_ok(int b, int h, int64_t n, int d, int e, int dtype, int seg_le
 
 static int chunk_fwd_impl(const char *me, const void *q, const void *k, const void *v, const float *s,
                           const float *kv_in, float *kv_out, void *o, float *seg_states, const Geom &g,
-                          int dtype, void *stream) {
+                          int dtype, void *stream, bool narrow = false) {
   int rc;
   if ((rc = check_alias(me, "kv", kv_in, kv_out, sizeof(float) * (size_t)g.b * g.h * g.dt * g.e, g, false))) return rc;
   if ((rc = check_aligned(me, "q", q, 16)) || (rc = check_aligned(me, "k", k, 16)) ||
@@ -592,7 +595,7 @@ static int chunk_fwd_impl(const char *me, const void *q, const void *k, const vo
   // (where a single launch leaves no segment states behind anyway, a few tokens take their own kernel)
   rc = step_eligible(g) && (g.fused || !seg_states) ? step_fwd(a, g, dtype, st)
        : mfma_eligible(g.dt, g.e, dtype)    ? mfma_fwd(a, g, dtype, st)
-       : mfma_f32_eligible(g.d, g.e, dtype) ? mfma_f32_fwd(a, g, st)
+       : narrow || mfma_f32_eligible(g.d, g.e, dtype) ? mfma_f32_fwd(a, g, st)
                                             : generic_fwd(a, g, dtype, st);
   if (rc > 0) set_error("%s: HIP error %d: %s", me, rc, hipGetErrorString((hipError_t)rc));
   return rc;
@@ -604,9 +607,9 @@ int lasp_chunk_fwd(const void *q, const void *k, const void *v, const float *s, 
   return lasp_chunk_fwd_twin(q, k, v, s, kv_in, kv_out, nullptr, o, seg_states, b, h, n, d, e, dtype, seg_len, stream);
 }
 
-int lasp_chunk_fwd_twin(const void *q, const void *k, const void *v, const float *s, const float *kv_in,
-                        float *kv_out, float *kv_twin, void *o, float *seg_states, int b, int h, int64_t n, int d, int e,
-                        int dtype, int seg_len, void *stream) {
+static int fwd_twin(const void *q, const void *k, const void *v, const float *s, const float *kv_in, float *kv_out,
+                    float *kv_twin, void *o, float *seg_states, int b, int h, int64_t n, int d, int e, int dtype, int seg_len,
+                    void *stream, bool narrow) {
   Geom g;
   int rc = make_geom(b, h, n, d, e, dtype, seg_len, &g);
   if (rc) return rc;
@@ -621,7 +624,27 @@ int lasp_chunk_fwd_twin(const void *q, const void *k, const void *v, const float
   }
   if ((rc = check_twin("lasp_chunk_fwd", "kv", kv_in, kv_out, kv_twin, sizeof(float) * (size_t)b * h * d * e))) return rc;
   g.twin = kv_twin;
-  return chunk_fwd_impl("lasp_chunk_fwd", q, k, v, s, kv_in, kv_out, o, seg_states, g, dtype, stream);
+  return chunk_fwd_impl("lasp_chunk_fwd", q, k, v, s, kv_in, kv_out, o, seg_states, g, dtype, stream, narrow);
+}
+
+int lasp_chunk_fwd_twin(const void *q, const void *k, const void *v, const float *s, const float *kv_in,
+                        float *kv_out, float *kv_twin, void *o, float *seg_states, int b, int h, int64_t n, int d, int e,
+                        int dtype, int seg_len, void *stream) {
+  return fwd_twin(q, k, v, s, kv_in, kv_out, kv_twin, o, seg_states, b, h, n, d, e, dtype, seg_len, stream, false);
+}
+
+static int check_narrow(const char *call, int d, int e, int dtype) {
+  if (narrow_eligible(d, e, dtype)) return 0;
+  set_error("%s: dtype %d, d=%d, e=%d (need float32 rows of a multiple of 4 features)", call, dtype, d, e);
+  return LASP_E_SHAPE;
+}
+
+int lasp_narrow_fwd(const void *q, const void *k, const void *v, const float *s, const float *kv_in, float *kv_out,
+                    float *kv_twin, void *o, float *seg_states, int b, int h, int64_t n, int d, int e, int dtype, int seg_len,
+                    void *stream) {
+  const int rc = check_narrow("lasp_narrow_fwd", d, e, dtype);
+  if (rc) return rc;
+  return fwd_twin(q, k, v, s, kv_in, kv_out, kv_twin, o, seg_states, b, h, n, d, e, dtype, seg_len, stream, true);
 }
 
 int lasp_step_fwd(const void *q, const void *k, const void *v, const float *s, const float *kv_in, float *kv_out, void *o,
@@ -673,11 +696,10 @@ int lasp_chunk_bwd(const void *q, const void *k, const void *v, const float *s, 
                              workspace_bytes, b, h, n, d, e, dtype, seg_len, stream);
 }
 
-int lasp_chunk_bwd_twin(const void *q, const void *k, const void *v, const float *s, const void *d_o,
-                        const float *kv_in, const float *dkv_in, void *dq, void *dk, void *dv,
-                        float *dkv_out, float *dkv_twin, const float *kv_seg_states, float *workspace,
-                        size_t workspace_bytes, int b, int h, int64_t n, int d, int e, int dtype,
-                        int seg_len, void *stream) {
+static int bwd_twin(const void *q, const void *k, const void *v, const float *s, const void *d_o, const float *kv_in,
+                    const float *dkv_in, void *dq, void *dk, void *dv, float *dkv_out, float *dkv_twin,
+                    const float *kv_seg_states, float *workspace, size_t workspace_bytes, int b, int h, int64_t n, int d, int e,
+                    int dtype, int seg_len, void *stream, bool narrow) {
   Geom g;
   int rc = make_geom(b, h, n, d, e, dtype, seg_len, &g);
   if (rc) return rc;
@@ -721,10 +743,29 @@ int lasp_chunk_bwd_twin(const void *q, const void *k, const void *v, const float
   if (need_kv) a.ws_kv = wp;
   hipStream_t st = (hipStream_t)stream;
   rc = mfma_eligible(d, e, dtype)       ? mfma_bwd(a, g, dtype, st)
-       : mfma_f32_eligible(d, e, dtype) ? mfma_f32_bwd(a, g, st)
+       : narrow || mfma_f32_eligible(d, e, dtype) ? mfma_f32_bwd(a, g, st)
                                         : generic_bwd(a, g, dtype, st);
   if (rc > 0) set_error("lasp_chunk_bwd: HIP error %d: %s", rc, hipGetErrorString((hipError_t)rc));
   return rc;
+}
+
+int lasp_chunk_bwd_twin(const void *q, const void *k, const void *v, const float *s, const void *d_o,
+                        const float *kv_in, const float *dkv_in, void *dq, void *dk, void *dv,
+                        float *dkv_out, float *dkv_twin, const float *kv_seg_states, float *workspace,
+                        size_t workspace_bytes, int b, int h, int64_t n, int d, int e, int dtype,
+                        int seg_len, void *stream) {
+  return bwd_twin(q, k, v, s, d_o, kv_in, dkv_in, dq, dk, dv, dkv_out, dkv_twin, kv_seg_states, workspace, workspace_bytes, b, h,
+                  n, d, e, dtype, seg_len, stream, false);
+}
+
+int lasp_narrow_bwd(const void *q, const void *k, const void *v, const float *s, const void *d_o, const float *kv_in,
+                    const float *dkv_in, void *dq, void *dk, void *dv, float *dkv_out, float *dkv_twin,
+                    const float *kv_seg_states, float *workspace, size_t workspace_bytes, int b, int h, int64_t n, int d, int e,
+                    int dtype, int seg_len, void *stream) {
+  const int rc = check_narrow("lasp_narrow_bwd", d, e, dtype);
+  if (rc) return rc;
+  return bwd_twin(q, k, v, s, d_o, kv_in, dkv_in, dq, dk, dv, dkv_out, dkv_twin, kv_seg_states, workspace, workspace_bytes, b, h,
+                  n, d, e, dtype, seg_len, stream, true);
 }
 
 }  // extern "C"

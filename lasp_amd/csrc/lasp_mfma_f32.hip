@@ -1,4 +1,4 @@
-// fp32 MFMA kernels for d = e = 128 (gfx950, wave64): the same decomposition
+// fp32 MFMA kernels for d, e <= 128, laid out for 128 (gfx950, wave64): the same decomposition
 // as the 16-bit kernels -- one routine evaluates a causal or anti-causal decayed linear
 // attention over a segment given the state entering it, and the four outputs of the
 // operator are instances of it (O: x=Q y=K z=V; dQ: x=dO y=V z=K with the state transposed;
@@ -155,11 +155,13 @@ __device__ __forceinline__ void reads_first() { __builtin_amdgcn_sched_barrier(0
 // A block of token rows as a buffer that ends with them: rows that a partial block does not have read as zeros and are not
 // stored, without a branch per access (after which a wait for the oldest access would have to wait for all of them).
 typedef __amdgpu_buffer_rsrc_t rows_t;
-__device__ __forceinline__ rows_t rows_of(const float *p, int count) {
+__device__ __forceinline__ rows_t buffer_of(const float *p, int bytes) {
   const uint64_t v = reinterpret_cast<uint64_t>(p);  // the same for every lane
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return __builtin_amdgcn_make_buffer_rsrc((void *)(((uint64_t)hi << 32) | lo), 0, count * F * 4, 0x00020000);
+  return __builtin_amdgcn_make_buffer_rsrc((void *)(((uint64_t)hi << 32) | lo), 0, bytes, 0x00020000);
 }
+__device__ __forceinline__ rows_t rows_of(const float *p, int count, int width) { return buffer_of(p, count * width * 4); }
+constexpr int NOWHERE = 1 << 30;  // an offset past the end of every such buffer: features that a narrow row does not have
 __device__ __forceinline__ f32x4 load16(rows_t rows, int off) {
   return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, off, 0, 0));
 }
@@ -183,17 +185,26 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
   return r;
 }
 
+// An offset that is worked out here, and not once for all blocks: the offsets of narrow rows are no constants, and registers are short
+template <bool NARROW>
+__device__ __forceinline__ int fresh(int off) {
+  if (NARROW) asm volatile("" : "+v"(off));
+  return off;
+}
 // The X (or Y) rows of a block: thread (cq, rq) holds features 4 cq .. + 3 of rows rq + 8 it
 struct Loader {
-  int from, to;  // the thread's place in a block of rows and in a tile
-  __device__ __forceinline__ explicit Loader(int tid) {
+  int from, to, step;  // the thread's place in a block of rows and in a tile; eight rows on
+  __device__ __forceinline__ Loader(int tid, int width) {
     const int cq = tid & 31, rq = tid >> 5, p = cq & 3;
-    from = rq * (F * 4) + cq * 16;
+    from = width == F || 4 * cq < width ? rq * (width * 4) + cq * 16 : NOWHERE;
+    step = 8 * width * 4;
     to = rq * ROW + (((2 * (cq >> 2) + (p & 1)) ^ swizzle(rq)) << 4) + ((p >> 1) << 3);
   }
+  template <bool NARROW>
   __device__ __forceinline__ void load(rows_t rows, f32x4 (&n)[4]) const {
+    const int at = fresh<NARROW>(from);
 #pragma unroll
-    for (int it = 0; it < 4; ++it) n[it] = load16(rows, from + it * (8 * F * 4));
+    for (int it = 0; it < 4; ++it) n[it] = load16(rows, at + it * step);
   }
   // half `k & 1` of row k >> 1, into `row`; the second half writes the row
   __device__ __forceinline__ void fill_half(char *tile, const f32x4 (&n)[4], int k, u32x2 (&row)[3]) const {
@@ -218,46 +229,75 @@ struct Loader {
   }
 };
 // A wave's own 32 columns of Z come straight from memory: lane (c, hh) holds tokens 16 u + 8 hh + j of column c in z[8 u + j]
-__device__ __forceinline__ void load_columns(rows_t rows, int lane_off, float (&z)[16]) {
+__device__ __forceinline__ int column_off(int lane, int w, int width) {
+  const int col = 32 * w + (lane & 31);
+  return width == F || col < width ? 8 * (lane >> 5) * (width * 4) + col * 4 : NOWHERE;
+}
+template <bool NARROW>
+__device__ __forceinline__ void load_columns(rows_t rows, int lane_off, int width, float (&z)[16]) {
+  const int at = fresh<NARROW>(lane_off);
 #pragma unroll
   for (int i = 0; i < 16; ++i)
-    z[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, lane_off + (16 * (i >> 3) + (i & 7)) * (F * 4), 0, 0));
+    z[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rows, at + (16 * (i >> 3) + (i & 7)) * (width * 4), 0, 0));
 }
 
+enum Mode {
+  M_ALIGNED,  // n is a multiple of 32, rows of 128 features
+  M_RAGGED,   // any n
+  // any n and rows of any multiples of 4 features, d and e, that 2, 3 or 4 tiles of 32 features hold
+  M_NARROW2,
+  M_NARROW3,
+  M_NARROW4,
+};
+constexpr bool narrow(int mode) { return mode >= M_NARROW2; }
+constexpr int tiles(int mode) { return narrow(mode) ? mode - M_NARROW2 + 2 : 4; }  // of 32 features
+// Narrow rows end after g.d (g.e) features: what is missing reads as zeros and is not stored, and stored states are d x e.  With two or
+// three tiles the state has as many rows, and the waves whose columns of Z are all missing only help with rows and scores.
+// Against rows padded to 128 features before the call (five tensors copied in, four copied out, and products of zeros), forward +
+// backward: b*h = 24, n = 2048: d = e = 64 348 -> 105 us, 80 359 -> 121, 96 371 -> 133, d = 128, e = 64 282 -> 146; n = 8192, d = e =
+// 64: 1035 -> 303.  Bound as above; with two tiles the matrix units of two SIMDs idle in the state's products.  The kernels are
+// instances per number of tiles because a number known only at run time cost up to 110 spilled registers.
+//
 // RAGGED: the chunk length is not a multiple of 32, so the last block of the last segment is
 // partial (missing rows read as zeros, stores masked, and -- going backwards, where that block
 // comes first -- the entering state sits `len` tokens ahead instead of 32).
-template <bool REV, bool TRANS, bool RAGGED>
+template <bool REV, bool TRANS, int MODE>
 __device__ __forceinline__ void
 sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float *__restrict__ Z,
            const float *__restrict__ S, const float *__restrict__ states, float *__restrict__ Out,
            const Geom &g, int item, char *smem) {
-  const int tid = threadIdx.x;
+  constexpr bool RAGGED = MODE != M_ALIGNED, NARROW = narrow(MODE);
+  constexpr int NT = tiles(MODE);
+  const int tid = fresh<NARROW>(threadIdx.x);  // (nothing of it is kept for another role's sweep)
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform: keeps it in an SGPR
   const int c = lane & 31, hh = lane >> 5;
 
+  // features of X and Y, and of Z and Out
+  const int xw = !NARROW ? F : TRANS ? g.e : g.d, zw = !NARROW ? F : TRANS ? g.d : g.e;
+  const bool active = NT == 4 || w < NT;
+
   const SegWork sw = seg_work(g, item);
-  const int64_t base = ((int64_t)sw.bh * g.n + sw.tok0) * F;
-  const Loader loader(tid);
+  const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
+  const Loader loader(tid, xw);
   const TokenReader tokens(lane);
-  const int z_off = 8 * hh * (F * 4) + (32 * w + c) * 4;
+  const int z_off = column_off(lane, w, zw);
 
   f32x4 nx[4], ny[4];
   float z[16];
   auto len_of = [&](int blk) __attribute__((always_inline)) { return RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK; };
-  auto rows = [&](const float *p, int blk) __attribute__((always_inline)) {
-    return rows_of(p + base + (int64_t)blk * (BLK * F), len_of(blk));
+  auto rows = [&](const float *p, int blk, int width) __attribute__((always_inline)) {
+    return rows_of(p + (row0 + (int64_t)blk * BLK) * width, len_of(blk), width);
   };
   // the block after this one, or none of its rows where there is none: as many accesses in flight on every path
-  auto next_rows = [&](const float *p, bool more, int blk) __attribute__((always_inline)) {
-    return rows_of(p + base + (int64_t)blk * (BLK * F), more ? len_of(blk) : 0);
+  auto next_rows = [&](const float *p, bool more, int blk, int width) __attribute__((always_inline)) {
+    return rows_of(p + (row0 + (int64_t)blk * BLK) * width, more ? len_of(blk) : 0, width);
   };
   const int first = REV ? sw.nblk - 1 : 0;
   const int step = REV ? -1 : 1;
-  loader.load(rows(X, first), nx);
-  loader.load(rows(Y, first), ny);
-  load_columns(rows(Z, first), z_off, z);
+  loader.load<NARROW>(rows(X, first, xw), nx);
+  loader.load<NARROW>(rows(Y, first, xw), ny);
+  load_columns<NARROW>(rows(Z, first, zw), z_off, zw, z);
 
   const float sl = S[sw.bh - quotient(sw.bh, g.by_h) * g.h] * LOG2E;
   // ---- constants (all exponents <= 0)
@@ -283,11 +323,28 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
   const int x_from = c * ROW + ((hh ^ swizzle(c)) << 4);
 
   // ---- state entering the segment: st[T][4g+r] = St[32T+8g+4hh+r][32w+c]
-  floatx16 st[4];
-  if (states) {
+  floatx16 st[NT];
+  if (NARROW && states) {
+    // (rows come in fours: a row that is missing is in a group of four that is)
+    const rows_t sp = buffer_of(states + ((int64_t)sw.bh * g.n_seg + sw.seg) * (g.d * g.e), g.d * g.e * 4);
+    const int col = 32 * w + c;
+    const int at = col < zw ? (TRANS ? col * xw : col) * 4 : NOWHERE;
+#pragma unroll
+    for (int T = 0; T < NT; ++T) {
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) {
+        const int row = 32 * T + 8 * gq + 4 * hh;
+        const int off = row < xw ? at + (TRANS ? row : row * zw) * 4 : NOWHERE;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          st[T][4 * gq + r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sp, off + (TRANS ? r : r * zw) * 4, 0, 0));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else if (states) {
     const float *sp = states + ((int64_t)sw.bh * g.n_seg + sw.seg) * (F * F);
 #pragma unroll
-    for (int T = 0; T < 4; ++T)
+    for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = 32 * T + 8 * (r >> 2) + 4 * hh + (r & 3);
@@ -296,7 +353,7 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       }
   } else {
 #pragma unroll
-    for (int T = 0; T < 4; ++T)
+    for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int r = 0; r < 16; ++r) st[T][r] = 0.f;
   }
@@ -331,8 +388,8 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       xs[0] = parts(smem + OFF_X, xq, PART);
       ys[0] = parts(smem + OFF_Y, yq, PART);
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        if (m < 3) {
+      for (int m = 0; m < NT; ++m) {
+        if (m < NT - 1) {
           xs[(m + 1) & 1] = parts(smem + OFF_X, xq ^ ((m + 1) << 6), PART);
           ys[(m + 1) & 1] = parts(smem + OFF_Y, yq ^ ((m + 1) << 6), PART);
         } else {
@@ -341,7 +398,9 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
         }
         reads_first();
         sc = product(ys[m & 1], xs[m & 1], sc, [&](int i) __attribute__((always_inline)) {
-          if (i % 3 == 0) scale_z(2 * m + i / 3);
+          constexpr int PER = (8 + NT - 1) / NT;  // pairs of Z for each of the NT products
+          const int pair = m * PER + i / (6 / PER);
+          if (i % (6 / PER) == 0 && i / (6 / PER) < PER && pair < 8) scale_z(pair);
         });
       }
 #pragma unroll
@@ -366,52 +425,56 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
     floatx16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    loader.load(next_rows(X, more, blk + step), nx);
+    loader.load<NARROW>(next_rows(X, more, blk + step, xw), nx);
     Split a0, a1, zu[2];
     f32x4 zp[4];
+    if (active) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) split_pair(a0, i, st[0][2 * i], st[0][2 * i + 1]);
+      for (int i = 0; i < 4; ++i) split_pair(a0, i, st[0][2 * i], st[0][2 * i + 1]);
 #pragma unroll
-    for (int T = 0; T < 4; ++T) {
-      acc = product(a0, xf[0], acc, [&](int i) __attribute__((always_inline)) {
-        if (i < 4) split_pair(a1, i, st[T][8 + 2 * i], st[T][9 + 2 * i]);
-      });
-      acc = product(a1, xf[1], acc, [&](int i) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 3 * i; r < 3 * i + 3 && r < 16; ++r) st[T][r] *= bd;
-      });
-      if (T < 3) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) xf[u] = parts(smem + OFF_X, x_from ^ ((2 * T + 2 + u) << 5), PART);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) zp[i] = *reinterpret_cast<const f32x4 *>(z_park + 1024 * i);
-      }
-      reads_first();
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        st[T] = product(yf[u], zs[u], st[T], [&](int i) __attribute__((always_inline)) {
-          if (T < 3) {
-            if (u == 0 && i < 4) split_pair(a0, i, st[T + 1][2 * i], st[T + 1][2 * i + 1]);
-          } else if (i < 4) {
-            const f32x4 &v = zp[2 * u + (i >> 1)];
-            split_pair(zu[u], i, (i & 1) ? v.z : v.x, (i & 1) ? v.w : v.y);
-          }
+      for (int T = 0; T < NT; ++T) {
+        acc = product(a0, xf[0], acc, [&](int i) __attribute__((always_inline)) {
+          if (i < 4) split_pair(a1, i, st[T][8 + 2 * i], st[T][9 + 2 * i]);
         });
-        if (T < 3) yf[u] = tokens.read(smem + OFF_Y, T + 1, u);
-        reads_first();
-      }
-      if (T == 1) loader.load(next_rows(Y, more, blk + step), ny);
-    }
+        acc = product(a1, xf[1], acc, [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] *= qd;
+          for (int r = 3 * i; r < 3 * i + 3 && r < 16; ++r) st[T][r] *= bd;
+        });
+        if (T < NT - 1) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) xf[u] = parts(smem + OFF_X, x_from ^ ((2 * T + 2 + u) << 5), PART);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) zp[i] = *reinterpret_cast<const f32x4 *>(z_park + 1024 * i);
+        }
+        reads_first();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          st[T] = product(yf[u], zs[u], st[T], [&](int i) __attribute__((always_inline)) {
+            if (T < NT - 1) {
+              if (u == 0 && i < 4) split_pair(a0, i, st[T + 1][2 * i], st[T + 1][2 * i + 1]);
+            } else if (i < 4) {
+              const f32x4 &v = zp[2 * u + (i >> 1)];
+              split_pair(zu[u], i, (i & 1) ? v.z : v.x, (i & 1) ? v.w : v.y);
+            }
+          });
+          if (T < NT - 1) yf[u] = tokens.read(smem + OFF_Y, T + 1, u);
+          reads_first();
+        }
+        if (T == (NT == 3 ? 2 : 1)) loader.load<NARROW>(next_rows(Y, more, blk + step, xw), ny);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] *= qd;
+    } else {
+      loader.load<NARROW>(next_rows(Y, more, blk + step, xw), ny);
+    }
     __syncthreads();  // the score tile is complete; X and Y are no longer read
     // (4) intra-block term
-    {
+    load_columns<NARROW>(next_rows(Z, more, blk + step, zw), z_off, zw, z);
+    if (active) {
       Split sf[2];
 #pragma unroll
       for (int u = 0; u < 2; ++u) sf[u] = parts(smem + OFF_SC, sc_from ^ (u << 5), SC_PART);
-      load_columns(next_rows(Z, more, blk + step), z_off, z);
       reads_first();
       u32x2 row[3];
 #pragma unroll
@@ -419,10 +482,13 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
         acc = product(zu[u], sf[u], acc, [&](int i) __attribute__((always_inline)) {  // and the next block's X
           if (6 * u + i < 8) loader.fill_half(smem + OFF_X, nx, 6 * u + i, row);
         });
+    } else {
+      loader.fill(smem + OFF_X, nx);
     }
     loader.fill(smem + OFF_Y, ny);
     // (5) output: lane (c, hh) holds, for token c, four consecutive columns per g
-    const rows_t out = rows_of(Out + base + (int64_t)blk * (BLK * F), len);
+    const int col0 = fresh<NARROW>(32 * w + 4 * hh);
+    const rows_t out = rows_of(Out + (row0 + (int64_t)blk * BLK) * zw, len, zw);
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) {
       f32x4 o;
@@ -430,23 +496,24 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       o.y = acc[4 * gq + 1];
       o.z = acc[4 * gq + 2];
       o.w = acc[4 * gq + 3];
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), out, c * (F * 4) + (32 * w + 4 * hh + 8 * gq) * 4, 0, 0);
+      const int col = col0 + 8 * gq, off = !NARROW || col < zw ? c * (zw * 4) + col * 4 : NOWHERE;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), out, off, 0, 0);
     }
     if (more) __syncthreads();  // the next block's X and Y are complete; the score tile is no longer read
   }
 }
 
-template <bool REV, bool TRANS, bool RAGGED>
+template <bool REV, bool TRANS, int MODE>
 __global__ void __launch_bounds__(NTHR, 2)
 la32_apply(const float *__restrict__ X, const float *__restrict__ Y, const float *__restrict__ Z,
            const float *__restrict__ S, const float *__restrict__ states, float *__restrict__ Out, Geom g) {
   extern __shared__ __align__(16) char smem[];
-  sweep_body<REV, TRANS, RAGGED>(X, Y, Z, S, states, Out, g, (int)blockIdx.x, smem);
+  sweep_body<REV, TRANS, MODE>(X, Y, Z, S, states, Out, g, (int)blockIdx.x, smem);
 }
 
 // dQ, dV and dK in one launch; the three workgroups of a (b*h, segment) sit 8 block indices
 // apart, i.e. on the same XCD
-template <bool RAGGED>
+template <int MODE>
 __global__ void __launch_bounds__(NTHR, 2)
 la32_bwd3(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
           const float *__restrict__ DO, const float *__restrict__ S, const float *__restrict__ kv_states,
@@ -459,18 +526,20 @@ la32_bwd3(const float *__restrict__ Q, const float *__restrict__ K, const float 
   const int item = n_items - 1 - (grp * 8 + (r & 7));
   if (item < 0) return;
   if (role == 0)
-    sweep_body<false, true, RAGGED>(DO, V, K, S, kv_states, DQ, g, item, smem);
+    sweep_body<false, true, MODE>(DO, V, K, S, kv_states, DQ, g, item, smem);
   else if (role == 1)
-    sweep_body<true, false, RAGGED>(K, Q, DO, S, dkv_states, DV, g, item, smem);
+    sweep_body<true, false, MODE>(K, Q, DO, S, dkv_states, DV, g, item, smem);
   else
-    sweep_body<true, true, RAGGED>(V, DO, Q, S, dkv_states, DK, g, item, smem);
+    sweep_body<true, true, MODE>(V, DO, Q, S, dkv_states, DK, g, item, smem);
 }
 
 // a segment's own state: causal sum_b l^(L-b) y_b^T z_b ; anti-causal sum_b l^b y_b^T z_b
-template <bool REV, bool RAGGED>
+template <bool REV, int MODE>
 __global__ void __launch_bounds__(NTHR, 2)
 la32_seg_state(const float *__restrict__ Y, const float *__restrict__ Z, const float *__restrict__ S,
                float *__restrict__ states, Geom g, int skip_seg) {
+  constexpr bool RAGGED = MODE != M_ALIGNED, NARROW = narrow(MODE);
+  constexpr int NT = tiles(MODE);
   __shared__ __align__(256) char smem[2][TILE];  // double-buffered Y
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -479,20 +548,22 @@ la32_seg_state(const float *__restrict__ Y, const float *__restrict__ Z, const f
 
   const SegWork sw = seg_work(g, (int)blockIdx.x);
   if (sw.seg == skip_seg) return;
-  const int64_t base = ((int64_t)sw.bh * g.n + sw.tok0) * F;
-  const Loader loader(tid);
+  const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
+  const int yw = NARROW ? g.d : F, zw = NARROW ? g.e : F;
+  const bool active = NT == 4 || w < NT;
+  const Loader loader(tid, yw);
   const TokenReader tokens(lane);
-  const int z_off = 8 * hh * (F * 4) + (32 * w + c) * 4;
+  const int z_off = column_off(lane, w, zw);
   auto len_of = [&](int blk) __attribute__((always_inline)) { return RAGGED && blk == sw.nblk - 1 ? sw.tail : BLK; };
-  auto rows = [&](const float *p, int blk) __attribute__((always_inline)) {
-    return rows_of(p + base + (int64_t)blk * (BLK * F), len_of(blk));
+  auto rows = [&](const float *p, int blk, int width) __attribute__((always_inline)) {
+    return rows_of(p + (row0 + (int64_t)blk * BLK) * width, len_of(blk), width);
   };
   f32x4 ny[4];
   float z[16];
   const int first = REV ? sw.nblk - 1 : 0;
   const int step = REV ? -1 : 1;
-  loader.load(rows(Y, first), ny);
-  load_columns(rows(Z, first), z_off, z);
+  loader.load<NARROW>(rows(Y, first, yw), ny);
+  load_columns<NARROW>(rows(Z, first, zw), z_off, zw, z);
 
   const float sl = S[sw.bh - quotient(sw.bh, g.by_h) * g.h] * LOG2E;
   const float blockdec = uniform_decay(sl, (float)BLK);
@@ -502,16 +573,16 @@ la32_seg_state(const float *__restrict__ Y, const float *__restrict__ Z, const f
     const int b = 16 * (i >> 3) + 8 * hh + (i & 7);
     zdec[i] = decay(sl, REV ? (float)b : (float)(BLK - b));
   }
-  floatx16 st[4];
+  floatx16 st[NT];
 #pragma unroll
-  for (int T = 0; T < 4; ++T)
+  for (int T = 0; T < NT; ++T)
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[T][r] = 0.f;
   loader.fill(smem[0], ny);
   __syncthreads();
   for (int it = 0, blk = first; it < sw.nblk; ++it, blk += step) {
     const bool more = it + 1 < sw.nblk;
-    if (more) loader.load(rows(Y, blk + step), ny);
+    if (more) loader.load<NARROW>(rows(Y, blk + step, yw), ny);
     const int len = len_of(blk);
     const float bd = RAGGED && len != BLK ? uniform_decay(sl, (float)len) : blockdec;
     if (RAGGED && !REV && len != BLK)  // going forwards a partial block is the last one: its tokens sit `len - b` before the segment's end
@@ -523,19 +594,20 @@ la32_seg_state(const float *__restrict__ Y, const float *__restrict__ Z, const f
     for (int u = 0; u < 2; ++u) yf[0][u] = tokens.read(tile, 0, u);
 #pragma unroll
     for (int i = 0; i < 8; ++i) split_pair(zs[i >> 2], i & 3, z[2 * i] * zdec[2 * i], z[2 * i + 1] * zdec[2 * i + 1]);
-    if (more) load_columns(rows(Z, blk + step), z_off, z);
+    if (more) load_columns<NARROW>(rows(Z, blk + step, zw), z_off, zw, z);
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[0][r] *= bd;
 #pragma unroll
-    for (int T = 0; T < 4; ++T) {
-      if (T < 3)
+    for (int T = 0; T < NT; ++T) {
+      if (!active) break;
+      if (T < NT - 1)
 #pragma unroll
         for (int u = 0; u < 2; ++u) yf[(T + 1) & 1][u] = tokens.read(tile, T + 1, u);
       reads_first();
 #pragma unroll
       for (int u = 0; u < 2; ++u)
         st[T] = product(yf[T & 1][u], zs[u], st[T], [&](int i) __attribute__((always_inline)) {
-          if (T < 3 && u == 0)
+          if (T < NT - 1 && u == 0)
 #pragma unroll
             for (int r = 3 * i; r < 3 * i + 3 && r < 16; ++r) st[T + 1][r] *= bd;
         });
@@ -543,63 +615,75 @@ la32_seg_state(const float *__restrict__ Y, const float *__restrict__ Z, const f
     if (more) loader.fill(smem[(it + 1) & 1], ny);
     __syncthreads();
   }
+  if (NARROW) {
+    const rows_t sp = buffer_of(states + ((int64_t)sw.bh * g.n_seg + sw.seg) * (yw * zw), yw * zw * 4);
+#pragma unroll
+    for (int T = 0; T < NT; ++T)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = 32 * T + 8 * (r >> 2) + 4 * hh + (r & 3), col = 32 * w + c;
+        const int off = row < yw && col < zw ? (row * zw + col) * 4 : NOWHERE;
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, (float)st[T][r]), sp, off, 0, 0);
+      }
+    return;
+  }
   float *sp = states + ((int64_t)sw.bh * g.n_seg + sw.seg) * (F * F);
 #pragma unroll
-  for (int T = 0; T < 4; ++T)
+  for (int T = 0; T < NT; ++T)
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       sp[(32 * T + 8 * (r >> 2) + 4 * hh + (r & 3)) * F + 32 * w + c] = st[T][r];
 }
 
-template <bool REV, bool RAGGED>
+template <bool REV, int MODE>
 int launch_state(const void *y, const void *z, const float *s, float *states, const Geom &g,
                  bool carry_wanted, hipStream_t st) {
   const unsigned grid = (unsigned)((int64_t)g.b * g.h * g.n_seg);
   const int skip_seg = carry_wanted ? -1 : (REV ? 0 : g.n_seg - 1);
   ProfScope prof(KC_STATE, st);
-  la32_seg_state<REV, RAGGED><<<grid, NTHR, 0, st>>>((const float *)y, (const float *)z, s, states, g,
+  la32_seg_state<REV, MODE><<<grid, NTHR, 0, st>>>((const float *)y, (const float *)z, s, states, g,
                                                      skip_seg);
   return (int)hipGetLastError();
 }
 
-template <bool RAGGED>
+template <int MODE>
 int fwd_r(const FwdArgs &a, const Geom &g, hipStream_t st) {
   int rc;
   const bool need_states = g.n_seg > 1 || a.kv_in || a.kv_out;
   if (need_states) {
-    if ((rc = launch_state<false, RAGGED>(a.k, a.v, a.s, a.seg_states, g, a.kv_out != nullptr, st))) return rc;
+    if ((rc = launch_state<false, MODE>(a.k, a.v, a.s, a.seg_states, g, a.kv_out != nullptr, st))) return rc;
     if ((rc = launch_segment_scan(a.seg_states, a.kv_in, a.kv_out, a.s, g, 0, st))) return rc;
   }
-  if ((rc = grant_lds<la32_apply<false, false, RAGGED>>(APPLY_LDS))) return rc;
+  if ((rc = grant_lds<la32_apply<false, false, MODE>>(APPLY_LDS))) return rc;
   const unsigned grid = (unsigned)((int64_t)g.b * g.h * g.n_seg);
   ProfScope prof(KC_APPLY, st);
-  la32_apply<false, false, RAGGED><<<grid, NTHR, APPLY_LDS, st>>>((const float *)a.q, (const float *)a.k,
+  la32_apply<false, false, MODE><<<grid, NTHR, APPLY_LDS, st>>>((const float *)a.q, (const float *)a.k,
                                                                   (const float *)a.v, a.s,
                                                                   need_states ? a.seg_states : nullptr,
                                                                   (float *)a.o, g);
   return (int)hipGetLastError();
 }
 
-template <bool RAGGED>
+template <int MODE>
 int bwd_r(const BwdArgs &a, const Geom &g, hipStream_t st) {
   int rc;
   const float *kv_states = a.kv_seg_states;
   if (!kv_states && (g.n_seg > 1 || a.kv_in)) {
-    if ((rc = launch_state<false, RAGGED>(a.k, a.v, a.s, a.ws_kv, g, false, st))) return rc;
+    if ((rc = launch_state<false, MODE>(a.k, a.v, a.s, a.ws_kv, g, false, st))) return rc;
     if ((rc = launch_segment_scan(a.ws_kv, a.kv_in, nullptr, a.s, g, 0, st))) return rc;
     kv_states = a.ws_kv;
   }
   const float *dkv_states = nullptr;
   if (g.n_seg > 1 || a.dkv_in || a.dkv_out) {
-    if ((rc = launch_state<true, RAGGED>(a.q, a.d_o, a.s, a.ws_dkv, g, a.dkv_out != nullptr, st))) return rc;
+    if ((rc = launch_state<true, MODE>(a.q, a.d_o, a.s, a.ws_dkv, g, a.dkv_out != nullptr, st))) return rc;
     if ((rc = launch_segment_scan(a.ws_dkv, a.dkv_in, a.dkv_out, a.s, g, 1, st))) return rc;
     dkv_states = a.ws_dkv;
   }
-  if ((rc = grant_lds<la32_bwd3<RAGGED>>(APPLY_LDS))) return rc;
+  if ((rc = grant_lds<la32_bwd3<MODE>>(APPLY_LDS))) return rc;
   const int64_t n_items = (int64_t)g.b * g.h * g.n_seg;
   const unsigned grid = (unsigned)(((n_items + 7) / 8) * 24);
   ProfScope prof(KC_BWD3, st);
-  la32_bwd3<RAGGED><<<grid, NTHR, APPLY_LDS, st>>>((const float *)a.q, (const float *)a.k,
+  la32_bwd3<MODE><<<grid, NTHR, APPLY_LDS, st>>>((const float *)a.q, (const float *)a.k,
                                                    (const float *)a.v, (const float *)a.d_o, a.s, kv_states,
                                                    dkv_states, (float *)a.dq, (float *)a.dk, (float *)a.dv, g);
   return (int)hipGetLastError();
@@ -608,11 +692,15 @@ int bwd_r(const BwdArgs &a, const Geom &g, hipStream_t st) {
 }  // namespace
 
 int mfma_f32_fwd(const FwdArgs &a, const Geom &g, hipStream_t st) {
-  return g.n % BLK != 0 ? fwd_r<true>(a, g, st) : fwd_r<false>(a, g, st);
+  if (g.d == F && g.e == F) return g.n % BLK != 0 ? fwd_r<M_RAGGED>(a, g, st) : fwd_r<M_ALIGNED>(a, g, st);
+  const int widest = g.d > g.e ? g.d : g.e;
+  return widest <= 64 ? fwd_r<M_NARROW2>(a, g, st) : widest <= 96 ? fwd_r<M_NARROW3>(a, g, st) : fwd_r<M_NARROW4>(a, g, st);
 }
 
 int mfma_f32_bwd(const BwdArgs &a, const Geom &g, hipStream_t st) {
-  return g.n % BLK != 0 ? bwd_r<true>(a, g, st) : bwd_r<false>(a, g, st);
+  if (g.d == F && g.e == F) return g.n % BLK != 0 ? bwd_r<M_RAGGED>(a, g, st) : bwd_r<M_ALIGNED>(a, g, st);
+  const int widest = g.d > g.e ? g.d : g.e;
+  return widest <= 64 ? bwd_r<M_NARROW2>(a, g, st) : widest <= 96 ? bwd_r<M_NARROW3>(a, g, st) : bwd_r<M_NARROW4>(a, g, st);
 }
 
 }  // namespace lasp

@@ -10,7 +10,7 @@
 // n = 512: 108 and 52 us (the kernels); eight chained chunks of 2048 tokens at b*h = 24: 762 and 674 us.
 //
 // "Usual case": contiguity aside, what the kernels take as it is -- device tensors of one type, fp32 with
-// d = e = 128 or 16 bits with widths that are multiples of 8, float32 slopes on the same device.  Everything else (padding, other
+// widths that are multiples of 4 or 16 bits with multiples of 8, float32 slopes on the same device.  Everything else (padding, other
 // types, errors to report; tensor subclasses, function transforms, tracing and forward-mode differentiation, which a
 // node built here would not be seen by) stays with lasp_amd/_abi.py and lasp_amd/_chain.py: the functions below return
 // None for it.
@@ -82,6 +82,9 @@ bool followed(const Tensor &t) { return at::isTensorSubclassLike(t) || t._fw_gra
 // What the library takes as a few tokens under their states, of any type and without a workspace.
 bool is_step(int64_t n, int64_t d, int64_t e) { return n <= LASP_STEP_TOKENS && d <= 128 && e <= 128 && e % 4 == 0; }
 
+// fp32 rows that the MFMA kernels take under a call of their own
+bool is_narrow(const Shape &sh) { return sh.dtype == LASP_DTYPE_F32 && (sh.d != 128 || sh.e != 128); }
+
 // The usual case, see above; fills `sh`.  `keep`: the segment states are kept for a backward.
 bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Shape &sh, bool keep = true) {
   if (torch::jit::tracer::isTracing() || followed(q) || followed(k) || followed(v) || followed(s)) return false;
@@ -95,7 +98,7 @@ bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s,
   const int dtype = dtype_code(q);
   const int64_t d = q.size(3), e = v.size(3);
   if (keep || dtype < 0 || !is_step(q.size(2), d, e))
-    if (dtype == LASP_DTYPE_F32 ? d != 128 || e != 128 : dtype < 0 || d % 8 || e % 8 || d > 1024 || e > 128) return false;
+    if (dtype == LASP_DTYPE_F32 ? d % 4 || e % 4 || d > 128 || e > 128 : dtype < 0 || d % 8 || e % 8 || d > 1024 || e > 128) return false;
   sh = shape_of(q, v);
   return true;
 }
@@ -168,7 +171,7 @@ Forward run_forward(const Shape &sh, const Tensor &q, const Tensor &k, const Ten
   kv_in = private_incoming(kv_in, kv_out, sh, p.seg_len, false);
   f.seg_len = p.seg_len;
   if (!p.fused && (p.n_seg > 1 || kv_in.defined() || kv_out.defined())) f.states = floats(p.bytes, q);
-  const int rc = lasp_chunk_fwd_twin(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(),
+  const int rc = (is_narrow(sh) ? lasp_narrow_fwd : lasp_chunk_fwd_twin)(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(),
                                      (const float *)data(kv_in), (float *)data(kv_out), (float *)data(kv_twin), f.o.data_ptr(),
                                      (float *)data(f.states), sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, p.seg_len, stream());
   if (rc) raise_lasp(rc, "lasp_chunk_fwd");
@@ -192,7 +195,7 @@ Backward run_backward(const Shape &sh, const Tensor &q, const Tensor &k, const T
   const size_t bytes = p.bytes * ((need_dkv ? 1 : 0) + (need_kv ? 1 : 0));
   Tensor ws;
   if (bytes) ws = floats(bytes, q);
-  const int rc = lasp_chunk_bwd_twin(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), d_o.data_ptr(),
+  const int rc = (is_narrow(sh) ? lasp_narrow_bwd : lasp_chunk_bwd_twin)(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), d_o.data_ptr(),
                                 (const float *)data(kv_in), (const float *)data(dkv_in), r.dq.data_ptr(), r.dk.data_ptr(),
                                 r.dv.data_ptr(), (float *)data(dkv_out), (float *)data(dkv_twin),
                                 p.fused ? nullptr : (const float *)data(states), (float *)data(ws), bytes, sh.b, sh.h, sh.n,
