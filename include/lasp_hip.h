@@ -108,6 +108,10 @@ const char *lasp_last_error(void);
 int lasp_plan(int b, int h, int64_t n, int d, int e, int dtype, int seg_len_or_0,
               int *seg_len, int *n_seg, size_t *state_bytes);
 
+/* The seg_len to pass for a forward without kv_in and kv_out and for its backward, where that differs from lasp_plan's
+ * default (float32 on the MFMA kernels: one segment, which needs no states); 0: the default is right. */
+int lasp_stateless_seg_len(int b, int h, int64_t n, int d, int e, int dtype);
+
 /* LASP_PATH_* for this shape under the default plan (seg_len = 0), or a negative LASP_E_* if it is
  * unsupported. */
 int lasp_kernel_path(int b, int h, int64_t n, int d, int e, int dtype);

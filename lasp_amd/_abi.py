@@ -54,6 +54,8 @@ def load() -> ctypes.CDLL:
     lib.lasp_plan.restype = _c_int
     lib.lasp_plan.argtypes = [_c_int, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int,
                               ctypes.POINTER(_c_int), ctypes.POINTER(_c_int), ctypes.POINTER(_c_size)]
+    lib.lasp_stateless_seg_len.restype = _c_int
+    lib.lasp_stateless_seg_len.argtypes = [_c_int, _c_int, _c_i64, _c_int, _c_int, _c_int]
     lib.lasp_kernel_path.restype = _c_int
     lib.lasp_kernel_path.argtypes = [_c_int, _c_int, _c_i64, _c_int, _c_int, _c_int]
     lib.lasp_inplace_ok.restype = _c_int
@@ -126,6 +128,12 @@ def plan(b: int, h: int, n: int, d: int, e: int, dtype: torch.dtype, seg_len: in
     if rc:
         _raise(rc, "lasp_plan")
     return sl.value, ns.value, sb.value
+
+
+@functools.lru_cache(maxsize=256)
+def stateless_seg_len(b, h, n, d, e, dtype) -> int:
+    """The segment length of a forward that neither takes nor leaves a state, 0 for the default plan's."""
+    return load().lasp_stateless_seg_len(b, h, n, d, e, DTYPE_CODE[dtype])
 
 
 @functools.lru_cache(maxsize=256)
@@ -373,6 +381,9 @@ def _pad_state(t, d, e):
 
 def chunk_fwd(q, k, v, s, kv_in=None, kv_out=None, seg_len: int = 0):
     """Forward of one chunk: (o, seg_states, seg_len).  See _chunk_fwd_exact; narrow heads are padded."""
+    if q.dim() == 4 and v.dim() == 4 and seg_len == 0 and kv_in is None and kv_out is None and q.dtype == torch.float32:
+        d, e = (_MFMA_F, _MFMA_F) if _pad_to_mfma(q, v) else (q.shape[3], v.shape[3])
+        seg_len = stateless_seg_len(*q.shape[:3], d, e, q.dtype)
     if q.dim() != 4 or v.dim() != 4 or not _pad_to_mfma(q, v):
         narrow = q.dim() == 4 and v.dim() == 4 and _narrow_rows(q, v)
         return _chunk_fwd_exact(q, k, v, s, kv_in, kv_out, seg_len, narrow)

@@ -207,6 +207,29 @@ int two_per_cu_seg_len(int b, int h, int64_t n) {
   return (int)best;
 }
 
+// A call of the fp32 MFMA kernels that neither takes nor leaves a state may run as one segment per (b, h), which spares the
+// pre-pass, the scan and the states themselves: worth it where that does not leave the chip emptier for it.  Compared are rounds of
+// the forward and the backward sweep times a segment's blocks (two more for a workgroup's start), and eight (ten for heads of up to 64
+// features) blocks' time for the four launches that fall away; workgroups of the latter share a CU at almost no loss, others hardly
+// gain from it, hence the places.  Taken only if it is 5 % better by that count.  Measured forward + backward over b*h = 16 ... 512, n =
+// 96 ... 2048, d = e = 128 and 64, segments against one: b*h = 192, n = 512: 309 and 238 us (64: 159 and 152); b*h = 64, n = 256:
+// 79 and 66; b*h = 48, n = 96: 56 and 30; b*h = 384, n = 1024: 1003 and 867; b*h = 96, n = 1024, where segments stay: 310 and 318
+// (64: 162 and 223).  Of 308 shapes 159 take it, none slower by more than 3 %.
+constexpr int64_t kMaxWhole = 2048;  // tokens, the range measured
+int whole_seg_len(int b, int h, int64_t n, int d, int e) {
+  const int64_t bh = (int64_t)b * h;
+  const bool small = d <= 64 && e <= 64;
+  const int64_t places = small ? 512 : 256, launches = small ? 10 : 8;
+  const int seg_len = two_per_cu_seg_len(b, h, n);
+  if (n <= seg_len || n > kMaxWhole) return 0;
+  auto cost = [&](int64_t segs, int64_t len) {
+    const int64_t groups = bh * segs, rounds = (groups + places - 1) / places + (3 * groups + places - 1) / places;
+    return rounds * ((len + 31) / 32 + 2) + (segs > 1 ? launches : 0);
+  };
+  if (cost(1, n) * 100 >= cost((n + seg_len - 1) / seg_len, seg_len) * 95) return 0;
+  return (int)((n + kSegQuantum - 1) / kSegQuantum) * kSegQuantum;
+}
+
 int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geom *g) {
   int rc = check_shape(b, h, n, d, e, dtype);
   if (rc) return rc;
@@ -561,6 +584,11 @@ int lasp_plan(int b, int h, int64_t n, int d, int e, int dtype, int seg_len_or_0
   if (n_seg) *n_seg = g.n_seg;
   if (state_bytes) *state_bytes = state_bytes_of(g);
   return 0;
+}
+
+int lasp_stateless_seg_len(int b, int h, int64_t n, int d, int e, int dtype) {
+  if (!mfma_f32_eligible(d, e, dtype) && !narrow_eligible(d, e, dtype)) return 0;
+  return check_shape(b, h, n, d, e, dtype) ? 0 : whole_seg_len(b, h, n, d, e);
 }
 
 int lasp_kernel_path(int b, int h, int64_t n, int d, int e, int dtype) {

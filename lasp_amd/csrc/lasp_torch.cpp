@@ -167,6 +167,7 @@ Forward run_forward(const Shape &sh, const Tensor &q, const Tensor &k, const Ten
     if (rc) raise_lasp(rc, "lasp_step_fwd");
     return f;
   }
+  if (seg_len == 0 && !kv_in.defined() && !kv_out.defined()) seg_len = lasp_stateless_seg_len(sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype);
   const Plan p = plan_of(sh, seg_len);
   kv_in = private_incoming(kv_in, kv_out, sh, p.seg_len, false);
   f.seg_len = p.seg_len;
