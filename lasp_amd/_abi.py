@@ -234,6 +234,11 @@ class _on_device:
         return False
 
 
+def _rows16(t):
+    """t, or a copy where it does not start at a multiple of 16 bytes (a view into a larger buffer)."""
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 def _chunk_fwd_exact(q, k, v, s, kv_in=None, kv_out=None, seg_len: int = 0, narrow: bool = False):
     """Enqueues the forward of one chunk.  Returns (o, seg_states, seg_len).
 
@@ -245,6 +250,8 @@ def _chunk_fwd_exact(q, k, v, s, kv_in=None, kv_out=None, seg_len: int = 0, narr
     dev = _check_dev(q, k, v, kv_in, kv_out)
     b, h, n, d, e = _shapes(q, k, v)
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    if narrow:
+        q, k, v = _rows16(q), _rows16(k), _rows16(v)
     s = _slopes(s, h, dev)
     _check_state("kv_in", kv_in, b, h, d, e)
     _check_state("kv_out", kv_out, b, h, d, e)
@@ -309,6 +316,8 @@ def _chunk_bwd_exact(q, k, v, s, do, kv_in=None, dkv_in=None, dkv_out=None, kv_s
     if do.shape != v.shape or do.dtype != q.dtype:
         raise LaspError(f"do must match v: {tuple(do.shape)} {do.dtype} vs {tuple(v.shape)} {q.dtype}")
     q, k, v, do = q.contiguous(), k.contiguous(), v.contiguous(), do.contiguous()
+    if narrow:
+        q, k, v, do = _rows16(q), _rows16(k), _rows16(v), _rows16(do)
     s = _slopes(s, h, dev)
     _check_state("kv_in", kv_in, b, h, d, e)
     _check_state("dkv_in", dkv_in, b, h, d, e)

@@ -85,6 +85,10 @@ bool is_step(int64_t n, int64_t d, int64_t e) { return n <= LASP_STEP_TOKENS && 
 // fp32 rows that the MFMA kernels take under a call of their own
 bool is_narrow(const Shape &sh) { return sh.dtype == LASP_DTYPE_F32 && (sh.d != 128 || sh.e != 128); }
 
+// What a narrow row's kernel fetches 16 bytes at a time: memory that starts elsewhere (a view into a larger buffer) is copied, as it
+// was when such rows were padded.
+Tensor rows(const Tensor &t, const Shape &sh) { return is_narrow(sh) && (uintptr_t)t.data_ptr() % 16 ? t.clone() : t; }
+
 // The usual case, see above; fills `sh`.  `keep`: the segment states are kept for a backward.
 bool regular(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Shape &sh, bool keep = true) {
   if (torch::jit::tracer::isTracing() || followed(q) || followed(k) || followed(v) || followed(s)) return false;
@@ -156,7 +160,7 @@ struct Forward {
   int seg_len = 0;
 };
 // q, k, v contiguous
-Forward run_forward(const Shape &sh, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, Tensor kv_in,
+Forward run_forward(const Shape &sh, Tensor q, Tensor k, Tensor v, const Tensor &s, Tensor kv_in,
                     const Tensor &kv_out, const Tensor &kv_twin, int seg_len, bool keep = true) {
   const auto stream = [&] { return c10::hip::getCurrentHIPStream(q.device().index()).stream(); };
   Forward f;
@@ -170,6 +174,7 @@ Forward run_forward(const Shape &sh, const Tensor &q, const Tensor &k, const Ten
   if (seg_len == 0 && !kv_in.defined() && !kv_out.defined()) seg_len = lasp_stateless_seg_len(sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype);
   const Plan p = plan_of(sh, seg_len);
   kv_in = private_incoming(kv_in, kv_out, sh, p.seg_len, false);
+  q = rows(q, sh), k = rows(k, sh), v = rows(v, sh);
   f.seg_len = p.seg_len;
   if (!p.fused && (p.n_seg > 1 || kv_in.defined() || kv_out.defined())) f.states = floats(p.bytes, q);
   const int rc = (is_narrow(sh) ? lasp_narrow_fwd : lasp_chunk_fwd_twin)(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(),
@@ -183,7 +188,7 @@ struct Backward {
   Tensor dq, dk, dv;
 };
 // q, k, v, d_o contiguous; `states` undefined: rebuilt
-Backward run_backward(const Shape &sh, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Tensor &d_o,
+Backward run_backward(const Shape &sh, Tensor q, Tensor k, Tensor v, const Tensor &s, Tensor d_o,
                       const Tensor &kv_in, Tensor dkv_in, const Tensor &dkv_out, const Tensor &dkv_twin, const Tensor &states, int seg_len) {
   const Plan p = plan_of(sh, seg_len);
   dkv_in = private_incoming(dkv_in, dkv_out, sh, p.seg_len, true);
@@ -196,6 +201,7 @@ Backward run_backward(const Shape &sh, const Tensor &q, const Tensor &k, const T
   const size_t bytes = p.bytes * ((need_dkv ? 1 : 0) + (need_kv ? 1 : 0));
   Tensor ws;
   if (bytes) ws = floats(bytes, q);
+  q = rows(q, sh), k = rows(k, sh), v = rows(v, sh), d_o = rows(d_o, sh);
   const int rc = (is_narrow(sh) ? lasp_narrow_bwd : lasp_chunk_bwd_twin)(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), d_o.data_ptr(),
                                 (const float *)data(kv_in), (const float *)data(dkv_in), r.dq.data_ptr(), r.dk.data_ptr(),
                                 r.dv.data_ptr(), (float *)data(dkv_out), (float *)data(dkv_twin),

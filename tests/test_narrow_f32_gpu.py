@@ -104,3 +104,28 @@ def test_native_and_python_paths_agree(d, e):
         grads2 = _abi.chunk_bwd(*leaves, s, inp["do"], kv_seg_states=states, seg_len=seg)
     for a, c in zip((o, *grads), (o2, *grads2)):
         assert torch.equal(a, c)
+
+
+def _shifted(t):
+    """The same numbers in a view that starts 4 bytes past a multiple of 16."""
+    room = torch.empty(t.numel() + 1, device="cuda")
+    out = room[1:].view(t.shape).copy_(t)
+    assert out.data_ptr() % 16 == 4
+    return out
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_rows_that_start_off_a_vector(native):
+    inp = {k: t.cuda() for k, t in make_inputs(1, H, 70, 64, 36, torch.float32, seed=3, scale=0.1, state=False).items() if t is not None}
+    s = lasp_amd.build_slope_tensor(H).cuda()
+    seen = []
+    for place in (torch.clone, _shifted):
+        q, k, v, do = (place(inp[x]) for x in ("q", "k", "v", "do"))
+        if native:
+            leaves = [t.requires_grad_() for t in (q, k, v)]
+            o = _native.ext().attention(*leaves, s)
+            seen.append((o, *torch.autograd.grad(o, leaves, do)))
+        else:
+            o, states, seg = _abi.chunk_fwd(q, k, v, s)
+            seen.append((o, *_abi.chunk_bwd(q, k, v, s, do, kv_seg_states=states, seg_len=seg)))
+    assert all(torch.equal(a, c) for a, c in zip(*seen))
