@@ -183,14 +183,18 @@ bool fused_eligible(int64_t n, int d, int e, int dtype, int seg_len_arg, int seg
 // per CU and are bound by arithmetic: what counts is that every CU gets the same number of workgroups.  Of the
 // power-of-two lengths that give the forward sweep at least one workgroup per CU, the one with the smallest
 // load per CU -- ceil(workgroups / 256) x (seg_len + 64 tokens for the state each workgroup loads and leaves) --
-// is taken, longer segments (fewer states to scan) winning ties; a single segment of 1024 tokens or more is
-// then cut in two when the chunk has more than one, because two workgroups on a CU fill each other's waits.
+// is taken, longer segments (fewer states to scan) winning ties; a segment of 1024 tokens or more that has a CU
+// to itself is then cut in two when the chunk has more than one, because two workgroups on a CU fill each other's
+// waits.  Heads of up to 96 features, whose states cost half as much or less to carry, gain from that from 512 tokens on:
+// fp32 forward + backward and forward alone with states, 512 and 256 tokens, b*h = 16, n = 8192: d = e = 32: 205 and 179 us, 74
+// and 59; 64: 212 and 191, 76 and 63; 96: 279 and 270, 93 and 83 (128: 357 and 375).  256 tokens stay: cut in two they take
+// 0.90 - 1.09 of the time.
 // Measured forward + backward in fp32, d = e = 128, this rule against the one of the 16-bit sweeps:
 // b*h = 24, n = 16384: 512 tokens, 1555 us against 1783 (1024: 384 workgroups, half the CUs with two);
 // b*h = 4, n = 8192: 128 tokens, 181 against 231; b*h = 8, n = 4096: 128, 173 against 228; b*h = 16, n = 1024:
 // 64, 108 against 176; b*h = 1, n = 8192: 64, 109 against 179; b*h = 24, n = 2048: 128, 272 against 280; equal
 // within 3 % on the other shapes tried (b*h = 1 ... 256, n = 1024 ... 262144).
-int two_per_cu_seg_len(int b, int h, int64_t n) {
+int two_per_cu_seg_len(int b, int h, int64_t n, int d, int e) {
   const int64_t bh = (int64_t)b * h;
   auto groups = [&](int64_t len) { return bh * ((n + len - 1) / len); };
   int64_t best = kSegQuantum, best_load = -1;
@@ -203,7 +207,8 @@ int two_per_cu_seg_len(int b, int h, int64_t n) {
     }
     if (len >= n) break;
   }
-  if (best >= kPreferredSeg && best < n && groups(best) <= kMinGroups) best /= 2;
+  const int64_t cut = d <= 96 && e <= 96 ? kPreferredSeg / 2 : kPreferredSeg;
+  if (best >= cut && best < n && groups(best) <= kMinGroups) best /= 2;
   return (int)best;
 }
 
@@ -214,13 +219,15 @@ int two_per_cu_seg_len(int b, int h, int64_t n) {
 // gain from it, hence the places.  Taken only if it is 5 % better by that count.  Measured forward + backward over b*h = 16 ... 512, n =
 // 96 ... 2048, d = e = 128 and 64, segments against one: b*h = 192, n = 512: 309 and 238 us (64: 159 and 152); b*h = 64, n = 256:
 // 79 and 66; b*h = 48, n = 96: 56 and 30; b*h = 384, n = 1024: 1003 and 867; b*h = 96, n = 1024, where segments stay: 310 and 318
-// (64: 162 and 223).  Of 308 shapes 159 take it, none slower by more than 3 %.
+// (64: 162 and 223).  Of 308 shapes 159 take it, none slower by more than 3 %.  Where 512-token segments are cut
+// in two (narrow heads, b*h = 128, n = 513 ... 1024) the choice is within 3 % of the better one on 47 of 52 shapes, at worst 10 % off (96
+// features, n = 850: 253 us where one segment takes 230).
 constexpr int64_t kMaxWhole = 2048;  // tokens, the range measured
 int whole_seg_len(int b, int h, int64_t n, int d, int e) {
   const int64_t bh = (int64_t)b * h;
   const bool small = d <= 64 && e <= 64;
   const int64_t places = small ? 512 : 256, launches = small ? 10 : 8;
-  const int seg_len = two_per_cu_seg_len(b, h, n);
+  const int seg_len = two_per_cu_seg_len(b, h, n, d, e);
   if (n <= seg_len || n > kMaxWhole) return 0;
   auto cost = [&](int64_t segs, int64_t len) {
     const int64_t groups = bh * segs, rounds = (groups + places - 1) / places + (3 * groups + places - 1) / places;
@@ -235,7 +242,7 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   if (rc) return rc;
   const int seg_len_arg = seg_len;
   const int width = sweep_width(d, e);
-  if (seg_len == 0) seg_len = mfma_eligible(d, e, dtype) ? default_seg_len(b, h, n, width == 64) : two_per_cu_seg_len(b, h, n);
+  if (seg_len == 0) seg_len = mfma_eligible(d, e, dtype) ? default_seg_len(b, h, n, width == 64) : two_per_cu_seg_len(b, h, n, d, e);
   if (seg_len < 0 || seg_len % kSegQuantum != 0) {
     set_error("seg_len=%d must be a positive multiple of %d (or 0 for the default)", seg_len,
               kSegQuantum);

@@ -129,3 +129,15 @@ def test_rows_that_start_off_a_vector(native):
             o, states, seg = _abi.chunk_fwd(q, k, v, s)
             seen.append((o, *_abi.chunk_bwd(q, k, v, s, do, kv_seg_states=states, seg_len=seg)))
     assert all(torch.equal(a, c) for a, c in zip(*seen))
+
+
+@pytest.mark.parametrize("d,e,b,n", [(64, 64, 16, 1800), (96, 80, 32, 600)])
+def test_segments_of_512_tokens_cut_in_two(d, e, b, n):
+    """The default plan where it halves a segment that has a CU to itself."""
+    h = 4
+    assert _abi.plan(b, h, n, d, e, torch.float32, 0)[0] == 256
+    assert _abi.plan(b, h, n, 128, 128, torch.float32, 0)[0] == 512
+    inp = make_inputs(b, h, n, d, e, torch.float32, seed=n, scale=0.1, state=True)
+    s = lasp_amd.build_slope_tensor(h)
+    ref = O.ref_chunked(inp["q"], inp["k"], inp["v"], s, inp["do"], inp["kv"], inp["dkv"], dtype=torch.float64)
+    check(_run(inp, s, 0), ref, (60 + 12 * -(-n // 32)) * 2.0 ** -24, what=f"d={d} e={e} n={n}")
