@@ -306,16 +306,18 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
   if (tid < BLK) *reinterpret_cast<float *>(smem + OFF_W + 4 * tid) = decay(sl, REV ? (float)tid : (float)(BLK - tid));
   // this wave's quadrant of the score tile: tokens b = 16 qb .. of Y, a = 16 qa .. of X
   const int qb = w >> 1, qa = w & 1;
-  const bool q_active = REV ? !(qb == 0 && qa == 1) : !(qb == 1 && qa == 0);
   const int q_lane = lane & 15, q_grp = lane >> 4;
   const int xq = (16 * qa + q_lane) * ROW + ((q_grp ^ swizzle(16 * qa + q_lane)) << 4);
   const int yq = (16 * qb + q_lane) * ROW + ((q_grp ^ swizzle(16 * qb + q_lane)) << 4);
-  float qmask[4];  // decay between the tokens of a score
+  // decay between the tokens of a score; -1: masked.  Such a score is left out and not multiplied by zero, which would take an
+  // infinity or a NaN (or what overflowed on the way to this score only) to tokens that do not see it.
+  float qmask[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int dist = (16 * qa + q_lane - 16 * qb - 4 * q_grp - r) * (REV ? -1 : 1);
-    qmask[r] = dist >= 0 ? decay(sl, (float)dist) : 0.f;
+    qmask[r] = dist >= 0 ? decay(sl, (float)dist) : -1.f;
   }
+  auto masked = [&](float score, int r) __attribute__((always_inline)) { return qmask[r] < 0.f ? 0.f : score * qmask[r]; };
   // rows of 64 bytes; unit u of row a lies at u ^ ((a >> 2) & 3)
   const int sc_at = (16 * qa + q_lane) * SC_ROW + (((2 * qb + (q_grp >> 1)) ^ ((q_lane >> 2) & 3)) << 4) + ((q_grp & 1) << 3);
   const int sc_from = c * SC_ROW + ((hh ^ ((c >> 2) & 3)) << 4);
@@ -412,9 +414,9 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       reads_first();
       u32x2 h, m, l;
       uint32_t a, b, d;
-      split2(sc[0] * qmask[0], sc[1] * qmask[1], a, b, d);
+      split2(masked(sc[0], 0), masked(sc[1], 1), a, b, d);
       h.x = a, m.x = b, l.x = d;
-      split2(sc[2] * qmask[2], sc[3] * qmask[3], a, b, d);
+      split2(masked(sc[2], 2), masked(sc[3], 3), a, b, d);
       h.y = a, m.y = b, l.y = d;
       char *at = smem + OFF_SC + sc_at;
       *reinterpret_cast<u32x2 *>(at) = h;

@@ -20,9 +20,9 @@ def _run(inp, s, seg):
     dev = {k: (t.cuda() if t is not None else None) for k, t in inp.items()}
     s = s.cuda()
     kv_out, dkv_out = (torch.empty_like(dev["kv"]) for _ in range(2)) if dev["kv"] is not None else (None, None)
-    o, states, seg_len = _abi._chunk_fwd_exact(dev["q"], dev["k"], dev["v"], s, kv_in=dev["kv"], kv_out=kv_out, seg_len=seg)
-    dq, dk, dv = _abi._chunk_bwd_exact(dev["q"], dev["k"], dev["v"], s, dev["do"], kv_in=dev["kv"], dkv_in=dev["dkv"],
-                                       dkv_out=dkv_out, kv_seg_states=states, seg_len=seg_len)[:3]
+    o, states, seg_len = _abi.chunk_fwd(dev["q"], dev["k"], dev["v"], s, kv_in=dev["kv"], kv_out=kv_out, seg_len=seg)
+    dq, dk, dv = _abi.chunk_bwd(dev["q"], dev["k"], dev["v"], s, dev["do"], kv_in=dev["kv"], dkv_in=dev["dkv"],
+                                dkv_out=dkv_out, kv_seg_states=states, seg_len=seg_len)
     return dict(o=o, kv_out=kv_out, dq=dq, dk=dk, dv=dv, dkv_out=dkv_out)
 
 
@@ -61,14 +61,48 @@ def test_lowest_value():
     check(got, ref, TOL, names=("o",))
 
 
-def test_nan_stays_behind():
-    """A NaN of a token reaches its own output and none of the blocks before it."""
-    inp = make_inputs(1, H, 96, 128, 128, torch.float32, seed=7, scale=0.1, state=False)
+T, CLEAN = 70, 64  # a token in the middle of a 32-token block, and where its block starts
+# what an input of token T reaches: outputs from there on (forwards), up to there (backwards), or its own only
+REACH = {("q", "o"): "own", ("k", "o"): "later", ("do", "dq"): "own", ("v", "dq"): "later", ("k", "dv"): "own", ("q", "dv"): "earlier",
+         ("v", "dk"): "own", ("do", "dk"): "earlier"}
+
+
+@pytest.mark.parametrize("d,e", [(128, 128), (64, 96)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("name", ["q", "k", "v", "do"])
+def test_nonfinite_inputs_stay_where_they_are_seen(name, value, d, e):
+    """A NaN or an infinity of a token reaches no token that does not see it, in its own block neither: where it is a factor of
+    the scores.  As a summed row (V, and K, Q, dO in their gradients) it meets the masked scores, which are zero, inside a product, and
+    other tokens of its block become NaN; no token of the blocks before (after, backwards) does."""
+    inp = make_inputs(1, H, 128, d, e, torch.float32, seed=7, scale=0.1, state=False)
     s = lasp_amd.build_slope_tensor(H)
-    clean = _run(inp, s, 64)["o"]
-    for name in ("q", "k", "v"):
-        bad = dict(inp, **{name: inp[name].clone()})
-        bad[name][:, :, 70, 9] = float("nan")
-        o = _run(bad, s, 64)["o"]
-        assert torch.isnan(o[:, :, 70]).any(-1).all()
-        assert torch.equal(o[:, :, :64], clean[:, :, :64])
+    clean = _run(inp, s, 64)
+    bad = dict(inp, **{name: inp[name].clone()})
+    bad[name][:, :, T, 9] = value
+    got = _run(bad, s, 64)
+    for (source, out), reach in REACH.items():
+        if source != name:
+            continue
+        seen = {"own": slice(T, T + 1), "later": slice(T, None), "earlier": slice(0, T + 1)}[reach]
+        assert not torch.isfinite(got[out][:, :, T]).all(-1).any(), out
+        same = got[out] == clean[out]
+        same[:, :, seen] = True
+        assert same.all(), (out, (~same).any(-1).nonzero()[:8].tolist())
+    if name == "v":
+        assert torch.equal(got["o"][:, :, :CLEAN], clean["o"][:, :, :CLEAN])
+
+
+@pytest.mark.parametrize("d,e", [(128, 128), (64, 96)])
+def test_masked_scores_that_overflow(d, e):
+    """Finite inputs whose product is too large for fp32 only between tokens that do not see each other."""
+    inp = make_inputs(1, H, 128, d, e, torch.float32, seed=8, scale=0.1, state=False)
+    inp["q"][:, :, T, 3], inp["do"][:, :, T, 3] = 1e20, 1e20
+    s = lasp_amd.build_slope_tensor(H)
+    clean = _run(inp, s, 64)
+    inp["k"][:, :, T + 5, 3], inp["v"][:, :, T + 5, 3] = 1e20, 1e20
+    got = _run(inp, s, 64)
+    for out in ("o", "dq"):
+        assert torch.isfinite(got[out][:, :, :T + 5]).all()
+        assert torch.equal(got[out][:, :, :T + 5], clean[out][:, :, :T + 5]), out
+    for out in ("dk", "dv"):
+        assert torch.isfinite(got[out][:, :, T + 1:]).all(), out
