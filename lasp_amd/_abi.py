@@ -154,11 +154,15 @@ def inplace_ok(b, h, n, d, e, dtype, seg_len: int, backward: bool) -> bool:
     return bool(rc)
 
 
-def _private_incoming(state_in, state_out, shape_key, seg_len, backward):
+def _private_incoming(state_in, state_out, shape_key, seg_len, backward, narrow=False):
     """`state_in`, or a copy of it when `state_out` is the same memory and the kernels this shape runs
-    on cannot update a state in place (the copy then plays the reference's in-place update)."""
-    if state_in is None or state_out is None or state_in.data_ptr() != state_out.data_ptr():
+    on cannot update a state in place (the copy then plays the reference's in-place update).  States of narrow float32
+    rows may also lie partly over each other, as they may for rows that are padded; the library refuses that."""
+    if state_in is None or state_out is None:
         return state_in
+    apart = state_out.data_ptr() - state_in.data_ptr()
+    if apart:
+        return state_in.clone() if narrow and abs(apart) < 4 * state_in.numel() else state_in
     return state_in if inplace_ok(*shape_key, seg_len, backward) else state_in.clone()
 
 
@@ -261,7 +265,7 @@ def _chunk_fwd_exact(q, k, v, s, kv_in=None, kv_out=None, seg_len: int = 0, narr
     if not fused:
         seg_len, n_seg, state_bytes = plan(b, h, n, d, e, q.dtype, seg_len)
     with _on_device(dev):
-        kv_in = _private_incoming(kv_in, kv_out, (b, h, n, d, e, q.dtype), seg_len, False)
+        kv_in = _private_incoming(kv_in, kv_out, (b, h, n, d, e, q.dtype), seg_len, False, narrow)
         o = torch.empty((b, h, n, e), dtype=q.dtype, device=dev)
         states = None
         if not fused and (n_seg > 1 or kv_in is not None or kv_out is not None):
@@ -334,7 +338,7 @@ def _chunk_bwd_exact(q, k, v, s, do, kv_in=None, dkv_in=None, dkv_out=None, kv_s
                             f"chunk_fwd returned for this shape, got {kv_seg_states.dtype} "
                             f"{tuple(kv_seg_states.shape)}")
     with _on_device(dev):
-        dkv_in = _private_incoming(dkv_in, dkv_out, (b, h, n, d, e, q.dtype), 0 if fused else seg_len, True)
+        dkv_in = _private_incoming(dkv_in, dkv_out, (b, h, n, d, e, q.dtype), 0 if fused else seg_len, True, narrow)
         dq = torch.empty_like(q)
         dk = torch.empty_like(k)
         dv = torch.empty_like(v)

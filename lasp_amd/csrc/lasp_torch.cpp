@@ -145,9 +145,12 @@ Plan plan_of(const Shape &sh, int seg_len) {
   return p;
 }
 
-// `in`, or a copy where `out` is the same memory and this shape's kernels cannot update a state in place
+// `in`, or a copy where `out` is the same memory and this shape's kernels cannot update a state in place.  States of narrow fp32 rows
+// may also lie partly over each other, as they may where rows are padded; the library refuses that.
 Tensor private_incoming(const Tensor &in, const Tensor &out, const Shape &sh, int seg_len, bool backward) {
-  if (!in.defined() || !out.defined() || in.data_ptr() != out.data_ptr()) return in;
+  if (!in.defined() || !out.defined()) return in;
+  const uintptr_t a = (uintptr_t)in.data_ptr(), b = (uintptr_t)out.data_ptr();
+  if (a != b) return is_narrow(sh) && a < b + out.nbytes() && b < a + in.nbytes() ? in.clone() : in;
   return lasp_inplace_ok(sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, seg_len, backward) == 1 ? in : in.clone();
 }
 

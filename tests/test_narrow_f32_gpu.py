@@ -131,6 +131,38 @@ def test_rows_that_start_off_a_vector(native):
     assert all(torch.equal(a, c) for a, c in zip(*seen))
 
 
+def _overlapping(state, apart):
+    """`state` and room for another that starts `apart` floats after it, in one buffer."""
+    first, second = max(-apart, 0), max(apart, 0)
+    room = torch.zeros(state.numel() + abs(apart), device="cuda")
+    views = [room[at:at + state.numel()].view(state.shape) for at in (first, second)]
+    views[0].copy_(state)
+    return views
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("apart", [4, -4, 64 * 36])
+def test_states_that_lie_partly_over_each_other(native, apart):
+    """As where rows are padded; states of full rows are refused."""
+    inp = {k: t.cuda() for k, t in make_inputs(1, H, 300, 64, 36, torch.float32, seed=4, scale=0.1, state=True).items()}
+    s = lasp_amd.build_slope_tensor(H).cuda()
+    calls = _native if native else _abi
+
+    def run(pair):
+        kv, kv_out = pair(inp["kv"])
+        o, _, _ = calls.chunk_fwd(inp["q"], inp["k"], inp["v"], s, kv_in=kv, kv_out=kv_out)
+        dkv, dkv_out = pair(inp["dkv"])
+        grads = calls.chunk_bwd(inp["q"], inp["k"], inp["v"], s, inp["do"], kv_in=inp["kv"], dkv_in=dkv, dkv_out=dkv_out)
+        return (o, kv_out, *grads, dkv_out)
+
+    got, want = run(lambda t: _overlapping(t, apart)), run(lambda t: (t.clone(), torch.empty_like(t)))
+    assert all(torch.equal(a, c) for a, c in zip(got, want))
+    full = torch.zeros(1, H, 64, 128, device="cuda")
+    kv, kv_out = _overlapping(torch.zeros(1, H, 128, 128, device="cuda"), apart)
+    with pytest.raises(_abi.LaspError, match="overlaps"):
+        calls.chunk_fwd(full, full, full, s, kv_in=kv, kv_out=kv_out)
+
+
 @pytest.mark.parametrize("d,e,b,n", [(64, 64, 16, 1800), (96, 80, 32, 600)])
 def test_segments_of_512_tokens_cut_in_two(d, e, b, n):
     """The default plan where it halves a segment that has a CU to itself."""
