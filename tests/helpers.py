@@ -39,6 +39,19 @@ def check(got: dict, ref: dict, tol: float, names=NAMES, what=""):
     return errs
 
 
+# What the three-part products of the fp32 MFMA kernels leave, as a 2-norm over an output's: some 60 roundings of 2^-25 (of 2^-24 at
+# most) of a partial sum, which add up like a random walk to 2.3e-7, and a few of operands and decays; measured 0.7e-7 to 2.2e-7 (n = 1 ...
+# 2048).  A product that lost its third parts (2^-17 of an operand) would show 5e-6 and more.
+NORM_F32 = 1e-6
+
+
+def check_norm(got: dict, ref: dict, tol: float, names=NAMES, what=""):
+    """Asserts |x - ref| <= tol |ref| in 2-norms over each whole output."""
+    errs = {name: float((got[name].cpu().double() - ref[name].double()).norm() / ref[name].double().norm())
+            for name in names if got.get(name) is not None}
+    assert all(v_ <= tol for v_ in errs.values()), f"{what}: 2-norm over {tol}: {errs}"
+
+
 def in_place_bits(inp, s, seg):
     """Outputs of a forward and two backwards (the forward's states, rebuilt ones) whose states are updated in place, each
     with that of separate buffers.  Where the library does not take a shape in place in a direction, that one is left out."""

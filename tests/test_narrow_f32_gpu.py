@@ -7,7 +7,7 @@ import torch
 import lasp_amd
 from lasp_amd import _abi, _native
 from oracle import lasp_oracle as O
-from tests.helpers import check, make_inputs
+from tests.helpers import NORM_F32, check, check_norm, make_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -36,7 +36,9 @@ def test_widths(d, e, n, state):
     s = lasp_amd.build_slope_tensor(H)
     ref = O.ref_chunked(inp["q"], inp["k"], inp["v"], s, inp["do"], inp["kv"], inp["dkv"], dtype=torch.float64)
     for cached in (True, False):
-        check(_run(inp, s, 64, cached), ref, TOL, what=f"d={d} e={e} n={n} cached={cached}")
+        got = _run(inp, s, 64, cached)
+        check(got, ref, TOL, what=f"d={d} e={e} n={n} cached={cached}")
+        check_norm(got, ref, NORM_F32, what=f"d={d} e={e} n={n} cached={cached}")
 
 
 @pytest.mark.parametrize("d,e", WIDTHS)

@@ -6,7 +6,7 @@ import torch
 import lasp_amd
 from lasp_amd import _abi
 from oracle import lasp_oracle as O
-from tests.helpers import check, make_inputs
+from tests.helpers import NORM_F32, check, check_norm, make_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -32,7 +32,9 @@ def test_lengths(n, state):
     inp = make_inputs(1, H, n, 128, 128, torch.float32, seed=n, scale=0.1, state=state)
     s = lasp_amd.build_slope_tensor(H)
     ref = O.ref_chunked(inp["q"], inp["k"], inp["v"], s, inp["do"], inp["kv"], inp["dkv"], dtype=torch.float64)
-    check(_run(inp, s, 64), ref, TOL, what=f"n={n}")
+    got = _run(inp, s, 64)
+    check(got, ref, TOL, what=f"n={n}")
+    check_norm(got, ref, NORM_F32, what=f"n={n}")
 
 
 def test_features_of_any_size():
@@ -46,6 +48,45 @@ def test_features_of_any_size():
     for out, by in (("dq", size), ("dk", 1 / size)):
         got[out], ref[out] = got[out].cpu() * by, ref[out] * by.double()
     check(got, ref, TOL, names=("o", "dq", "dk", "dv"))
+    check_norm(got, ref, NORM_F32, names=("o", "dq", "dk", "dv"))
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("value", [1.0077972, 0.7071068, 0.1, 3.14159265])
+def test_equal_numbers(d, value):
+    """Every product is the same, and so is what it leaves out: nothing averages.  The omitted partial products are at most 2^-22 of
+    a product, in each of the up to three products that an output passes through, beside the roundings of the sums, all of one sign."""
+    n = 64
+    inp = {x: torch.full((1, H, n, d), value) for x in ("q", "k", "v", "do")}
+    inp.update(kv=None, dkv=None)
+    s = lasp_amd.build_slope_tensor(H)
+    ref = O.ref_chunked(inp["q"], inp["k"], inp["v"], s, inp["do"], dtype=torch.float64)
+    check_norm(_run(inp, s, 64), ref, 3 * 2.0 ** -22 + NORM_F32, what=f"{value}")
+
+
+@pytest.mark.parametrize("n,d", [(1, 128), (3, 128), (3, 64)])
+def test_short_sums(n, d):
+    """Sums of one or a few products, in which no error averages: features of which one is not zero."""
+    inp = make_inputs(16, H, n, d, d, torch.float32, seed=n, state=False)
+    for x in ("q", "k"):
+        inp[x][..., 1:] = 0
+    s = lasp_amd.build_slope_tensor(H)
+    ref = O.ref_chunked(inp["q"], inp["k"], inp["v"], s, inp["do"], dtype=torch.float64)
+    check_norm(_run(inp, s, 64), ref, NORM_F32, what=f"n={n} d={d}")
+
+
+@pytest.mark.parametrize("power", [-109, -115, -120])
+def test_small_operands(power):
+    """Numbers below 2^-110 have parts under bf16's smallest, 2^-133: they are held to 2^-134 (to the bit above), here in q and in what
+    is made of it and k, whose size makes up for it: rows, weighted rows and states, each off by 2^-134 of 2^power."""
+    inp = make_inputs(1, H, 130, 128, 128, torch.float32, seed=9, state=False)
+    inp["q"], inp["k"] = inp["q"] * 2.0 ** power, inp["k"] * 2.0 ** 100
+    s = lasp_amd.build_slope_tensor(H)
+    ref = O.ref_chunked(inp["q"], inp["k"], inp["v"], s, inp["do"], dtype=torch.float64)
+    got = _run(inp, s, 64)
+    tol = NORM_F32 + (3 * 2.0 ** (-134 - power) if power < -110 else 0)
+    check_norm(got, ref, tol, names=("o", "dk", "dv"))
+    check_norm(got, ref, NORM_F32, names=("dq",))
 
 
 def test_lowest_value():
