@@ -317,7 +317,8 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
     const int dist = (16 * qa + q_lane - 16 * qb - 4 * q_grp - r) * (REV ? -1 : 1);
     qmask[r] = dist >= 0 ? decay(sl, (float)dist) : -1.f;
   }
-  auto masked = [&](float score, int r) __attribute__((always_inline)) { return qmask[r] < 0.f ? 0.f : score * qmask[r]; };
+  // (selected before the product, which the compiler fuses with the first subtraction of the split: its rounding is not felt)
+  auto masked = [&](float score, int r) __attribute__((always_inline)) { return (qmask[r] < 0.f ? 0.f : score) * qmask[r]; };
   // rows of 64 bytes; unit u of row a lies at u ^ ((a >> 2) & 3)
   const int sc_at = (16 * qa + q_lane) * SC_ROW + (((2 * qb + (q_grp >> 1)) ^ ((q_lane >> 2) & 3)) << 4) + ((q_grp & 1) << 3);
   const int sc_from = c * SC_ROW + ((hh ^ ((c >> 2) & 3)) << 4);
