@@ -51,7 +51,7 @@ BYTES_FWD_PER_TH = 1024        # read Q,K,V + write O, bf16
 BYTES_BWD_PER_TH = 1792        # read Q,K,V,dO + write dQ,dK,dV
 HBM_PEAK_GBS = 8000.0
 MFMA_BF16_PEAK_TFLOPS = 2500.0
-MFMA_F32_PEAK_TFLOPS = 157.3
+F32_PRODUCTS = 6  # bf16 products that the fp32 kernels make of one
 HBM_PROFILE = os.path.join(ROOT, "profiles", "pmc_hbm_bytes_config2.txt")
 
 
@@ -295,7 +295,7 @@ def other_configs(dev):
     for t in (q, k, v):
         t.requires_grad_(True)
     r = with_bytes(rates(gpu_time(single_pass_step(lasp_amd, q, k, v, do, slopes(h).to(dev)), 50), b, h, n), b, h, n, 4)
-    r["frac_f32_mfma_peak"] = r["tflops"] / MFMA_F32_PEAK_TFLOPS
+    r["frac_bf16_mfma_peak"] = r["tflops"] * F32_PRODUCTS / MFMA_BF16_PEAK_TFLOPS
     out["config0_fp32_single_pass"] = r
     del q, k, v, do
 

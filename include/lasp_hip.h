@@ -30,6 +30,11 @@
  * fp32).  With fp16 I/O any of them beyond 65504 in magnitude becomes inf -- a large
  * caller-supplied kv_in, or a slow-decay head with positive-mean feature maps over a
  * long chunk; bf16 has the range of fp32 and no such limit.
+ * The fp32 MFMA kernels multiply numbers split into three bf16 parts.  They take all
+ * finite numbers, those below 2^-110 in magnitude to the nearest multiple of 2^-133; an
+ * infinity, and a sum that overflows, makes NaN (not an infinity) of what it takes part
+ * in.  What is not finite reaches the tokens that see it and, where it is summed as a row
+ * (v in o, k in dq, q in dk, do in dv), others of its block of 32 tokens.
  *
  * Every call only ENQUEUES work on `stream` (a hipStream_t; NULL = the default
  * stream); nothing is allocated, freed or synchronised, pointers are borrowed
@@ -109,7 +114,8 @@ int lasp_plan(int b, int h, int64_t n, int d, int e, int dtype, int seg_len_or_0
               int *seg_len, int *n_seg, size_t *state_bytes);
 
 /* The seg_len to pass for a forward without kv_in and kv_out and for its backward, where that differs from lasp_plan's
- * default (float32 on the MFMA kernels: one segment, which needs no states); 0: the default is right. */
+ * default (float32 on the MFMA kernels, i.e. lasp_chunk_* for d = e = 128 and lasp_narrow_* for narrower rows: one segment, which
+ * needs no states); 0: the default is right. */
 int lasp_stateless_seg_len(int b, int h, int64_t n, int d, int e, int dtype);
 
 /* LASP_PATH_* for this shape under the default plan (seg_len = 0), or a negative LASP_E_* if it is

@@ -188,12 +188,16 @@ bool fused_eligible(int64_t n, int d, int e, int dtype, int seg_len_arg, int seg
 // waits.  Heads of up to 96 features, whose states cost half as much or less to carry, gain from that from 512 tokens on:
 // fp32 forward + backward and forward alone with states, 512 and 256 tokens, b*h = 16, n = 8192: d = e = 32: 205 and 179 us, 74
 // and 59; 64: 212 and 191, 76 and 63; 96: 279 and 270, 93 and 83 (128: 357 and 375).  256 tokens stay: cut in two they take
-// 0.90 - 1.09 of the time.
-// Measured forward + backward in fp32, d = e = 128, this rule against the one of the 16-bit sweeps:
-// b*h = 24, n = 16384: 512 tokens, 1555 us against 1783 (1024: 384 workgroups, half the CUs with two);
-// b*h = 4, n = 8192: 128 tokens, 181 against 231; b*h = 8, n = 4096: 128, 173 against 228; b*h = 16, n = 1024:
-// 64, 108 against 176; b*h = 1, n = 8192: 64, 109 against 179; b*h = 24, n = 2048: 128, 272 against 280; equal
-// within 3 % on the other shapes tried (b*h = 1 ... 256, n = 1024 ... 262144).
+// 0.90 - 1.09 of the time.  The generic kernels, which share the plan, gain more (fp32 and bf16 heads of 30 to 96 features, b*h = 8 ... 128,
+// 512 and 256 tokens: forward 0.51 - 0.55 of the time, forward + backward 0.52 - 0.69); the states of such a plan, at most 512, fit the
+// library's scratch array as those of half as many did.
+// Measured forward + backward in fp32, d = e = 128, replayed from a graph: b*h = 24, n = 16384: 512 tokens, 1051 us (256: 1114,
+// 1024, 384 workgroups, half the CUs with two: 1089); b*h = 4, n = 8192: 128 tokens, 129 (64: 152, 256: 143); b*h = 8, n = 4096: 128, 127
+// (151 and 143); b*h = 16, n = 1024: 64, 89 (128: 92); b*h = 64, n = 4096: 512, 694 (744 and 713); b*h = 256, n = 4096: 4096, 2249 (2048:
+// 2524).  Over 27 shapes (b*h = 1 ... 256, n = 300 ... 262144) against 64, 128, ... 2048 tokens and the length that the 16-bit kernels
+// would take, the rule has the best or comes within 2 % on 21 at d = e = 128, and on 24 at 64; within 8 % on the others (d = e = 128: b*h =
+// 96, n = 1024: 318 against 298 for 256 tokens; b*h = 1, n = 8192: 89 against 84 for 128; b*h = 48, n = 3000: 451 against 428 for 640; b*h = 24,
+// n = 2048: 181 against 173 for 320) but for b*h = 160, n = 700, where one segment is better (343 against 273), see below.
 int two_per_cu_seg_len(int b, int h, int64_t n, int d, int e) {
   const int64_t bh = (int64_t)b * h;
   auto groups = [&](int64_t len) { return bh * ((n + len - 1) / len); };
@@ -221,7 +225,9 @@ int two_per_cu_seg_len(int b, int h, int64_t n, int d, int e) {
 // 79 and 66; b*h = 48, n = 96: 56 and 30; b*h = 384, n = 1024: 1003 and 867; b*h = 96, n = 1024, where segments stay: 310 and 318
 // (64: 162 and 223).  Of 308 shapes 159 take it, none slower by more than 3 %.  Where 512-token segments are cut
 // in two (narrow heads, b*h = 128, n = 513 ... 1024) the choice is within 3 % of the better one on 47 of 52 shapes, at worst 10 % off (96
-// features, n = 850: 253 us where one segment takes 230).
+// features, n = 850: 253 us where one segment takes 230).  A forward alone, whose backward may or may not follow, takes the same plan: over
+// 219 shapes that run as one segment 0.74 of the segments' time on average, faster or equal within 3 % on 204, at worst 1.28 (b*h = 48,
+// n = 400, d = e = 96: 45 us against 35).
 constexpr int64_t kMaxWhole = 2048;  // tokens, the range measured
 int whole_seg_len(int b, int h, int64_t n, int d, int e) {
   const int64_t bh = (int64_t)b * h;

@@ -5,14 +5,20 @@
 // dV: x=K y=Q z=dO anti-causal; dK: x=V y=dO z=Q anti-causal, state transposed) -- but with
 // full-precision arithmetic, for inputs whose tolerance (1e-3) rules out 16-bit operands.
 //
-// The matrix unit multiplies fp32 at a sixteenth of its bf16 rate, so every operand is split into three bf16 numbers,
-// x = h + m + l: h is x cut off after 8 bits, m what is left rounded to 8 bits, l the rest, and |x - h - m - l| <= 2^-25 |x|, no
-// more than fp32 itself rounds x by.  A product is the six of the nine partial products that reach 2^-24 of the whole, the small
-// ones first, in the unit's fp32 accumulators; m l and l m, left out, are of either sign and 2^-25 of a term as a rule (2^-23 at
-// most).  Sums of a few wide products round less often than sums of many narrow ones: the errors against 64 bits (2-norms) are
-// 0.71 - 0.83 of those with v_mfma_f32_32x32x2_f32, used before (n = 64 ... 7168, with and without states, 2.3e-7 against 2.9e-7
-// at b*h = 24, n = 2048).  All finite numbers are taken; an infinite one makes NaN of what it takes part in, where the fp32
-// instruction could leave an infinity.
+// The matrix unit multiplies fp32 at a sixteenth of its bf16 rate, so every operand is split into three bf16 numbers (Henry,
+// Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", 2019), x = h
+// + m + l: h is x cut off after 8 bits, m what is left rounded to 8 bits, l the rest.  The three hold x exactly from 2^-110 on;
+// below, where l and then m fall under bf16's smallest number, 2^-133, they are off by up to 2^-134 (1e-6 of an operand at
+// 2^-115, 4e-5 at 2^-120).  A product is the six of the nine partial products that reach 2^-24 of the whole, the small ones
+// first, in the unit's fp32 accumulators; m l and l m, left out, are 2^-25 of a term as a rule and of either sign, and at most
+// 2^-22 together.  With these two added the errors are the same within 5 % from n = 16 on and up to a quarter less below, and
+// 0.6 - 1.04 of themselves for rows of equal numbers, whose errors do not average. Sums of a few wide products round less often
+// than sums of many narrow ones: 2-norms of the errors against 64 bits are 0.62 - 0.86 of those with v_mfma_f32_32x32x2_f32,
+// used before, for random numbers, d = 64 and 128, n = 2 ... 2048 (n = 1: 0.64 - 1.03; no decay, n = 2048: 3.7e-7 against
+// 4.4e-7), and 0.09 - 1.0 for rows of equal numbers.  Products of single features go either way (n = 1: dv 6.9e-8 against
+// 3.3e-8, dq 1.0e-7 against 1.6e-7).  All finite numbers are taken; an infinite one, or a sum that overflows, makes NaN of what
+// it takes part in, where the fp32 instruction could leave an infinity.  Neither reaches a token that does not see it through a
+// score, but a row of Z that is not finite meets the masked scores, zeros, of its block in a product.
 //
 // The state tiles feed the state-term product straight from registers (see the order of features below), each split anew for
 // every block.  The LDS holds the X and Y rows of a block, split, and the masked 32 x 32 score tile, split, of which each of the
@@ -22,10 +28,11 @@
 //
 // What bounds it: a wave and block take 132 matrix instructions (3840 cycles of its SIMD's matrix unit) and some 870 others on
 // the vector unit, two thirds of them for splitting; one of those costs about 4 cycles of issue and a matrix instruction 11, so
-// that a block cannot take less than 4900 cycles.  It takes 8100 (two workgroups per CU, n = 16384).  The splitting stands between
-// the matrix instructions, one by one: 9200 with each operand split in one go.  Against v_mfma_f32_32x32x2_f32 (10 240
-// cycles of matrix unit per block), forward + backward: b*h = 24, n = 2048: 170 - 180 us against 231; n = 16384: 1034
-// against 1384.
+// that a block cannot take less than 4900 cycles.  At n = 16384, with two workgroups per CU, it takes a CU 8200 in the forward
+// sweep and 7000 in the backward, the matrix units busy 47 and 55 % of the time (75 and 81 % of 13 700 and 12 600 with
+// v_mfma_f32_32x32x2_f32, 10 240 cycles of matrix unit per block).  The splitting stands between the matrix instructions, one
+// by one: 9200 with each operand split in one go. Against v_mfma_f32_32x32x2_f32, forward + backward: b*h = 24, n = 2048: 172 -
+// 182 us against 227 - 231; n = 16384: 1034 - 1072 against 1365.
 #include "lasp_common.h"
 
 namespace lasp {
