@@ -352,7 +352,6 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   g->n = n;
   g->d = d < kMaxFeature ? d : kMaxFeature;
   g->dt = d;
-  g->add = 0;
   g->e = e;
   g->seg_len = seg_len;
   g->n_seg = (int)n_seg_final;

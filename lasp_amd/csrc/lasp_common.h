@@ -73,7 +73,6 @@ struct Geom {
                 // generic kernels, 128 x 128 or 64 x 64 (zero beyond d, e) for the MFMA kernels
   int width;    // 16-bit MFMA kernels: the width they are laid out for, 128 or 64; else 0
   int dt;       // features in a row of q and k: d, or more where the head is wide and d is the slice at hand
-  int add;      // the sweep adds its O (dV) to what a slice before it left there
   int fused;    // the chunk is served by the single-launch kernels, which use no workspace
   int combine;  // few segments: no scan launch, the sweep workgroups gather the segments' own states
   int bypass;   // the scan leaves out heads whose state dies within one segment (see state_dies_in_segment)

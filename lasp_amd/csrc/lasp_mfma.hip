@@ -3,7 +3,7 @@
 // (one partial last block) and M_NARROW (rows of d, e < W features, multiples of 8, read
 // zero-extended to W and written back at their own width; any chunk length).
 //
-// One device routine, `ws_body`, evaluates a causal (or anti-causal) decayed linear
+// A sweep (`sweep_body` for W = 128, `ws_body` for W = 64) evaluates a causal (or anti-causal) decayed linear
 // attention over a segment of 64-token blocks given the state entering it:
 //
 //   causal       out_a = sum_{b<=a} l^(a-b) (x_a . y_b) z_b + l^a      x_a St
@@ -20,15 +20,14 @@
 // `la_seg_state` computes a segment's own contribution to St (the pre-pass whose
 // results the decayed scan stitches together).
 //
-// Work split inside a 512-thread workgroup (8 waves, one workgroup per CU): four "math"
-// waves own the state and the output -- wave w columns [32w, 32w+32), as four 32x32 fp32
-// MFMA accumulator tiles that never leave registers -- and four "feed" waves fetch and
-// transpose the next block, compute the 64x64 score tile (one 32x32 quadrant per wave;
-// masked, rounded to 16 bits and shared through LDS) and store the outputs.  All products are arranged so that an accumulator tile can be fed
-// back as an MFMA operand without a shuffle: v_mfma_f32_32x32x16_bf16 leaves
-// C[8g+4hh+r][c] in register 4g+r of lane (c, hh) -- four consecutive rows per
-// lane -- and the contraction index of the following product is permuted to
-// match on both operands.
+// Work split inside a 512-thread workgroup (8 waves): four "math" waves own the state and the output (W = 128: wave w columns
+// [32w, 32w+32), as four 32x32 fp32 MFMA accumulator tiles that never leave registers) and four "feed" waves see to the
+// blocks to come, compute the 64x64 score tile (one 32x32 quadrant per wave; masked, rounded to 16 bits and shared through
+// LDS) and store the outputs.  All products are arranged so that an accumulator tile can be fed back as an MFMA operand
+// without a shuffle: v_mfma_f32_32x32x16_bf16 leaves C[8g+4hh+r][c] in register 4g+r of lane (c, hh) -- four consecutive
+// rows per lane -- and the contraction index of the following product is permuted to match on both operands.
+#include <type_traits>
+
 #include "lasp_common.h"
 
 namespace lasp {
@@ -47,11 +46,9 @@ typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 typedef uint16_t elem16_t;  // raw bits of one bf16 or fp16 element
 
 constexpr int BLK = 64;     // tokens per block
-constexpr int LDT = 128;    // bytes per row of a feature-major tile (64 tokens), XOR-swizzled
-constexpr int LDSC = 144;   // bytes per row of the score tile (128 + 16)
 constexpr float LOG2E = kLog2e;
 constexpr float SKIP_LOG2 = kSkipLog2;  // decay weights below 2^-SKIP_LOG2 are treated as zero (see la_seg_state)
-enum Mode { M_ALIGNED = 0, M_RAGGED = 1, M_NARROW = 2 };
+enum Mode { M_ALIGNED = 0, M_RAGGED = 1, M_NARROW = 2, M_ADDING = 3 };
 // where a sweep takes the state entering its segment from (see ws_body)
 enum Source { SRC_SCANNED = 0, SRC_WALK = 1, SRC_COMBINE = 2 };
 
@@ -105,81 +102,36 @@ __device__ __forceinline__ gmem_ptr uniform_ptr(const char *p) {
 __device__ __forceinline__ void reads_first() { __builtin_amdgcn_sched_barrier(0); }
 __device__ __forceinline__ u32x4 lds16(const char *p) { return *reinterpret_cast<const u32x4 *>(p); }
 
+typedef short v4i16 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4i16 *lds_v4i16;
+// The transposing 8-byte read works in groups of 16 lanes: lane i of a group receives, as element j,
+// element (i % 4) of what lane (4 j + i / 4) of the group addressed.  With lane s of a group addressing
+// token T + s / 4, features f + 4 (s % 4) .. + 3, lane i ends up with feature f + i of tokens T .. T + 3.
+__device__ __forceinline__ u32x2 lds_tr8(const char *p) {
+  const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(p));
+  return __builtin_bit_cast(u32x2, r);
+}
+
 // element x (0..7) of a 16-byte group of 16-bit elements, widened to fp32
 template <class E>
 __device__ __forceinline__ float elem_f32(const u32x4 &q, int x) {
   const uint32_t w = (x >> 1) == 0 ? q.x : (x >> 1) == 1 ? q.y : (x >> 1) == 2 ? q.z : q.w;
   return E::widen(w, x & 1);
 }
-__device__ __forceinline__ uint32_t elem_bits(const u32x4 &q, int x) {
-  const uint32_t w = (x >> 1) == 0 ? q.x : (x >> 1) == 1 ? q.y : (x >> 1) == 2 ? q.z : q.w;
-  return (x & 1) ? (w >> 16) : (w & 0xffffu);
-}
-
-// Feature order inside LDS rows and registers.  A thread never holds eight consecutive
-// features: its 16 bytes are features {16G+4j .. +3} and {16G+8+4j .. +3} (G = 0..7,
-// j = 0..1), fetched as two 8-byte loads.  Token-major rows store these 16-byte units at
-// index 2G+j, so that lane half hh of an MFMA operand, reading unit 2k+hh, receives
-// features {16k+4hh .. +3, 16k+8+4hh .. +3}: exactly the rows 8g+4hh+r (g = 2u, 2u+1)
-// that the same lane holds of a 32x32 accumulator tile.  Accumulators can therefore be
-// multiplied against LDS rows with single 16-byte reads, and one set of X fragments
-// serves both the score product and the state product.
-struct LoaderRole {
-  int G, j;    // feature group and half handled by this thread
-  int rowq;    // X: row within a 16-row band; Y/Z: group of four rows
-};
-// X tile: W / 8 consecutive lanes fetch one row of W features
-template <int W>
-__device__ __forceinline__ LoaderRole x_role(int tid) {
-  LoaderRole r;
-  r.G = (tid >> 1) & (W / 16 - 1);
-  r.j = tid & 1;
-  r.rowq = tid / (W / 8);
-  return r;
-}
-// Y / Z tiles (also stored transposed): lane bits are dealt so that any 16 consecutive
-// lanes cover 8 feature units x 2 row groups -- 16 distinct 8-byte slots of the
-// feature-major tile, i.e. conflict-free ds_write_b64.  A tile of W features takes 2 W threads.
-template <int W>
-__device__ __forceinline__ LoaderRole yz_role(int tid) {
-  LoaderRole r;
-  r.j = tid & 1;
-  r.G = W == 128 ? ((tid >> 1) & 3) | (((tid >> 4) & 1) << 2) : (tid >> 1) & 3;
-  r.rowq = ((tid >> 3) & 1) | ((W == 128 ? tid >> 5 : tid >> 4) << 1);
-  return r;
-}
-
-// byte offset of 16-byte granule g16 (8 tokens) of feature row f in a feature-major tile.
-// The XOR term varies with f bits 0-2 (consecutive rows read by consecutive lanes) and
-// with bits 2,4,5 (the rows written by 16 consecutive loader lanes).
-__device__ __forceinline__ int tr_off(int f, int g16) {
-  return f * LDT + (((g16 ^ (f & 7) ^ ((f >> 4) & 3)) & 7) << 4);
+// a 16-byte group of 16-bit elements, each times w
+template <class E>
+__device__ __forceinline__ u32x4 scaled(const u32x4 &q, float w) {
+  u32x4 o;
+  o.x = E::pack(elem_f32<E>(q, 0) * w, elem_f32<E>(q, 1) * w);
+  o.y = E::pack(elem_f32<E>(q, 2) * w, elem_f32<E>(q, 3) * w);
+  o.z = E::pack(elem_f32<E>(q, 4) * w, elem_f32<E>(q, 5) * w);
+  o.w = E::pack(elem_f32<E>(q, 6) * w, elem_f32<E>(q, 7) * w);
+  return o;
 }
 
 // l^x for x >= 0
 __device__ __forceinline__ float decay(float s_log2e, float x) {
   return __builtin_amdgcn_exp2f(-s_log2e * x);
-}
-
-// Writes four rows (tokens 4*rowq .. +3) x the thread's eight features into a
-// feature-major tile: eight 8-byte stores, one per feature, each holding the four
-// tokens; `w[r]` scales token r before rounding (SCALE), else bits are moved as is.
-template <class E, bool SCALE>
-__device__ __forceinline__ void store_transposed(char *tile, const u32x4 (&rows)[4],
-                                                 const LoaderRole &role, const float (&w)[4]) {
-#pragma unroll
-  for (int x = 0; x < 8; ++x) {
-    const int f = 16 * role.G + 8 * (x >> 2) + 4 * role.j + (x & 3);
-    u32x2 out;
-    if (SCALE) {
-      out.x = E::pack(elem_f32<E>(rows[0], x) * w[0], elem_f32<E>(rows[1], x) * w[1]);
-      out.y = E::pack(elem_f32<E>(rows[2], x) * w[2], elem_f32<E>(rows[3], x) * w[3]);
-    } else {
-      out.x = elem_bits(rows[0], x) | (elem_bits(rows[1], x) << 16);
-      out.y = elem_bits(rows[2], x) | (elem_bits(rows[3], x) << 16);
-    }
-    *reinterpret_cast<u32x2 *>(tile + tr_off(f, role.rowq >> 1) + ((role.rowq & 1) << 3)) = out;
-  }
 }
 
 // A block of token rows as a buffer that ends with them: a lane that addresses past the end -- a row that a partial block
@@ -193,26 +145,6 @@ __device__ __forceinline__ rows_t rows_of(const void *p, int bytes) {
   const gmem_ptr u = uniform_ptr(reinterpret_cast<const char *>(p));
   return __builtin_amdgcn_make_buffer_rsrc((void *)(const char *)u, 0, bytes, 0x00020000);
 }
-// A thread's two 8-byte pieces of a row: 16 bytes apart, the second `hi_step` after the first
-__device__ __forceinline__ u32x4 load_row_pieces(rows_t rows, uint32_t lane_off, uint32_t hi_step) {
-  const u32x2 lo = __builtin_amdgcn_raw_buffer_load_b64(rows, (int)lane_off, 0, 0);
-  const u32x2 hi = __builtin_amdgcn_raw_buffer_load_b64(rows, (int)(lane_off + hi_step), 0, 0);
-  u32x4 r;
-  r.x = lo.x;
-  r.y = lo.y;
-  r.z = hi.x;
-  r.w = hi.y;
-  return r;
-}
-// where the thread's first piece lies in a block, `row` rows down (rows of `units` 8-byte units, of which `width` are read),
-// and how far its second piece is from it
-__device__ __forceinline__ uint32_t lane_offset(const LoaderRole &role, int row, int units, int width) {
-  return 4 * role.G + role.j < width ? (uint32_t)((row * units + 4 * role.G + role.j) * 8) : kOutside;
-}
-__device__ __forceinline__ uint32_t second_piece(const LoaderRole &role, int width) {
-  return 4 * role.G + 2 + role.j < width ? 16u : kOutside;
-}
-
 struct SegWork {
   int bh, seg;
   int64_t tok0;  // first token of the segment
@@ -234,17 +166,16 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
 }
 
 // ------------------------------------------------------------------------------
-// Every sweep kernel below is an instance of ws_body<E, REV, TRANS, SRC, MODE>.
-//
-// W.  The width the arithmetic is laid out for: 128, or 64 where neither d nor e is larger.
+// Every sweep kernel below is an instance of sweep_body (W = 128) or ws_body (W = 64, where neither d nor e is larger),
+// <E, REV, TRANS, SRC, MODE>.
 //
 // MODE.  M_RAGGED: the chunk length is not a multiple of 64, so the last block of the last segment is
 // partial (rows past its end read as zeros, stores are masked, and the decay factors of that one block use
 // its true length).  M_NARROW: in addition X and Y rows hold `fa` features, Z and Out rows `fb`
-// (multiples of 8, at most W), read zero-extended to W and written back at their own width; the upper
-// half of the feature steps and state tiles, and waves whose columns lie in the zero extension, are skipped
-// when they would only see zeros.  The slices of a wide head (d > 128) run in this mode too, their rows being g.dt
-// features apart.  M_ALIGNED carries none of that bookkeeping; fa and fb are read in M_NARROW only.
+// (multiples of 8, at most W), read zero-extended to W and written back at their own width; math
+// waves of the 128-wide form whose columns all lie in the zero extension only take part in the barriers.  The slices of a wide
+// head (d > 128) run in this mode too, their rows being g.dt features apart; M_ADDING: slices after the first, which add their
+// O (dV) to what the slices before left there.  M_ALIGNED carries none of that bookkeeping; fa and fb are read from M_NARROW on.
 //
 // SRC says where the state entering the segment comes from.
 // SRC_SCANNED: `states` holds it, left there by the decayed scan over the segments' own states.
@@ -260,16 +191,15 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
 // In the last two the workgroup of the segment visited last writes the state it ends with to
 // `carry_out` (non-transposed roles only).
 // ------------------------------------------------------------------------------
-// The sweep, with the work of a block split between two groups of waves.  A workgroup whose waves all run
-// fill -> products -> store one after the other spends most of a block waiting for its own LDS round trips
-// (measured on such a form of this kernel: 5806 against 3700 clock ticks per block alone on a CU); here 512
-// threads form one workgroup per CU:
-//   waves 0-3 ("feed"): global loads, the LDS tiles of the NEXT block (transposes and decay scaling
-//     included), the masked score tile of the current block, the coalesced output stores;
-//   waves 4-7 ("math"): own the state and the output accumulators (wave 4 + w: columns [32w, 32w + 32)):
-//     state term, intra-block term, state update, output staging.
-// The tiles are double-buffered (two sets of X, Y token-major and Y^T, Z^T feature-major, 144 384 B
-// with the score tile), and a block takes two barriers:
+// The 64-wide sweep.  512 threads, two workgroups per CU, the work of a block split between two groups of waves (a workgroup
+// whose waves all run fill -> products -> store one after the other spends most of a block waiting for its own LDS round trips):
+//   waves 0-3 ("feed"): global loads, the LDS tiles of the NEXT block (waves 0, 1 fetch Y, waves 2, 3 Z, which they also write
+//     scaled by the state update's decay), the masked score tile of the current block, the coalesced output stores;
+//   waves 4-7 ("math"): state term, intra-block term, state update, output staging.  Wave 4 + w owns one 32 x 32 tile of the
+//     output -- columns [32 (w & 1), + 32) of tokens [32 (w >> 1), + 32) -- and the 64 x 32 state columns it needs (both token
+//     halves keep those: 8 products per block and wave, against a reduction through LDS).
+// All tiles are token-major; what contracts over tokens is read transposed.  They are double-buffered (two sets of X, Y, Z and scaled
+// Z, 73 728 B with the score tile), and a block takes two barriers:
 //     feed: store O(t-1), score(t),   | math: state term(t), state update(t)
 //           fill Y, Z(t+1),           |
 //           issue loads Y, Z(t+2)     |
@@ -278,35 +208,26 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
 //           issue loads X(t+2)        |       (no longer read)
 //   ---- barrier ----
 // O(t-1) waits in the X tile of the set that the fill of X(t+1) overwrites after the first barrier; the set's other tiles
-// were last read before the second barrier of block t-1.
-// What bounds a block: with long chunks HBM; otherwise the LDS, which moves some 330 KB per block (every math wave reads
-// all of X and Y^T), and the round trips that nothing covers.  Against a form that updated the state after the first barrier,
-// filled all tiles there and read LDS operand by operand (forward + backward): b*h = 16, n = 65536: 773 us against 815;
-// b*h = 36, n = 5003: 170 against 184; d = e = 64, b*h = 64, n = 4096: 107 against 112; forward with a state, b*h = 16,
-// n = 2000: 25.3 against 26.2.  Half of that comes from loads and stores without branches (see rows_of): in the ragged
-// form each of the 24 loads of a block had been one of its own, and every fill waited for everything in flight.
-// Both groups run their own loop; each executes exactly 1 + 2 * nblk barriers.
-//
-// W = 64 keeps that split with a quarter of the state and half of every tile: 78 848 B of LDS and at most 128
-// registers, so two workgroups share a CU and fill each other's waits.  A feed wave then fetches either Y (waves
-// 0, 1) or Z (waves 2, 3), and a math wave owns one 32 x 32 tile of the output -- columns [32 (w & 1), + 32) of tokens
-// [32 (w >> 1), + 32) -- and the 64 x 32 state columns it needs (both token halves keep those: 8 products per block and
-// wave, against a reduction through LDS).  Rows of 64 features ran on the W = 128 kernels before, where two of the four
-// math waves own columns that do not exist and one workgroup holds the CU (forward + backward, b*h = 64, n = 4096: 210 us
-// against 118; b*h = 16, n = 65536: 692 against 390).
+// were last read before the second barrier of block t-1.  Both groups run their own loop; each executes exactly
+// 1 + 2 * nblk barriers.  At most 128 registers, so that two workgroups share a CU and fill each other's waits; bound by HBM on
+// long chunks.  In us, with tiles transposed in registers on the way to LDS and as it is: backward sweep, b*h = 24, n = 2048:
+// 14.0 and 12.8, b*h = 16, n = 16384: 54.2 and 51.8, b*h = 64, n = 4096: 54.8 and 52.5; one launch for b*h = 96, n = 512:
+// 17.1 and 16.8 (forward 10.2 and 9.9).  The 128-wide form's pipeline, whose math waves scale Z themselves, twice here, took 56 to 59 for
+// b*h = 64 where this one takes 52.5.
 constexpr int WS_THREADS = 512;
-template <int W>
 struct WsLds {
-  static constexpr int LDN = 2 * W + 16;  // bytes per row of a token-major tile (rows shift 4 banks)
-  static constexpr int XN = 0, YN = BLK * LDN, YT = 2 * BLK * LDN, ZT = YT + W * LDT;
-  static constexpr int SET = ZT + W * LDT;         // one block's tiles
-  static constexpr int SC = 2 * SET;               // the score tile
-  static constexpr int BYTES = SC + BLK * LDSC;    // W = 128: 144 384 B, one workgroup per CU; 64: 78 848 B, two
+  static constexpr int W = 64, ROW = 2 * W, TILE = BLK * ROW;
+  static constexpr int X = 0, Y = TILE, Z = 2 * TILE, ZS = 3 * TILE, SET = 4 * TILE;  // one block's tiles; ZS: Z scaled
+  static constexpr int SC = 2 * SET, SC_ROW = 2 * BLK;  // the score tile
+  static constexpr int BYTES = SC + BLK * SC_ROW;       // 73 728 B: two workgroups per CU
+  // Unit u (16 bytes) of row r lies at u ^ swizzle(r): the rows that a phase of a 16-byte read takes one unit of, and the four rows
+  // x 64 bytes that half a wave reads transposed, fall on disjoint banks (two rows to a set of banks).
+  static __device__ __forceinline__ int swizzle(int row) { return ((row & 2) << 1) | ((row >> 2) & 3); }
 };
 // workgroups of a sweep that share a CU, and with them the waves per SIMD the registers must leave room for
 constexpr int ws_waves_per_simd(int w) { return w == 64 ? 4 : 1; }
 
-template <class E, bool REV, bool TRANS, int SRC, int MODE, int W>
+template <class E, bool REV, bool TRANS, int SRC, int MODE>
 __device__ __forceinline__ void
 ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z,
         const float *__restrict__ S, const float *__restrict__ states, elem16_t *__restrict__ Out, const Geom &g,
@@ -314,15 +235,14 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
         float *__restrict__ carry_out = nullptr) {
   constexpr bool RAGGED = MODE != M_ALIGNED, NARROW = MODE == M_NARROW;
   constexpr bool LEAVES_STATE = SRC != SRC_SCANNED;  // the sweep's final state is the chunk's outgoing one
-  using L = WsLds<W>;
-  constexpr int NT = W / 32;           // 32-row tiles of a wave's state columns
-  constexpr int NI = W == 128 ? 2 : 1;  // 32-token halves of the output a math wave owns
+  using L = WsLds;
+  constexpr int W = L::W;
+  constexpr int NT = W / 32;  // 32-row tiles of a wave's state columns
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int w = w8 & 3;                     // feed: score quadrant
-  const int wcol = W == 128 ? w : w & 1;    // math: column block
-  const int ih = W == 128 ? 0 : w >> 1;     // math: (first) token half
+  const int w = w8 & 3;                   // feed: score quadrant
+  const int wcol = w & 1, ih = w >> 1;    // math: column block and token half
   const int c = lane & 31, hh = lane >> 5;
 
   const SegWork sw = seg_work(g, item);
@@ -367,50 +287,39 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   if (w8 < 4) {
     // ================================ feed waves ================================
     const int ftid = tid;  // 0..255
-    constexpr int XI = W / 32;           // X rows per thread
-    constexpr int XROWS = 2048 / W;      // X rows that the feed threads fetch at a time
-    constexpr bool SPLIT = W == 64;      // a thread fetches Y or Z, not both
-    const bool zfeed = SPLIT && w8 >= 2;
-    const LoaderRole xr = x_role<W>(ftid), yr = yz_role<W>(SPLIT ? ftid & 127 : ftid);
-    const int chunk = ftid & (W / 8 - 1), rowq = ftid / (W / 8);
-    const int xu = xp / 4, zu = zp / 4;  // 8-byte units from row to row
-    const int qI = w >> 1, qJ = w & 1;
-    const bool q_active = REV ? !(qI == 1 && qJ == 0) : !(qI == 0 && qJ == 1);
-    const int yu = zfeed ? zu : xu;      // SPLIT: of the tile that this wave fetches through ny
-    const int xw = NARROW ? fa / 4 : W / 4, zw = NARROW ? fb / 4 : W / 4, yw = zfeed ? zw : xw;  // 8-byte units read of a row
-    uint32_t x_off[XI], y_off[4], z_off[4];
+    const bool zfeed = w8 >= 2;  // a wave fetches Y or Z, not both
+    // 16 bytes per thread and row: rows xr and xr + 32 of X, yr + 16 r of Y or Z
+    const int unit = ftid & 7, xr = ftid >> 3, yr = (ftid & 127) >> 3;
+    const int yp = zfeed ? zp : xp, yw = zfeed ? fb : fa;
+    uint32_t x_off[2], y_off[4], o_off[2];
 #pragma unroll
-    for (int it = 0; it < XI; ++it) x_off[it] = lane_offset(xr, xr.rowq + XROWS * it, xu, xw);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      y_off[r] = lane_offset(yr, 4 * yr.rowq + r, yu, yw);
-      z_off[r] = lane_offset(yr, 4 * yr.rowq + r, zu, zw);
+    for (int i = 0; i < 2; ++i) {
+      x_off[i] = !NARROW || unit * 8 < fa ? (uint32_t)((xr + 32 * i) * xp * 2 + unit * 16) : kOutside;
+      o_off[i] = !NARROW || unit * 8 < fb ? (uint32_t)((xr + 32 * i) * zp * 2 + unit * 16) : kOutside;
     }
-    const uint32_t x_hi = NARROW ? second_piece(xr, xw) : 16, y_hi = NARROW ? second_piece(yr, yw) : 16,
-                   z_hi = NARROW ? second_piece(yr, zw) : 16;
-    const elem16_t *Xg = X + row0 * xp, *Yg = zfeed ? Z + row0 * zp : Y + row0 * xp, *Zg = Z + row0 * zp;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      y_off[r] = !NARROW || unit * 8 < yw ? (uint32_t)((yr + 16 * r) * yp * 2 + unit * 16) : kOutside;
+    const int x_to = xr * L::ROW + ((unit ^ L::swizzle(xr)) << 4), y_to = yr * L::ROW + ((unit ^ L::swizzle(yr)) << 4);
+    const elem16_t *Xg = X + row0 * xp, *Yg = zfeed ? Z + row0 * zp : Y + row0 * xp;
     elem16_t *Og = Out + row0 * zp;
 
-    // the block in flight, two 8-byte pieces per row (see LoaderRole); SPLIT: ny holds Y or Z
-    u32x4 nx[XI], ny[4], nz[4];
+    u32x4 nx[2], ny[4];  // the block in flight; ny: Y or Z
     // block k of the run as a buffer; none of its rows where it is not `wanted`
-    auto rows = [&](const elem16_t *base, int k, int units, bool wanted) __attribute__((always_inline)) {
+    auto rows = [&](const elem16_t *base, int k, int pitch, bool wanted) __attribute__((always_inline)) {
       const int blk = first_blk + k * step;
-      return rows_of(base + (int64_t)blk * BLK * units * 4, wanted ? len_of(blk) * units * 8 : 0);
+      return rows_of(base + (int64_t)blk * BLK * pitch, wanted ? len_of(blk) * pitch * 2 : 0);
     };
     // Always the same number of loads (see rows_of); walk blocks (k < runup) need no X tile
     auto issue_x = [&](int k) __attribute__((always_inline)) {
-      const rows_t x = rows(Xg, k, xu, k < run && (SRC != SRC_WALK || k >= runup));
+      const rows_t x = rows(Xg, k, xp, k < run && (SRC != SRC_WALK || k >= runup));
 #pragma unroll
-      for (int it = 0; it < XI; ++it) nx[it] = load_row_pieces(x, x_off[it], x_hi);
+      for (int i = 0; i < 2; ++i) nx[i] = __builtin_amdgcn_raw_buffer_load_b128(x, (int)x_off[i], 0, 0);
     };
     auto issue_yz = [&](int k) __attribute__((always_inline)) {
-      const rows_t y = rows(Yg, k, yu, k < run), z = rows(Zg, k, zu, k < run);
+      const rows_t y = rows(Yg, k, yp, k < run);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        ny[r] = load_row_pieces(y, y_off[r], y_hi);
-        if (!SPLIT) nz[r] = load_row_pieces(z, z_off[r], z_hi);
-      }
+      for (int r = 0; r < 4; ++r) ny[r] = __builtin_amdgcn_raw_buffer_load_b128(y, (int)y_off[r], 0, 0);
     };
     // The slope comes as a lane's load in front of the first block's: as a scalar one, whose waits know no order, it would
     // have to arrive before the first of these loads could leave.
@@ -423,86 +332,75 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     const float sl = slope * LOG2E;
     float kdec[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int b = 4 * yr.rowq + r;
-      kdec[r] = decay(sl, REV ? (float)b : (float)(BLK - b));
-    }
-    // writes the block held in nx / ny / nz into a tile set: token-major X ...
+    for (int r = 0; r < 4; ++r) kdec[r] = decay(sl, REV ? (float)(yr + 16 * r) : (float)(BLK - yr - 16 * r));
+    // writes the block held in nx and ny into a tile set: X ...
     auto fill_x = [&](char *set, int k) __attribute__((always_inline)) {
       if (SRC != SRC_WALK || k >= runup) {  // a walk block is only multiplied into the state
 #pragma unroll
-        for (int it = 0; it < XI; ++it)
-          *reinterpret_cast<u32x4 *>(set + L::XN + (xr.rowq + XROWS * it) * L::LDN + (2 * xr.G + xr.j) * 16) = nx[it];
+        for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4 *>(set + L::X + x_to + 32 * i * L::ROW) = nx[i];
       }
     };
-    // ... token-major Y, and feature-major Y (scaled by the key decay) and Z
+    // ... and Y, or Z as it is and scaled by the key decay
     auto fill_yz = [&](char *set, int k) __attribute__((always_inline)) {
-      if ((SRC != SRC_WALK || k >= runup) && !zfeed) {
+      char *to = set + (zfeed ? L::Z : L::Y) + y_to;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          *reinterpret_cast<u32x4 *>(set + L::YN + (4 * yr.rowq + r) * L::LDN + (2 * yr.G + yr.j) * 16) = ny[r];
-      }
-      if (zfeed) {
-        store_transposed<E, false>(set + L::ZT, ny, yr, kdec);
-        return;
-      }
+      for (int r = 0; r < 4; ++r) *reinterpret_cast<u32x4 *>(to + 16 * r * L::ROW) = ny[r];
+      if (!zfeed) return;
       const int len = len_of(first_blk + k * step);
+      float kd[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) kd[r] = kdec[r];
       if (LEAVES_STATE && RAGGED && !REV && len != BLK) {
         // the chunk's partial last block, going forwards: its tokens sit `len - b` before the chunk end, which
         // matters here because the state it leaves is the outgoing one
-        float kd[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) kd[r] = decay(sl, (float)max(len - (4 * yr.rowq + r), 0));
-        store_transposed<E, true>(set + L::YT, ny, yr, kd);
-      } else {
-        store_transposed<E, true>(set + L::YT, ny, yr, kdec);
+        for (int r = 0; r < 4; ++r) kd[r] = decay(sl, (float)max(len - (yr + 16 * r), 0));
       }
-      if (!SPLIT) store_transposed<E, false>(set + L::ZT, nz, yr, kdec);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) *reinterpret_cast<u32x4 *>(set + L::ZS + y_to + 16 * r * L::ROW) = scaled<E>(ny[r], kd[r]);
     };
-    // the output tile staged in `set`'s X region -> global rows of block k of the run
-    uint32_t o_off[XI];
-#pragma unroll
-    for (int r4 = 0; r4 < XI; ++r4)
-      o_off[r4] = !NARROW || chunk < fb / 8 ? (uint32_t)(((rowq + XROWS * r4) * zu * 8) + chunk * 16) : kOutside;
+    // the output tile staged in `set`'s X tile -> global rows of block k of the run
     auto store_out = [&](const char *set, int k, bool wanted) __attribute__((always_inline)) {
-      const rows_t out = rows(Og, k, zu, wanted);
+      const rows_t out = rows(Og, k, zp, wanted);
 #pragma unroll
-      for (int r4 = 0; r4 < XI; ++r4)
-        __builtin_amdgcn_raw_buffer_store_b128(
-            *reinterpret_cast<const u32x4 *>(set + L::XN + (rowq + XROWS * r4) * L::LDN + chunk * 16), out, (int)o_off[r4], 0,
-            2 /* non-temporal */);
+      for (int i = 0; i < 2; ++i)
+        __builtin_amdgcn_raw_buffer_store_b128(lds16(set + L::X + x_to + 32 * i * L::ROW), out, (int)o_off[i], 0,
+                                               2 /* non-temporal */);
     };
     // this wave's quadrant of the transposed score tile: sc[4g+r] = y_b . x_a, b = 32qJ+8g+4hh+r, a = 32qI+c
+    const int qI = w >> 1, qJ = w & 1;
+    const bool q_active = REV ? !(qI == 1 && qJ == 0) : !(qI == 0 && qJ == 1);
+    float mask[16];  // decay between the tokens of a score; negative: masked
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int a = 32 * qI + c, b = 32 * qJ + 8 * (r >> 2) + 4 * hh + (r & 3), dist = REV ? b - a : a - b;
+      mask[r] = dist >= 0 ? decay(sl, (float)dist) : -1.f;
+    }
+    const int q_at = c * L::ROW + ((hh ^ L::swizzle(c)) << 4);
+    const int sc_at = (32 * qI + c) * L::SC_ROW + ((4 * qJ ^ ((c >> 1) & 7)) << 4) + 8 * hh;
     auto score = [&](const char *set) __attribute__((always_inline)) {
       if (!q_active) return;
       floatx16 sc;
 #pragma unroll
       for (int r = 0; r < 16; ++r) sc[r] = 0.f;
-      const char *xa = set + L::XN + (32 * qI + c) * L::LDN + hh * 16;
-      const char *ya = set + L::YN + (32 * qJ + c) * L::LDN + hh * 16;
       u32x4 yf[W / 16], xf[W / 16];
 #pragma unroll
       for (int ks = 0; ks < W / 16; ++ks) {
-        yf[ks] = lds16(ya + ks * 32);
-        xf[ks] = lds16(xa + ks * 32);
+        yf[ks] = lds16(set + L::Y + 32 * qJ * L::ROW + (q_at ^ (ks << 5)));
+        xf[ks] = lds16(set + L::X + 32 * qI * L::ROW + (q_at ^ (ks << 5)));
       }
       reads_first();
 #pragma unroll
       for (int ks = 0; ks < W / 16; ++ks) sc = E::mfma(yf[ks], xf[ks], sc);
-      const int a = 32 * qI + c;
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
         float m[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int b = 32 * qJ + 8 * gq + 4 * hh + r;
-          const int dist = REV ? b - a : a - b;
-          m[r] = dist >= 0 ? sc[4 * gq + r] * decay(sl, (float)dist) : 0.f;
-        }
+        for (int r = 0; r < 4; ++r) m[r] = mask[4 * gq + r] >= 0.f ? sc[4 * gq + r] * mask[4 * gq + r] : 0.f;
         u32x2 o;
         o.x = E::pack(m[0], m[1]);
         o.y = E::pack(m[2], m[3]);
-        *reinterpret_cast<u32x2 *>(smem + L::SC + a * LDSC + (32 * qJ + 8 * gq + 4 * hh) * 2) = o;
+        *reinterpret_cast<u32x2 *>(smem + L::SC + (sc_at ^ (gq << 4))) = o;
       }
     };
 
@@ -522,13 +420,13 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     }
     for (; k < run; ++k) {
       char *cur = smem + (k & 1) * L::SET, *nxt = smem + ((k + 1) & 1) * L::SET;
-      // per block: 4 stores, 16 loads of Y and Z, 8 of X, in this order, so the waits of the fills leave what was issued
+      // per block: 2 stores, 4 loads of Y or Z, 2 of X, in this order, so the waits of the fills leave what was issued
       // after their own loads in flight
       store_out(nxt, k - 1, k > runup);
       score(cur);
       if (k + 1 < run) fill_yz(nxt, k + 1);
       issue_yz(k + 2);
-      __syncthreads();  // first barrier of a sweep block: score tile complete; `cur` and the output staged in `nxt` no longer read
+      __syncthreads();  // first barrier of a sweep block: score tile complete; X of `cur` and the output staged in `nxt` no longer read
       if (k + 1 < run) fill_x(nxt, k + 1);
       issue_x(k + 2);
       __syncthreads();  // second barrier: next block visible; output of this block staged
@@ -538,42 +436,33 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   }
 
   // ================================== math waves ==================================
+  // (rows and columns of the state: see sweep_body)
+  const int col = 32 * wcol + 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3);
   const float sl = S[head] * LOG2E;
   const float blockdec = decay(sl, (float)BLK);
-  float qdec[NI];
-#pragma unroll
-  for (int I = 0; I < NI; ++I) {
-    const int a = 32 * (ih + I) + c;
-    qdec[I] = decay(sl, REV ? (float)(BLK - a) : (float)a);
-  }
-  // state entering the segment: st[T][4g+r] = St[32T+8g+4hh+r][32 wcol + c]
+  const int a_own = 32 * ih + c;  // the token whose output the lane holds
+  const float qdec = decay(sl, REV ? (float)(BLK - a_own) : (float)a_own);
   floatx16 st[NT];
 #pragma unroll
   for (int T = 0; T < NT; ++T)
 #pragma unroll
     for (int r = 0; r < 16; ++r) st[T][r] = 0.f;
-  // M_NARROW: a wave whose 32 columns all lie past the width of Z has nothing to compute (it still takes part in
-  // every barrier); the upper half of the features is skipped as a whole when the rows are no wider
-  const bool wave_active = !NARROW || W == 64 || 32 * wcol < fb;  // (at W = 64 the skipping costs registers that two workgroups per CU do not have)
-  constexpr int PARTS = NARROW ? 2 : 1;  // M_NARROW takes the lower and the upper features one after the other
-  const bool upper_half = !NARROW || W == 64 || fa > W / 2;
-  // st <- f * st + M (`fresh`: st <- M, which leaves the loads in flight until a product needs them: the feed waves go on
-  // with the first block meanwhile), M being the W x W fp32 tile whose element (row, col) is src[row * ld + col], or for a
-  // transposed role src[col * ld + row]; `bounded`: src holds only fa x fb (transposed: fb x fa) elements
+  // st <- f * st + M (`fresh`: st <- M, which leaves the loads in flight until a product needs them), M being the W x W fp32
+  // tile whose element (row, col) is src[row * ld + col], or for a transposed role src[col * ld + row]; `bounded`: src holds
+  // only fa x fb (transposed: fb x fa) elements
   auto add_state_ld = [&](const float *src, int ld, float f, bool bounded, bool fresh) __attribute__((always_inline)) {
     typedef const __attribute__((address_space(1))) float *gmem_f32;
-    const uint32_t lane_off =
-        (uint32_t)(TRANS ? (32 * wcol + c) * ld + 4 * hh : 4 * hh * ld + 32 * wcol + c) * (uint32_t)sizeof(float);
-    const bool col_ok = !bounded || 32 * wcol + c < fb;
+    const uint32_t lane_off = (uint32_t)(TRANS ? col * ld + 8 * hh : 8 * hh * ld + col) * (uint32_t)sizeof(float);
+    const bool col_ok = !bounded || col < fb;
 #pragma unroll
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
-        const int band = 32 * T + 8 * gq;
+        const int band = 32 * T + 16 * (gq >> 1) + 4 * (gq & 1);
         const gmem_ptr bp = uniform_ptr(reinterpret_cast<const char *>(src + (TRANS ? band : (int64_t)band * ld)));
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const bool ok = col_ok && (!bounded || band + 4 * hh + r < fa);
+          const bool ok = col_ok && (!bounded || band + 8 * hh + r < fa);
           const float own =
               ok ? *reinterpret_cast<gmem_f32>(bp + lane_off + (uint32_t)(TRANS ? r : r * ld) * sizeof(float)) : 0.f;
           st[T][4 * gq + r] = fresh ? own : fmaf(f, st[T][4 * gq + r], own);
@@ -637,58 +526,46 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       }
     }
   }
-  // St <- l^64 St + (scaled Y)^T Z from the feature-major tiles of `set`
-  auto update_state = [&](const char *set, const u32x4 (&zf)[4], float bd) __attribute__((always_inline)) {
+  const int s16 = lane & 15, q4 = s16 & 3, ch = (lane >> 4) & 1;
+  const int t_row = 8 * hh + (s16 >> 2), t_swz = L::swizzle(t_row);
+  const int y_at = t_row * L::ROW + (((2 * ch + (q4 & 1)) ^ t_swz) << 4) + ((q4 >> 1) << 3);
+  const int z_at = t_row * L::ROW + (((4 * wcol + 2 * (q4 & 1) + ch) ^ t_swz) << 4) + ((q4 >> 1) << 3);
+  const int x_at = a_own * L::ROW + ((hh ^ L::swizzle(c)) << 4);
+  const int o_at = a_own * L::ROW + (((4 * wcol + 2 * hh) ^ L::swizzle(c)) << 4);
+  const int sc_at = a_own * L::SC_ROW + ((hh ^ ((c >> 1) & 7)) << 4);
+  // operand over tokens 16 u + 8 hh .. + 7 of a tile
+  auto tokens = [&](const char *tile, int at, int u) __attribute__((always_inline)) {
+    const u32x2 lo = lds_tr8(tile + at + 16 * u * L::ROW), hi = lds_tr8(tile + (at ^ 16) + (16 * u + 4) * L::ROW);
+    u32x4 r;
+    r.x = lo.x;
+    r.y = lo.y;
+    r.z = hi.x;
+    r.w = hi.y;
+    return r;
+  };
+  // St <- l^64 St + Y^T (scaled Z)
+  auto update_state = [&](const char *set, float bd) __attribute__((always_inline)) {
+    u32x4 yf[4][NT], zs[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      zs[u] = tokens(set + L::ZS, z_at, u);
+#pragma unroll
+      for (int T = 0; T < NT; ++T) yf[u][T] = tokens(set + L::Y, y_at ^ (T << 6), u);
+    }
 #pragma unroll
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int r = 0; r < 16; ++r) st[T][r] *= bd;
+    reads_first();
 #pragma unroll
-    for (int part = 0; part < PARTS; ++part) {
-      if (part > 0 && !upper_half) break;  // state rows past the width of Y stay zero
-      constexpr int TP = NT / PARTS;
-      u32x4 yf[4][TP];
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int T = 0; T < TP; ++T) yf[u][T] = lds16(set + L::YT + tr_off(32 * (part * TP + T) + c, 2 * u + hh));
-      reads_first();
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int T = 0; T < TP; ++T) st[part * TP + T] = E::mfma(yf[u][T], zf[u], st[part * TP + T]);
-    }
+      for (int T = 0; T < NT; ++T) st[T] = E::mfma(yf[u][T], zs[u], st[T]);
   };
-  // Slices of a wide head after the first add to what the slices before them left in Out (its rows are whole
-  // features of v, so only the non-transposed roles).  A block's old output is fetched while the block before it is
-  // computed; the lane holds the columns that its accumulators hold.
-  constexpr bool MAY_ADD = NARROW && !TRANS && W == 128;
-  const bool adds = MAY_ADD && g.add != 0;
-  u32x2 old[NI][4];
-  auto fetch_old = [&](int blk) __attribute__((always_inline)) {
-    const int len = len_of(blk);
-    const elem16_t *rows = Out + (row0 + (int64_t)blk * BLK) * zp + 32 * wcol + 4 * hh;
-    const u32x2 zero = {0u, 0u};
-#pragma unroll
-    for (int I = 0; I < NI; ++I)
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        const int row = 32 * (ih + I) + c;
-        const bool ok = row < len && 32 * wcol + 8 * gq + 4 * hh < fb;
-        old[I][gq] = ok ? *reinterpret_cast<const u32x2 *>(rows + (int64_t)row * zp + 8 * gq) : zero;
-      }
-  };
-  if (adds) fetch_old(blk0);
   __syncthreads();  // barrier 0
   for (int k = 0; k < runup; ++k) {  // walk
-    const char *set = smem + (k & 1) * L::SET;
-    if (wave_active) {
-      const int len = len_of(first_blk + k * step);
-      u32x4 zf[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) zf[u] = lds16(set + L::ZT + tr_off(32 * wcol + c, 2 * u + hh));
-      update_state(set, zf, RAGGED && len != BLK ? decay(sl, (float)len) : blockdec);
-    }
+    const int len = len_of(first_blk + k * step);
+    update_state(smem + (k & 1) * L::SET, RAGGED && len != BLK ? decay(sl, (float)len) : blockdec);
     __syncthreads();  // walk barrier k
   }
   for (int it = 0; it < nblk; ++it) {
@@ -697,105 +574,66 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
     // state where the sweep leaves it); going backwards it comes first and the entering state sits `len` (not 64)
     // tokens ahead.
     const int len = len_of(blk0 + it * step);
-    float qd[NI];
-#pragma unroll
-    for (int I = 0; I < NI; ++I) qd[I] = qdec[I];
-    float bd = blockdec;
+    float qd = qdec, bd = blockdec;
     if (RAGGED && REV && len != BLK) {
-#pragma unroll
-      for (int I = 0; I < NI; ++I) qd[I] = decay(sl, (float)max(len - 32 * (ih + I) - c, 0));
+      qd = decay(sl, (float)max(len - a_own, 0));
       bd = decay(sl, (float)len);
     }
     if (LEAVES_STATE && RAGGED && !REV && len != BLK) bd = decay(sl, (float)len);
-    // state term, transposed: acc[I][4g+r] = sum_f St[f][32 wcol + 8g+4hh+r] x_a[f], a = 32 (ih + I) + c
-    floatx16 acc[NI];
+    // state term, transposed: acc[4g+r] = sum_f St[f][column] x_a[f], a = a_own
+    floatx16 acc;
 #pragma unroll
-    for (int I = 0; I < NI; ++I)
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    // all X fragments are requested before the first product
+    u32x4 xf[W / 16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[I][r] = 0.f;
-    if (wave_active) {
-      // all X fragments (of a part) are requested before the first product (these waves have the registers for it)
-      const char *x0 = cur + L::XN + (32 * ih + c) * L::LDN + hh * 16;
+    for (int ks = 0; ks < W / 16; ++ks) xf[ks] = lds16(cur + L::X + (x_at ^ (ks << 5)));
+    reads_first();
 #pragma unroll
-      for (int part = 0; part < PARTS; ++part) {
-        if (part > 0 && !upper_half) break;
-        constexpr int KS = W / 16 / PARTS;
-        u32x4 xf[KS][NI];
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-          for (int I = 0; I < NI; ++I) xf[ks][I] = lds16(x0 + 32 * I * L::LDN + (part * KS + ks) * 32);
-        reads_first();
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const int T = (part * KS + ks) >> 1, u = ks & 1;
-          u32x4 a;
-          a.x = E::pack(st[T][8 * u + 0], st[T][8 * u + 1]);
-          a.y = E::pack(st[T][8 * u + 2], st[T][8 * u + 3]);
-          a.z = E::pack(st[T][8 * u + 4], st[T][8 * u + 5]);
-          a.w = E::pack(st[T][8 * u + 6], st[T][8 * u + 7]);
-#pragma unroll
-          for (int I = 0; I < NI; ++I) acc[I] = E::mfma(a, xf[ks][I], acc[I]);
-        }
-      }
+    for (int ks = 0; ks < W / 16; ++ks) {
+      const int T = ks >> 1, u = ks & 1;
+      u32x4 a;
+      a.x = E::pack(st[T][8 * u + 0], st[T][8 * u + 1]);
+      a.y = E::pack(st[T][8 * u + 2], st[T][8 * u + 3]);
+      a.z = E::pack(st[T][8 * u + 4], st[T][8 * u + 5]);
+      a.w = E::pack(st[T][8 * u + 6], st[T][8 * u + 7]);
+      acc = E::mfma(a, xf[ks], acc);
     }
 #pragma unroll
-    for (int I = 0; I < NI; ++I)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[I][r] *= qd[I];
-    if (adds) {
-#pragma unroll
-      for (int I = 0; I < NI; ++I)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[I][r] += E::widen((r & 2) ? old[I][r >> 2].y : old[I][r >> 2].x, r & 1);
-      if (it + 1 < nblk) fetch_old(blk0 + (it + 1) * step);
-    }
+    for (int r = 0; r < 16; ++r) acc[r] *= qd;
+    update_state(cur, bd);
     u32x4 zf[4];
-    if (wave_active) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) zf[u] = lds16(cur + L::ZT + tr_off(32 * wcol + c, 2 * u + hh));
-      update_state(cur, zf, bd);
-    }
+    for (int u = 0; u < 4; ++u) zf[u] = tokens(cur + L::Z, z_at, u);
     __syncthreads();  // barrier 2 it + 1: score tile complete
-    if (wave_active) {
-      // intra-block term: acc[I] += Z^T[32 wcol.., tokens] * score[a][tokens]
-      u32x4 sf[4][NI];
+    // intra-block term: acc += Z^T[32 wcol.., tokens] * score[a][tokens]
+    u32x4 sf[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 4; ++u) sf[u] = lds16(smem + L::SC + (sc_at ^ (u << 5)));
+    reads_first();
 #pragma unroll
-        for (int I = 0; I < NI; ++I) sf[u][I] = lds16(smem + L::SC + (32 * (ih + I) + c) * LDSC + (16 * u + 8 * hh) * 2);
-      reads_first();
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int I = 0; I < NI; ++I) {
-          const bool needed = REV ? (ih + I == 0 || u >= 2) : (ih + I == 1 || u < 2);
-          if (needed) acc[I] = E::mfma(zf[u], sf[u][I], acc[I]);
-        }
+    for (int u = 0; u < 4; ++u) {
+      const bool needed = REV ? (ih == 0 || u >= 2) : (ih == 1 || u < 2);
+      if (needed) acc = E::mfma(zf[u], sf[u], acc);
     }
-    // stage the output tile (token-major) in the X region of this block
-    if (wave_active)
+    // stage the output in the X tile of this block: the lane holds columns 32 wcol + 16 hh .. + 15
 #pragma unroll
-    for (int I = 0; I < NI; ++I)
+    for (int p = 0; p < 2; ++p) {
+      u32x4 o;
 #pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        u32x2 o;
-        o.x = E::pack(acc[I][4 * gq + 0], acc[I][4 * gq + 1]);
-        o.y = E::pack(acc[I][4 * gq + 2], acc[I][4 * gq + 3]);
-        *reinterpret_cast<u32x2 *>(cur + L::XN + (32 * (ih + I) + c) * L::LDN + (32 * wcol + 8 * gq + 4 * hh) * 2) = o;
-      }
+      for (int i = 0; i < 4; ++i) o[i] = E::pack(acc[8 * p + 2 * i], acc[8 * p + 2 * i + 1]);
+      *reinterpret_cast<u32x4 *>(cur + L::X + (o_at ^ (p << 4))) = o;
+    }
     __syncthreads();  // barrier 2 it + 2
   }
   // the segment visited last leaves the chunk's outgoing state
   if (SRC != SRC_SCANNED && !TRANS && carry_out != nullptr && sw.seg == (REV ? 0 : g.n_seg - 1) && ih == 0) {
     float *cp = carry_out + (int64_t)sw.bh * g.dt * g.e, *tp = g.twin ? g.twin + (int64_t)sw.bh * g.dt * g.e : nullptr;
-    const int col = 32 * wcol + c;
 #pragma unroll
     for (int T = 0; T < NT; ++T)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int row = 32 * T + 8 * (r >> 2) + 4 * hh + (r & 3);
+        const int row = 32 * T + 16 * (r >> 3) + 8 * hh + 4 * ((r >> 2) & 1) + (r & 3);
         if (!NARROW || (row < fa && col < fb)) {
           cp[row * (NARROW ? fb : W) + col] = st[T][r];
           if (tp) tp[row * (NARROW ? fb : W) + col] = st[T][r];
@@ -803,6 +641,688 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       }
   }
 }
+
+// LDS of the 128-wide sweep: three sets of token-major X, Y and Z tiles, and the score tile.
+struct SweepLds {
+  static constexpr int ROW = 256, TILE = BLK * ROW;
+  static constexpr int X = 0, Y = TILE, Z = 2 * TILE, SET = 3 * TILE;
+  static constexpr int SC = 3 * SET, SC_ROW = 2 * BLK;
+  static constexpr int KDEC = SC + BLK * SC_ROW;  // decay between each token of a block and the state that the block leaves,
+  static constexpr int KDEC_TAIL = KDEC + 4 * BLK;  // ... and of the chunk's partial last block
+  static constexpr int BYTES = KDEC_TAIL + 4 * BLK;  // 156 160 B: one workgroup per CU
+};
+// unit u (16 bytes) of row r of such a tile lies at u ^ swizzle(r)
+__device__ __forceinline__ int swizzle(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+__device__ __forceinline__ uint32_t lds_address(const char *p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p;
+}
+__device__ __forceinline__ u32x4 row_buffer(const void *p, int bytes) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  u32x4 r;
+  r.x = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  r.y = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  r.z = (uint32_t)__builtin_amdgcn_readfirstlane(bytes);
+  r.w = 0x00020000u;
+  return r;
+}
+// 16 bytes per lane from memory to LDS, lane after lane from `lds` on
+__device__ __forceinline__ void load_to_lds(u32x4 rows, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rows)
+               : "memory", "m0");
+}
+// A barrier that the wave's LDS accesses have to be done for, but the N youngest (they are answered in order)
+template <int N>
+__device__ __forceinline__ void barrier_before() {
+  asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// ------------------------------------------------------------------------------
+// The 128-wide sweep.  512 threads, one workgroup per CU, two groups of waves:
+//   waves 0-3 ("feed"): loads, which go from memory straight to LDS, two blocks ahead; the masked score tile; the output stores;
+//   waves 4-7 ("math"): own the state and the output (wave 4 + w: 32 columns from 32 w on): state term, state update, the
+//     scores' part of the output ("intra"), which follows while the next block is under way.
+// A block takes two barriers:
+//     feed: score(t) up to its products,  | math: upper half of the state update(t-1), intra(t-1), first half of the state
+//           load Y, Z(t+2)                |       term(t), stage O(t-1) in the X tile of block t-1
+//   ---- barrier m ----
+//     feed: mask and write score(t),      | math: second half of the state term(t), lower half of the state update(t)
+//           store O(t-1), load X(t+2)     |
+//   ---- barrier b ----
+// Every tile lies token-major, as in memory: what contracts over tokens is read transposed (ds_read_b64_tr_b16), the state update's
+// decay goes to the 32 columns of Z that only one wave reads, and no wave moves a tile through its registers.
+//
+// What bounds a block.  The issue of the math waves' instructions, some 300 on the vector unit (about 4.4 cycles each behind one
+// another), 38 products (9) and 70 LDS accesses; then the LDS, which moves some 330 KB a block.  So the vector work is dealt out
+// between the products by hand (see `slot`), reads are asked for a phase ahead, and what a block's first reads would wait for is
+// covered by products held back from the block before.  Neither stores nor loads to registers stand in the math waves: behind the feed waves' loads
+// each of them waits its turn in the memory pipeline (with the outputs stored from there, the state term took 2660 cycles at
+// n = 65536 instead of 700; so does any register spilled to scratch).
+//   Cycles a block, alone on a CU: 3200 (4250 with tiles that went through registers, transposed on the way, and the state update
+// and both halves of the output between the same two barriers).  Sweep kernels in us, that form and this one: b*h = 16, n = 65536:
+// forward 193 and 196, backward 507 and 460 (HBM: 2.7 GB); n = 16384 in 256 segments: 48 and 46, 136 and 113; b*h = 36, n = 5003:
+// 34.8 and 32.4, 97 and 84.6; b*h = 24, n = 2048, 7 segments: 14.6 and 13.4, 30.4 and 27.7; two slices of d = 256, b*h = 8,
+// n = 8192: 40 and 34, 97 and 82.
+// ------------------------------------------------------------------------------
+template <class E, bool REV, bool TRANS, int SRC, int MODE>
+__device__ __forceinline__ void
+sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z,
+           const float *__restrict__ S, const float *__restrict__ states, elem16_t *__restrict__ Out, const Geom &g,
+           int fa, int fb, int item, char *smem, const float *__restrict__ carry_in,
+           float *__restrict__ carry_out = nullptr) {
+  constexpr bool RAGGED = MODE != M_ALIGNED, NARROW = MODE >= M_NARROW;
+  constexpr bool LEAVES_STATE = SRC != SRC_SCANNED;  // the sweep's final state is the chunk's outgoing one
+  using L = SweepLds;
+  constexpr int W = 128;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = w8 & 3;
+  const int c = lane & 31, hh = lane >> 5;
+
+  const SegWork sw = seg_work(g, item);
+  const int head = sw.bh - quotient(sw.bh, g.by_h) * g.h;
+  const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
+  // elements from row to row of X and Y, and of Z and Out: q, k and their gradients have rows of g.dt features, of which
+  // a slice of a wide head reads and writes fa (fb)
+  const int xp = NARROW ? (TRANS ? g.e : g.dt) : W, zp = NARROW ? (TRANS ? g.dt : g.e) : W;
+  const int nblk = sw.nblk;
+  const int step = REV ? -1 : 1;
+  const int blk0 = REV ? nblk - 1 : 0;
+  const int total_blk = (int)((g.n + BLK - 1) / BLK);  // blocks in the chunk
+  const int seg_blk0 = (int)(sw.tok0 / BLK);           // the segment's first block
+  const int chunk_tail = (int)(g.n - (int64_t)(total_blk - 1) * BLK);
+  // tokens in a block (numbered relative to the segment): a partial block is the chunk's last one
+  auto len_of = [&](int blk) __attribute__((always_inline)) {
+    if (!RAGGED) return BLK;
+    return seg_blk0 + blk == total_blk - 1 ? chunk_tail : BLK;
+  };
+  // SRC_WALK: the state entering the segment is rebuilt by walking `runup` blocks outside it first (before it,
+  // or after it going backwards), as far as the head's decay reaches, from the chunk's incoming state if the
+  // walk gets to the chunk's end, else from zero.  Blocks are numbered relative to the segment; walk and sweep
+  // form one run of runup + nblk blocks, first_blk, first_blk + step, ..., of which the first `runup` only
+  // update the state.
+  int runup = 0;
+  bool take_carry = false;
+  if (SRC == SRC_WALK) {
+    const int avail = REV ? total_blk - (seg_blk0 + nblk) : seg_blk0;
+    int reach = avail;
+    const float sl = S[head] * LOG2E;
+    if (sl > 0.f) {
+      const float x = SKIP_LOG2 / (sl * (float)BLK);  // blocks over which a weight falls to 2^-SKIP_LOG2
+      if (x < (float)avail) reach = (int)x + 1;
+    }
+    runup = __builtin_amdgcn_readfirstlane(min(reach, avail));
+    take_carry = carry_in != nullptr && runup == avail;
+  }
+  const int first_blk = blk0 - runup * step;
+  const int run = runup + nblk;  // blocks in the whole run
+
+  if (w8 < 4) {
+    // ================================ feed waves ================================
+    // Wave w loads rows 16 w .. + 15 of every tile, four of them at a time: lane l's 16 bytes land at unit l % 16 of row l / 16.
+    uint32_t x_off[4], z_off[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 16 * w + 4 * i + (lane >> 4), unit = (lane & 15) ^ swizzle(row);
+      x_off[i] = !NARROW || unit * 8 < fa ? (uint32_t)(row * xp * 2 + unit * 16) : kOutside;
+      z_off[i] = !NARROW || unit * 8 < fb ? (uint32_t)(row * zp * 2 + unit * 16) : kOutside;
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_address(smem) + 16 * w * L::ROW);
+    const elem16_t *Xg = X + row0 * xp, *Yg = Y + row0 * xp, *Zg = Z + row0 * zp;
+    auto fetch_tile = [&](const elem16_t *base, int blk, int pitch, const uint32_t (&off)[4], uint32_t lds)
+                          __attribute__((always_inline)) {
+      const u32x4 rows = row_buffer(base + (int64_t)blk * BLK * pitch, len_of(blk) * pitch * 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) load_to_lds(rows, off[i], lds + 4 * i * L::ROW);
+    };
+    // block k of the run into set `set`: four loads of X (none for a block that is only walked over), eight of Y and Z
+    auto fetch_x = [&](int k, int set) __attribute__((always_inline)) {
+      if (SRC != SRC_WALK || k >= runup) fetch_tile(Xg, first_blk + k * step, xp, x_off, lds0 + set * L::SET + L::X);
+    };
+    auto fetch_yz = [&](int k, int set) __attribute__((always_inline)) {
+      const int blk = first_blk + k * step;
+      fetch_tile(Yg, blk, xp, x_off, lds0 + set * L::SET + L::Y);
+      fetch_tile(Zg, blk, zp, z_off, lds0 + set * L::SET + L::Z);
+    };
+    fetch_x(0, 0);
+    fetch_yz(0, 0);
+    if (run > 1) {
+      fetch_x(1, 1);
+      fetch_yz(1, 1);
+    }
+    const float *late = S + head;  // (asked for behind the first loads: it would have to arrive before they could leave)
+    asm volatile("" : "+s"(late));
+    const float sl = *late * LOG2E;
+    if (tid < BLK) {
+      *reinterpret_cast<float *>(smem + L::KDEC + 4 * tid) = decay(sl, REV ? (float)tid : (float)(BLK - tid));
+      if (RAGGED) *reinterpret_cast<float *>(smem + L::KDEC_TAIL + 4 * tid) = decay(sl, REV ? (float)tid : (float)max(chunk_tail - tid, 0));
+    }
+    // this wave's quadrant of the transposed score tile: sc[4g+r] = y_b . x_a, b = 32qJ+8g+4hh+r, a = 32qI+c
+    const int qI = w >> 1, qJ = w & 1;
+    const bool q_active = REV ? !(qI == 1 && qJ == 0) : !(qI == 0 && qJ == 1);
+    float mask[16];  // decay between the tokens of a score; negative: masked
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int a = 32 * qI + c, b = 32 * qJ + 8 * (r >> 2) + 4 * hh + (r & 3), dist = REV ? b - a : a - b;
+      mask[r] = dist >= 0 ? decay(sl, (float)dist) : -1.f;
+    }
+    const int x_at = 32 * qI * L::ROW + c * L::ROW + ((hh ^ swizzle(c)) << 4);
+    const int y_at = 32 * qJ * L::ROW + c * L::ROW + ((hh ^ swizzle(c)) << 4);
+    const int sc_at = (32 * qI + c) * L::SC_ROW + ((4 * qJ ^ ((c >> 1) & 7)) << 4) + 8 * hh;
+    floatx16 sc;
+    auto write_scores = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) {
+        float m[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m[r] = mask[4 * gq + r] >= 0.f ? sc[4 * gq + r] * mask[4 * gq + r] : 0.f;
+        u32x2 o;
+        o.x = E::pack(m[0], m[1]);
+        o.y = E::pack(m[2], m[3]);
+        *reinterpret_cast<u32x2 *>(smem + L::SC + (sc_at ^ (gq << 4))) = o;
+      }
+    };
+    // the rows of output staged in a set's X tile, where this wave will load X: row by row to where the rows of Z lie
+    elem16_t *Og = Out + row0 * zp;
+    const char *const o_from = smem + L::X + 16 * w * L::ROW + lane * 16;
+    u32x4 out[4];
+    auto read_out = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[i] = lds16(o_from + set * L::SET + 4 * i * L::ROW);
+    };
+    auto store_out = [&](int k) __attribute__((always_inline)) {
+      const int blk = first_blk + k * step;
+      const rows_t rows = rows_of(Og + (int64_t)blk * BLK * zp, len_of(blk) * zp * 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_raw_buffer_store_b128(out[i], rows, (int)z_off[i], 0, 2 /* non-temporal */);
+    };
+    // Everything that this wave has asked for but the loads of block 1 has arrived
+    if (run == 1)
+      wait_loads<0>();
+    else if (SRC != SRC_WALK || runup <= 1)
+      wait_loads<12>();
+    else
+      wait_loads<8>();
+    __syncthreads();  // block 0 of the run visible
+    int set = 0, spare = 2;  // of block k, and of the blocks before it and two after it
+    int k = 0;
+    for (; SRC == SRC_WALK && k < runup; ++k) {
+      if (k + 2 < run) {
+        fetch_x(k + 2, spare);
+        fetch_yz(k + 2, spare);
+      }
+      if (k + 2 >= run)
+        wait_loads<0>();
+      else if (k + 2 >= runup)
+        wait_loads<12>();
+      else
+        wait_loads<8>();
+      __syncthreads();  // block k + 1 visible; the tiles of block k no longer read
+      spare = set;
+      set = set == 2 ? 0 : set + 1;
+    }
+    for (; k < run; ++k) {
+      u32x4 yf[8], xf[8];
+      if (q_active) {
+        const char *from = smem + set * L::SET;
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+          yf[ks] = lds16(from + L::Y + (y_at ^ (ks << 5)));
+          xf[ks] = lds16(from + L::X + (x_at ^ (ks << 5)));
+        }
+      }
+      if (k + 2 < run) fetch_yz(k + 2, spare);
+      if (q_active) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) sc = E::mfma(yf[ks], xf[ks], sc);
+      }
+      __syncthreads();  // the scores of block k - 1 no longer read, its output staged
+      if (q_active) write_scores();
+      if (k > runup) {
+        read_out(spare);
+        store_out(k - 1);
+      }
+      if (k + 2 < run) fetch_x(k + 2, spare);
+      // all but what was asked for since: four stores, 12 loads
+      if (k + 2 < run) {
+        if (k > runup)
+          wait_loads<16>();
+        else
+          wait_loads<12>();
+      } else if (k + 1 < run) {
+        if (k > runup)
+          wait_loads<4>();
+        else
+          wait_loads<0>();
+      }
+      __syncthreads();  // block k + 1 and the scores of block k visible; the tiles of block k no longer read
+      spare = set;
+      set = set == 2 ? 0 : set + 1;
+    }
+    __syncthreads();  // the last block's output staged
+    read_out(spare);
+    store_out(run - 1);
+    return;
+  }
+
+  // ================================== math waves ==================================
+  __builtin_amdgcn_s_setprio(2);  // a block waits for these waves: b*h = 16, n = 65536, backward sweep 460 us, 475 without
+  // Registers and rows.  An accumulator tile holds rows 8g + 4hh + r in register 4g + r of lane (c, hh).  Which feature
+  // of Y (state row) and which column of Z (state column, output column) a row or lane stands for is chosen by the addresses of
+  // the transposing reads: state row 32T + 16(g / 2) + 8hh + 4(g % 2) + r, so that the eight rows of a k-step are eight
+  // features in a row, as X has them in memory; column 16 hh' + 4 g + r for lane c = 8g + 4hh' + r, so that a lane of the output tile holds
+  // 16 columns in a row of its token.
+  const int col = 32 * w + 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3);
+  const float sl = S[head] * LOG2E;
+  const float blockdec = decay(sl, (float)BLK);
+  float qdec[2];
+#pragma unroll
+  for (int I = 0; I < 2; ++I) qdec[I] = decay(sl, REV ? (float)(BLK - 32 * I - c) : (float)(32 * I + c));
+  floatx16 st[4];
+#pragma unroll
+  for (int T = 0; T < 4; ++T)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st[T][r] = 0.f;
+  // st <- f * st + M (`fresh`: st <- M, which leaves the loads in flight until a product needs them), M being the W x W fp32
+  // tile whose element (row, col) is src[row * ld + col], or for a transposed role src[col * ld + row]; `bounded`: src holds
+  // only fa x fb (transposed: fb x fa) elements
+  auto add_state_ld = [&](const float *src, int ld, float f, bool bounded, bool fresh) __attribute__((always_inline)) {
+    typedef const __attribute__((address_space(1))) float *gmem_f32;
+    const uint32_t lane_off = (uint32_t)(TRANS ? col * ld + 8 * hh : 8 * hh * ld + col) * (uint32_t)sizeof(float);
+    const bool col_ok = !bounded || col < fb;
+#pragma unroll
+    for (int T = 0; T < 4; ++T)
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) {
+        const int band = 32 * T + 16 * (gq >> 1) + 4 * (gq & 1);
+        const gmem_ptr bp = uniform_ptr(reinterpret_cast<const char *>(src + (TRANS ? band : (int64_t)band * ld)));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const bool ok = col_ok && (!bounded || band + 8 * hh + r < fa);
+          const float own =
+              ok ? *reinterpret_cast<gmem_f32>(bp + lane_off + (uint32_t)(TRANS ? r : r * ld) * sizeof(float)) : 0.f;
+          st[T][4 * gq + r] = fresh ? own : fmaf(f, st[T][4 * gq + r], own);
+        }
+      }
+  };
+  // a state of the workspace (W x W, zero beyond fa x fb) / the chunk's incoming state (fa x fb, unpadded)
+  auto add_state = [&](const float *src, float f, bool fresh = false) __attribute__((always_inline)) {
+    add_state_ld(src, W, f, false, fresh);
+  };
+  auto add_carry = [&]() __attribute__((always_inline)) {
+    add_state_ld(carry_in + (int64_t)sw.bh * g.dt * g.e, NARROW ? (TRANS ? fa : fb) : W, 0.f, NARROW, true);
+  };
+  if (SRC == SRC_WALK) {
+    if (take_carry) add_carry();
+  } else if (SRC == SRC_SCANNED) {
+    if (states) {
+      // the scanned state of this segment, or for a head the scan leaves out (state_dies_in_segment), whose
+      // own states are still where the pre-pass put them, the own state of the segment visited before it
+      // (the chunk's incoming state for the first one)
+      // The workspace holds one state per segment of the pre-pass, of which this sweep segment spans
+      // `sub` (a power of two; 1 unless the plan cut long segments finer for the pre-pass): the state that
+      // enters it is the one entering its first piece in sweep order.
+      const int sub = g.seg_len / g.pre_len;
+      const int piece = REV ? min(sw.seg * sub + sub, g.pre_n) - 1 : sw.seg * sub;
+      const float *src = states + ((int64_t)sw.bh * g.pre_n + piece) * (W * W);
+      bool from_carry = false;
+      if (state_dies_in_segment(S[head], g)) {
+        const int nb = REV ? piece + 1 : piece - 1;
+        if (nb < 0 || nb >= g.pre_n)
+          from_carry = true;
+        else
+          src = states + ((int64_t)sw.bh * g.pre_n + nb) * (W * W);
+      }
+      // (for such a head the scan kernel has parked the chunk's incoming state in the slot of the piece it
+      // visits last, so that nothing reads `carry_in`'s memory once the outgoing state may have replaced it)
+      if (from_carry) src = states + ((int64_t)sw.bh * g.pre_n + (REV ? 0 : g.pre_n - 1)) * (W * W);
+      if (!from_carry || carry_in != nullptr) add_state(src, 0.f, true);
+    }
+  } else {
+    // `states` holds the segments' OWN states.  The scan's recurrence, St <- l^len_j St + own_j over the
+    // segments visited before this one, is run here -- over as many of them as the head's decay reaches:
+    // an own state further back arrives weighted below 2^-SKIP_LOG2 (everything between it and this
+    // segment is a full-length segment) and is left out, and so is the chunk's incoming state unless the
+    // walk starts at the chunk's end.  These waves have the time: the feed waves are fetching block 0.
+    const int n_before = REV ? g.n_seg - 1 - sw.seg : sw.seg;
+    int first = 0;
+    if (sl > 0.f) {
+      const float segs = SKIP_LOG2 / (sl * (float)g.seg_len);  // full segments over which a weight falls to 2^-SKIP_LOG2
+      if (segs < (float)n_before) first = n_before - ((int)segs + 1);
+    }
+    first = __builtin_amdgcn_readfirstlane(first);
+    if (first == 0 && carry_in) add_carry();
+    if (states) {
+      const float *base = states + (int64_t)sw.bh * g.n_seg * (W * W);
+      const float full = decay(sl, (float)g.seg_len);
+      const float last = decay(sl, (float)(g.n - (int64_t)(g.n_seg - 1) * g.seg_len));
+      for (int i = first; i < n_before; ++i) {
+        const int j = REV ? g.n_seg - 1 - i : i;
+        add_state(base + (int64_t)j * (W * W), j == g.n_seg - 1 ? last : full);
+      }
+    }
+  }
+  const int s16 = lane & 15, q4 = s16 & 3, ch = (lane >> 4) & 1;
+  const int t_row = 8 * hh + (s16 >> 2), t_swz = swizzle(t_row);
+  const int y_at = t_row * L::ROW + (((2 * ch + (q4 & 1)) ^ t_swz) << 4) + ((q4 >> 1) << 3);
+  const int z_at = t_row * L::ROW + (((4 * w + 2 * (q4 & 1) + ch) ^ t_swz) << 4) + ((q4 >> 1) << 3);
+  const int x_at = c * L::ROW + ((hh ^ swizzle(c)) << 4);
+  const int sc_at = c * L::SC_ROW + ((hh ^ ((c >> 1) & 7)) << 4);
+  // operand over tokens 16 u + 8 hh .. + 7 of a tile
+  auto tokens = [&](const char *tile, int at, int u) __attribute__((always_inline)) {
+    const u32x2 lo = lds_tr8(tile + at + 16 * u * L::ROW), hi = lds_tr8(tile + (at ^ 16) + (16 * u + 4) * L::ROW);
+    u32x4 r;
+    r.x = lo.x;
+    r.y = lo.y;
+    r.z = hi.x;
+    r.w = hi.y;
+    return r;
+  };
+  // Work for the vector unit is dealt out by hand between the products: one of 32 x 32 x 16 keeps the matrix unit busy for 32
+  // cycles, in which the wave that issued it can issue some seven other instructions; the scheduler would put all of them in front.
+  auto slot = [](floatx16 &sum, const u32x4 &a, const u32x4 &b, auto &&work) __attribute__((always_inline)) {
+    sum = E::mfma(a, b, sum);
+    work();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // rows r0 .. + 3 of tile T of the state
+  auto decay_state = [&](int T, int r0, float bd) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = r0; r < r0 + 4; ++r) {
+      float x = st[T][r] * bd;
+      asm volatile("" : "+v"(x));
+      st[T][r] = x;
+    }
+  };
+  // operand of k-step ks of the state term
+  auto pack_state = [&](int ks) __attribute__((always_inline)) {
+    const int T = ks >> 1, r = 8 * (ks & 1);
+    u32x4 a;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t x = E::pack(st[T][r + 2 * i], st[T][r + 2 * i + 1]);
+      asm volatile("" : "+v"(x));
+      a[i] = x;
+    }
+    return a;
+  };
+  // Z^T scaled by its tokens' decay to the block's end: the decays of step u, pair i of it.  (Where a sweep leaves the state, the
+  // tokens of the chunk's partial last block, going forwards, lie `len` - b before the end; elsewhere nothing after that block
+  // uses the state.)
+  const int kdec_at = L::KDEC + 32 * hh;
+  auto read_kdec = [&](int u, int len, u32x4 (&kd)[2]) __attribute__((always_inline)) {
+    const char *from = smem + kdec_at + (LEAVES_STATE && RAGGED && len != BLK ? L::KDEC_TAIL - L::KDEC : 0) + 64 * u;
+    kd[0] = lds16(from);
+    kd[1] = lds16(from + 16);
+  };
+  auto scale_z = [&](const u32x4 (&zf)[4], u32x4 (&zs)[4], const u32x4 (&kd)[2], int u, int i) __attribute__((always_inline)) {
+    const u32x4 &q = kd[i >> 1];
+    const float w0 = __uint_as_float((i & 1) ? q.z : q.x), w1 = __uint_as_float((i & 1) ? q.w : q.y);
+    uint32_t x = E::pack(elem_f32<E>(zf[u], 2 * i) * w0, elem_f32<E>(zf[u], 2 * i + 1) * w1);
+    asm volatile("" : "+v"(x));
+    zs[u][i] = x;
+  };
+  // operand over tokens 16 u .. of the 32 rows of state tile T
+  auto read_y = [&](const char *tile, int lane_at, int T, int u) __attribute__((always_inline)) {
+    return tokens(tile, lane_at ^ (T << 6), u);
+  };
+  // an offset whose variants are worked out where they are used and not kept in registers
+  auto fresh = [](int at) __attribute__((always_inline)) {
+    asm volatile("" : "+v"(at));
+    return at;
+  };
+  // Slices of a wide head after the first add to what the slices before them left in Out (its rows are whole
+  // features of v, so only the non-transposed roles).  A block's old output is fetched while the block before it is
+  // computed; the lane holds the columns that its accumulators hold.
+  constexpr bool ADDS = MODE == M_ADDING && !TRANS;
+  u32x4 old[2][2] = {};
+  auto fetch_old = [&](int blk) __attribute__((always_inline)) {
+    const rows_t rows = rows_of(Out + (row0 + (int64_t)blk * BLK) * zp, len_of(blk) * zp * 2);
+#pragma unroll
+    for (int I = 0; I < 2; ++I)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int first = 32 * w + 16 * hh + 8 * p;
+        old[I][p] = __builtin_amdgcn_raw_buffer_load_b128(
+            rows, first < fb ? (32 * I + c) * zp * 2 + first * 2 : (int)kOutside, 0, 0);
+      }
+  };
+  // Unit j of 8 of a block's output on its way into an X tile: four for the 32 tokens that `first` names, then four for the others
+  const int o_at = c * L::ROW + (((4 * w + 2 * hh) ^ swizzle(c)) << 4);
+  auto pack_out = [&](const floatx16 (&acc)[2], int first, int j, char *tile, u32x4 &o) __attribute__((always_inline)) {
+    const int lane_at = fresh(o_at);
+    const int I = j < 4 ? first : 1 - first, i = j & 3;
+    o[2 * (i & 1)] = E::pack(acc[I][4 * i], acc[I][4 * i + 1]);
+    o[2 * (i & 1) + 1] = E::pack(acc[I][4 * i + 2], acc[I][4 * i + 3]);
+    if (i & 1) *reinterpret_cast<u32x4 *>(tile + 32 * I * L::ROW + (lane_at ^ ((i >> 1) << 4))) = o;
+  };
+  if (NARROW && 32 * w >= fb) {  // a wave whose columns all lie past the width of Z only takes part in the barriers
+    for (int i = 0; i < 2 + runup + 2 * nblk; ++i) __syncthreads();
+    return;
+  }
+  __syncthreads();  // block 0 of the run visible
+  int set_i = 0, k = 0;
+  for (; SRC == SRC_WALK && k < runup; ++k) {  // walk
+    const char *set = smem + set_i * L::SET;
+    set_i = set_i == 2 ? 0 : set_i + 1;
+    {
+      const int len = len_of(first_blk + k * step);
+      const float bd = RAGGED && len != BLK ? decay(sl, (float)len) : blockdec;
+      const int y_lane = fresh(y_at);
+      u32x4 zf[4], zs[4], yf[2][4][2], kd[4][2];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) zf[u] = tokens(set + L::Z, z_at, u);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int T = 0; T < 2; ++T) yf[0][u][T] = read_y(set + L::Y, y_lane, T, u);
+      reads_first();
+#pragma unroll
+      for (int r = 0; r < 16; r += 4) decay_state(0, r, bd), decay_state(1, r, bd);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) read_kdec(u, len, kd[u]);
+      reads_first();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) scale_z(zf, zs, kd[0], 0, i);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int u = j >> 1, T = j & 1;
+        slot(st[T], yf[0][u][T], zs[u], [&]() __attribute__((always_inline)) {
+          decay_state(2 + (j >> 2), 4 * (j & 3), bd);
+          if (u < 3) scale_z(zf, zs, kd[u + 1], u + 1, 2 * T), scale_z(zf, zs, kd[u + 1], u + 1, 2 * T + 1);
+          yf[1][u][T] = read_y(set + L::Y, y_lane, 2 + T, u);
+        });
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) st[2 + (j & 1)] = E::mfma(yf[1][j >> 1][j & 1], zs[j >> 1], st[2 + (j & 1)]);
+    }
+    __syncthreads();
+  }
+  // What a block leaves to the next one's time: of its output, the scores' part (they are computed meanwhile), of the state
+  // update, the upper half of the rows, whose products cover the time that the next block's first reads take.
+  floatx16 acc[2];  // the output without that part, not yet scaled by ...
+  float qd[2] = {1.f, 1.f};
+  u32x4 zf[4], zs[4], yf1[4][2];
+#pragma unroll
+  for (int I = 0; I < 2; ++I)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[I][r] = 0.f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) zf[u] = zs[u] = yf1[u][0] = yf1[u][1] = u32x4{0u, 0u, 0u, 0u};
+  // acc[I] += Z^T[32 w .., tokens] * score[a][tokens] of the block before
+  auto read_scores = [&](const char *tile, u32x4 (&sf)[4][2]) __attribute__((always_inline)) {
+    const int lane_at = fresh(sc_at);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int I = 0; I < 2; ++I)
+        if (REV ? (I == 0 || u >= 2) : (I == 1 || u < 2)) sf[u][I] = lds16(tile + 32 * I * L::SC_ROW + (lane_at ^ (u << 5)));
+  };
+  // the six products of (row half I of the output, tokens 16 u ..) that the mask leaves
+  constexpr int INTRA_U[2][6] = {{0, 1, 0, 1, 2, 3}, {2, 3, 0, 1, 2, 3}}, INTRA_I[2][6] = {{0, 0, 1, 1, 1, 1}, {1, 1, 0, 0, 0, 0}};
+  constexpr int FIRST = REV ? 1 : 0;  // the half that is finished first
+  auto scale_acc = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 4 * (j & 3); r < 4 * (j & 3) + 4; ++r) {
+      float x = ADDS ? fmaf(acc[j >> 2][r], qd[j >> 2], elem_f32<E>(old[j >> 2][r >> 3], r & 7)) : acc[j >> 2][r] * qd[j >> 2];
+      asm volatile("" : "+v"(x));
+      acc[j >> 2][r] = x;
+    }
+  };
+  for (; k < run; ++k) {
+    const char *set = smem + set_i * L::SET;
+    char *const staged = smem + (set_i == 0 ? 2 : set_i - 1) * L::SET + L::X;  // where the output of the block before goes
+    set_i = set_i == 2 ? 0 : set_i + 1;
+    const int blk = first_blk + k * step;
+    const int len = len_of(blk);
+    // A partial block is the chunk's last one.  Going forwards nothing after it uses the state (but the outgoing
+    // state where the sweep leaves it); going backwards it comes first and the entering state sits `len` (not 64)
+    // tokens ahead.
+    float qn[2] = {qdec[0], qdec[1]};
+    float bd = blockdec;
+    if (RAGGED && REV && len != BLK) {
+#pragma unroll
+      for (int I = 0; I < 2; ++I) qn[I] = decay(sl, (float)max(len - 32 * I - c, 0));
+      bd = decay(sl, (float)len);
+    }
+    if (LEAVES_STATE && RAGGED && !REV && len != BLK) bd = decay(sl, (float)len);
+    {
+      u32x4 sf[4][2], xf[2][4][2], yf0[4][2], zn[4], a[4], kd[4][2];
+      const int x_lane = fresh(x_at), y_lane = fresh(y_at), z_lane = fresh(z_at);
+      auto read_x = [&](int ks, int I) __attribute__((always_inline)) {
+        return lds16(set + L::X + 32 * I * L::ROW + (x_lane ^ (ks << 5)));
+      };
+      read_scores(smem + L::SC, sf);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) xf[0][j >> 1][j & 1] = read_x(j >> 1, j & 1);
+      reads_first();
+      // (1) the block before: the rest of its state update, the scores
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        slot(st[2 + (j & 1)], yf1[j >> 1][j & 1], zs[j >> 1], [&]() __attribute__((always_inline)) {
+          scale_acc(j);
+          if (j >= 4) xf[0][j >> 1][j & 1] = read_x(j >> 1, j & 1);
+        });
+      }
+#pragma unroll
+      for (int j = 0; j < 6; ++j) {
+        slot(acc[INTRA_I[REV][j]], zf[INTRA_U[REV][j]], sf[INTRA_U[REV][j]][INTRA_I[REV][j]], [&]() __attribute__((always_inline)) {
+          if (j < 4) a[j] = pack_state(j);
+          if (j >= 2) zn[j - 2] = tokens(set + L::Z, z_lane, j - 2);
+          if (j >= 2 && j < 4) decay_state(0, 8 * (j - 2), bd), decay_state(0, 8 * (j - 2) + 4, bd);
+          if (j >= 4) decay_state(1, 8 * (j - 4), bd), decay_state(1, 8 * (j - 4) + 4, bd);
+        });
+      }
+      // (2) state term, transposed: term[I][4g+r] = sum_f St[f][column] x_a[f], a = 32 I + c
+      floatx16 term[2];
+#pragma unroll
+      for (int I = 0; I < 2; ++I)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) term[I][r] = 0.f;
+      u32x4 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int ks = j >> 1, I = j & 1;
+        slot(term[I], a[ks], xf[0][ks][I], [&]() __attribute__((always_inline)) {
+          if (j >= 1 && j < 5) {
+            pack_out(acc, FIRST, 2 * j - 2, staged, o);
+            pack_out(acc, FIRST, 2 * j - 1, staged, o);
+          }
+          if (j == 2) read_kdec(0, len, kd[0]);
+          if (j == 3) read_kdec(1, len, kd[1]);
+          if (j == 4) __builtin_amdgcn_sched_barrier(0);
+          if (j >= 4) {
+            xf[1][j - 4][0] = read_x(j, 0);
+            xf[1][j - 4][1] = read_x(j, 1);
+          }
+          if (j >= 5) a[j - 5] = pack_state(j - 1);
+        });
+      }
+      if (ADDS) fetch_old(blk);
+      barrier_before<8>();  // the scores are read and the output is staged (the eight youngest reads may be on their way)
+      auto second_half = [&](int j) __attribute__((always_inline)) {
+        decay_state(2 + (j >> 2), 4 * (j & 3), bd);
+        yf0[j >> 1][j & 1] = read_y(set + L::Y, y_lane, j & 1, j >> 1);
+        scale_z(zn, zs, kd[j >> 2], j >> 2, j & 3);
+        if (j == 4) read_kdec(2, len, kd[2]), read_kdec(3, len, kd[3]);
+      };
+      a[3] = pack_state(7);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        slot(term[j & 1], a[j >> 1], xf[1][j >> 1][j & 1], [&]() __attribute__((always_inline)) { second_half(j); });
+      // (3) state update, the lower half of the rows
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int u = j >> 1, T = j & 1;
+        slot(st[T], yf0[u][T], zs[u], [&]() __attribute__((always_inline)) {
+          if (j < 4) scale_z(zn, zs, kd[2], 2, j), scale_z(zn, zs, kd[3], 3, j);
+          if (j < 4) {
+            yf1[j][0] = read_y(set + L::Y, y_lane, 2, j);
+            yf1[j][1] = read_y(set + L::Y, y_lane, 3, j);
+          }
+        });
+      }
+#pragma unroll
+      for (int I = 0; I < 2; ++I) {
+        acc[I] = term[I];
+        qd[I] = qn[I];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) zf[u] = zn[u];
+    }
+    __syncthreads();
+  }
+  {
+    u32x4 sf[4][2], o;
+    read_scores(smem + L::SC, sf);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (LEAVES_STATE) st[2 + (j & 1)] = E::mfma(yf1[j >> 1][j & 1], zs[j >> 1], st[2 + (j & 1)]);
+      scale_acc(j);
+    }
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+      acc[INTRA_I[REV][j]] = E::mfma(zf[INTRA_U[REV][j]], sf[INTRA_U[REV][j]][INTRA_I[REV][j]], acc[INTRA_I[REV][j]]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) pack_out(acc, FIRST, j, smem + (set_i == 0 ? 2 : set_i - 1) * L::SET + L::X, o);
+    __syncthreads();
+  }
+  // the segment visited last leaves the chunk's outgoing state
+  if (SRC != SRC_SCANNED && !TRANS && carry_out != nullptr && sw.seg == (REV ? 0 : g.n_seg - 1)) {
+    float *cp = carry_out + (int64_t)sw.bh * g.dt * g.e, *tp = g.twin ? g.twin + (int64_t)sw.bh * g.dt * g.e : nullptr;
+#pragma unroll
+    for (int T = 0; T < 4; ++T)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = 32 * T + 16 * (r >> 3) + 8 * hh + 4 * ((r >> 2) & 1) + (r & 3);
+        if (!NARROW || (row < fa && col < fb)) {
+          cp[row * (NARROW ? fb : W) + col] = st[T][r];
+          if (tp) tp[row * (NARROW ? fb : W) + col] = st[T][r];
+        }
+      }
+  }
+}
+
+// (both round the same operand of every product and add in the same order: rows of 64 features give the bits of rows extended by zeros)
+template <class E, bool REV, bool TRANS, int SRC, int MODE, int W>
+__device__ __forceinline__ void
+any_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z,
+         const float *__restrict__ S, const float *__restrict__ states, elem16_t *__restrict__ Out, const Geom &g,
+         int fa, int fb, int item, char *smem, const float *__restrict__ carry_in,
+         float *__restrict__ carry_out = nullptr) {
+  if constexpr (W == 128)
+    sweep_body<E, REV, TRANS, SRC, MODE>(X, Y, Z, S, states, Out, g, fa, fb, item, smem, carry_in, carry_out);
+  else
+    ws_body<E, REV, TRANS, SRC, MODE>(X, Y, Z, S, states, Out, g, fa, fb, item, smem, carry_in, carry_out);
+}
+template <int W>
+constexpr int sweep_lds() { return W == 128 ? SweepLds::BYTES : WsLds::BYTES; }
 
 template <class E, bool REV, bool TRANS, int SRC, int MODE, int W>
 __global__ void __launch_bounds__(WS_THREADS, ws_waves_per_simd(W))
@@ -812,7 +1332,7 @@ la_apply(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const e
   extern __shared__ __align__(16) char smem[];
   // SRC_COMBINE: later segments have more states to gather first, so they are started first
   const int item = SRC == SRC_COMBINE ? g.b * g.h * g.n_seg - 1 - (int)blockIdx.x : (int)blockIdx.x;
-  ws_body<E, REV, TRANS, SRC, MODE, W>(X, Y, Z, S, states, Out, g, g.d, g.e, item, smem, carry_in, carry_out);
+  any_body<E, REV, TRANS, SRC, MODE, W>(X, Y, Z, S, states, Out, g, g.d, g.e, item, smem, carry_in, carry_out);
 }
 
 // A whole short chunk in one launch: every workgroup rebuilds the state entering its segment (SRC_WALK), so
@@ -829,7 +1349,7 @@ la_fused_fwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
   const int group = quotient(slot, g.by_seg), bh = group * 8 + xcd;
   if (bh >= g.b * g.h) return;
   const int item = bh * g.n_seg + (g.n_seg - 1 - (slot - group * g.n_seg));
-  ws_body<E, false, false, SRC_WALK, MODE, W>(Q, K, V, S, nullptr, O, g, g.d, g.e, item, smem, kv_in, kv_out);
+  any_body<E, false, false, SRC_WALK, MODE, W>(Q, K, V, S, nullptr, O, g, g.d, g.e, item, smem, kv_in, kv_out);
 }
 
 // The (b, h) from bh0 on are cut into segments of their own (n_seg of seg_len tokens): see launch_fused_bwd.
@@ -860,13 +1380,13 @@ la_fused_bwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
   if (bh >= g.b * g.h) return;
   const int k = triple - group * g.n_seg;  // k-th longest walk of its role
   if (role == 0)
-    ws_body<E, false, true, SRC_WALK, MODE, W>(DO, V, K, S, nullptr, DQ, g, g.e, g.d, bh * g.n_seg + g.n_seg - 1 - k, smem,
+    any_body<E, false, true, SRC_WALK, MODE, W>(DO, V, K, S, nullptr, DQ, g, g.e, g.d, bh * g.n_seg + g.n_seg - 1 - k, smem,
                                             kv_in);
   else if (role == 1)
-    ws_body<E, true, false, SRC_WALK, MODE, W>(K, Q, DO, S, nullptr, DV, g, g.d, g.e, bh * g.n_seg + k, smem, dkv_in,
+    any_body<E, true, false, SRC_WALK, MODE, W>(K, Q, DO, S, nullptr, DV, g, g.d, g.e, bh * g.n_seg + k, smem, dkv_in,
                                             dkv_out);
   else
-    ws_body<E, true, true, SRC_WALK, MODE, W>(V, DO, Q, S, nullptr, DK, g, g.e, g.d, bh * g.n_seg + k, smem, dkv_in);
+    any_body<E, true, true, SRC_WALK, MODE, W>(V, DO, Q, S, nullptr, DK, g, g.e, g.d, bh * g.n_seg + k, smem, dkv_in);
 }
 
 // The three gradients in one launch.  Workgroups come in triples (dQ, dV, dK) that work on the same
@@ -887,11 +1407,11 @@ la_bwd3(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const el
   const int item = n_items - 1 - (grp * 8 + (r & 7));
   if (item < 0) return;
   if (role == 0)
-    ws_body<E, false, true, SRC, MODE, W>(DO, V, K, S, kv_states, DQ, g, g.e, g.d, item, smem, kv_in);
+    any_body<E, false, true, SRC, MODE, W>(DO, V, K, S, kv_states, DQ, g, g.e, g.d, item, smem, kv_in);
   else if (role == 1)
-    ws_body<E, true, false, SRC, MODE, W>(K, Q, DO, S, dkv_states, DV, g, g.d, g.e, item, smem, dkv_in, dkv_out);
+    any_body<E, true, false, SRC, MODE, W>(K, Q, DO, S, dkv_states, DV, g, g.d, g.e, item, smem, dkv_in, dkv_out);
   else
-    ws_body<E, true, true, SRC, MODE, W>(V, DO, Q, S, dkv_states, DK, g, g.e, g.d, item, smem, dkv_in);
+    any_body<E, true, true, SRC, MODE, W>(V, DO, Q, S, dkv_states, DK, g, g.e, g.d, item, smem, dkv_in);
 }
 
 // ------------------------------------------------------------------------------
@@ -942,15 +1462,6 @@ constexpr int STATE_DEPTH_LONG = 4, STATE_DEPTH_SHORT = 2;
 constexpr int STATE_WHOLE = 512;
 constexpr int STATE_LONG_WALK = 1024;  // tokens per segment from which the deeper pipeline is used
 
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4i16 *lds_v4i16;
-// The transposing 8-byte read works in groups of 16 lanes: lane i of a group receives, as element j,
-// element (i % 4) of what lane (4 j + i / 4) of the group addressed.  With lane s of a group addressing
-// token T + s / 4, features f + 4 (s % 4) .. + 3, lane i ends up with feature f + i of tokens T .. T + 3.
-__device__ __forceinline__ u32x2 lds_tr8(const char *p) {
-  const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(p));
-  return __builtin_bit_cast(u32x2, r);
-}
 // MFMA operand of lane (c, hh): feature f0 + c, tokens t0 + 8 hh .. + 7 (`lane_part` holds the lane's share
 // of the address, see la_seg_state; rows LDR bytes apart)
 template <int LDR>
@@ -1072,14 +1583,6 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
         if (half_of(r) == half) nt[r] = __builtin_amdgcn_raw_buffer_load_b128(rows, (int)t_off[r], 0, 0);
     }
   };
-  auto scaled = [&](const u32x4 &q, float w) __attribute__((always_inline)) {
-    u32x4 o;
-    o.x = E::pack(elem_f32<E>(q, 0) * w, elem_f32<E>(q, 1) * w);
-    o.y = E::pack(elem_f32<E>(q, 2) * w, elem_f32<E>(q, 3) * w);
-    o.z = E::pack(elem_f32<E>(q, 4) * w, elem_f32<E>(q, 5) * w);
-    o.w = E::pack(elem_f32<E>(q, 6) * w, elem_f32<E>(q, 7) * w);
-    return o;
-  };
   char *const my_rows = smem + (zgrp ? L::TILE : 0) + rq * L::LDR + ((cq * 16) ^ L::row_swap(rq));
   auto fill_lds = [&](int buf, const u32x4 (&nt)[4], int i) __attribute__((always_inline)) {
     char *dst = my_rows + buf * (2 * L::TILE);
@@ -1088,7 +1591,7 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
       const int len = len_of(block_of(BPS * i + half_of(r)));
       const bool partial = RAGGED && !REV && len != BLK;
       u32x4 v = nt[r];
-      if (!zgrp) v = scaled(v, partial ? decay(sl, (float)max(len - row_of(r), 0)) : kdec[BPS == 1 ? r : r & 1]);
+      if (!zgrp) v = scaled<E>(v, partial ? decay(sl, (float)max(len - row_of(r), 0)) : kdec[BPS == 1 ? r : r & 1]);
       *reinterpret_cast<u32x4 *>(dst + ROWS * r * L::LDR) = v;
     }
   };
@@ -1177,11 +1680,11 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
 template <class E, bool REV, bool TRANS, int SRC, int MODE, int W>
 int launch_apply(const void *x, const void *y, const void *z, const float *s, const float *states,
                     const float *carry_in, float *carry_out, void *out, const Geom &g, hipStream_t st) {
-  int rc = grant_lds<la_apply<E, REV, TRANS, SRC, MODE, W>>(WsLds<W>::BYTES);
+  int rc = grant_lds<la_apply<E, REV, TRANS, SRC, MODE, W>>(sweep_lds<W>());
   if (rc) return rc;
   const unsigned grid = (unsigned)((int64_t)g.b * g.h * g.n_seg);
   ProfScope prof(KC_APPLY, st);
-  la_apply<E, REV, TRANS, SRC, MODE, W><<<grid, WS_THREADS, WsLds<W>::BYTES, st>>>(
+  la_apply<E, REV, TRANS, SRC, MODE, W><<<grid, WS_THREADS, sweep_lds<W>(), st>>>(
       (const elem16_t *)x, (const elem16_t *)y, (const elem16_t *)z, s, states, carry_in, carry_out, (elem16_t *)out, g);
   return (int)hipGetLastError();
 }
@@ -1189,12 +1692,12 @@ int launch_apply(const void *x, const void *y, const void *z, const float *s, co
 template <class E, int SRC, int MODE, int W>
 int launch_bwd3(const BwdArgs &a, const float *kv_states, const float *dkv_states, const Geom &g,
                    hipStream_t st) {
-  int rc = grant_lds<la_bwd3<E, SRC, MODE, W>>(WsLds<W>::BYTES);
+  int rc = grant_lds<la_bwd3<E, SRC, MODE, W>>(sweep_lds<W>());
   if (rc) return rc;
   const int64_t n_items = (int64_t)g.b * g.h * g.n_seg;
   const unsigned grid = (unsigned)(((n_items + 7) / 8) * 24);
   ProfScope prof(KC_BWD3, st);
-  la_bwd3<E, SRC, MODE, W><<<grid, WS_THREADS, WsLds<W>::BYTES, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
+  la_bwd3<E, SRC, MODE, W><<<grid, WS_THREADS, sweep_lds<W>(), st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
                                                          (const elem16_t *)a.v, (const elem16_t *)a.d_o, a.s,
                                                          kv_states, dkv_states, a.kv_in, a.dkv_in, a.dkv_out,
                                                          (elem16_t *)a.dq, (elem16_t *)a.dk, (elem16_t *)a.dv, g);
@@ -1235,11 +1738,11 @@ int launch_state(const void *y, const void *z, const float *s, float *states, co
 
 template <class E, int MODE, int W>
 int launch_fused_fwd(const FwdArgs &a, const Geom &g, hipStream_t st) {
-  int rc = grant_lds<la_fused_fwd<E, MODE, W>>(WsLds<W>::BYTES);
+  int rc = grant_lds<la_fused_fwd<E, MODE, W>>(sweep_lds<W>());
   if (rc) return rc;
   const unsigned grid = (unsigned)((((int64_t)g.b * g.h + 7) / 8) * 8 * g.n_seg);  // whole groups of 8 (b, h)
   ProfScope prof(KC_FUSED, st);
-  la_fused_fwd<E, MODE, W><<<grid, WS_THREADS, WsLds<W>::BYTES, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
+  la_fused_fwd<E, MODE, W><<<grid, WS_THREADS, sweep_lds<W>(), st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
                                                          (const elem16_t *)a.v, a.s, a.kv_in, a.kv_out,
                                                          (elem16_t *)a.o, g);
   return (int)hipGetLastError();
@@ -1290,14 +1793,14 @@ Fine fused_bwd_tail(const Geom &g) {
 
 template <class E, int MODE, int W>
 int launch_fused_bwd(const BwdArgs &a, const Geom &g_fwd, hipStream_t st) {
-  int rc = grant_lds<la_fused_bwd<E, MODE, W>>(WsLds<W>::BYTES);
+  int rc = grant_lds<la_fused_bwd<E, MODE, W>>(sweep_lds<W>());
   if (rc) return rc;
   const Geom g = fused_bwd_geom(g_fwd);
   const Fine fine = fused_bwd_tail(g);
   const int64_t tail8 = ((int64_t)g.b * g.h - fine.bh0 + 7) / 8 * 8;
   const unsigned grid = (unsigned)(3 * ((int64_t)fine.bh0 * g.n_seg + tail8 * fine.n_seg));
   ProfScope prof(KC_FUSED, st);
-  la_fused_bwd<E, MODE, W><<<grid, WS_THREADS, WsLds<W>::BYTES, st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
+  la_fused_bwd<E, MODE, W><<<grid, WS_THREADS, sweep_lds<W>(), st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
                                                          (const elem16_t *)a.v, (const elem16_t *)a.d_o, a.s,
                                                          a.kv_in, a.dkv_in, a.dkv_out, (elem16_t *)a.dq,
                                                          (elem16_t *)a.dk, (elem16_t *)a.dv, g, fine);
@@ -1321,7 +1824,6 @@ Geom pre_pass_geom(const Geom &g) {
 Geom slice_geom(const Geom &g, int i) {
   Geom gs = g;
   gs.d = g.dt - i * kMaxWidth < kMaxWidth ? g.dt - i * kMaxWidth : kMaxWidth;
-  gs.add = i > 0;
   if (g.twin) gs.twin = g.twin + (int64_t)i * kMaxWidth * g.e;
   return gs;
 }
@@ -1358,7 +1860,9 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
   int rc = 0;
   const int slices = (int)slices_of(g);
   if (g.fused) {
-    for (int i = 0; i < slices && !rc; ++i) rc = launch_fused_fwd<E, MODE, W>(slice_args(a, g, i), slice_geom(g, i), st);
+    rc = launch_fused_fwd<E, MODE, W>(slice_args(a, g, 0), slice_geom(g, 0), st);
+    if constexpr (MODE == M_NARROW && W == kMaxWidth)
+      for (int i = 1; i < slices && !rc; ++i) rc = launch_fused_fwd<E, M_ADDING, W>(slice_args(a, g, i), slice_geom(g, i), st);
     return rc;
   }
   if constexpr (MODE != M_NARROW) if (g.combine) {  // (the plan combines full-width heads only)
@@ -1377,12 +1881,15 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
     if ((rc = launch_state<E, false, MODE, W>(a.k, a.v, a.s, a.seg_states, gp, a.kv_out != nullptr, sub, st))) return rc;
     if ((rc = launch_segment_scan(a.seg_states, a.kv_in, a.kv_out, a.s, gp, 0, st))) return rc;
   }
-  for (int i = 0; i < slices && !rc; ++i) {
+  auto sweep = [&](auto mode, int i) {
     const FwdArgs as = slice_args(a, g, i);
-    rc = launch_apply<E, false, false, SRC_SCANNED, MODE, W>(
+    return launch_apply<E, false, false, SRC_SCANNED, decltype(mode)::value, W>(
         as.q, as.k, as.v, as.s, need_states ? state_slice(as.seg_states, g, i) : nullptr, as.kv_in, nullptr, as.o,
         slice_geom(g, i), st);
-  }
+  };
+  rc = sweep(std::integral_constant<int, MODE>(), 0);
+  if constexpr (MODE == M_NARROW && W == kMaxWidth)
+    for (int i = 1; i < slices && !rc; ++i) rc = sweep(std::integral_constant<int, M_ADDING>(), i);
   return rc;
 }
 
@@ -1391,7 +1898,9 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
   int rc = 0;
   const int slices = (int)slices_of(g);
   if (g.fused) {
-    for (int i = 0; i < slices && !rc; ++i) rc = launch_fused_bwd<E, MODE, W>(slice_args(a, g, i), slice_geom(g, i), st);
+    rc = launch_fused_bwd<E, MODE, W>(slice_args(a, g, 0), slice_geom(g, 0), st);
+    if constexpr (MODE == M_NARROW && W == kMaxWidth)
+      for (int i = 1; i < slices && !rc; ++i) rc = launch_fused_bwd<E, M_ADDING, W>(slice_args(a, g, i), slice_geom(g, i), st);
     return rc;
   }
   if constexpr (MODE != M_NARROW) if (g.combine) {
@@ -1418,9 +1927,13 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
     if ((rc = launch_segment_scan(a.ws_dkv, a.dkv_in, a.dkv_out, a.s, gp, 1, st))) return rc;
     dkv_states = a.ws_dkv;
   }
-  for (int i = 0; i < slices && !rc; ++i)
-    rc = launch_bwd3<E, SRC_SCANNED, MODE, W>(slice_args(a, g, i), state_slice(kv_states, g, i),
-                                              state_slice(dkv_states, g, i), slice_geom(g, i), st);
+  auto sweep = [&](auto mode, int i) {
+    return launch_bwd3<E, SRC_SCANNED, decltype(mode)::value, W>(slice_args(a, g, i), state_slice(kv_states, g, i),
+                                                                 state_slice(dkv_states, g, i), slice_geom(g, i), st);
+  };
+  rc = sweep(std::integral_constant<int, MODE>(), 0);
+  if constexpr (MODE == M_NARROW && W == kMaxWidth)
+    for (int i = 1; i < slices && !rc; ++i) rc = sweep(std::integral_constant<int, M_ADDING>(), i);
   return rc;
 }
 
