@@ -1750,10 +1750,16 @@ int launch_fused_fwd(const FwdArgs &a, const Geom &g, hipStream_t st) {
 
 // The backward's three workgroups per segment should fit the chip in one round (one workgroup per CU, two at W = 64), and
 // nothing ties its segments to the forward's: no states are handed over on this path.
+// All workgroups of a (b, h) run on one XCD, so from 20 (b, h) on it is the XCDs with most of them that have to have the places: bf16,
+// d = e = 128, counted over the chip and by XCD: b*h = 20, n = 1024 27.5 and 22.6 us, b*h = 25, n = 768 23.9 and 19.9, b*h = 28, n =
+// 1024 27.9 and 25.0, b*h = 42, n = 2048 61.6 and 57.8.  Fewer (b, h) have more, shorter segments, and those that wait for a place are
+// the ones without a walk: b*h = 12, n = 1024 20.1 and 20.6, b*h = 18 21.6 and 22.2.  At W = 64 the two count alike (14.7 and 15.0 at
+// worst).
+constexpr int64_t kFitByXcd = 20;
 Geom fused_bwd_geom(const Geom &g) {
   Geom gb = g;
-  const int64_t bh = (int64_t)g.b * g.h;
-  int64_t fit = (g.width == 64 ? 512 : 256) / (3 * bh);  // segments per (b, h) in one round
+  const int64_t bh = (int64_t)g.b * g.h, placed = g.width == 128 && bh >= kFitByXcd ? (bh + 7) / 8 * 8 : bh;
+  int64_t fit = (g.width == 64 ? 512 : 256) / (3 * placed);  // segments per (b, h) in one round
   if (fit < 1) fit = 1;
   if (fit < g.n_seg) {
     int64_t len = (g.n + fit - 1) / fit;
