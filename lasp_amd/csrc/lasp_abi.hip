@@ -771,10 +771,15 @@ static int bwd_twin(const void *q, const void *k, const void *v, const float *s,
     return rc;
   if ((rc = check_device(me, q))) return rc;
   (void)hipGetLastError();  // an earlier, unrelated error of this thread is not this call's
+  bool planned = seg_len == 0;
+  if (!planned && g.width) {  // (callers pass the forward's seg_len on)
+    Geom own;
+    planned = make_geom(b, h, n, d, e, dtype, 0, &own) == 0 && !own.fused && own.seg_len == g.seg_len;
+  }
   BwdArgs a{q,  k,  v,       s,
             d_o, kv_in, dkv_in, dq,
             dk, dv, dkv_out, kv_seg_states,
-            nullptr, nullptr};
+            nullptr, nullptr, planned};
   float *wp = workspace;
   if (need_dkv) {
     a.ws_dkv = wp;

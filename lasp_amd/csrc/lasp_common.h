@@ -123,6 +123,7 @@ struct BwdArgs {
   const float *kv_seg_states;  // may be NULL
   float *ws_kv;                // used when kv_seg_states is NULL
   float *ws_dkv;
+  bool planned;                // seg_len is the one that the default plan has
 };
 
 int generic_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st);

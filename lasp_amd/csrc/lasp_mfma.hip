@@ -1899,11 +1899,34 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
   return rc;
 }
 
+// Chunks whose forward takes pre-pass, scan and sweep run their backward in one launch all the same where that is faster: it reads q
+// and dO once less, passes no states through memory, and three workgroups per segment fill the chip with a third of the segments,
+// so that little is walked twice.  Its time goes with the chunk's length, as a workgroup walks and sweeps all of it, that of the
+// three kernels with n b h: the line is n = 88 b*h.  bf16, d = e = 128, backward with states, three kernels and one launch, in us:
+// b*h = 16, n = 1536 32.4 and 28.1, n = 2560 39.6 and 41.8; b*h = 24, n = 2048 44.6 and 40.1, n = 3072 55.0 and 56.9; b*h = 36,
+// n = 2048 65.4 and 46.4, n = 3072 82.2 and 70.2; b*h = 60, n = 2048 90.2 and 68.2, n = 4096 146 and 123; b*h = 160, n = 3072 268 and
+// 227; without decay b*h = 24, n = 2048 46.2 and 40.9; d = e = 96: b*h = 36, n = 2500 62.2 and 52.3.  At the longest chunks of the rule
+// b*h = 80 still gains (n = 6144: 262 and 237), b*h = 128 no longer (396 both).  Heads of up to 64 features do not (b*h = 24, n = 2048:
+// 23.1 and 29.1).
+// Only with the segments that the library plans by itself (others are asked for to get the three kernels), and not where the
+// outgoing state lies over an incoming one: nothing orders the workgroup that writes it and those that read the other.
+constexpr int64_t kWholeBwdPerHead = 88, kWholeBwdMax = 6144;
+bool whole_bwd(const BwdArgs &a, const Geom &g) {
+  const int64_t bh = (int64_t)g.b * g.h;
+  if (!a.planned || g.width != kMaxWidth || g.dt > kMaxWidth || g.n > kWholeBwdMax || g.n > kWholeBwdPerHead * bh) return false;
+  const size_t bytes = sizeof(float) * (size_t)bh * g.dt * g.e;
+  auto apart = [&](const float *in, const float *out) {
+    const uintptr_t i = (uintptr_t)in, o = (uintptr_t)out;
+    return !in || !out || i + bytes <= o || o + bytes <= i;
+  };
+  return apart(a.dkv_in, a.dkv_out) && apart(a.kv_in, a.dkv_out) && apart(a.kv_in, g.twin);
+}
+
 template <class E, int MODE, int W>
 int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
   int rc = 0;
   const int slices = (int)slices_of(g);
-  if (g.fused) {
+  if (g.fused || whole_bwd(a, g)) {
     rc = launch_fused_bwd<E, MODE, W>(slice_args(a, g, 0), slice_geom(g, 0), st);
     if constexpr (MODE == M_NARROW && W == kMaxWidth)
       for (int i = 1; i < slices && !rc; ++i) rc = launch_fused_bwd<E, M_ADDING, W>(slice_args(a, g, i), slice_geom(g, i), st);
