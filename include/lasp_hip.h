@@ -201,9 +201,11 @@ int lasp_chunk_fwd_static(const void *q, const void *k, const void *v, const flo
  * (lasp/lasp_fuse.py:352-353) under the same rule as kv_out / kv_in in the forward.
  * kv_seg_states: the array lasp_chunk_fwd left in `seg_states` for the same
  * inputs, seg_len and kv_in, or NULL to recompute it (then `workspace` must
- * hold 2 * state_bytes, else 1 * state_bytes).  kv_in is passed in either case: where the
- * 16-bit kernels run a medium chunk's backward in one launch (default seg_len, dkv_out apart from
- * kv_in and dkv_in), they walk from it and leave the states and the workspace alone.
+ * hold 2 * state_bytes, else 1 * state_bytes).  Given the states of more than four segments, or of rows
+ * narrower than the 64 or 128 features that a kernel works on, the 16-bit kernels take the state that entered the
+ * chunk from them: kv_in must be passed as in the forward, but its memory may have been written since.
+ * (Other plans read kv_in.)  The 16-bit kernels may run a chunk of a few thousand tokens in one launch here
+ * too, which leaves the workspace alone; results agree to rounding.
  */
 int lasp_chunk_bwd(const void *q, const void *k, const void *v, const float *s,
                    const void *d_o, const float *kv_in, const float *dkv_in,

@@ -62,6 +62,10 @@ __host__ __device__ inline int quotient(int n, Divisor d) {
   return (int)(((uint32_t)(((uint64_t)(uint32_t)n * d.mul) >> 32) + (uint32_t)n) >> d.shift);
 }
 
+// The incoming state that dQ starts from in a backward of one launch: the chunk's kv_in; the states that the forward's scan left,
+// for a call with a kv_in, or without (where a head outside the scan has parked none, see state_dies_in_segment).
+enum Kept { KEPT_NONE = 0, KEPT_STATES = 1, KEPT_STATES_ONLY = 2 };
+
 // One chunk's geometry, passed by value to every kernel.
 struct Geom {
   int b, h;
@@ -80,6 +84,7 @@ struct Geom {
                 // segments are cut finer for the pre-pass (16-bit scan path only)
   Divisor by_seg, by_h;  // n_seg and h
   int pre_n;    // ceil(n / pre_len): states per (b, h) in the workspace
+  int kept;     // a backward in one launch: what its kv_in is, see Kept
   float *twin;  // where an outgoing state is written a second time (NULL: nowhere): the copy that a caller keeping the state
                 // would hand on.  A copy of its own is a launch of 3.6 us for 24 states (4.6 for 16 beside long sweeps)
                 // and its host call; eight chained chunks of 2048 tokens, b*h = 24: 675 us, 651 without them

@@ -187,7 +187,8 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
 //   segment (follow it, going backwards) and only updating the state: no X tile, no score, no
 //   output.  The walk starts from `carry_in`, or from zero as many blocks back as the head's decay
 //   reaches (weights below 2^-SKIP_LOG2 are dropped).  One launch then does a whole chunk; the
-//   repeated walks make it a tool for short chunks.
+//   repeated walks make it a tool for short chunks.  In the 128-wide dQ sweep `carry_in` may be the states that
+//   the forward's scan left (g.kept): it then starts from the one among them that entered the chunk.
 // In the last two the workgroup of the segment visited last writes the state it ends with to
 // `carry_out` (non-transposed roles only).
 // ------------------------------------------------------------------------------
@@ -714,6 +715,7 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
            float *__restrict__ carry_out = nullptr) {
   constexpr bool RAGGED = MODE != M_ALIGNED, NARROW = MODE >= M_NARROW;
   constexpr bool LEAVES_STATE = SRC != SRC_SCANNED;  // the sweep's final state is the chunk's outgoing one
+  constexpr bool MAY_BE_KEPT = SRC == SRC_WALK && !REV && TRANS;  // dQ, see Geom::kept
   using L = SweepLds;
   constexpr int W = 128;
   const int tid = threadIdx.x;
@@ -746,10 +748,12 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
   // update the state.
   int runup = 0;
   bool take_carry = false;
+  float slope = 0.f;
   if (SRC == SRC_WALK) {
     const int avail = REV ? total_blk - (seg_blk0 + nblk) : seg_blk0;
     int reach = avail;
-    const float sl = S[head] * LOG2E;
+    slope = S[head];
+    const float sl = slope * LOG2E;
     if (sl > 0.f) {
       const float x = SKIP_LOG2 / (sl * (float)BLK);  // blocks over which a weight falls to 2^-SKIP_LOG2
       if (x < (float)avail) reach = (int)x + 1;
@@ -959,7 +963,17 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
     add_state_ld(carry_in + (int64_t)sw.bh * g.dt * g.e, NARROW ? (TRANS ? fa : fb) : W, 0.f, NARROW, true);
   };
   if (SRC == SRC_WALK) {
-    if (take_carry) add_carry();
+    const float *src = carry_in + (int64_t)sw.bh * g.dt * g.e;
+    int ld = NARROW ? (TRANS ? fa : fb) : W;
+    if (MAY_BE_KEPT && g.kept) {
+      // the state that entered the chunk lies in the slot of the first piece, or of the last one for a head outside the scan (see below).
+      // (By the slope at hand: asked for again it would have to arrive before these loads could leave.)
+      const bool parked = state_dies_in_segment(slope, g);
+      if (parked && g.kept == KEPT_STATES_ONLY) take_carry = false;
+      src = carry_in + ((int64_t)sw.bh * g.pre_n + (parked ? g.pre_n - 1 : 0)) * (W * W);
+      ld = W;
+    }
+    if (take_carry) add_state_ld(src, ld, 0.f, NARROW, true);
   } else if (SRC == SRC_SCANNED) {
     if (states) {
       // the scanned state of this segment, or for a head the scan leaves out (state_dies_in_segment), whose
@@ -1358,7 +1372,8 @@ struct Fine {
   Divisor by_seg;
 };
 
-// roles as in la_bwd3 (the dV role leaves dKV_out); all roles and segments of one (b, h) on one XCD
+// roles as in la_bwd3 (the dV role leaves dKV_out); all roles and segments of one (b, h) on one XCD.  With g.kept set, kv_in holds the
+// scanned states that the forward left, of which dQ takes the one that entered the chunk
 template <class E, int MODE, int W>
 __global__ void __launch_bounds__(WS_THREADS, ws_waves_per_simd(W))
 la_fused_bwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const elem16_t *__restrict__ V,
@@ -1926,11 +1941,23 @@ template <class E, int MODE, int W>
 int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
   int rc = 0;
   const int slices = (int)slices_of(g);
-  if (g.fused || whole_bwd(a, g)) {
+  if (g.fused) {
     rc = launch_fused_bwd<E, MODE, W>(slice_args(a, g, 0), slice_geom(g, 0), st);
     if constexpr (MODE == M_NARROW && W == kMaxWidth)
       for (int i = 1; i < slices && !rc; ++i) rc = launch_fused_bwd<E, M_ADDING, W>(slice_args(a, g, i), slice_geom(g, i), st);
     return rc;
+  }
+  if (whole_bwd(a, g)) {
+    // Kept states say what entered the chunk, whatever kv_in's memory holds by now (gathered ones do not: there kv_in is read, as
+    // their sweeps do).  They come in kv_in's place: a pointer of their own among the kernel's arguments, read before the state can
+    // be, took the launch at b*h = 16, n = 1024 from 19.4 to 19.9 us.
+    BwdArgs aw = a;
+    Geom gw = slice_geom(g, 0);
+    if (a.kv_seg_states && !g.combine) {
+      gw.kept = a.kv_in ? KEPT_STATES : KEPT_STATES_ONLY;
+      aw.kv_in = a.kv_seg_states;
+    }
+    return launch_fused_bwd<E, MODE, W>(aw, gw, st);
   }
   if constexpr (MODE != M_NARROW) if (g.combine) {
     const float *kv_states = a.kv_seg_states;
