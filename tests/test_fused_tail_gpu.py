@@ -1,7 +1,5 @@
 """Short chunks whose (b, h) fill more than one round of the chip in the backward: the (b, h) of the last, partly filled round
 are cut into segments, the others run whole.  Every (b, h) against the oracle in 64 bits."""
-import statistics
-
 import pytest
 import torch
 
@@ -57,4 +55,7 @@ def test_a_last_round_is_cut_only_where_that_pays(gpu_device):
             stop.record()
             stop.synchronize()
             times[bh].append(start.elapsed_time(stop))
-    assert statistics.median(times[240]) < statistics.median(times[256])
+    # The fastest of each, not the medians: some cards lower their clock a few bursts into this test, from where on both take the same
+    # time (first bursts 0.59 and 0.63 ms, third 0.80 and 0.79, medians 0.646 and 0.646).  Cut too finely, 240 (b, h) took 1.11 times
+    # what they take (n = 1024: 63.9 us and 57.4), more than the 0.93 that lie between the two here.
+    assert min(times[240]) < min(times[256])
