@@ -1790,15 +1790,17 @@ Geom fused_bwd_geom(const Geom &g) {
 // long as a full one.  Their (b, h) are cut into as many segments as fill the places that are left: walks over the blocks before
 // a segment cost less than half of sweeping them.  Backward kernel, bf16, uncut and cut.  d = e = 128: n = 512, b*h = 88: 35.4 and
 // 25.2 us, 96: 35.3 and 28.9, 120 (two segments only): 35.8 and 33.0, 172: 53.0 and 43.9; n = 1024, b*h = 96: 67.8 and 51.6, 120:
-// 70.8 and 69.6; never slower over b*h = 88 ... 512, n = 64 ... 1536.  d = e = 64: the places count one workgroup per CU, not
+// 70.8 and 69.6; never slower over b*h = 88 ... 512, n = 64 ... 1536.  At W = 128 the places are counted by XCD (see fused_bwd_geom):
+// 81 to 85 (b, h) overflow one of them, though 3 b*h <= 256 (b*h = 84: n = 512 uncut 34.9, cut 26.9; n = 2048 127 and 88), as 169 and
+// 170 do with two rounds (n = 2048: 198 and 178).  d = e = 64: the places count one workgroup per CU, not
 // two: a last round of at most 256 has the CUs to itself and runs at up to twice the pace of a full one, which is all that cutting
 // it further can win (n = 1024: b*h = 171 uncut 50.2, cut for one per CU 38.5, for two 40.6; 200: 52.6, 50.4 and 51.1; 216, left
 // uncut with one per CU: 53.8 and 57.1; 240: 58.3 and 63.9).
 Fine fused_bwd_tail(const Geom &g) {
-  const int64_t bh = (int64_t)g.b * g.h, slots = g.width == 64 ? 512 : 256;
+  const int64_t bh = (int64_t)g.b * g.h, slots = g.width == 64 ? 512 : 256, placed = g.width == 64 ? bh : (bh + 7) / 8 * 8;
   Fine f = {(int)((bh + 7) / 8 * 8), g.seg_len, g.n_seg, g.by_seg};  // nothing is cut
-  if (g.n_seg > 1 || 3 * bh <= slots) return f;
-  const int64_t whole = 3 * bh / slots * slots;  // workgroups in whole rounds
+  if (g.n_seg > 1 || 3 * placed <= slots) return f;
+  const int64_t whole = 3 * placed / slots * slots;  // workgroups in whole rounds
   const int64_t bh0 = whole / 24 * 8;            // whole groups of 8
   const int64_t rest = (bh - bh0 + 7) / 8 * 8, room = 256 + (g.width == 64 ? 0 : whole - 3 * bh0);
   const int64_t nblk = (g.n + BLK - 1) / BLK;
@@ -1917,19 +1919,47 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
 // Chunks whose forward takes pre-pass, scan and sweep run their backward in one launch all the same where that is faster: it reads q
 // and dO once less, passes no states through memory, and three workgroups per segment fill the chip with a third of the segments,
 // so that little is walked twice.  Its time goes with the chunk's length, as a workgroup walks and sweeps all of it, that of the
-// three kernels with n b h: the line is n = 88 b*h.  bf16, d = e = 128, backward with states, three kernels and one launch, in us:
-// b*h = 16, n = 1536 32.4 and 28.1, n = 2560 39.6 and 41.8; b*h = 24, n = 2048 44.6 and 40.1, n = 3072 55.0 and 56.9; b*h = 36,
-// n = 2048 65.4 and 46.4, n = 3072 82.2 and 70.2; b*h = 60, n = 2048 90.2 and 68.2, n = 4096 146 and 123; b*h = 160, n = 3072 268 and
-// 227; without decay b*h = 24, n = 2048 46.2 and 40.9; d = e = 96: b*h = 36, n = 2500 62.2 and 52.3.  At the longest chunks of the rule
-// b*h = 80 still gains (n = 6144: 262 and 237), b*h = 128 no longer (396 both).  Heads of up to 64 features do not (b*h = 24, n = 2048:
-// 23.1 and 29.1).
-// Only with the segments that the library plans by itself (others are asked for to get the three kernels), and not where the
+// three kernels with n b h: no chunk beyond n = 88 b*h.  Up to there, bf16, backward with states, three kernels and one launch in us:
+//   Whole rows, all (b, h) in one round (up to 80): always.  b*h = 24, n = 2048 40.9 and 35.1, n = 2112 42 and 37; b*h = 36, n = 2048
+// 59.0 and 42.3; b*h = 48, n = 4224 118 and 111 (the nearest); b*h = 60, n = 4096 131 and 119; b*h = 80, n = 6144 247 and 234.
+//   Whole rows, more rounds than one: the three kernels come down to few, well-filled rounds too, above all where they gather four
+// segments or fewer.  Up to 4096 tokens the one launch is at worst even (b*h = 104: 216 and 217) and as a rule faster (b*h = 88,
+// n = 3072 154 and 149, b*h = 112, n = 4096 239 and 227, b*h = 160, n = 3072 257 and 222); beyond, it is where they scan and b*h > 128
+// (b*h = 144, n = 6144 449 and 425, b*h = 192, n = 5003 500 and 479), and elsewhere it may lose what it wins (b*h = 128, n = 4608 296
+// and 305, n = 6144 386 and 400, b*h = 192, n = 4608 423 and 441, b*h = 168, n = 5632 443 and 454, but b*h = 144, n = 4608 348 and 322,
+// b*h = 256 573 and 547).  81 to 85 (b, h) are one round of three segments for the three kernels and one and a half here: up to
+// 2304 tokens (b*h = 84, n = 2048 100 and 86; b*h = 82 99 and 99, n = 4096 172 and 181).
+//   Narrow rows, whose three kernels scan whatever the number of segments: with more rounds than one always (d = e = 96, b*h = 128,
+// n = 3072 185 and 160, b*h = 84, n = 4096 154 and 133); with one, by the blocks that a workgroup of either form goes through in a row --
+// one launch a segment and the longest walk before it, at 0.35 of a block swept, the three kernels their rounds of segments, three
+// blocks more for each start, and pre-pass and scan.  Fitted over 631 shapes, four widths (b*h = 18 ... 80, n = 1100 ... 6144), 4 %
+// off at one deviation.  d = 128, e = 64: b*h = 24, n = 2048 40.1 and 38.5; b*h = 28, n = 2464 45 and 47; b*h = 44, n = 3872 91 and 96;
+// b*h = 60, n = 4096 132 and 102.
+// Of 1034 measured shapes 831 take one launch, the slowest beside its three kernels at 1.024.  Heads of up to 64 features stay (b*h = 24,
+// n = 2048: 23.1 and 29.1).
+// Only with the segments of the library's own plan (others are asked for to get the three kernels), and not where the
 // outgoing state lies over an incoming one: nothing orders the workgroup that writes it and those that read the other.
 constexpr int64_t kWholeBwdPerHead = 88, kWholeBwdMax = 6144;
+constexpr int64_t kWholeBwdRounds = 4096, kWholeBwdOverXcd = 2304, kWholeBwdMany = 128;
+bool whole_bwd_pays(const Geom &g) {
+  const int64_t bh = (int64_t)g.b * g.h, placed = (bh + 7) / 8 * 8;
+  if (g.n > kWholeBwdMax || g.n > kWholeBwdPerHead * bh) return false;
+  const bool one_round = 3 * placed <= 256;
+  if (g.dt == kMaxWidth && g.e == kMaxWidth) {
+    if (one_round) return true;
+    if (3 * bh <= 256) return g.n <= kWholeBwdOverXcd;
+    return g.n <= kWholeBwdRounds || (bh > kWholeBwdMany && !g.combine);
+  }
+  if (!one_round) return true;
+  const Geom gb = fused_bwd_geom(g);
+  const double len = gb.seg_len / BLK, walk = (gb.n_seg - 1) * len, blocks = (double)((g.n + BLK - 1) / BLK);
+  const double rounds = (double)((3 * bh * g.n_seg + 255) / 256);
+  const double three = rounds * (g.seg_len / BLK + 3) + (double)(bh * g.n_seg) / 13 + (double)bh * blocks / 116;
+  return 1.44 * (len + 0.35 * walk) + 6 < three;
+}
 bool whole_bwd(const BwdArgs &a, const Geom &g) {
-  const int64_t bh = (int64_t)g.b * g.h;
-  if (!a.planned || g.width != kMaxWidth || g.dt > kMaxWidth || g.n > kWholeBwdMax || g.n > kWholeBwdPerHead * bh) return false;
-  const size_t bytes = sizeof(float) * (size_t)bh * g.dt * g.e;
+  if (!a.planned || g.width != kMaxWidth || g.dt > kMaxWidth || !whole_bwd_pays(g)) return false;
+  const size_t bytes = sizeof(float) * (size_t)g.b * g.h * g.dt * g.e;
   auto apart = [&](const float *in, const float *out) {
     const uintptr_t i = (uintptr_t)in, o = (uintptr_t)out;
     return !in || !out || i + bytes <= o || o + bytes <= i;
