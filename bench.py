@@ -12,7 +12,8 @@ Prints ONE JSON line (metric = fwd+bwd tokens/s) that also carries
                   bytes per launch / its mean launch duration (HIP events around
                   every launch, on the launch stream); roofline_fwd: the same for la_apply.
                   `traffic` is read from the rocprofv3 counter summary under profiles/
-                  and is null when that summary was taken with another segment plan.
+                  and is null when that summary was taken with another segment plan or another
+                  state of the kernels' source.
   cpu_baseline -- the CPU oracle (fp32 torch port of the same recurrence) timed on
                   the host cores on a bounded number of passes of the same workload.
   other_configs -- forward+backward times of the other benchmark configurations
@@ -32,6 +33,7 @@ job sits in the settled regime, so that is what the timed steps measure; `settle
 recorded in the output, and --settle-ms 0 shows the transient.
 """
 import argparse
+import hashlib
 import json
 import os
 import re
@@ -71,25 +73,36 @@ def device_inputs(dev, b, h, n, d, dtype, seed, scale):
     return [(torch.randn(b, h, n, d, generator=g, device=dev) * scale).to(dtype) for _ in range(4)]
 
 
+def kernel_code():
+    """A short hash of the sweep kernels' source without its comments."""
+    code = hashlib.sha256()
+    for name in ("lasp_common.h", "lasp_mfma.hip"):
+        with open(os.path.join(ROOT, "lasp_amd", "csrc", name)) as f:
+            code.update("".join(re.sub(r"//.*", "", f.read()).split()).encode())
+    return code.hexdigest()[:16]
+
+
 def read_traffic_profile(path=HBM_PROFILE):
     """HBM bytes per launch from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary.
 
-    The file states the segment plan it was taken with (`plan: seg_len=.. n_seg=..`), the scale factor of
-    each counter (from a plain device copy of known size) and one `traffic <kernel> fetch_kib=.. write_kib=..`
-    line per kernel.  Returns {"seg_len", "n_seg", "kernels": {name: bytes}} or None if there is no such file."""
+    The file states the segment plan it was taken with (`plan: seg_len=.. n_seg=..`), the kernels' source (`code: ..`, see
+    kernel_code), the scale factor of each counter (from a plain device copy of known size) and one
+    `traffic <kernel> fetch_kib=.. write_kib=..` line per kernel.  Returns {"seg_len", "n_seg", "code", "kernels": {name: bytes}}
+    or None if there is no such file."""
     try:
         text = open(path).read()
     except OSError:
         return None
     plan = re.search(r"plan:\s*seg_len=(\d+)\s+n_seg=(\d+)", text)
     scale = re.search(r"scale:\s*fetch=([0-9.]+)\s+write=([0-9.]+)", text)
-    if not plan or not scale:
+    code = re.search(r"^code:\s*(\w+)", text, flags=re.M)
+    if not plan or not scale or not code:
         return None
     f_scale, w_scale = float(scale.group(1)), float(scale.group(2))
     kernels = {}
     for m in re.finditer(r"^traffic\s+(\S+)\s+fetch_kib=([0-9.]+)\s+write_kib=([0-9.]+)", text, flags=re.M):
         kernels[m.group(1)] = int((float(m.group(2)) * f_scale + float(m.group(3)) * w_scale) * 1024)
-    return {"seg_len": int(plan.group(1)), "n_seg": int(plan.group(2)), "kernels": kernels}
+    return {"seg_len": int(plan.group(1)), "n_seg": int(plan.group(2)), "code": code.group(1), "kernels": kernels}
 
 
 CEILING_PROFILE = os.path.join(ROOT, "profiles", "stream_probe_hbm_ceiling.txt")
@@ -507,7 +520,7 @@ def main():
     kernel_sum_ms = sum(ms for ms, cnt in prof.values()) / args.steps
 
     profile = read_traffic_profile()
-    same_plan = profile is not None and (profile["seg_len"], profile["n_seg"]) == (seg_len, n_seg)
+    same_plan = profile is not None and (profile["seg_len"], profile["n_seg"], profile["code"]) == (seg_len, n_seg, kernel_code())
 
     ceilings = read_ceiling_profile()
 

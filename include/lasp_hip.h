@@ -91,7 +91,9 @@ extern "C" {
                                per direction; NO workspace is read or written (seg_states,
                                kv_seg_states and workspace may be NULL and are ignored) and the forward
                                leaves no segment states behind.  An explicit seg_len selects
-                               LASP_PATH_MFMA instead. */
+                               LASP_PATH_MFMA instead.  (On LASP_PATH_MFMA too a backward may be one
+                               launch, of chunks up to 6144 tokens with the plan's segments, given or
+                               not: workspaces and states are asked for and used as described below.) */
 
 int lasp_abi_version(void);
 
@@ -130,7 +132,9 @@ int lasp_kernel_path(int b, int h, int64_t n, int d, int e, int dtype);
  * there it is 1.  Where the sweeps themselves combine the states (LASP_PATH_MFMA_FUSED, and chunks
  * of at most 4 segments on the 16-bit kernels) several workgroups read the incoming state and
  * another one writes the outgoing state when it is done, with nothing ordering the two: it is 0
- * unless a single workgroup does both (forward with one segment).  The reference updates in place
+ * unless a single workgroup does both (forward with one segment).  A forward in place leaves KV_out where
+ * kv_in was: its backward may still be given that buffer as kv_in where it is given the segment states of more
+ * than four segments (see lasp_chunk_bwd), else it needs a copy of the incoming state.  The reference updates in place
  * (lasp/lasp_fuse.py:126-127,352-353); a caller that wants that where this returns 0 passes a
  * copy of the incoming state as kv_in / dkv_in.
  */

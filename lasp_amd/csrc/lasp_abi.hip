@@ -68,7 +68,7 @@ constexpr int kPreMaxSeg = 2304;        // longest segment the pre-pass walks in
                                         // are still cut in 2, 4, ... and not in twice as many pieces
 
 // The 16-bit MFMA kernels work on 128 features, or 64 where neither d nor e is larger, and read narrower rows
-// zero-extended (wider ones in slices of 128); their 8-byte loads and 16-byte stores need every row to start on such
+// zero-extended (wider ones in slices of 128); their 16-byte loads and stores need every row to start on such
 // a boundary.
 bool mfma_eligible(int d, int e, int dtype) {
   return (dtype == LASP_DTYPE_BF16 || dtype == LASP_DTYPE_F16) && d % 8 == 0 && e % 8 == 0;
@@ -156,12 +156,12 @@ int default_seg_len(int b, int h, int64_t n, bool narrow64) {
 // Short chunks given to the library with the default plan run as ONE launch per direction: every
 // workgroup rebuilds the state entering its segment by walking the blocks before it, which saves
 // the pre-pass, its launch and the workspace.  The walk is serial work on the critical path (0.7 us
-// per 64-token block: the math waves multiply a block into the state while the feed waves fetch and
-// transpose the next one), and the single launch wins up to walks of about 16 blocks.  Forward +
+// per 64-token block: the math waves multiply a block into the state while the feed waves fetch those
+// to come), and the single launch wins up to walks of about 16 blocks.  Forward +
 // backward replayed from a graph over rotating inputs, scan path against single launch: b*h = 24:
 // n = 512 44 / 33 us, 768 48 / 40, 1024 59 / 46, 1536 70 / 69, 2048 81 / 87; b*h = 128, n = 1024:
-// 172 / 133; b*h = 16, n = 2048: 66 / 76; b*h = 4, n = 2048: 45 / 70.  An explicit seg_len always
-// selects the pre-pass / sweep kernels.
+// 172 / 133; b*h = 16, n = 2048: 66 / 76; b*h = 4, n = 2048: 45 / 70 (on sweeps before the present ones).  An explicit
+// seg_len always selects the pre-pass / sweep kernels (the backward of a planned length may be one launch all the same, see whole_bwd).
 constexpr int64_t kFusedMaxTokens = 2048;
 constexpr int kFusedMaxWalk = 16;  // blocks
 // With few segments the 16-bit sweeps of full-width heads gather the segments' own states themselves
@@ -388,7 +388,7 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   return 0;
 }
 
-// The kernels fetch rows of q/k/v/do with 8-byte loads and store o/dq/dk/dv with 16-byte stores,
+// The kernels fetch rows of q/k/v/do with 8- and 16-byte loads and store o/dq/dk/dv with 16-byte stores,
 // and read states as floats: tensors must start on a 16-byte boundary, states on a 4-byte one.
 int check_aligned(const char *call, const char *name, const void *p, size_t align) {
   if (p && ((uintptr_t)p % align) != 0) {

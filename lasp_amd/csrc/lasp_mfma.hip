@@ -695,17 +695,22 @@ __device__ __forceinline__ void wait_loads() {
 // Every tile lies token-major, as in memory: what contracts over tokens is read transposed (ds_read_b64_tr_b16), the state update's
 // decay goes to the 32 columns of Z that only one wave reads, and no wave moves a tile through its registers.
 //
-// What bounds a block.  The issue of the math waves' instructions, some 300 on the vector unit (about 4.4 cycles each behind one
-// another), 38 products (9) and 70 LDS accesses; then the LDS, which moves some 330 KB a block.  So the vector work is dealt out
+// What bounds a block.  The issue of the math waves' instructions, some 300 on the vector unit, 38 products and 70 LDS accesses
+// in each; then the LDS, which moves some 330 KB a block, counted access by access.  So the vector work is dealt out
 // between the products by hand (see `slot`), reads are asked for a phase ahead, and what a block's first reads would wait for is
 // covered by products held back from the block before.  Neither stores nor loads to registers stand in the math waves: behind the feed waves' loads
-// each of them waits its turn in the memory pipeline (with the outputs stored from there, the state term took 2660 cycles at
-// n = 65536 instead of 700; so does any register spilled to scratch).
-//   Cycles a block, alone on a CU: 3200 (4250 with tiles that went through registers, transposed on the way, and the state update
-// and both halves of the output between the same two barriers).  Sweep kernels in us, that form and this one: b*h = 16, n = 65536:
-// forward 193 and 196, backward 507 and 460 (HBM: 2.7 GB); n = 16384 in 256 segments: 48 and 46, 136 and 113; b*h = 36, n = 5003:
-// 34.8 and 32.4, 97 and 84.6; b*h = 24, n = 2048, 7 segments: 14.6 and 13.4, 30.4 and 27.7; two slices of d = 256, b*h = 8,
+// each of them waits its turn in the memory pipeline (and so does any register spilled to scratch).
+//   Cycles a block, alone on a CU: 3100 (4130 with tiles that went through registers, transposed on the way, and the state update
+// and both halves of the output between the same two barriers); LDS busy for 1410 of them (1860), 180 in conflicts (240).  Sweep
+// kernels in us, that form and this one, one after the other on one card: b*h = 16, n = 65536: forward 194.3 and 195.7 (0.7 % lost),
+// backward 481 and 437 (the forward moves its bytes at 5.6 TB/s either way; of the backward's 2.69 GB beyond L2 the
+// memory-side cache serves a part); n = 16384 in 256 segments: 48 and 46, 136 and 113; b*h = 36,
+// n = 5003: 34.8 and 32.4, 97 and 84.6; b*h = 24, n = 2048, 7 segments: 14.6 and 13.4, 30.4 and 27.7; two slices of d = 256, b*h = 8,
 // n = 8192: 40 and 34, 97 and 82.
+//   Rows of X and Y of at most 64 features (d = 128, e = 64 backwards) have two of four state tiles of zeros, which that form left out
+// and this one multiplies: a branch there would cut the hand-made order.  Whole calls, forward and backward, b*h = 16, n = 65536:
+// d = 128, e = 64 188 and 188, 451 and 391; 64 x 128 187 and 189, 435 and 378; b*h = 24, n = 2048, 128 x 64 27.7 and 25.9,
+// 40.0 and 36.5.
 // ------------------------------------------------------------------------------
 template <class E, bool REV, bool TRANS, int SRC, int MODE>
 __device__ __forceinline__ void
@@ -1937,6 +1942,9 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
 // b*h = 60, n = 4096 132 and 102.
 // Of 1034 measured shapes 831 take one launch, the slowest beside its three kernels at 1.024.  Heads of up to 64 features stay (b*h = 24,
 // n = 2048: 23.1 and 29.1).
+// DKV_out is summed over the whole chunk in one accumulator of 32 bits: without decay, b*h = 24, n = 2048, it is 2.9e-7 off (2-norm, against
+// 64 bits) where sums of segments are 1.0e-7, at n = 6144, b*h = 80, 5.0e-7 and 4.3e-7; as chunks of that length are in one launch
+// of either direction.  With decay it is 1.6e-3 off either way (bf16), the rounding of its decayed operand, and no other output differs.
 // Only with the segments of the library's own plan (others are asked for to get the three kernels), and not where the
 // outgoing state lies over an incoming one: nothing orders the workgroup that writes it and those that read the other.
 constexpr int64_t kWholeBwdPerHead = 88, kWholeBwdMax = 6144;

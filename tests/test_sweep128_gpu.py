@@ -27,8 +27,8 @@ def test_few_blocks(gpu_device, n, seg, d, e, dtype):
         return dict(o=o, kv_out=kvo.clone(), dq=dq, dk=dk, dv=dv, dkv_out=dkvo.clone())
 
     got = run()
-    # the bound of every 16-bit parity test: a few roundings of 2^-9 (2^-12 in fp16), of the products' operands and the output
-    check(got, oracle(inp, s), 2e-2, what=f"n={n} seg={seg} d={d} e={e} {dtype}")
+    # the bound of every 16-bit parity test: a few roundings of 2^-9, of the products' operands and the output; in fp16 of an eighth each
+    check(got, oracle(inp, s), 2e-2 if dtype == torch.bfloat16 else 2e-2 / 8, what=f"n={n} seg={seg} d={d} e={e} {dtype}")
     for _ in range(3):  # no sum depends on which wave comes first
         for name, x in run().items():
             assert torch.equal(x, got[name]), name
