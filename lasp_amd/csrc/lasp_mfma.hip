@@ -1933,7 +1933,7 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
 // (b*h = 144, n = 6144 449 and 425, b*h = 192, n = 5003 500 and 479), and elsewhere it may lose what it wins (b*h = 128, n = 4608 296
 // and 305, n = 6144 386 and 400, b*h = 192, n = 4608 423 and 441, b*h = 168, n = 5632 443 and 454, but b*h = 144, n = 4608 348 and 322,
 // b*h = 256 573 and 547).  81 to 85 (b, h) are one round of three segments for the three kernels and one and a half here: up to
-// 2304 tokens (b*h = 84, n = 2048 100 and 86; b*h = 82 99 and 99, n = 4096 172 and 181).
+// 2560 tokens (b*h = 84 120 and 103; b*h = 82 118 and 120, n = 3072 135 and 141).
 //   Narrow rows, whose three kernels scan whatever the number of segments: with more rounds than one always (d = e = 96, b*h = 128,
 // n = 3072 185 and 160, b*h = 84, n = 4096 154 and 133); with one, by the blocks that a workgroup of either form goes through in a row --
 // one launch a segment and the longest walk before it, at 0.35 of a block swept, the three kernels their rounds of segments, three
@@ -1948,7 +1948,7 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
 // Only with the segments of the library's own plan (others are asked for to get the three kernels), and not where the
 // outgoing state lies over an incoming one: nothing orders the workgroup that writes it and those that read the other.
 constexpr int64_t kWholeBwdPerHead = 88, kWholeBwdMax = 6144;
-constexpr int64_t kWholeBwdRounds = 4096, kWholeBwdOverXcd = 2304, kWholeBwdMany = 128;
+constexpr int64_t kWholeBwdRounds = 4096, kWholeBwdOverXcd = 2560, kWholeBwdMany = 128;
 bool whole_bwd_pays(const Geom &g) {
   const int64_t bh = (int64_t)g.b * g.h, placed = (bh + 7) / 8 * 8;
   if (g.n > kWholeBwdMax || g.n > kWholeBwdPerHead * bh) return false;

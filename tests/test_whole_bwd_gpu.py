@@ -70,7 +70,7 @@ def test_matches_oracle_and_the_three_kernels(gpu_device, b, h, n, d, e, one, dt
 
 @pytest.mark.parametrize("b,h,n,d,e,one", [
     (5, 16, 6144, 128, 128, True), (5, 16, 6145, 128, 128, False),    # one round of whole rows, the longest chunk
-    (7, 12, 2304, 128, 128, True), (7, 12, 2305, 128, 128, False),    # more than an XCD has places for
+    (7, 12, 2560, 128, 128, True), (7, 12, 2561, 128, 128, False),    # more than an XCD has places for
     (8, 12, 4096, 128, 128, True), (8, 12, 4097, 128, 128, False),    # more rounds than one
     (3, 43, 5120, 128, 128, True), (8, 18, 4608, 128, 128, False),    # ... of more than 128 (b, h): scanned, gathered
     (1, 28, 1792, 128, 64, True), (1, 28, 2464, 128, 64, False),      # narrow rows, one round
