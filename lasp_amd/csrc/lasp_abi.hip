@@ -155,12 +155,12 @@ int default_seg_len(int b, int h, int64_t n, bool narrow64) {
 
 // Short chunks given to the library with the default plan run as ONE launch per direction: every
 // workgroup rebuilds the state entering its segment by walking the blocks before it, which saves
-// the pre-pass, its launch and the workspace.  The walk is serial work on the critical path (0.7 us
+// the pre-pass, its launch and the workspace.  The walk is serial work on the critical path (0.57 us
 // per 64-token block: the math waves multiply a block into the state while the feed waves fetch those
 // to come), and the single launch wins up to walks of about 16 blocks.  Forward +
 // backward replayed from a graph over rotating inputs, scan path against single launch: b*h = 24:
 // n = 512 44 / 33 us, 768 48 / 40, 1024 59 / 46, 1536 70 / 69, 2048 81 / 87; b*h = 128, n = 1024:
-// 172 / 133; b*h = 16, n = 2048: 66 / 76; b*h = 4, n = 2048: 45 / 70 (on sweeps before the present ones).  An explicit
+// 172 / 133; b*h = 16, n = 2048: 66 / 76; b*h = 4, n = 2048: 45 / 70 (on sweeps before the present ones, whose walks took 0.7).  An explicit
 // seg_len always selects the pre-pass / sweep kernels (the backward of a planned length may be one launch all the same, see whole_bwd).
 constexpr int64_t kFusedMaxTokens = 2048;
 constexpr int kFusedMaxWalk = 16;  // blocks

@@ -1127,42 +1127,6 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
   }
   __syncthreads();  // block 0 of the run visible
   int set_i = 0, k = 0;
-  for (; SRC == SRC_WALK && k < runup; ++k) {  // walk
-    const char *set = smem + set_i * L::SET;
-    set_i = set_i == 2 ? 0 : set_i + 1;
-    {
-      const int len = len_of(first_blk + k * step);
-      const float bd = RAGGED && len != BLK ? decay(sl, (float)len) : blockdec;
-      const int y_lane = fresh(y_at);
-      u32x4 zf[4], zs[4], yf[2][4][2], kd[4][2];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) zf[u] = tokens(set + L::Z, z_at, u);
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int T = 0; T < 2; ++T) yf[0][u][T] = read_y(set + L::Y, y_lane, T, u);
-      reads_first();
-#pragma unroll
-      for (int r = 0; r < 16; r += 4) decay_state(0, r, bd), decay_state(1, r, bd);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) read_kdec(u, len, kd[u]);
-      reads_first();
-#pragma unroll
-      for (int i = 0; i < 4; ++i) scale_z(zf, zs, kd[0], 0, i);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int u = j >> 1, T = j & 1;
-        slot(st[T], yf[0][u][T], zs[u], [&]() __attribute__((always_inline)) {
-          decay_state(2 + (j >> 2), 4 * (j & 3), bd);
-          if (u < 3) scale_z(zf, zs, kd[u + 1], u + 1, 2 * T), scale_z(zf, zs, kd[u + 1], u + 1, 2 * T + 1);
-          yf[1][u][T] = read_y(set + L::Y, y_lane, 2 + T, u);
-        });
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) st[2 + (j & 1)] = E::mfma(yf[1][j >> 1][j & 1], zs[j >> 1], st[2 + (j & 1)]);
-    }
-    __syncthreads();
-  }
   // What a block leaves to the next one's time: of its output, the scores' part (they are computed meanwhile), of the state
   // update, the upper half of the rows, whose products cover the time that the next block's first reads take.
   floatx16 acc[2];  // the output without that part, not yet scaled by ...
@@ -1194,6 +1158,58 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
       acc[j >> 2][r] = x;
     }
   };
+  if (SRC == SRC_WALK && runup > 0) {
+    // A walk block: the upper half of the rows of the state update of the block before, whose products cover the time that this block's
+    // first reads take, then the lower half of its own.  What bounds it is the issue of a math wave's instructions, alone on its SIMD but
+    // for a feed wave: 16 products, 40 LDS reads and 190 on the vector unit, 0.57 us a block where reads, scaling and products that
+    // followed one another took 0.69 (the loads alone would allow 0.35; scaling Z in the feed waves instead took 0.71, loads three blocks
+    // ahead instead of two 0.57).  Backwards in one launch, in us: b*h = 24, n = 2048 36.8 -> 34.5, b*h = 20, n = 1024 21.5 -> 20.7;
+    // forwards, b*h = 48, n = 1024 20.0 -> 18.5.
+    u32x4 kd[4][2], zr[4], zt[4], yf0[4][2];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) read_kdec(u, BLK, kd[u]);  // (partial only going backwards, where the tokens' decays are the same)
+    auto walk = [&](u32x4 (&before)[4], u32x4 (&now)[4]) __attribute__((always_inline)) {
+      const char *set = smem + set_i * L::SET;
+      set_i = set_i == 2 ? 0 : set_i + 1;
+      const int len = len_of(first_blk + k * step);
+      const float bd = RAGGED && len != BLK ? decay(sl, (float)len) : blockdec;
+      const int y_lane = fresh(y_at), z_lane = fresh(z_at);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) zr[u] = tokens(set + L::Z, z_lane, u);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        slot(st[2 + (j & 1)], yf1[j >> 1][j & 1], before[j >> 1], [&]() __attribute__((always_inline)) {
+          if (j < 2) zr[2 + j] = tokens(set + L::Z, z_lane, 2 + j);
+          if (j >= 2 && j < 6) {
+            yf0[j - 2][0] = read_y(set + L::Y, y_lane, 0, j - 2);
+            yf0[j - 2][1] = read_y(set + L::Y, y_lane, 1, j - 2);
+          }
+          decay_state(j >> 2, 4 * (j & 3), bd);
+          if (j >= 4) scale_z(zr, now, kd[(j - 4) >> 1], (j - 4) >> 1, 2 * (j & 1)), scale_z(zr, now, kd[(j - 4) >> 1], (j - 4) >> 1, 2 * (j & 1) + 1);
+        });
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int u = j >> 1, T = j & 1;
+        slot(st[T], yf0[u][T], now[u], [&]() __attribute__((always_inline)) {
+          if (j < 4) scale_z(zr, now, kd[2 + (j >> 1)], 2 + (j >> 1), 2 * (j & 1)), scale_z(zr, now, kd[2 + (j >> 1)], 2 + (j >> 1), 2 * (j & 1) + 1);
+          decay_state(2 + (j >> 2), 4 * (j & 3), bd);
+          yf1[u][T] = read_y(set + L::Y, y_lane, 2 + T, u);
+        });
+      }
+      __syncthreads();
+      ++k;
+    };
+    for (; k + 1 < runup;) {
+      walk(zs, zt);
+      walk(zt, zs);
+    }
+    if (k < runup) {
+      walk(zs, zt);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) zs[u] = zt[u];
+    }
+  }
   for (; k < run; ++k) {
     const char *set = smem + set_i * L::SET;
     char *const staged = smem + (set_i == 0 ? 2 : set_i - 1) * L::SET + L::X;  // where the output of the block before goes
