@@ -296,10 +296,6 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
   auto rows = [&](const float *p, int blk, int width) __attribute__((always_inline)) {
     return rows_of(p + (row0 + (int64_t)blk * BLK) * width, len_of(blk), width);
   };
-  // the block after this one, or none of its rows where there is none: as many accesses in flight on every path
-  auto next_rows = [&](const float *p, bool more, int blk, int width) __attribute__((always_inline)) {
-    return rows_of(p + (row0 + (int64_t)blk * BLK) * width, more ? len_of(blk) : 0, width);
-  };
   const int first = REV ? sw.nblk - 1 : 0;
   const int step = REV ? -1 : 1;
   loader.load<NARROW>(rows(X, first, xw), nx);
@@ -314,8 +310,13 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
   // this wave's quadrant of the score tile: tokens b = 16 qb .. of Y, a = 16 qa .. of X
   const int qb = w >> 1, qa = w & 1;
   const int q_lane = lane & 15, q_grp = lane >> 4;
-  const int xq = (16 * qa + q_lane) * ROW + ((q_grp ^ swizzle(16 * qa + q_lane)) << 4);
-  const int yq = (16 * qb + q_lane) * ROW + ((q_grp ^ swizzle(16 * qb + q_lane)) << 4);
+  // the lane's operands: a token of quadrant row q of X or Y, and token lane % 32 of X
+  auto quadrant_at = [](int lane, int q) {
+    const int token = 16 * q + (lane & 15);
+    return token * ROW + (((lane >> 4) ^ swizzle(token)) << 4);
+  };
+  auto row_at = [](int lane) { return (lane & 31) * ROW + (((lane >> 5) ^ swizzle(lane & 31)) << 4); };
+  const int xq = quadrant_at(lane, qa), yq = quadrant_at(lane, qb);
   // decay between the tokens of a score; -1: masked.  Such a score is left out and not multiplied by zero, which would take an
   // infinity or a NaN (or what overflowed on the way to this score only) to tokens that do not see it.
   float qmask[4];
@@ -327,10 +328,15 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
   // (selected before the product, which the compiler fuses with the first subtraction of the split: its rounding is not felt)
   auto masked = [&](float score, int r) __attribute__((always_inline)) { return (qmask[r] < 0.f ? 0.f : score) * qmask[r]; };
   // rows of 64 bytes; unit u of row a lies at u ^ ((a >> 2) & 3)
-  const int sc_at = (16 * qa + q_lane) * SC_ROW + (((2 * qb + (q_grp >> 1)) ^ ((q_lane >> 2) & 3)) << 4) + ((q_grp & 1) << 3);
-  const int sc_from = c * SC_ROW + ((hh ^ ((c >> 2) & 3)) << 4);
+  auto quadrant_scores_at = [&](int lane) __attribute__((always_inline)) {
+    const int q_lane = lane & 15, q_grp = lane >> 4;
+    return (16 * qa + q_lane) * SC_ROW + (((2 * qb + (q_grp >> 1)) ^ ((q_lane >> 2) & 3)) << 4) + ((q_grp & 1) << 3);
+  };
+  const int sc_at = quadrant_scores_at(lane);
+  auto scores_at = [](int lane) { return (lane & 31) * SC_ROW + (((lane >> 5) ^ ((lane >> 2) & 3)) << 4); };  // token lane % 32's
+  const int sc_from = scores_at(lane);
   char *const z_park = smem + OFF_Z + w * 4096 + lane * 16;
-  const int x_from = c * ROW + ((hh ^ swizzle(c)) << 4);
+  const int x_from = row_at(lane);
 
   // ---- state entering the segment: st[T][4g+r] = St[32T+8g+4hh+r][32w+c]
   floatx16 st[NT];
@@ -371,8 +377,25 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
   loader.fill(smem + OFF_Y, ny);
   __syncthreads();
 
-  for (int it = 0, blk = first; it < sw.nblk; ++it, blk += step) {
-    const bool more = it + 1 < sw.nblk;
+  // output: lane (c, hh) holds, for token c, four consecutive columns per g
+  auto store = [&](const floatx16 &acc, int blk, int lane) __attribute__((always_inline)) {
+    const int c = lane & 31, col0 = fresh<NARROW>(32 * w + 4 * (lane >> 5));
+    const rows_t out = rows_of(Out + (row0 + (int64_t)blk * BLK) * zw, len_of(blk), zw);
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      f32x4 o;
+      o.x = acc[4 * gq + 0];
+      o.y = acc[4 * gq + 1];
+      o.z = acc[4 * gq + 2];
+      o.w = acc[4 * gq + 3];
+      const int col = col0 + 8 * gq, off = !NARROW || col < zw ? c * (zw * 4) + col * 4 : NOWHERE;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), out, off, 0, 0);
+    }
+  };
+
+  int blk = first;
+#pragma unroll 1
+  for (int it = 0; it < sw.nblk - 1; ++it, blk += step) {
     const int len = len_of(blk);
     float qd = qdec, bd = blockdec;
     if (RAGGED && REV && len != BLK) {
@@ -415,7 +438,6 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       }
 #pragma unroll
       for (int u = 0; u < 2; ++u) yf[u] = tokens.read(smem + OFF_Y, 0, u);
-      // z is wanted once more, for the intra-block term; until then it gives its registers away
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         *reinterpret_cast<f32x4 *>(z_park + 1024 * i) = f32x4{z[4 * i], z[4 * i + 1], z[4 * i + 2], z[4 * i + 3]};
@@ -435,7 +457,7 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
     floatx16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    loader.load<NARROW>(next_rows(X, more, blk + step, xw), nx);
+    loader.load<NARROW>(rows(X, blk + step, xw), nx);
     Split a0, a1, zu[2];
     f32x4 zp[4];
     if (active) {
@@ -471,16 +493,16 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
           if (T < NT - 1) yf[u] = tokens.read(smem + OFF_Y, T + 1, u);
           reads_first();
         }
-        if (T == (NT == 3 ? 2 : 1)) loader.load<NARROW>(next_rows(Y, more, blk + step, xw), ny);
+        if (T == (NT == 3 ? 2 : 1)) loader.load<NARROW>(rows(Y, blk + step, xw), ny);
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] *= qd;
     } else {
-      loader.load<NARROW>(next_rows(Y, more, blk + step, xw), ny);
+      loader.load<NARROW>(rows(Y, blk + step, xw), ny);
     }
     __syncthreads();  // the score tile is complete; X and Y are no longer read
     // (4) intra-block term
-    load_columns<NARROW>(next_rows(Z, more, blk + step, zw), z_off, zw, z);
+    load_columns<NARROW>(rows(Z, blk + step, zw), z_off, zw, z);
     if (active) {
       Split sf[2];
 #pragma unroll
@@ -496,20 +518,87 @@ sweep_body(const float *__restrict__ X, const float *__restrict__ Y, const float
       loader.fill(smem + OFF_X, nx);
     }
     loader.fill(smem + OFF_Y, ny);
-    // (5) output: lane (c, hh) holds, for token c, four consecutive columns per g
-    const int col0 = fresh<NARROW>(32 * w + 4 * hh);
-    const rows_t out = rows_of(Out + (row0 + (int64_t)blk * BLK) * zw, len, zw);
+    store(acc, blk, lane);  // (5)
+    __syncthreads();  // the next block's X and Y are complete; the score tile is no longer read
+  }
+  // The segment's last block leaves no state behind: its update, 48 of 132 products, and what is split and scaled for it are left out.
+  // Forward + backward in us, with that update and without, the same bits: b*h = 24, n = 2048 (four blocks to a segment) 183.7 and 174.8,
+  // n = 16384 (16 blocks) 1061 and 1045; b*h = 16, n = 1024 (two) 85.6 and 79.9.
+  {
+    float qd = qdec;
+    if (RAGGED && REV && len_of(blk) != BLK) qd = decay(sl, (float)max(len_of(blk) - c, 0));
+    Split xf[2][2], zu[2];
+    // (the lane's offsets are worked out here: kept through the blocks before, they would go to scratch)
+    const int late = fresh<true>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+    const int x_at = row_at(late);
+    {
+      floatx4 sc = {0.f, 0.f, 0.f, 0.f};
+      Split ys[2], xs[2];
+      const int xl = quadrant_at(late, qa), yl = quadrant_at(late, qb);
+      xs[0] = parts(smem + OFF_X, xl, PART);
+      ys[0] = parts(smem + OFF_Y, yl, PART);
 #pragma unroll
-    for (int gq = 0; gq < 4; ++gq) {
-      f32x4 o;
-      o.x = acc[4 * gq + 0];
-      o.y = acc[4 * gq + 1];
-      o.z = acc[4 * gq + 2];
-      o.w = acc[4 * gq + 3];
-      const int col = col0 + 8 * gq, off = !NARROW || col < zw ? c * (zw * 4) + col * 4 : NOWHERE;
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), out, off, 0, 0);
+      for (int m = 0; m < NT; ++m) {
+        if (m < NT - 1) {
+          xs[(m + 1) & 1] = parts(smem + OFF_X, xl ^ ((m + 1) << 6), PART);
+          ys[(m + 1) & 1] = parts(smem + OFF_Y, yl ^ ((m + 1) << 6), PART);
+        } else {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) xf[0][u] = parts(smem + OFF_X, x_at ^ (u << 5), PART);
+        }
+        reads_first();
+        sc = product(ys[m & 1], xs[m & 1], sc, [](int) {});
+      }
+      u32x2 h, m, l;
+      uint32_t a, b, d;
+      split2(masked(sc[0], 0), masked(sc[1], 1), a, b, d);
+      h.x = a, m.x = b, l.x = d;
+      split2(masked(sc[2], 2), masked(sc[3], 3), a, b, d);
+      h.y = a, m.y = b, l.y = d;
+      char *at = smem + OFF_SC + quadrant_scores_at(late);
+      *reinterpret_cast<u32x2 *>(at) = h;
+      *reinterpret_cast<u32x2 *>(at + SC_PART) = m;
+      *reinterpret_cast<u32x2 *>(at + 2 * SC_PART) = l;
     }
-    if (more) __syncthreads();  // the next block's X and Y are complete; the score tile is no longer read
+    floatx16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    if (active) {
+      Split a0, a1;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) split_pair(a0, i, st[0][2 * i], st[0][2 * i + 1]);
+#pragma unroll
+      for (int T = 0; T < NT; ++T) {
+        if (T < NT - 1)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) xf[(T + 1) & 1][u] = parts(smem + OFF_X, x_at ^ ((2 * T + 2 + u) << 5), PART);
+        reads_first();
+        auto split_z = [&](int k) __attribute__((always_inline)) {
+          if (k < 8) split_pair(zu[k >> 2], k & 3, z[2 * k], z[2 * k + 1]);
+        };
+        constexpr int PER = 8 / NT + (8 % NT > 0);  // pairs of Z beside each of the NT pairs of products
+        acc = product(a0, xf[T & 1][0], acc, [&](int i) __attribute__((always_inline)) {
+          if (i < 4) split_pair(a1, i, st[T][8 + 2 * i], st[T][9 + 2 * i]);
+          if (i >= 4 && i - 4 < PER) split_z(T * PER + i - 4);
+        });
+        acc = product(a1, xf[T & 1][1], acc, [&](int i) __attribute__((always_inline)) {
+          if (T < NT - 1 && i < 4) split_pair(a0, i, st[T < NT - 1 ? T + 1 : T][2 * i], st[T < NT - 1 ? T + 1 : T][2 * i + 1]);
+          if (i >= 4 && i - 2 < PER) split_z(T * PER + i - 2);
+        });
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] *= qd;
+    }
+    __syncthreads();  // the score tile is complete
+    if (active) {
+      Split sf[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) sf[u] = parts(smem + OFF_SC, scores_at(late) ^ (u << 5), SC_PART);
+      reads_first();
+#pragma unroll
+      for (int u = 0; u < 2; ++u) acc = product(zu[u], sf[u], acc, [](int) {});
+    }
+    store(acc, blk, late);
   }
 }
 
