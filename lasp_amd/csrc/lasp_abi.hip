@@ -378,6 +378,7 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   }
   g->pre_n = (int)((n + g->pre_len - 1) / g->pre_len);
   g->kept = KEPT_NONE;
+  g->cut = Cut{0, 0, 0};
   g->twin = nullptr;
   g->by_seg = divisor_of((uint32_t)g->n_seg);
   g->by_h = divisor_of((uint32_t)h);

@@ -66,6 +66,14 @@ __host__ __device__ inline int quotient(int n, Divisor d) {
 // for a call with a kv_in, or without (where a head outside the scan has parked none, see state_dies_in_segment).
 enum Kept { KEPT_NONE = 0, KEPT_STATES = 1, KEPT_STATES_ONLY = 2 };
 
+// Where the segments of a single-launch kernel begin, in blocks of 64 tokens from the end at which its walks start: at most eight
+// segments, 16 bits each.  Taken by heads whose decay reaches over `from` blocks and more.
+struct Cut {
+  uint64_t lo, hi;
+  int from;
+  __host__ __device__ int start(int j) const { return (int)((j < 4 ? lo : hi) >> (16 * (j & 3))) & 0xffff; }
+};
+
 // One chunk's geometry, passed by value to every kernel.
 struct Geom {
   int b, h;
@@ -85,6 +93,7 @@ struct Geom {
   Divisor by_seg, by_h;  // n_seg and h
   int pre_n;    // ceil(n / pre_len): states per (b, h) in the workspace
   int kept;     // a backward in one launch: what its kv_in is, see Kept
+  Cut cut;      // single-launch kernels only
   float *twin;  // where an outgoing state is written a second time (NULL: nowhere): the copy that a caller keeping the state
                 // would hand on.  A copy of its own is a launch of 3.6 us for 24 states (4.6 for 16 beside long sweeps)
                 // and its host call; eight chained chunks of 2048 tokens, b*h = 24: 675 us, 651 without them

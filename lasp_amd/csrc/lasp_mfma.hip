@@ -165,6 +165,36 @@ __device__ __forceinline__ SegWork seg_work(const Geom &g, int item) {
   return r;
 }
 
+// blocks over which a head's decay falls to 2^-SKIP_LOG2, or `all` where it takes that many and more
+__device__ __forceinline__ int reach_of(float slope, int all) {
+  const float sl = slope * LOG2E;
+  if (!(sl > 0.f)) return all;
+  const float x = SKIP_LOG2 / (sl * (float)BLK);
+  return x < (float)all ? (int)x + 1 : all;
+}
+// The same of a kernel that walks to its segment (SRC_WALK): segments of equal length for heads whose decay ends the walks soon, those of
+// g.cut, shorter the longer the walk before them, for the others.
+__device__ __forceinline__ SegWork walk_work(const Geom &g, int item, bool rev, int reach) {
+  SegWork r;
+  r.bh = quotient(item, g.by_seg);
+  r.seg = item - r.bh * g.n_seg;
+  const int total = (int)((g.n + BLK - 1) / BLK);
+  int b0, b1;
+  if (reach >= g.cut.from) {
+    const int j = rev ? g.n_seg - 1 - r.seg : r.seg;  // segments visited before it
+    const int from = g.cut.start(j), to = j + 1 < g.n_seg ? g.cut.start(j + 1) : total;
+    b0 = rev ? total - to : from;
+    b1 = rev ? total - from : to;
+  } else {
+    b0 = quotient(r.seg * total, g.by_seg);
+    b1 = quotient((r.seg + 1) * total, g.by_seg);
+  }
+  r.tok0 = (int64_t)b0 * BLK;
+  r.nblk = b1 - b0;
+  r.tail = b1 == total ? (int)(g.n - (int64_t)(total - 1) * BLK) : BLK;
+  return r;
+}
+
 // ------------------------------------------------------------------------------
 // Every sweep kernel below is an instance of sweep_body (W = 128) or ws_body (W = 64, where neither d nor e is larger),
 // <E, REV, TRANS, SRC, MODE>.
@@ -246,8 +276,15 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   const int wcol = w & 1, ih = w >> 1;    // math: column block and token half
   const int c = lane & 31, hh = lane >> 5;
 
-  const SegWork sw = seg_work(g, item);
-  const int head = sw.bh - quotient(sw.bh, g.by_h) * g.h;
+  const int bh = quotient(item, g.by_seg), head = bh - quotient(bh, g.by_h) * g.h;
+  const int total_blk = (int)((g.n + BLK - 1) / BLK);  // blocks in the chunk
+  float slope = 0.f;
+  int reach = 0;
+  if (SRC == SRC_WALK) {
+    slope = S[head];
+    reach = __builtin_amdgcn_readfirstlane(reach_of(slope, total_blk));
+  }
+  const SegWork sw = SRC == SRC_WALK ? walk_work(g, item, REV, reach) : seg_work(g, item);
   const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
   // elements from row to row of X and Y, and of Z and Out: q, k and their gradients have rows of g.dt features, of which
   // a slice of a wide head reads and writes fa (fb)
@@ -261,7 +298,6 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   // walk gets to the chunk's end, else from zero.  Blocks are numbered relative to the segment; walk and sweep
   // form one run of runup + nblk blocks, first_blk, first_blk + step, ..., of which the first `runup` only
   // update the state (one barrier each, both groups).
-  const int total_blk = (int)((g.n + BLK - 1) / BLK);  // blocks in the chunk
   const int seg_blk0 = (int)(sw.tok0 / BLK);           // the segment's first block
   const int chunk_tail = (int)(g.n - (int64_t)(total_blk - 1) * BLK);
   // tokens in a block (numbered relative to the segment): a partial block is the chunk's last one
@@ -273,13 +309,7 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
   bool take_carry = false;
   if (SRC == SRC_WALK) {
     const int avail = REV ? total_blk - (seg_blk0 + nblk) : seg_blk0;
-    int reach = avail;
-    const float sl = S[head] * LOG2E;
-    if (sl > 0.f) {
-      const float x = SKIP_LOG2 / (sl * (float)BLK);  // blocks over which a weight falls to 2^-SKIP_LOG2
-      if (x < (float)avail) reach = (int)x + 1;
-    }
-    runup = __builtin_amdgcn_readfirstlane(min(reach, avail));
+    runup = min(reach, avail);
     take_carry = carry_in != nullptr && runup == avail;
   }
   const int first_blk = blk0 - runup * step;
@@ -729,8 +759,15 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
   const int w = w8 & 3;
   const int c = lane & 31, hh = lane >> 5;
 
-  const SegWork sw = seg_work(g, item);
-  const int head = sw.bh - quotient(sw.bh, g.by_h) * g.h;
+  const int bh = quotient(item, g.by_seg), head = bh - quotient(bh, g.by_h) * g.h;
+  const int total_blk = (int)((g.n + BLK - 1) / BLK);  // blocks in the chunk
+  float slope = 0.f;
+  int reach = 0;
+  if (SRC == SRC_WALK) {
+    slope = S[head];
+    reach = __builtin_amdgcn_readfirstlane(reach_of(slope, total_blk));
+  }
+  const SegWork sw = SRC == SRC_WALK ? walk_work(g, item, REV, reach) : seg_work(g, item);
   const int64_t row0 = (int64_t)sw.bh * g.n + sw.tok0;
   // elements from row to row of X and Y, and of Z and Out: q, k and their gradients have rows of g.dt features, of which
   // a slice of a wide head reads and writes fa (fb)
@@ -738,7 +775,6 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
   const int nblk = sw.nblk;
   const int step = REV ? -1 : 1;
   const int blk0 = REV ? nblk - 1 : 0;
-  const int total_blk = (int)((g.n + BLK - 1) / BLK);  // blocks in the chunk
   const int seg_blk0 = (int)(sw.tok0 / BLK);           // the segment's first block
   const int chunk_tail = (int)(g.n - (int64_t)(total_blk - 1) * BLK);
   // tokens in a block (numbered relative to the segment): a partial block is the chunk's last one
@@ -753,17 +789,9 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
   // update the state.
   int runup = 0;
   bool take_carry = false;
-  float slope = 0.f;
   if (SRC == SRC_WALK) {
     const int avail = REV ? total_blk - (seg_blk0 + nblk) : seg_blk0;
-    int reach = avail;
-    slope = S[head];
-    const float sl = slope * LOG2E;
-    if (sl > 0.f) {
-      const float x = SKIP_LOG2 / (sl * (float)BLK);  // blocks over which a weight falls to 2^-SKIP_LOG2
-      if (x < (float)avail) reach = (int)x + 1;
-    }
-    runup = __builtin_amdgcn_readfirstlane(min(reach, avail));
+    runup = min(reach, avail);
     take_carry = carry_in != nullptr && runup == avail;
   }
   const int first_blk = blk0 - runup * step;
@@ -1389,8 +1417,9 @@ la_fused_fwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
 
 // The (b, h) from bh0 on are cut into segments of their own (n_seg of seg_len tokens): see launch_fused_bwd.
 struct Fine {
-  int bh0, seg_len, n_seg;
+  int bh0, n_seg;
   Divisor by_seg;
+  Cut cut;
 };
 
 // roles as in la_bwd3 (the dV role leaves dKV_out); all roles and segments of one (b, h) on one XCD.  With g.kept set, kv_in holds the
@@ -1405,9 +1434,9 @@ la_fused_bwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
   const int before = 3 * fine.bh0 * g.n_seg;  // workgroups of the (b, h) before bh0, a multiple of 8
   const bool cut = (int)blockIdx.x >= before;
   if (cut) {
-    g.seg_len = fine.seg_len;
     g.n_seg = fine.n_seg;
     g.by_seg = fine.by_seg;
+    g.cut = fine.cut;
   }
   const int local = (int)blockIdx.x - (cut ? before : 0);
   const int xcd = local & 7, slot = local >> 3;
@@ -1772,11 +1801,57 @@ int launch_state(const void *y, const void *z, const float *s, float *states, co
   return launch_state_skipping<E, REV, MODE, W>(y, z, s, states, g, carry_wanted ? -1 : (REV ? 0 : g.n_seg - 1), st, sub);
 }
 
+// How a single launch cuts a (b, h).  Segments of equal length leave the first one's workgroup idle while the last one's walks; so the
+// first is the longest (32 blocks in three segments: 16, 10 and 6 and not 11, 11 and 10).  A walk block takes 0.57 us, a swept one 1.35;
+// with 30 or 55 instead of 42 % the launches below take 0.99 - 1.09 of their time, with 70 % up to 1.25.  More than eight segments have
+// nothing left to do.  In us, equal segments (forwards of 256 tokens, whatever the chip had room for) and these: forwards, b*h = 8, n = 256 8.5
+// and 6.5, b*h = 16, n = 1024 17.6 and 15.6, b*h = 20, n = 700 14.7 and 13.2, b*h = 128, n = 1024 44.8 and 33.4, b*h = 160, n = 512 26.9 and
+// 20.5; backwards, b*h = 8, n = 256 9.3 and 7.1, b*h = 24, n = 2048 33.2 and 30.2, b*h = 20, n = 1024 20.5 and 18.8, b*h = 36, n = 3000 63.5
+// and 61.2; d = e = 64, b*h = 16, n = 1024 14.0 and 12.6 forwards, 13.6 and 13.4 backwards.  Of 31 such shapes none is slower by more than
+// 1.6 %.
+constexpr int CUT_MOST = 8;
+constexpr int CUT_SWEEP = 100, CUT_WALK = 42;  // a block's time, swept and walked over
+// A (b, h) of `total` blocks in at most `most` segments, each as long as the walk before it leaves it time: the least time in which that
+// covers all of them.
+void cut_in(int total, int64_t most, int *n_seg, Divisor *by_seg, Cut *cut) {
+  const int m = (int)(most < 1 ? 1 : most > CUT_MOST ? CUT_MOST : most);
+  // segments that cover the blocks in `time` (0: they don't), and where they start
+  auto cover = [&](int64_t time, uint64_t (&starts)[2]) {
+    starts[0] = starts[1] = 0;
+    int64_t at = 0;
+    for (int k = 0; k < m; ++k) {
+      const int64_t len = (time - at * CUT_WALK) / CUT_SWEEP;
+      if (len < 1) return 0;
+      starts[k >> 2] |= (uint64_t)at << (16 * (k & 3));
+      at += len;
+      if (at >= total) return k + 1;
+    }
+    return 0;
+  };
+  uint64_t starts[2];
+  int64_t lo = 0, hi = (int64_t)total * CUT_SWEEP;  // too little, enough
+  while (hi - lo > 1) {
+    const int64_t mid = (lo + hi) / 2;
+    (cover(mid, starts) ? hi : lo) = mid;
+  }
+  const int k = cover(hi, starts);
+  // equal segments take as long for a head that walks over this many blocks
+  const int64_t spare = hi - (int64_t)((total + k - 1) / k) * CUT_SWEEP;
+  *n_seg = k;
+  *by_seg = divisor_of((uint32_t)k);
+  *cut = Cut{starts[0], starts[1], k > 1 ? (int)(spare / CUT_WALK) + 1 : 0};
+}
+int blocks_of(const Geom &g) { return (int)((g.n + BLK - 1) / BLK); }
+
 template <class E, int MODE, int W>
-int launch_fused_fwd(const FwdArgs &a, const Geom &g, hipStream_t st) {
+int launch_fused_fwd(const FwdArgs &a, const Geom &g_plan, hipStream_t st) {
   int rc = grant_lds<la_fused_fwd<E, MODE, W>>(sweep_lds<W>());
   if (rc) return rc;
-  const unsigned grid = (unsigned)((((int64_t)g.b * g.h + 7) / 8) * 8 * g.n_seg);  // whole groups of 8 (b, h)
+  Geom g = g_plan;
+  const int64_t bh8 = ((int64_t)g.b * g.h + 7) / 8 * 8;
+  // (one segment that takes a state may be asked to leave it in its place: no other workgroup may have to read it)
+  if (!(g.n_seg == 1 && a.kv_in)) cut_in(blocks_of(g), (W == 64 ? 512 : 256) / bh8, &g.n_seg, &g.by_seg, &g.cut);
+  const unsigned grid = (unsigned)(bh8 * g.n_seg);  // whole groups of 8 (b, h)
   ProfScope prof(KC_FUSED, st);
   la_fused_fwd<E, MODE, W><<<grid, WS_THREADS, sweep_lds<W>(), st>>>((const elem16_t *)a.q, (const elem16_t *)a.k,
                                                          (const elem16_t *)a.v, a.s, a.kv_in, a.kv_out,
@@ -1792,18 +1867,13 @@ int launch_fused_fwd(const FwdArgs &a, const Geom &g, hipStream_t st) {
 // the ones without a walk: b*h = 12, n = 1024 20.1 and 20.6, b*h = 18 21.6 and 22.2.  At W = 64 the two count alike (14.7 and 15.0 at
 // worst).
 constexpr int64_t kFitByXcd = 20;
+int64_t fused_bwd_fit(const Geom &g) {  // segments per (b, h) in one round
+  const int64_t bh = (int64_t)g.b * g.h, placed = g.width == 128 && bh >= kFitByXcd ? (bh + 7) / 8 * 8 : bh;
+  return (g.width == 64 ? 512 : 256) / (3 * placed);
+}
 Geom fused_bwd_geom(const Geom &g) {
   Geom gb = g;
-  const int64_t bh = (int64_t)g.b * g.h, placed = g.width == 128 && bh >= kFitByXcd ? (bh + 7) / 8 * 8 : bh;
-  int64_t fit = (g.width == 64 ? 512 : 256) / (3 * placed);  // segments per (b, h) in one round
-  if (fit < 1) fit = 1;
-  if (fit < g.n_seg) {
-    int64_t len = (g.n + fit - 1) / fit;
-    len = ((len + BLK - 1) / BLK) * BLK;
-    gb.seg_len = (int)len;
-    gb.n_seg = (int)((g.n + len - 1) / len);
-    gb.by_seg = divisor_of((uint32_t)gb.n_seg);
-  }
+  cut_in(blocks_of(g), fused_bwd_fit(g), &gb.n_seg, &gb.by_seg, &gb.cut);
   return gb;
 }
 
@@ -1819,19 +1889,14 @@ Geom fused_bwd_geom(const Geom &g) {
 // uncut with one per CU: 53.8 and 57.1; 240: 58.3 and 63.9).
 Fine fused_bwd_tail(const Geom &g) {
   const int64_t bh = (int64_t)g.b * g.h, slots = g.width == 64 ? 512 : 256, placed = g.width == 64 ? bh : (bh + 7) / 8 * 8;
-  Fine f = {(int)((bh + 7) / 8 * 8), g.seg_len, g.n_seg, g.by_seg};  // nothing is cut
+  Fine f = {(int)((bh + 7) / 8 * 8), g.n_seg, g.by_seg, g.cut};  // nothing is cut
   if (g.n_seg > 1 || 3 * placed <= slots) return f;
   const int64_t whole = 3 * placed / slots * slots;  // workgroups in whole rounds
   const int64_t bh0 = whole / 24 * 8;            // whole groups of 8
   const int64_t rest = (bh - bh0 + 7) / 8 * 8, room = 256 + (g.width == 64 ? 0 : whole - 3 * bh0);
-  const int64_t nblk = (g.n + BLK - 1) / BLK;
-  int64_t n_seg = rest > 0 ? room / (3 * rest) : 1;
-  if (n_seg > nblk) n_seg = nblk;
-  if (n_seg < 2) return f;
-  f.bh0 = (int)bh0;
-  f.seg_len = (int)((nblk + n_seg - 1) / n_seg) * BLK;
-  f.n_seg = (int)((g.n + f.seg_len - 1) / f.seg_len);
-  f.by_seg = divisor_of((uint32_t)f.n_seg);
+  if (rest <= 0 || room / (3 * rest) < 2) return f;
+  cut_in(blocks_of(g), room / (3 * rest), &f.n_seg, &f.by_seg, &f.cut);
+  if (f.n_seg > 1) f.bh0 = (int)bh0;
   return f;
 }
 
@@ -1975,8 +2040,10 @@ bool whole_bwd_pays(const Geom &g) {
     return g.n <= kWholeBwdRounds || (bh > kWholeBwdMany && !g.combine);
   }
   if (!one_round) return true;
-  const Geom gb = fused_bwd_geom(g);
-  const double len = gb.seg_len / BLK, walk = (gb.n_seg - 1) * len, blocks = (double)((g.n + BLK - 1) / BLK);
+  // (counted with segments of equal length, as when the rule was fitted)
+  const int64_t fit = fused_bwd_fit(g), segs = fit < 1 ? 1 : fit < g.n_seg ? fit : g.n_seg, seg_blk = (blocks_of(g) + segs - 1) / segs;
+  const double len = fit < g.n_seg ? (double)seg_blk : g.seg_len / BLK, walk = ((fit < g.n_seg ? (blocks_of(g) + seg_blk - 1) / seg_blk : g.n_seg) - 1) * len;
+  const double blocks = blocks_of(g);
   const double rounds = (double)((3 * bh * g.n_seg + 255) / 256);
   const double three = rounds * (g.seg_len / BLK + 3) + (double)(bh * g.n_seg) / 13 + (double)bh * blocks / 116;
   return 1.44 * (len + 0.35 * walk) + 6 < three;
