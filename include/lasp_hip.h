@@ -161,6 +161,16 @@ int lasp_chunk_fwd(const void *q, const void *k, const void *v, const float *s,
                    void *stream);
 
 /*
+ * lasp_chunk_fwd_twin for 16-bit chunks of medium length, in one launch that needs no workspace and leaves no segment states.
+ * lasp_whole_ok says whether a shape is taken (1, 0, or a negative LASP_E_*): where that is the faster forward and, with
+ * `backward_follows`, where lasp_chunk_bwd, given no kv_seg_states, runs in one launch too and so does not have to rebuild them.
+ * Other shapes return LASP_E_SHAPE; kv_out may not overlap kv_in (LASP_E_ALIAS).
+ */
+int lasp_whole_ok(int b, int h, int64_t n, int d, int e, int dtype, int backward_follows);
+int lasp_whole_fwd(const void *q, const void *k, const void *v, const float *s, const float *kv_in, float *kv_out, float *kv_twin,
+                   void *o, int b, int h, int64_t n, int d, int e, int dtype, void *stream);
+
+/*
  * A few tokens under their states, as a serving loop's step has them: lasp_chunk_fwd for n <= LASP_STEP_TOKENS, d <= 128
  * and e a multiple of 4, any element type, in one launch that holds the states in registers.  No workspace, and no segment
  * states left for a backward; kv_out may be the same buffer as kv_in.  Any other shape returns LASP_E_SHAPE.  (On

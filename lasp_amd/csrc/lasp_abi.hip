@@ -620,9 +620,18 @@ int lasp_inplace_ok(int b, int h, int64_t n, int d, int e, int dtype, int seg_le
   return inplace_ok(g, backward != 0) ? 1 : 0;
 }
 
+int lasp_whole_ok(int b, int h, int64_t n, int d, int e, int dtype, int backward_follows) {
+  if (!mfma_eligible(d, e, dtype)) return 0;
+  Geom g;
+  const int rc = make_geom(b, h, n, d, e, dtype, 0, &g);
+  if (rc) return rc;
+  return mfma_whole(g, backward_follows != 0) ? 1 : 0;
+}
+
+enum Through { THROUGH_PLAN, THROUGH_NARROW, THROUGH_WHOLE };
 static int chunk_fwd_impl(const char *me, const void *q, const void *k, const void *v, const float *s,
                           const float *kv_in, float *kv_out, void *o, float *seg_states, const Geom &g,
-                          int dtype, void *stream, bool narrow = false) {
+                          int dtype, void *stream, Through through = THROUGH_PLAN) {
   int rc;
   if ((rc = check_alias(me, "kv", kv_in, kv_out, sizeof(float) * (size_t)g.b * g.h * g.dt * g.e, g, false))) return rc;
   if ((rc = check_aligned(me, "q", q, 16)) || (rc = check_aligned(me, "k", k, 16)) ||
@@ -635,9 +644,10 @@ static int chunk_fwd_impl(const char *me, const void *q, const void *k, const vo
   FwdArgs a{q, k, v, s, kv_in, kv_out, o, seg_states};
   hipStream_t st = (hipStream_t)stream;
   // (where a single launch leaves no segment states behind anyway, a few tokens take their own kernel)
-  rc = step_eligible(g) && (g.fused || !seg_states) ? step_fwd(a, g, dtype, st)
+  rc = through == THROUGH_WHOLE ? mfma_whole_fwd(a, g, dtype, st)
+       : step_eligible(g) && (g.fused || !seg_states) ? step_fwd(a, g, dtype, st)
        : mfma_eligible(g.dt, g.e, dtype)    ? mfma_fwd(a, g, dtype, st)
-       : narrow || mfma_f32_eligible(g.d, g.e, dtype) ? mfma_f32_fwd(a, g, st)
+       : through == THROUGH_NARROW || mfma_f32_eligible(g.d, g.e, dtype) ? mfma_f32_fwd(a, g, st)
                                             : generic_fwd(a, g, dtype, st);
   if (rc > 0) set_error("%s: HIP error %d: %s", me, rc, hipGetErrorString((hipError_t)rc));
   return rc;
@@ -666,7 +676,8 @@ static int fwd_twin(const void *q, const void *k, const void *v, const float *s,
   }
   if ((rc = check_twin("lasp_chunk_fwd", "kv", kv_in, kv_out, kv_twin, sizeof(float) * (size_t)b * h * d * e))) return rc;
   g.twin = kv_twin;
-  return chunk_fwd_impl("lasp_chunk_fwd", q, k, v, s, kv_in, kv_out, o, seg_states, g, dtype, stream, narrow);
+  return chunk_fwd_impl("lasp_chunk_fwd", q, k, v, s, kv_in, kv_out, o, seg_states, g, dtype, stream,
+                        narrow ? THROUGH_NARROW : THROUGH_PLAN);
 }
 
 int lasp_chunk_fwd_twin(const void *q, const void *k, const void *v, const float *s, const float *kv_in,
@@ -704,6 +715,32 @@ int lasp_step_fwd(const void *q, const void *k, const void *v, const float *s, c
     return LASP_E_NULL;
   }
   return chunk_fwd_impl("lasp_step_fwd", q, k, v, s, kv_in, kv_out, o, nullptr, g, dtype, stream);
+}
+
+int lasp_whole_fwd(const void *q, const void *k, const void *v, const float *s, const float *kv_in, float *kv_out, float *kv_twin,
+                   void *o, int b, int h, int64_t n, int d, int e, int dtype, void *stream) {
+  const char *me = "lasp_whole_fwd";
+  Geom g;
+  int rc = make_geom(b, h, n, d, e, dtype, 0, &g);
+  if (rc) return rc;
+  if (!mfma_eligible(d, e, dtype) || !mfma_whole(g, false)) {
+    set_error("%s: b=%d h=%d n=%lld d=%d e=%d dtype=%d does not run in one launch (see lasp_whole_ok)", me, b, h, (long long)n, d, e, dtype);
+    return LASP_E_SHAPE;
+  }
+  if (!q || !k || !v || !s || !o) {
+    set_error("%s: q, k, v, s and o must not be NULL", me);
+    return LASP_E_NULL;
+  }
+  const size_t bytes = sizeof(float) * (size_t)b * h * d * e;
+  const uintptr_t in = (uintptr_t)kv_in, out = (uintptr_t)kv_out;
+  if (kv_in && kv_out && in < out + bytes && out < in + bytes) {
+    set_error("%s: kv_out = %p overlaps kv_in = %p: other workgroups may still have to read the incoming state when the outgoing one is written",
+              me, (const void *)kv_out, (const void *)kv_in);
+    return LASP_E_ALIAS;
+  }
+  if ((rc = check_twin(me, "kv", kv_in, kv_out, kv_twin, bytes))) return rc;
+  g.twin = kv_twin;
+  return chunk_fwd_impl(me, q, k, v, s, kv_in, kv_out, o, nullptr, g, dtype, stream, THROUGH_WHOLE);
 }
 
 int lasp_chunk_fwd_static(const void *q, const void *k, const void *v, const float *s, const float *kv_in,

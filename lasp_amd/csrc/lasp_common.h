@@ -146,6 +146,10 @@ int mfma_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st);  // bf
 int mfma_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st);
 int mfma_f16_fwd(const FwdArgs &a, const Geom &g, hipStream_t st);
 int mfma_f16_bwd(const BwdArgs &a, const Geom &g, hipStream_t st);
+// 16-bit chunks whose forward takes one launch where no segment states are wanted (and whose backward then takes one as well)
+bool mfma_whole(const Geom &g, bool backward_follows);
+int mfma_whole_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st);
+int mfma_f16_whole_fwd(const FwdArgs &a, const Geom &g, hipStream_t st);
 int mfma_f32_fwd(const FwdArgs &a, const Geom &g, hipStream_t st);
 int mfma_f32_bwd(const BwdArgs &a, const Geom &g, hipStream_t st);
 

@@ -2058,6 +2058,23 @@ bool whole_bwd(const BwdArgs &a, const Geom &g) {
   return apart(a.dkv_in, a.dkv_out) && apart(a.kv_in, a.dkv_out) && apart(a.kv_in, g.twin);
 }
 
+// A forward that keeps no states may run in one launch as well, where the three kernels are not faster: each workgroup walks or sweeps all
+// of its (b, h), so again up to n = 88 b*h (80 for narrow rows) and 6144 tokens.  Up to 64 (b, h) and beyond 4096 tokens four gathered
+// segments fill the chip as well (b*h = 60, n = 4700 75.8 and 79.7 us).  bf16, forward with states, three kernels and one launch in us:
+// b*h = 24, n = 2048 27.9 and 24.9, b*h = 48, n = 2048 39.9 and 28.2, b*h = 64, n = 3100 61.9 and 57.2, b*h = 56, n = 3600 62.6 and 61.8 (the
+// nearest), b*h = 112, n = 3600 115 and 99, b*h = 200, n = 5400 295 and 222; d = 96, b*h = 80, n = 2600 72.9 and 47.1.  Of 160 shapes that
+// take it (four widths, b*h = 13 ... 512, n = 1100 ... 6144) the slowest is at 1.006 of its three kernels, the mean at 0.84.
+// KV_out is one sum over the whole chunk, as DKV_out is backwards: without decay 2.9e-7 off 64 bits at b*h = 24, n = 2048 where sums of
+// segments are 1.0e-7, 5.0e-7 and 3.7e-7 at b*h = 120, n = 6000; with decay 1.66e-3 (bf16) and 2.07e-4 (fp16) either way, the rounding
+// of its operand, and O 1.7e-3 to 2.7e-3 either way.
+constexpr int64_t kWholeFwdNarrow = 80, kWholeFwdGathered = 64;
+bool whole_fwd_pays(const Geom &g) {
+  const int64_t bh = (int64_t)g.b * g.h;
+  const bool full = g.dt == kMaxWidth && g.e == kMaxWidth;
+  if (g.n > kWholeBwdMax || g.n > (full ? kWholeBwdPerHead : kWholeFwdNarrow) * bh) return false;
+  return !full || bh > kWholeFwdGathered || g.n <= kWholeBwdRounds;
+}
+
 template <class E, int MODE, int W>
 int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
   int rc = 0;
@@ -2145,6 +2162,14 @@ template <class E>
 int bwd_w(const BwdArgs &a, const Geom &g, hipStream_t st) {
   return g.width == 64 ? bwd_m<E, 64>(a, g, st) : bwd_m<E, 128>(a, g, st);
 }
+template <class E>
+int whole_fwd_w(const FwdArgs &a, const Geom &g, hipStream_t st) {
+  switch (mode_of(g)) {
+    case M_ALIGNED: return launch_fused_fwd<E, M_ALIGNED, kMaxWidth>(a, g, st);
+    case M_RAGGED: return launch_fused_fwd<E, M_RAGGED, kMaxWidth>(a, g, st);
+    default: return launch_fused_fwd<E, M_NARROW, kMaxWidth>(a, g, st);
+  }
+}
 
 }  // namespace
 
@@ -2152,12 +2177,19 @@ int bwd_w(const BwdArgs &a, const Geom &g, hipStream_t st) {
 #ifdef LASP_MFMA_F16
 int mfma_f16_fwd(const FwdArgs &a, const Geom &g, hipStream_t st) { return fwd_w<ElemF16>(a, g, st); }
 int mfma_f16_bwd(const BwdArgs &a, const Geom &g, hipStream_t st) { return bwd_w<ElemF16>(a, g, st); }
+int mfma_f16_whole_fwd(const FwdArgs &a, const Geom &g, hipStream_t st) { return whole_fwd_w<ElemF16>(a, g, st); }
 #else
 int mfma_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
   return dtype == LASP_DTYPE_F16 ? mfma_f16_fwd(a, g, st) : fwd_w<ElemBF16>(a, g, st);
 }
 int mfma_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
   return dtype == LASP_DTYPE_F16 ? mfma_f16_bwd(a, g, st) : bwd_w<ElemBF16>(a, g, st);
+}
+bool mfma_whole(const Geom &g, bool backward_follows) {
+  return !g.fused && g.width == kMaxWidth && g.dt <= kMaxWidth && whole_fwd_pays(g) && (!backward_follows || whole_bwd_pays(g));
+}
+int mfma_whole_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
+  return dtype == LASP_DTYPE_F16 ? mfma_f16_whole_fwd(a, g, st) : whole_fwd_w<ElemBF16>(a, g, st);
 }
 #endif
 

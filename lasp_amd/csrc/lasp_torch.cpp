@@ -162,13 +162,21 @@ struct Forward {
   Tensor o, states;
   int seg_len = 0;
 };
+bool apart(const Tensor &a, const Tensor &b) {
+  if (!a.defined() || !b.defined()) return true;
+  const uintptr_t x = (uintptr_t)a.data_ptr(), y = (uintptr_t)b.data_ptr();
+  return x + a.nbytes() <= y || y + b.nbytes() <= x;
+}
+// What a forward leaves for a backward: nothing; what `run_backward` below needs to be fast, which is nothing where both run in one launch;
+// the segment states, for a caller who may hand them on.
+enum Keep { KEEP_NOTHING, KEEP_WHAT_PAYS, KEEP_STATES };
 // q, k, v contiguous
 Forward run_forward(const Shape &sh, Tensor q, Tensor k, Tensor v, const Tensor &s, Tensor kv_in,
-                    const Tensor &kv_out, const Tensor &kv_twin, int seg_len, bool keep = true) {
+                    const Tensor &kv_out, const Tensor &kv_twin, int seg_len, Keep keep = KEEP_STATES) {
   const auto stream = [&] { return c10::hip::getCurrentHIPStream(q.device().index()).stream(); };
   Forward f;
   f.o = at::empty(v.sizes(), v.options());
-  if (!keep && seg_len == 0 && !kv_twin.defined() && is_step(sh.n, sh.d, sh.e)) {
+  if (keep == KEEP_NOTHING && seg_len == 0 && !kv_twin.defined() && is_step(sh.n, sh.d, sh.e)) {
     const int rc = lasp_step_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), (const float *)data(kv_in),
                                  (float *)data(kv_out), f.o.data_ptr(), sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, stream());
     if (rc) raise_lasp(rc, "lasp_step_fwd");
@@ -176,6 +184,13 @@ Forward run_forward(const Shape &sh, Tensor q, Tensor k, Tensor v, const Tensor 
   }
   if (seg_len == 0 && !kv_in.defined() && !kv_out.defined()) seg_len = lasp_stateless_seg_len(sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype);
   const Plan p = plan_of(sh, seg_len);
+  if (!p.fused && keep != KEEP_STATES && seg_len == 0 && sh.dtype != LASP_DTYPE_F32 && apart(kv_in, kv_out) &&
+      lasp_whole_ok(sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, keep == KEEP_WHAT_PAYS) == 1) {
+    const int rc = lasp_whole_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), (const float *)s.data_ptr(), (const float *)data(kv_in),
+                                  (float *)data(kv_out), (float *)data(kv_twin), f.o.data_ptr(), sh.b, sh.h, sh.n, sh.d, sh.e, sh.dtype, stream());
+    if (rc) raise_lasp(rc, "lasp_whole_fwd");
+    return f;
+  }
   kv_in = private_incoming(kv_in, kv_out, sh, p.seg_len, false);
   q = rows(q, sh), k = rows(k, sh), v = rows(v, sh);
   f.seg_len = p.seg_len;
@@ -276,7 +291,7 @@ struct Chain {
 };
 
 Forward forward_call(const Shape &sh, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Chain &chain,
-                     bool keep) {
+                     Keep keep) {
   Forward f;
   {
     at::AutoDispatchBelowADInplaceOrView below_autograd;
@@ -292,7 +307,7 @@ Forward forward_call(const Shape &sh, const Tensor &q, const Tensor &k, const Te
 struct LaspChunk : public torch::autograd::Function<LaspChunk> {
   static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &s, const Shape &sh,
                         const Chain &chain) {
-    const Forward f = forward_call(sh, q, k, v, s, chain, true);
+    const Forward f = forward_call(sh, q, k, v, s, chain, KEEP_WHAT_PAYS);
     variable_list saved{q, k, v, s};
     if (f.states.defined()) saved.push_back(f.states);
     if (chain.kv_in.defined()) saved.push_back(chain.kv_in);
@@ -357,7 +372,7 @@ std::optional<Tensor> operator_call(const Tensor &q, const Tensor &k, const Tens
   check_state("kv_twin", chain.kv_twin, sh, q);
   const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() || s.requires_grad());
   c10::OptionalDeviceGuard guard(q.device());
-  return grad ? LaspChunk::apply(q, k, v, s, sh, chain) : forward_call(sh, q, k, v, s, chain, false).o;
+  return grad ? LaspChunk::apply(q, k, v, s, sh, chain) : forward_call(sh, q, k, v, s, chain, KEEP_NOTHING).o;
 }
 
 Tensor or_none(const std::optional<Tensor> &t) { return t ? *t : Tensor(); }
@@ -405,7 +420,7 @@ PYBIND11_MODULE(_lasp_torch, m) {
         if (!regular(q, k, v, s, sh, keep) || !state_ok(in, sh, q) || !state_ok(out, sh, q)) return std::nullopt;
         c10::OptionalDeviceGuard guard(q.device());
         at::AutoDispatchBelowADInplaceOrView below_autograd;
-        Forward f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, in, out, Tensor(), seg_len, keep);
+        Forward f = run_forward(sh, q.contiguous(), k.contiguous(), v.contiguous(), s, in, out, Tensor(), seg_len, keep ? KEEP_STATES : KEEP_NOTHING);
         return std::make_tuple(f.o, or_nothing(f.states), f.seg_len);
       },
       unlocked());
