@@ -515,8 +515,8 @@ ws_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const el
       // own states are still where the pre-pass put them, the own state of the segment visited before it
       // (the chunk's incoming state for the first one)
       // The workspace holds one state per segment of the pre-pass, of which this sweep segment spans
-      // `sub` (a power of two; 1 unless the plan cut long segments finer for the pre-pass): the state that
-      // enters it is the one entering its first piece in sweep order.
+      // `sub` (1 unless the plan cut long segments finer for the pre-pass, or a backward sweeps several of the
+      // forward's in a row): the state that enters it is the one entering its first piece in sweep order.
       const int sub = g.seg_len / g.pre_len;
       const int piece = REV ? min(sw.seg * sub + sub, g.pre_n) - 1 : sw.seg * sub;
       const float *src = states + ((int64_t)sw.bh * g.pre_n + piece) * (W * W);
@@ -1013,8 +1013,8 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
       // own states are still where the pre-pass put them, the own state of the segment visited before it
       // (the chunk's incoming state for the first one)
       // The workspace holds one state per segment of the pre-pass, of which this sweep segment spans
-      // `sub` (a power of two; 1 unless the plan cut long segments finer for the pre-pass): the state that
-      // enters it is the one entering its first piece in sweep order.
+      // `sub` (1 unless the plan cut long segments finer for the pre-pass, or a backward sweeps several of the
+      // forward's in a row): the state that enters it is the one entering its first piece in sweep order.
       const int sub = g.seg_len / g.pre_len;
       const int piece = REV ? min(sw.seg * sub + sub, g.pre_n) - 1 : sw.seg * sub;
       const float *src = states + ((int64_t)sw.bh * g.pre_n + piece) * (W * W);
@@ -2075,6 +2075,38 @@ bool whole_fwd_pays(const Geom &g) {
   return !full || bh > kWholeFwdGathered || g.n <= kWholeBwdRounds;
 }
 
+// Segments of the backward sweeps: m of the plan's in a row.  The plan's segments give the forward a workgroup per CU; three roles of them
+// take one round and a half to three, each with its start-up -- the first tiles, the entering state, the last stores -- of about five
+// blocks' time, and half of a last round is empty.  The states lie at the plan's segments either way (a sweep takes the one that enters
+// its first), so the forward, the pre-passes and the scans stay as they are.  m is the one with the least rounds x (blocks + 5), a round
+// being 32 workgroups on each XCD, as launch_bwd3 deals items out, if that saves 3 %.  bf16, backward with states, us, m = 1 and m:
+// b*h = 4, n = 8192 38.2 and 34.0 (m = 2: one round of 8 blocks for two of 4), b*h = 8, n = 3784 35.5 and 31.1 (2), b*h = 16, n = 8192 87.9
+// and 81.2 (4: one round of 32 for three of 8), b*h = 20, n = 3757, d = 96 52.7 and 43.3 (3), b*h = 16, n = 1536, d = 192 55.9 and 47.9 (2).
+// A last segment of the plan's less than a fifth full makes no round of its own (b*h = 10, n = 8226: 3.4 % slower with m = 3).  Over 225 shapes
+// (b*h = 3 ... 48, n = 1523 ... 31484) 0.956 of the time on average, 0.954 with the best m of each, none slower.  Slices of a wide head, whose
+// sweeps fetch narrow rows, lose from 28 blocks on (b*h = 32, n = 4096, d = 256 1.012 and up).  Heads of up to 64 features run two workgroups to a
+// CU and lose with any m (1.03 and up on 24 shapes).
+constexpr int kSweepStart = 5, kSweepBlocks = 40, kSweepBlocksSlice = 24, kSweepRow = 8;
+template <int W>
+Geom bwd_sweep_geom(const Geom &g) {
+  Geom gs = g;
+  if (W != kMaxWidth) return gs;
+  const int64_t blk = g.seg_len / BLK, most = g.dt > kMaxWidth ? kSweepBlocksSlice : kSweepBlocks;
+  const bool sliver = g.n_seg > 1 && (g.n - (int64_t)(g.n_seg - 1) * g.seg_len) * 5 < g.seg_len;
+  auto cost = [&](int m) {
+    const int segs = m > 1 ? (g.n_seg + m - 1) / m : sliver ? g.n_seg - 1 : g.n_seg;
+    const int64_t items = (int64_t)g.b * g.h * segs, per_xcd = 3 * ((items + 7) / 8);
+    return (per_xcd + 31) / 32 * (m * blk + kSweepStart);
+  };
+  int best = 1;
+  for (int m = 2; m <= kSweepRow && m <= g.n_seg && m * blk <= most; ++m)
+    if (best == 1 ? cost(m) * 100 < cost(1) * 97 : cost(m) < cost(best)) best = m;
+  gs.seg_len = best * g.seg_len;
+  gs.n_seg = (g.n_seg + best - 1) / best;
+  gs.by_seg = divisor_of((uint32_t)gs.n_seg);
+  return gs;
+}
+
 template <class E, int MODE, int W>
 int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
   int rc = 0;
@@ -2107,8 +2139,8 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
     return launch_bwd3<E, SRC_COMBINE, MODE, W>(a, g.n_seg > 1 ? kv_states : nullptr,
                                                 g.n_seg > 1 ? a.ws_dkv : nullptr, g, st);
   }
-  const Geom gp = pre_pass_geom(g);
-  const int sub = g.seg_len / g.pre_len;  // pre-pass segments per sweep segment
+  const Geom gp = pre_pass_geom(g), gw = bwd_sweep_geom<W>(g);
+  const int sub = gw.seg_len / g.pre_len;  // pre-pass segments per sweep segment
   const float *kv_states = a.kv_seg_states;
   if (!kv_states && (g.n_seg > 1 || a.kv_in)) {
     if ((rc = launch_state<E, false, MODE, W>(a.k, a.v, a.s, a.ws_kv, gp, false, sub, st))) return rc;
@@ -2123,7 +2155,7 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
   }
   auto sweep = [&](auto mode, int i) {
     return launch_bwd3<E, SRC_SCANNED, decltype(mode)::value, W>(slice_args(a, g, i), state_slice(kv_states, g, i),
-                                                                 state_slice(dkv_states, g, i), slice_geom(g, i), st);
+                                                                 state_slice(dkv_states, g, i), slice_geom(gw, i), st);
   };
   rc = sweep(std::integral_constant<int, MODE>(), 0);
   if constexpr (MODE == M_NARROW && W == kMaxWidth)
