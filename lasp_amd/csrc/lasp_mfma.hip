@@ -1470,6 +1470,15 @@ la_bwd3(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const el
   const int grp = blockIdx.x / 24, r = blockIdx.x - grp * 24;
   const int role = r >> 3;
   const int item = n_items - 1 - (grp * 8 + (r & 7));
+  if (SRC == SRC_SCANNED && W == kMaxWidth) {
+    int len = g.rev_len, n = g.rev_n;
+    // (asked for here, with the arguments that everything waits for: where a role needs them they cost every call 0.5 us)
+    asm volatile("" : "+s"(len), "+s"(n));
+    if (role != 0) {
+      g.pre_len = len;
+      g.pre_n = n;
+    }
+  }
   if (item < 0) return;
   if (role == 0)
     any_body<E, false, true, SRC, MODE, W>(DO, V, K, S, kv_states, DQ, g, g.e, g.d, item, smem, kv_in);
@@ -1925,6 +1934,25 @@ Geom pre_pass_geom(const Geom &g) {
   gp.by_seg = divisor_of((uint32_t)gp.n_seg);
   return gp;
 }
+// The same for DKV in a backward whose sweeps (`gw`) go over several of the forward's segments in a row: nothing but those sweeps reads
+// its states, so they may lie as far apart as the sweeps start.  Fewer of them are written by the pre-pass, read and written by the scan;
+// the pre-pass's walks are longer and fewer.  The least 20 x blocks of a walk + walks is taken (a block takes some 0.6 us, a state
+// 0.03), for a wide head, whose slices wait for one another's bytes, if it saves a ninth.  Backward with states, us, states at the forward's segments and by this rule: b*h = 8, n = 8192, d = 256 102.2
+// and 94.8 (512 tokens apart, not 256; 1024 97.9), d = 192 93.1 and 87.2; d = 256, b*h = 16, n = 4000 96.6 and 89.0, b*h = 32, n = 2339
+// 113.5 and 105.7, b*h = 4, n = 7593 56.4 and 51.0; d = 128, b*h = 8, n = 3784 30.1 and 28.3, b*h = 4, n = 7521 33.1 and 30.1.
+// b*h = 16, n = 8192 stays at 512 (82.6, 1024 83.3).  Over 53 shapes (b*h = 4 ... 32, n = 1594 ... 14632, six of seven of them with d > 128) that
+// would take fewer states without the ninth 0.96 of the time on average; wide heads that save less came out between 0.96 and 1.02.
+constexpr int kRevBlock = 20;
+Geom rev_pass_geom(const Geom &g, const Geom &gw) {
+  Geom gp = g;
+  const int64_t heads = (int64_t)g.b * g.h * slices_of(g);
+  auto cost = [&](int len) { return kRevBlock * (int64_t)(len / BLK) + heads * ((g.n + len - 1) / len); };
+  const int64_t enough = g.dt > kMaxWidth ? cost(g.pre_len) * 8 / 9 : cost(g.pre_len);
+  for (int len = 2 * g.pre_len; len <= gw.seg_len; len += g.pre_len)
+    if (gw.seg_len % len == 0 && cost(len) < enough && cost(len) < cost(gp.pre_len)) gp.pre_len = len;
+  gp.pre_n = (int)((g.n + gp.pre_len - 1) / gp.pre_len);
+  return pre_pass_geom(gp);
+}
 
 // A wide head (d > 128) is swept one slice of 128 features of q and k after the other, straight from and to their rows
 // (b*h = 8, n = 8192, d = 256, e = 128, forward + backward: 197 us, against 383 with slices copied out and summed outside):
@@ -1940,9 +1968,9 @@ const void *row_slice(const void *p, int i) { return (const elem16_t *)p + i * k
 void *row_slice(void *p, int i) { return (elem16_t *)p + i * kMaxWidth; }
 template <class T>  // of the chunk's d x e states
 T *carry_slice(T *p, const Geom &g, int i) { return p ? p + (int64_t)i * kMaxWidth * g.e : p; }
-template <class T>  // of the workspace
-T *state_slice(T *p, const Geom &g, int i) {
-  return p ? p + (int64_t)i * g.b * g.h * g.pre_n * kMaxWidth * kMaxWidth : p;
+template <class T>  // of the workspace, which holds `n` states per (b, h)
+T *state_slice(T *p, const Geom &g, int n, int i) {
+  return p ? p + (int64_t)i * g.b * g.h * n * kMaxWidth * kMaxWidth : p;
 }
 FwdArgs slice_args(const FwdArgs &a, const Geom &g, int i) {
   FwdArgs r = a;
@@ -1993,7 +2021,7 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
   auto sweep = [&](auto mode, int i) {
     const FwdArgs as = slice_args(a, g, i);
     return launch_apply<E, false, false, SRC_SCANNED, decltype(mode)::value, W>(
-        as.q, as.k, as.v, as.s, need_states ? state_slice(as.seg_states, g, i) : nullptr, as.kv_in, nullptr, as.o,
+        as.q, as.k, as.v, as.s, need_states ? state_slice(as.seg_states, g, g.pre_n, i) : nullptr, as.kv_in, nullptr, as.o,
         slice_geom(g, i), st);
   };
   rc = sweep(std::integral_constant<int, MODE>(), 0);
@@ -2139,7 +2167,11 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
     return launch_bwd3<E, SRC_COMBINE, MODE, W>(a, g.n_seg > 1 ? kv_states : nullptr,
                                                 g.n_seg > 1 ? a.ws_dkv : nullptr, g, st);
   }
-  const Geom gp = pre_pass_geom(g), gw = bwd_sweep_geom<W>(g);
+  const Geom gp = pre_pass_geom(g);
+  Geom gw = bwd_sweep_geom<W>(g);
+  const Geom gr = W == kMaxWidth ? rev_pass_geom(g, gw) : gp;
+  gw.rev_len = gr.seg_len;
+  gw.rev_n = gr.n_seg;
   const int sub = gw.seg_len / g.pre_len;  // pre-pass segments per sweep segment
   const float *kv_states = a.kv_seg_states;
   if (!kv_states && (g.n_seg > 1 || a.kv_in)) {
@@ -2149,13 +2181,13 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
   }
   const float *dkv_states = nullptr;
   if (g.n_seg > 1 || a.dkv_in || a.dkv_out) {
-    if ((rc = launch_state<E, true, MODE, W>(a.q, a.d_o, a.s, a.ws_dkv, gp, a.dkv_out != nullptr, sub, st))) return rc;
-    if ((rc = launch_segment_scan(a.ws_dkv, a.dkv_in, a.dkv_out, a.s, gp, 1, st))) return rc;
+    if ((rc = launch_state<E, true, MODE, W>(a.q, a.d_o, a.s, a.ws_dkv, gr, a.dkv_out != nullptr, gw.seg_len / gr.seg_len, st))) return rc;
+    if ((rc = launch_segment_scan(a.ws_dkv, a.dkv_in, a.dkv_out, a.s, gr, 1, st))) return rc;
     dkv_states = a.ws_dkv;
   }
   auto sweep = [&](auto mode, int i) {
-    return launch_bwd3<E, SRC_SCANNED, decltype(mode)::value, W>(slice_args(a, g, i), state_slice(kv_states, g, i),
-                                                                 state_slice(dkv_states, g, i), slice_geom(gw, i), st);
+    return launch_bwd3<E, SRC_SCANNED, decltype(mode)::value, W>(slice_args(a, g, i), state_slice(kv_states, g, g.pre_n, i),
+                                                                 state_slice(dkv_states, g, gr.n_seg, i), slice_geom(gw, i), st);
   };
   rc = sweep(std::integral_constant<int, MODE>(), 0);
   if constexpr (MODE == M_NARROW && W == kMaxWidth)
