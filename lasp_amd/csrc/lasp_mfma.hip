@@ -1937,9 +1937,10 @@ Geom pre_pass_geom(const Geom &g) {
 // The same for DKV in a backward whose sweeps (`gw`) go over several of the forward's segments in a row: nothing but those sweeps reads
 // its states, so they may lie as far apart as the sweeps start.  Fewer of them are written by the pre-pass, read and written by the scan;
 // the pre-pass's walks are longer and fewer.  The least 20 x blocks of a walk + walks is taken (a block takes some 0.6 us, a state
-// 0.03), for a wide head, whose slices wait for one another's bytes, if it saves a ninth.  Backward with states, us, states at the forward's segments and by this rule: b*h = 8, n = 8192, d = 256 102.2
-// and 94.8 (512 tokens apart, not 256; 1024 97.9), d = 192 93.1 and 87.2; d = 256, b*h = 16, n = 4000 96.6 and 89.0, b*h = 32, n = 2339
-// 113.5 and 105.7, b*h = 4, n = 7593 56.4 and 51.0; d = 128, b*h = 8, n = 3784 30.1 and 28.3, b*h = 4, n = 7521 33.1 and 30.1.
+// 0.03), for a wide head, whose slices wait for one another's bytes, if it saves a ninth.  Backward with states, us, states at the forward's
+// segments and by this rule: b*h = 8, n = 8192, d = 256 102.2 and 94.8 (512 tokens apart, not 256; 1024 97.9), d = 192 93.1 and 87.2;
+// d = 256, b*h = 16, n = 4000 96.6 and 89.0, b*h = 32, n = 2339 113.5 and 105.7, b*h = 4, n = 7593 56.4 and 51.0; d = 128, b*h = 8, n = 3784
+// 30.1 and 28.3, b*h = 4, n = 7521 33.1 and 30.1.
 // b*h = 16, n = 8192 stays at 512 (82.6, 1024 83.3).  Over 53 shapes (b*h = 4 ... 32, n = 1594 ... 14632, six of seven of them with d > 128) that
 // would take fewer states without the ninth 0.96 of the time on average; wide heads that save less came out between 0.96 and 1.02.
 constexpr int kRevBlock = 20;
