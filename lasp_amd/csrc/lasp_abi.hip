@@ -379,6 +379,7 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   g->pre_n = (int)((n + g->pre_len - 1) / g->pre_len);
   g->rev_len = g->pre_len;
   g->rev_n = g->pre_n;
+  g->stay = 1 << 30;
   g->kept = KEPT_NONE;
   g->cut = Cut{0, 0, 0};
   g->twin = nullptr;

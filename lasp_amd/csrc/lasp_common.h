@@ -93,6 +93,7 @@ struct Geom {
   Divisor by_seg, by_h;  // n_seg and h
   int pre_n;    // ceil(n / pre_len): states per (b, h) in the workspace
   int rev_len, rev_n;  // the same of a 16-bit backward's own states (DKV), which may lie further apart
+  int stay;     // forward sweeps and dQ: blocks at a segment's end that are loaded to stay in the memory-side cache (see launch_apply)
   int kept;     // a backward in one launch: what its kv_in is, see Kept
   Cut cut;      // single-launch kernels only
   float *twin;  // where an outgoing state is written a second time (NULL: nowhere): the copy that a caller keeping the state

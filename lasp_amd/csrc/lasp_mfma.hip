@@ -701,6 +701,11 @@ __device__ __forceinline__ void load_to_lds(u32x4 rows, uint32_t off, uint32_t l
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(rows)
                : "memory", "m0");
 }
+// ... that the caches need not keep
+__device__ __forceinline__ void load_to_lds_once(u32x4 rows, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(lds), "v"(off), "s"(rows)
+               : "memory", "m0");
+}
 // A barrier that the wave's LDS accesses have to be done for, but the N youngest (they are answered in order)
 template <int N>
 __device__ __forceinline__ void barrier_before() {
@@ -812,8 +817,13 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
     auto fetch_tile = [&](const elem16_t *base, int blk, int pitch, const uint32_t (&off)[4], uint32_t lds)
                           __attribute__((always_inline)) {
       const u32x4 rows = row_buffer(base + (int64_t)blk * BLK * pitch, len_of(blk) * pitch * 2);
+      if (SRC != SRC_WALK && !REV && blk < nblk - g.stay) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) load_to_lds(rows, off[i], lds + 4 * i * L::ROW);
+        for (int i = 0; i < 4; ++i) load_to_lds_once(rows, off[i], lds + 4 * i * L::ROW);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) load_to_lds(rows, off[i], lds + 4 * i * L::ROW);
+      }
     };
     // block k of the run into set `set`: four loads of X (none for a block that is only walked over), eight of Y and Z
     auto fetch_x = [&](int k, int set) __attribute__((always_inline)) {
@@ -1751,11 +1761,28 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
   }
 }
 
+// What the loads of a sweep leave in the 256 MB memory-side cache.  A forward's q, k and v are read again by the backward, if that follows
+// soon, and it begins at the ends of the segments.  Where they exceed the cache, only the last blocks of the segments are loaded as usual, as
+// many as have 160 MB; the blocks before them, which would not last, are loaded as data that is read once (`nt`), and come faster for it.
+// Forwards, us: b*h = 32, n = 16384 138 -> 126, b*h = 16, n = 65536 245 -> 222, b*h = 64, n = 8192 134 -> 126; with the backward 394 -> 385,
+// 732 -> 698, 384 -> 378.  With every block read once b*h = 32's forward takes 128 and its backward 16 more.  Tensors that fit the cache lose:
+// b*h = 36, n = 5003, d = e = 128, every block read once 164.5 -> 168.1 in both directions, b*h = 16, n = 16384, 160 of 201 MB as usual, 237.7 ->
+// 239.8.  Of 64, 96, 128, 160, 192 and 256 MB the forwards are the faster the less stays (b*h = 32: 0.91 of the time with 64, 0.95 with 192), the
+// backwards the slower (b*h = 64, n = 4096: 1.03 of both with 64, 0.99 to 1.01 from 96 on).
+// In a backward the three roles' workgroups of a round go over their segments' q, k, v and dO at about the same time, dQ's in the other
+// direction: where these exceed the cache, dQ's loads leave nothing behind (b*h = 16, n = 65536: both directions 718 -> 706; b*h = 32, n = 16384,
+// where they do not, 393 -> 396).
+// Non-temporal loads in the pre-pass (0.95 of the speed at d = 256, 0.985 at n = 65536) or in all roles (0.90 to 0.96), and stores that are not
+// non-temporal (0.95 to 0.98 beyond 200 MB of tensors) lose.
+constexpr int64_t kCacheBytes = (int64_t)256 << 20, kStayBytes = (int64_t)160 << 20;
 template <class E, bool REV, bool TRANS, int SRC, int MODE, int W>
 int launch_apply(const void *x, const void *y, const void *z, const float *s, const float *states,
-                    const float *carry_in, float *carry_out, void *out, const Geom &g, hipStream_t st) {
+                    const float *carry_in, float *carry_out, void *out, const Geom &g_plan, hipStream_t st) {
   int rc = grant_lds<la_apply<E, REV, TRANS, SRC, MODE, W>>(sweep_lds<W>());
   if (rc) return rc;
+  Geom g = g_plan;
+  const int64_t row = (int64_t)g.b * g.h * 2 * (2 * g.d + g.e);  // bytes of a token's q, k and v
+  if (row * g.n > kCacheBytes) g.stay = (int)(kStayBytes / (row * g.n_seg * BLK));
   const unsigned grid = (unsigned)((int64_t)g.b * g.h * g.n_seg);
   ProfScope prof(KC_APPLY, st);
   la_apply<E, REV, TRANS, SRC, MODE, W><<<grid, WS_THREADS, sweep_lds<W>(), st>>>(
@@ -1764,10 +1791,12 @@ int launch_apply(const void *x, const void *y, const void *z, const float *s, co
 }
 
 template <class E, int SRC, int MODE, int W>
-int launch_bwd3(const BwdArgs &a, const float *kv_states, const float *dkv_states, const Geom &g,
+int launch_bwd3(const BwdArgs &a, const float *kv_states, const float *dkv_states, const Geom &g_sweep,
                    hipStream_t st) {
   int rc = grant_lds<la_bwd3<E, SRC, MODE, W>>(sweep_lds<W>());
   if (rc) return rc;
+  Geom g = g_sweep;
+  if (256 / 3 * (int64_t)g.seg_len * 4 * (g.d + g.e) > kCacheBytes) g.stay = 0;  // dQ's
   const int64_t n_items = (int64_t)g.b * g.h * g.n_seg;
   const unsigned grid = (unsigned)(((n_items + 7) / 8) * 24);
   ProfScope prof(KC_BWD3, st);
