@@ -876,6 +876,11 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
     elem16_t *Og = Out + row0 * zp;
     const char *const o_from = smem + L::X + 16 * w * L::ROW + lane * 16;
     u32x4 out[4];
+    // Output is not read again here, and its stores say so, but the dV that the next slice of a wide head adds to: where the L2s hold it, it
+    // stays there.  Backward, us, d = 256: b*h = 8, n = 8192 94.5 -> 87.5, b*h = 32, n = 3000 130 -> 120; beyond, b*h = 24, n = 12000 308 -> 313,
+    // and in the forward, b*h = 4, n = 15761 60.1 -> 61.3, it would lose.
+    constexpr int64_t L2_BYTES = (int64_t)32 << 20;
+    const bool again = MODE == M_NARROW && REV && !TRANS && g.dt > W && (int64_t)(g.b * g.h) * g.n * g.e * 2 <= L2_BYTES;
     auto read_out = [&](int set) __attribute__((always_inline)) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) out[i] = lds16(o_from + set * L::SET + 4 * i * L::ROW);
@@ -883,9 +888,13 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
     auto store_out = [&](int k) __attribute__((always_inline)) {
       const int blk = first_blk + k * step;
       const rows_t rows = rows_of(Og + (int64_t)blk * BLK * zp, len_of(blk) * zp * 2);
+      if (again) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        __builtin_amdgcn_raw_buffer_store_b128(out[i], rows, (int)z_off[i], 0, 2 /* non-temporal */);
+        for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b128(out[i], rows, (int)z_off[i], 0, 0);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b128(out[i], rows, (int)z_off[i], 0, 2 /* non-temporal */);
+      }
     };
     // Everything that this wave has asked for but the loads of block 1 has arrived
     if (run == 1)
