@@ -229,6 +229,13 @@ int lasp_chunk_bwd(const void *q, const void *k, const void *v, const float *s,
                    int dtype, int seg_len, void *stream);
 
 /*
+ * How lasp_chunk_bwd goes over a chunk on the 16-bit kernels (a pure function of its arguments, for tests and measurements): the tokens
+ * of one workgroup's sweep, a multiple of seg_len, and the tokens from one DKV state to the next, which divide them.  Both 0 where it
+ * does not run a pre-pass, a scan and a sweep.
+ */
+int lasp_bwd_rows(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, int *row_tokens, int *piece_tokens);
+
+/*
  * lasp_chunk_fwd / lasp_chunk_bwd that leave the outgoing state in two places: kv_out (dkv_out), which must then be
  * wanted, and kv_twin (dkv_twin), a buffer of the same size that overlaps neither state of the call.  For a caller that
  * keeps the state and hands a copy to the next chunk; NULL is the plain call.

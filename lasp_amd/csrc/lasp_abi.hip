@@ -392,6 +392,13 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
   return 0;
 }
 
+// Whether `seg_len`, which gave `g`, is the library's own choice: callers pass a forward's on to its backward.
+bool is_planned(const Geom &g, int dtype, int seg_len) {
+  if (seg_len == 0 || !g.width) return seg_len == 0;
+  Geom own;
+  return make_geom(g.b, g.h, g.n, g.dt, g.e, dtype, 0, &own) == 0 && !own.fused && own.seg_len == g.seg_len;
+}
+
 // The kernels fetch rows of q/k/v/do with 8- and 16-byte loads and store o/dq/dk/dv with 16-byte stores,
 // and read states as floats: tensors must start on a 16-byte boundary, states on a 4-byte one.
 int check_aligned(const char *call, const char *name, const void *p, size_t align) {
@@ -623,6 +630,17 @@ int lasp_inplace_ok(int b, int h, int64_t n, int d, int e, int dtype, int seg_le
   return inplace_ok(g, backward != 0) ? 1 : 0;
 }
 
+int lasp_bwd_rows(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, int *row_tokens, int *piece_tokens) {
+  Geom g;
+  const int rc = make_geom(b, h, n, d, e, dtype, seg_len, &g);
+  if (rc) return rc;
+  int row = 0, piece = 0;
+  if (mfma_eligible(d, e, dtype)) mfma_bwd_rows(g, is_planned(g, dtype, seg_len), &row, &piece);
+  if (row_tokens) *row_tokens = row;
+  if (piece_tokens) *piece_tokens = piece;
+  return 0;
+}
+
 int lasp_whole_ok(int b, int h, int64_t n, int d, int e, int dtype, int backward_follows) {
   if (!mfma_eligible(d, e, dtype)) return 0;
   Geom g;
@@ -813,11 +831,7 @@ static int bwd_twin(const void *q, const void *k, const void *v, const float *s,
     return rc;
   if ((rc = check_device(me, q))) return rc;
   (void)hipGetLastError();  // an earlier, unrelated error of this thread is not this call's
-  bool planned = seg_len == 0;
-  if (!planned && g.width) {  // (callers pass the forward's seg_len on)
-    Geom own;
-    planned = make_geom(b, h, n, d, e, dtype, 0, &own) == 0 && !own.fused && own.seg_len == g.seg_len;
-  }
+  const bool planned = is_planned(g, dtype, seg_len);
   BwdArgs a{q,  k,  v,       s,
             d_o, kv_in, dkv_in, dq,
             dk, dv, dkv_out, kv_seg_states,

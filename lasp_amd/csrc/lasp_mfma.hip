@@ -2288,6 +2288,13 @@ int mfma_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
 int mfma_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
   return dtype == LASP_DTYPE_F16 ? mfma_f16_bwd(a, g, st) : bwd_w<ElemBF16>(a, g, st);
 }
+void mfma_bwd_rows(const Geom &g, bool planned, int *row, int *piece) {
+  *row = *piece = 0;
+  if (g.fused || g.combine || (planned && g.width == kMaxWidth && g.dt <= kMaxWidth && whole_bwd_pays(g))) return;
+  const Geom gw = g.width == 64 ? bwd_sweep_geom<64>(g) : bwd_sweep_geom<kMaxWidth>(g);
+  *row = gw.seg_len;
+  *piece = g.width == 64 ? g.pre_len : rev_pass_geom(g, gw).seg_len;
+}
 bool mfma_whole(const Geom &g, bool backward_follows) {
   return !g.fused && g.width == kMaxWidth && g.dt <= kMaxWidth && whole_fwd_pays(g) && (!backward_follows || whole_bwd_pays(g));
 }

@@ -3,7 +3,7 @@ for heads that the scan takes and heads that it leaves out, one piece from the o
 import pytest
 import torch
 
-from helpers import check, make_inputs, oracle
+from helpers import bwd_rows, check, make_inputs, oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +45,59 @@ def test_matches_oracle(gpu_device, b, h, n, d, e, seg_len, dtype, decay):
     bare = dict(inp, kv=torch.zeros_like(inp["kv"]), dkv=torch.zeros_like(inp["dkv"]))
     want, got = oracle(bare, s), run(False)
     check(got, {k: want[k] for k in got}, TOL[dtype], what=what + ", no states")
+
+
+def chunk_bwd_over(fill, inp, s, kv_in, dkv_in, dkv_out, seg_len):
+    """lasp_chunk_bwd without kept states, in a workspace that holds `fill` everywhere: (dq, dk, dv)."""
+    from lasp_amd import _abi
+
+    q, v = inp["q"], inp["v"]
+    b, h, n, d, e = *q.shape, v.shape[-1]
+    seg_len, _, nbytes = _abi.plan(b, h, n, d, e, q.dtype, seg_len)
+    ws = torch.full((2 * nbytes // 4,), fill, device=q.device)
+    dq, dk, dv = [torch.empty_like(t) for t in (q, q, v)]
+    p = lambda t: None if t is None else t.data_ptr()
+    rc = _abi.load().lasp_chunk_bwd(p(q), p(inp["k"]), p(v), p(s), p(inp["do"]), p(kv_in), p(dkv_in), p(dq), p(dk), p(dv), p(dkv_out),
+                                    None, p(ws), 2 * nbytes, b, h, n, d, e, _abi.DTYPE_CODE[q.dtype], seg_len,
+                                    torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _abi.load().lasp_last_error()
+    return dq, dk, dv
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,h,n,d,e,seg_len", [
+    (2, 24, 320, 128, 128, 64), (1, 64, 449, 256, 128, 64),  # five segments, eight with one token in the last
+    (1, 41, 431, 96, 80, 64),                                # narrow rows
+    (4, 16, 1536, 512, 128, 0),                              # the library's own plan
+])
+def test_one_row_of_segments(gpu_device, b, h, n, d, e, seg_len, dtype):
+    """A sweep over the whole chunk, whose DKV states may be a single one: it has no neighbour to take a state from, so no head, whatever
+    the next one or the workspace holds, leaves anything but its own sum."""
+    assert bwd_rows(b, h, n, d, e, dtype, seg_len)[0] >= n
+    inp = make_inputs(b, h, n, d, e, dtype, seed=n + d + e, scale=0.3, state=True, state_std=1.0)
+    # every state dies within the chunk; the slowest is at 2^-25 after it, which a head 2^20 times as large would show
+    s = torch.linspace(0.5, 25 / (1.4427 * n), h)
+    loud = torch.arange(b * h).view(b, h) % 3 == 1
+    if dtype == torch.bfloat16:
+        inp["do"][loud] *= 2.0 ** 20
+        inp["dkv"][loud] *= 2.0 ** 20
+    dev, sd = {k: v.to(gpu_device) for k, v in inp.items()}, s.to(gpu_device)
+    what = f"b={b} h={h} n={n} d={d} e={e} {dtype}"
+
+    def run(do, carried, fill=float("nan")):
+        kv, dkv = (dev["kv"], dev["dkv"]) if carried else (None, None)
+        out = torch.full_like(dev["kv"], float("nan"))
+        grads = chunk_bwd_over(fill, dict(dev, do=do), sd, kv, dkv, out, seg_len)
+        bare = chunk_bwd_over(fill, dict(dev, do=do), sd, kv, dkv, None, seg_len)  # (the outgoing state not wanted)
+        return dict(zip(("dq", "dk", "dv"), grads), dkv_out=out), dict(zip(("dq", "dk", "dv"), bare))
+
+    for carried in (True, False):
+        want = oracle(inp if carried else dict(inp, kv=torch.zeros_like(inp["kv"]), dkv=torch.zeros_like(inp["dkv"])), s)
+        got, bare = run(dev["do"], carried)
+        check(got, {k: want[k] for k in got}, TOL[dtype], what=what)
+        check(bare, {k: want[k] for k in bare}, TOL[dtype], what=what + ", no outgoing state")
+        # heads that overflow leave the others' bits alone
+        do = dev["do"].clone()
+        do[loud.to(gpu_device)] = float("inf")
+        for name, x in run(do, carried, fill=0.0)[0].items():
+            assert torch.equal(x[~loud.to(gpu_device)], got[name][~loud.to(gpu_device)]), (what, name)
