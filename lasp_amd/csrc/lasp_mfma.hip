@@ -2132,7 +2132,7 @@ bool whole_bwd(const BwdArgs &a, const Geom &g) {
 // nearest), b*h = 112, n = 3600 115 and 99, b*h = 200, n = 5400 295 and 222; d = 96, b*h = 80, n = 2600 72.9 and 47.1.  Of 160 shapes that
 // take it (four widths, b*h = 13 ... 512, n = 1100 ... 6144) the slowest is at 1.006 of its three kernels, the mean at 0.84.
 // KV_out is one sum over the whole chunk, as DKV_out is backwards: without decay 2.9e-7 off 64 bits at b*h = 24, n = 2048 where sums of
-// segments are 1.0e-7, 5.0e-7 and 3.7e-7 at b*h = 120, n = 6000; with decay 1.66e-3 (bf16) and 2.07e-4 (fp16) either way, the rounding
+// segments are 1.0e-7, 5.0e-7 and 3.7e-7 at b*h = 120, n = 6000, so the operators take it only where no state leaves; with decay 1.66e-3 (bf16) and 2.07e-4 (fp16) either way, the rounding
 // of its operand, and O 1.7e-3 to 2.7e-3 either way.
 constexpr int64_t kWholeFwdNarrow = 80, kWholeFwdGathered = 64;
 bool whole_fwd_pays(const Geom &g) {
