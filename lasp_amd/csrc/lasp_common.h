@@ -150,7 +150,7 @@ int mfma_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st);
 int mfma_f16_fwd(const FwdArgs &a, const Geom &g, hipStream_t st);
 int mfma_f16_bwd(const BwdArgs &a, const Geom &g, hipStream_t st);
 // tokens that one backward sweep goes over, and that its DKV states lie apart; 0 where the backward is one launch or gathers its states
-void mfma_bwd_rows(const Geom &g, bool planned, int *row, int *piece);
+void mfma_bwd_rows(const Geom &g, bool planned, bool state_leaves, int *row, int *piece);
 // 16-bit chunks whose forward takes one launch where no segment states are wanted (and whose backward then takes one as well)
 bool mfma_whole(const Geom &g, bool backward_follows);
 int mfma_whole_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st);

@@ -1972,10 +1972,11 @@ Geom pre_pass_geom(const Geom &g) {
   gp.by_seg = divisor_of((uint32_t)gp.n_seg);
   return gp;
 }
-// The same for DKV in a backward whose sweeps (`gw`) go over several of the forward's segments in a row: nothing but those sweeps reads
-// its states, so they may lie as far apart as the sweeps start.  Fewer of them are written by the pre-pass, read and written by the scan;
-// the pre-pass's walks are longer and fewer.  The least 20 x blocks of a walk + walks is taken (a block takes some 0.6 us, a state
-// 0.03), for a wide head, whose slices wait for one another's bytes, if it saves a ninth.  Backward with states, us, states at the forward's
+// The same for DKV in a backward whose sweeps (`gw`) go over several of the forward's segments in a row and which leaves no state: nothing
+// but those sweeps reads its states, so they may lie as far apart as the sweeps start.  (Not where DKV_out leaves, the sum of longer
+// pieces: without decay up to 1.13 times as far from 64 bits, fp16, b*h = 16, n = 1536, d = 192 1.09e-7 and 0.96e-7.)  Fewer of them are
+// written by the pre-pass, read and written by the scan; the pre-pass's walks are longer and fewer.  The least 20 x blocks of a walk + walks is taken (a block takes some 0.6 us, a state
+// 0.03), for a wide head, whose slices wait for one another's bytes, if it saves a ninth.  Backward with kept states, us, states at the forward's
 // segments and by this rule: b*h = 8, n = 8192, d = 256 102.2 and 94.8 (512 tokens apart, not 256; 1024 97.9), d = 192 93.1 and 87.2;
 // d = 256, b*h = 16, n = 4000 96.6 and 89.0, b*h = 32, n = 2339 113.5 and 105.7, b*h = 4, n = 7593 56.4 and 51.0; d = 128, b*h = 8, n = 3784
 // 30.1 and 28.3, b*h = 4, n = 7521 33.1 and 30.1.
@@ -2144,9 +2145,10 @@ bool whole_fwd_pays(const Geom &g) {
 
 // Segments of the backward sweeps: m of the plan's in a row.  The plan's segments give the forward a workgroup per CU; three roles of them
 // take one round and a half to three, each with its start-up -- the first tiles, the entering state, the last stores -- of about five
-// blocks' time, and half of a last round is empty.  The states lie at the plan's segments either way (a sweep takes the one that enters
-// its first), so the forward, the pre-passes and the scans stay as they are.  m is the one with the least rounds x (blocks + 5), a round
-// being 32 workgroups on each XCD, as launch_bwd3 deals items out, if that saves 3 %.  bf16, backward with states, us, m = 1 and m:
+// blocks' time, and half of a last round is empty.  The KV states lie at the plan's segments either way (a sweep takes the one that enters
+// its first), so the forward and the KV pre-pass and scan stay as they are; DKV's lie at them or as rev_pass_geom says, at lengths that
+// divide a sweep's and that the plan's pieces divide: at most as many, so that they fit the workspace, and as few as one.  m is the one with the least rounds x (blocks + 5), a round
+// being 32 workgroups on each XCD, as launch_bwd3 deals items out, if that saves 3 %.  bf16, backward with kept states, us, m = 1 and m:
 // b*h = 4, n = 8192 38.2 and 34.0 (m = 2: one round of 8 blocks for two of 4), b*h = 8, n = 3784 35.5 and 31.1 (2), b*h = 16, n = 8192 87.9
 // and 81.2 (4: one round of 32 for three of 8), b*h = 20, n = 3757, d = 96 52.7 and 43.3 (3), b*h = 16, n = 1536, d = 192 55.9 and 47.9 (2).
 // A last segment of the plan's less than a fifth full makes no round of its own (b*h = 10, n = 8226: 3.4 % slower with m = 3).  Over 225 shapes
@@ -2208,7 +2210,7 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
   }
   const Geom gp = pre_pass_geom(g);
   Geom gw = bwd_sweep_geom<W>(g);
-  const Geom gr = W == kMaxWidth ? rev_pass_geom(g, gw) : gp;
+  const Geom gr = W == kMaxWidth && !a.dkv_out ? rev_pass_geom(g, gw) : gp;
   gw.rev_len = gr.seg_len;
   gw.rev_n = gr.n_seg;
   const int sub = gw.seg_len / g.pre_len;  // pre-pass segments per sweep segment
@@ -2288,12 +2290,12 @@ int mfma_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
 int mfma_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
   return dtype == LASP_DTYPE_F16 ? mfma_f16_bwd(a, g, st) : bwd_w<ElemBF16>(a, g, st);
 }
-void mfma_bwd_rows(const Geom &g, bool planned, int *row, int *piece) {
+void mfma_bwd_rows(const Geom &g, bool planned, bool state_leaves, int *row, int *piece) {
   *row = *piece = 0;
   if (g.fused || g.combine || (planned && g.width == kMaxWidth && g.dt <= kMaxWidth && whole_bwd_pays(g))) return;
   const Geom gw = g.width == 64 ? bwd_sweep_geom<64>(g) : bwd_sweep_geom<kMaxWidth>(g);
   *row = gw.seg_len;
-  *piece = g.width == 64 ? g.pre_len : rev_pass_geom(g, gw).seg_len;
+  *piece = g.width == 64 || state_leaves ? g.pre_len : rev_pass_geom(g, gw).seg_len;
 }
 bool mfma_whole(const Geom &g, bool backward_follows) {
   return !g.fused && g.width == kMaxWidth && g.dt <= kMaxWidth && whole_fwd_pays(g) && (!backward_follows || whole_bwd_pays(g));

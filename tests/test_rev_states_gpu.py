@@ -47,6 +47,31 @@ def test_matches_oracle(gpu_device, b, h, n, d, e, seg_len, dtype, decay):
     check(got, {k: want[k] for k in got}, TOL[dtype], what=what + ", no states")
 
 
+@pytest.mark.parametrize("b,h,n,d,e,seg_len", [(1, 16, 1088, 128, 128, 64), (2, 16, 449, 128, 128, 64), (1, 10, 1300, 192, 128, 64),
+                                               (1, 12, 1999, 96, 128, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_state_that_leaves_is_a_sum_of_the_same_pieces(gpu_device, b, h, n, d, e, seg_len, dtype):
+    """DKV_out has the bits that a call of few heads gives, whose sweeps go over one segment each: its pieces are the forward's, also where
+    the states that only the sweeps read would lie further apart."""
+    from lasp_amd import _abi
+
+    row, piece = bwd_rows(b, h, n, d, e, dtype, seg_len, False)
+    assert row >= piece > seg_len and bwd_rows(b, h, n, d, e, dtype, seg_len, True) == (row, seg_len)
+    assert bwd_rows(1, 1, n, d, e, dtype, seg_len, False) == (seg_len, seg_len)
+    dev = make_inputs(b, h, n, d, e, dtype, seed=n + d, scale=0.3, state=True, state_std=1.0, device=gpu_device)
+    s = torch.linspace(0.05, 0.0, h, device=gpu_device)
+
+    def run(part, s):
+        out = torch.full_like(part["kv"], float("nan"))
+        _abi.chunk_bwd(part["q"], part["k"], part["v"], s, part["do"], part["kv"], part["dkv"], out, None, seg_len)
+        return out
+
+    whole = run(dev, s)
+    for i in range(h):
+        one = run({k: v[:1, i:i + 1].contiguous() for k, v in dev.items()}, s[i:i + 1].contiguous())
+        assert torch.equal(one, whole[:1, i:i + 1]), i
+
+
 def chunk_bwd_over(fill, inp, s, kv_in, dkv_in, dkv_out, seg_len):
     """lasp_chunk_bwd without kept states, in a workspace that holds `fill` everywhere: (dq, dk, dv)."""
     from lasp_amd import _abi
@@ -73,7 +98,7 @@ def chunk_bwd_over(fill, inp, s, kv_in, dkv_in, dkv_out, seg_len):
 def test_one_row_of_segments(gpu_device, b, h, n, d, e, seg_len, dtype):
     """A sweep over the whole chunk, whose DKV states may be a single one: it has no neighbour to take a state from, so no head, whatever
     the next one or the workspace holds, leaves anything but its own sum."""
-    assert bwd_rows(b, h, n, d, e, dtype, seg_len)[0] >= n
+    assert bwd_rows(b, h, n, d, e, dtype, seg_len, False) == (-(-n // seg_len) * seg_len if seg_len else n,) * 2
     inp = make_inputs(b, h, n, d, e, dtype, seed=n + d + e, scale=0.3, state=True, state_std=1.0)
     # every state dies within the chunk; the slowest is at 2^-25 after it, which a head 2^20 times as large would show
     s = torch.linspace(0.5, 25 / (1.4427 * n), h)
