@@ -1,5 +1,5 @@
 """The single-launch kernels cut a (b, h) into segments that are shorter the longer the walk before them, for heads whose decay reaches
-far, and into equal ones for the others: both in one call, at sizes around the smallest and the largest number of segments."""
+far, and into equal ones for the others: both in one call, at sizes from one block on."""
 import pytest
 import torch
 
@@ -15,7 +15,7 @@ REL = {torch.bfloat16: 1.2e-2, torch.float16: 1.6e-3}
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("b,h,n,d,e", [
     (1, 6, 64, 128, 128), (1, 6, 65, 128, 128), (2, 4, 256, 128, 128),  # one block, two, four
-    (1, 5, 1000, 128, 128), (4, 8, 1024, 128, 128),                     # seven segments forwards, the last of one block
+    (1, 5, 1000, 128, 128), (4, 8, 1024, 128, 128),                     # six segments forwards, the last three of one block
     (5, 32, 500, 128, 128), (1, 130, 128, 128, 128),                    # one segment each, and in the backward a cut last round
     (1, 16, 1024, 64, 64), (3, 40, 700, 64, 48),                        # the 64-wide kernels
     (1, 6, 900, 96, 40), (1, 3, 600, 192, 128),                         # narrow rows, slices of wide ones

@@ -11,19 +11,26 @@ pytestmark = pytest.mark.gpu
 TOL = {torch.bfloat16: 2e-2, torch.float16: 2e-2 / 8}
 
 
+# (b, h, n, d, e, seg_len): segments from one DKV state to the next where none leaves, as the rule has them, and how many states that are
+SHAPES = {
+    (1, 16, 1088, 128, 128, 64): (4, 5), (2, 8, 1100, 128, 128, 64): (4, 5),  # the last piece one block; one block and 12 tokens
+    (1, 12, 897, 128, 128, 64): (3, 5), (1, 16, 641, 128, 64, 64): (3, 4),    # one token in the last segment
+    (1, 12, 1999, 128, 128, 64): (3, 11),                                     # sweeps over six, pieces of three
+    (2, 16, 449, 128, 128, 64): (4, 2), (1, 20, 520, 128, 128, 64): (3, 3),
+    (1, 8, 700, 256, 128, 64): (2, 6), (1, 10, 1300, 192, 128, 64): (3, 7), (1, 16, 385, 200, 72, 64): (2, 4),  # slices
+    (1, 8, 3784, 128, 128, 0): (2, 10), (1, 16, 1536, 192, 128, 0): (2, 4),   # default plans
+}
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("b,h,n,d,e,seg_len", [
-    (1, 16, 1088, 128, 128, 64), (2, 8, 1100, 128, 128, 64),  # four of the forward's segments each; the last piece one block and 12 tokens
-    (1, 12, 897, 128, 128, 64), (1, 16, 641, 128, 64, 64),    # three; one token in the last one
-    (1, 12, 1999, 128, 128, 64),                              # sweeps over six, pieces of three
-    (2, 16, 449, 128, 128, 64), (1, 20, 520, 128, 128, 64),   # two pieces, three
-    (1, 8, 700, 256, 128, 64), (1, 10, 1300, 192, 128, 64), (1, 16, 385, 200, 72, 64),  # slices
-    (1, 8, 3784, 128, 128, 0), (1, 16, 1536, 192, 128, 0),    # default plans
-])
+@pytest.mark.parametrize("b,h,n,d,e,seg_len", SHAPES)
 @pytest.mark.parametrize("decay", [(0.4, 0.003), (0.9, 0.08), (0.0, 0.0)])
 def test_matches_oracle(gpu_device, b, h, n, d, e, seg_len, dtype, decay):
     from lasp_amd import _abi
 
+    apart, states = SHAPES[b, h, n, d, e, seg_len]
+    piece = bwd_rows(b, h, n, d, e, dtype, seg_len, False)[1]
+    assert (piece, -(-n // piece)) == (apart * _abi.plan(b, h, n, d, e, dtype, seg_len)[0], states)
     inp = make_inputs(b, h, n, d, e, dtype, seed=n + d + e, scale=0.3, state=True, state_std=1.0)
     dev = {k: v.to(gpu_device) for k, v in inp.items()}
     s = torch.linspace(*decay, h)

@@ -3,7 +3,7 @@ takes them, in either element type, for every width that has them, from kept sta
 import pytest
 import torch
 
-from helpers import check, make_inputs, oracle
+from helpers import bwd_rows, check, make_inputs, oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -12,20 +12,31 @@ pytestmark = pytest.mark.gpu
 TOL = {torch.bfloat16: 2e-2, torch.float16: 2e-2 / 8}
 
 
+# (b, h, n, d, e, seg_len): segments in a row, as the rule has them
+SHAPES = {
+    (1, 4, 7168, 128, 128, 0): 2, (1, 4, 6800, 128, 128, 0): 2,      # rows of the library's own segments; a ragged last one
+    (1, 5, 2600, 128, 128, 192): 1,                                  # one round as it is
+    (1, 2, 8129, 96, 80, 256): 1,                                    # ... of narrow rows, one token in the last segment
+    (1, 16, 1600, 192, 128, 0): 2, (1, 3, 4161, 256, 72, 128): 2,    # slices
+    (1, 10, 2570, 128, 128, 256): 2,                                 # a last segment too small to count
+    (1, 7, 1280, 128, 64, 64): 2, (1, 1, 4096, 128, 128, 64): 1,
+    (1, 3, 520, 128, 128, 64): 1, (1, 6, 2049, 64, 64, 192): 1,      # the last one: heads that never take it
+    (1, 27, 309, 128, 128, 64): 3, (1, 27, 309, 256, 72, 64): 3,     # a second row of two segments, the last ragged
+    (1, 9, 553, 96, 80, 64): 2, (1, 41, 309, 96, 80, 64): 5,         # narrow rows
+    (1, 27, 919, 128, 128, 64): 8,                                   # the most in a row, twice
+    (1, 41, 431, 128, 128, 64): 7, (1, 41, 492, 128, 128, 64): 8,    # rows that are the whole chunk
+    (1, 57, 2225, 128, 128, 512): 5, (1, 57, 1378, 256, 64, 192): 8,  # rows of 40 blocks, and of 24 of a slice: the longest
+}
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("b,h,n,d,e,seg_len", [
-    (1, 4, 7168, 128, 128, 0), (1, 4, 6800, 128, 128, 0),     # two in a row; an odd number of segments, the last one ragged
-    (1, 5, 2600, 128, 128, 192),                              # 14 of 192, three in a row, the last row short
-    (1, 2, 8129, 96, 80, 256),                                # narrow rows, one token in the last segment
-    (1, 16, 1600, 192, 128, 0), (1, 3, 4161, 256, 72, 128),   # slices
-    (1, 10, 2570, 128, 128, 256),                             # a last segment too small to count
-    (1, 7, 1280, 128, 64, 64), (1, 1, 4096, 128, 128, 64),    # eight in a row; a row of four blocks
-    (1, 3, 520, 128, 128, 64), (1, 6, 2049, 64, 64, 192),     # rows that are the whole chunk; heads that never take it
-])
+@pytest.mark.parametrize("b,h,n,d,e,seg_len", SHAPES)
 @pytest.mark.parametrize("decay", [True, False])
 def test_matches_oracle(gpu_device, b, h, n, d, e, seg_len, dtype, decay):
     from lasp_amd import _abi
 
+    segment = _abi.plan(b, h, n, d, e, dtype, seg_len)[0]
+    assert bwd_rows(b, h, n, d, e, dtype, seg_len, True)[0] == SHAPES[b, h, n, d, e, seg_len] * segment
     inp = make_inputs(b, h, n, d, e, dtype, seed=n + d + e, scale=0.3, state=True, state_std=1.0)
     dev = {k: v.to(gpu_device) for k, v in inp.items()}
     s = torch.linspace(0.4, 0.003, h) if decay else torch.zeros(h)  # heads that the scan leaves out, and heads that it does not
@@ -45,7 +56,7 @@ def test_matches_oracle(gpu_device, b, h, n, d, e, seg_len, dtype, decay):
     check(got, {k: want[k] for k in got}, TOL[dtype], what=what)
     for name, x in run(True, False, seg_len).items():  # the states are the same ones
         assert torch.equal(x, got[name]), (what, name)
-    other = 2560 if n > 2560 else 512  # swept one by one: longer than any row
+    other = 2560 if n > 2560 else 512  # swept one by one
     check(got, run(True, True, other), TOL[dtype], what=what + ", other segments")
 
     bare = dict(inp, kv=torch.zeros_like(inp["kv"]), dkv=torch.zeros_like(inp["dkv"]))

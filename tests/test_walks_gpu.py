@@ -1,5 +1,6 @@
-"""Walks over the blocks before (after) a segment, of every length from none on: the last few (b, h) of these backwards are cut into
-segments of one block.  The products of a walk block are split over two blocks' time, so that odd and even walks end differently."""
+"""Walks over the blocks before (after) a segment, of every length from none to seven: the last few (b, h) of these backwards are cut, eight
+blocks for heads whose decay reaches far at 0, 3, 5, 6 and 7, for the others into equal segments whose walks end at the reach.  The products
+of a walk block are split over two blocks' time, so that odd and even walks end differently."""
 import pytest
 import torch
 
@@ -14,10 +15,10 @@ REL = {torch.bfloat16: 1.2e-2, torch.float16: 1.6e-3}
 
 @pytest.mark.parametrize("h,n,d,e,dtype", [
     (82, 450, 128, 128, torch.bfloat16),  # eight blocks, the last with two tokens
-    (81, 448, 128, 128, torch.float16),   # seven whole ones
-    (83, 130, 96, 72, torch.bfloat16),    # narrow rows, at most two
+    (81, 448, 128, 128, torch.float16),   # seven whole ones, cut at 0, 3, 5 and 6
+    (83, 130, 96, 72, torch.bfloat16),    # narrow rows, walks of none, one and two
 ])
-@pytest.mark.parametrize("slope", [0.0, 0.01, 0.2])  # walks to the chunk's end, and as far as the decay reaches
+@pytest.mark.parametrize("slope", [0.0, 0.01, 0.07, 0.2])  # walks to the chunk's end; as far as the decay reaches, four blocks and two
 def test_walks_of_every_length(gpu_device, h, n, d, e, dtype, slope):
     g = torch.Generator().manual_seed(h + n)
     mk = lambda w: (torch.randn(1, h, n, w, generator=g) / w ** 0.5).to(dtype)

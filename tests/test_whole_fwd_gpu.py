@@ -31,6 +31,7 @@ def close(got, want, dtype, what):
 @pytest.mark.parametrize("b,h,n,d,e,whole", [
     (2, 12, 2048, 128, 128, True), (1, 16, 1408, 128, 128, True), (1, 16, 1409, 128, 128, False),
     (1, 30, 2111, 128, 128, True), (2, 40, 1601, 96, 80, True),  # a partial last block, narrow rows
+    (1, 32, 2816, 128, 128, True),                               # 44 blocks, the fewest that a forward cuts into eight segments, the most
     (1, 90, 2100, 128, 64, True), (2, 12, 2048, 64, 64, False),  # more (b, h) than places for two segments; the 64-wide kernels
 ])
 def test_attention(gpu_device, b, h, n, d, e, whole, dtype):
