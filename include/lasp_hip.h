@@ -232,10 +232,9 @@ int lasp_chunk_bwd(const void *q, const void *k, const void *v, const float *s,
 
 /*
  * How lasp_chunk_bwd goes over a chunk on the 16-bit kernels (a pure function of its arguments, for tests and measurements): the tokens
- * of one workgroup's sweep, a multiple of seg_len, and the tokens from one DKV state to the next, which divide them and are the
- * forward's where a state leaves (dkv_out).  Both 0 where it does not run a pre-pass, a scan and a sweep.
+ * of one workgroup's sweep, a multiple of seg_len, or 0 where it does not run a pre-pass, a scan and a sweep.
  */
-int lasp_bwd_rows(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, int state_leaves, int *row_tokens, int *piece_tokens);
+int lasp_bwd_rows(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, int *row_tokens);
 
 /*
  * lasp_chunk_fwd / lasp_chunk_bwd that leave the outgoing state in two places: kv_out (dkv_out), which must then be

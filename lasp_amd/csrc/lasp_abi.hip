@@ -377,8 +377,6 @@ int make_geom(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, Geo
     if (pre <= kPreMaxSeg) g->pre_len = pre;
   }
   g->pre_n = (int)((n + g->pre_len - 1) / g->pre_len);
-  g->rev_len = g->pre_len;
-  g->rev_n = g->pre_n;
   g->stay = 1 << 30;
   g->kept = KEPT_NONE;
   g->cut = Cut{0, 0, 0};
@@ -630,14 +628,11 @@ int lasp_inplace_ok(int b, int h, int64_t n, int d, int e, int dtype, int seg_le
   return inplace_ok(g, backward != 0) ? 1 : 0;
 }
 
-int lasp_bwd_rows(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, int state_leaves, int *row_tokens, int *piece_tokens) {
+int lasp_bwd_rows(int b, int h, int64_t n, int d, int e, int dtype, int seg_len, int *row_tokens) {
   Geom g;
   const int rc = make_geom(b, h, n, d, e, dtype, seg_len, &g);
   if (rc) return rc;
-  int row = 0, piece = 0;
-  if (mfma_eligible(d, e, dtype)) mfma_bwd_rows(g, is_planned(g, dtype, seg_len), state_leaves != 0, &row, &piece);
-  if (row_tokens) *row_tokens = row;
-  if (piece_tokens) *piece_tokens = piece;
+  if (row_tokens) *row_tokens = mfma_eligible(d, e, dtype) ? mfma_bwd_row(g, is_planned(g, dtype, seg_len)) : 0;
   return 0;
 }
 

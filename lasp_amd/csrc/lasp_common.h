@@ -92,7 +92,6 @@ struct Geom {
                 // segments are cut finer for the pre-pass (16-bit scan path only)
   Divisor by_seg, by_h;  // n_seg and h
   int pre_n;    // ceil(n / pre_len): states per (b, h) in the workspace
-  int rev_len, rev_n;  // the same of a 16-bit backward's own states (DKV), which may lie further apart
   int stay;     // forward sweeps and dQ: blocks at a segment's end that are loaded to stay in the memory-side cache (see launch_apply)
   int kept;     // a backward in one launch: what its kv_in is, see Kept
   Cut cut;      // single-launch kernels only
@@ -114,11 +113,10 @@ constexpr int kMaxWidth = 128;  // features that one sweep works on
 // end, so the state entering segment j is the OWN state of the segment before it (after it, going
 // backwards) and, for the first segment visited, the chunk's incoming state.  The scan kernel
 // leaves those heads' own states in place and only forms their outgoing carry; the sweeps read the
-// neighbour's own state.  Both sides must take the same decision, hence this one function.  A backward whose DKV states lie
-// as far apart as the whole chunk has one piece and no neighbour: there every head takes part.
+// neighbour's own state.  Both sides must take the same decision, hence this one function.
 __device__ __forceinline__ bool state_dies_in_segment(float slope, const Geom &g) {
   const int64_t last_len = g.n - (int64_t)(g.pre_n - 1) * g.pre_len;  // segments of the pre-pass and the scan
-  return g.bypass != 0 && g.pre_n > 1 && slope * kLog2e * (float)last_len > kSkipLog2;
+  return g.bypass != 0 && slope * kLog2e * (float)last_len > kSkipLog2;
 }
 
 // Host-side launchers (each returns a hipError_t as int, or a negative LASP_E_*).
@@ -149,8 +147,7 @@ int mfma_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st);  // bf
 int mfma_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st);
 int mfma_f16_fwd(const FwdArgs &a, const Geom &g, hipStream_t st);
 int mfma_f16_bwd(const BwdArgs &a, const Geom &g, hipStream_t st);
-// tokens that one backward sweep goes over, and that its DKV states lie apart; 0 where the backward is one launch or gathers its states
-void mfma_bwd_rows(const Geom &g, bool planned, bool state_leaves, int *row, int *piece);
+int mfma_bwd_row(const Geom &g, bool planned);  // tokens that one backward sweep goes over; 0 where the backward is one launch or gathers its states
 // 16-bit chunks whose forward takes one launch where no segment states are wanted (and whose backward then takes one as well)
 bool mfma_whole(const Geom &g, bool backward_follows);
 int mfma_whole_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st);

@@ -1489,15 +1489,6 @@ la_bwd3(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, const el
   const int grp = blockIdx.x / 24, r = blockIdx.x - grp * 24;
   const int role = r >> 3;
   const int item = n_items - 1 - (grp * 8 + (r & 7));
-  if (SRC == SRC_SCANNED && W == kMaxWidth) {
-    int len = g.rev_len, n = g.rev_n;
-    // (asked for here, with the arguments that everything waits for: where a role needs them they cost every call 0.5 us)
-    asm volatile("" : "+s"(len), "+s"(n));
-    if (role != 0) {
-      g.pre_len = len;
-      g.pre_n = n;
-    }
-  }
   if (item < 0) return;
   if (role == 0)
     any_body<E, false, true, SRC, MODE, W>(DO, V, K, S, kv_states, DQ, g, g.e, g.d, item, smem, kv_in);
@@ -1972,27 +1963,6 @@ Geom pre_pass_geom(const Geom &g) {
   gp.by_seg = divisor_of((uint32_t)gp.n_seg);
   return gp;
 }
-// The same for DKV in a backward whose sweeps (`gw`) go over several of the forward's segments in a row and which leaves no state: nothing
-// but those sweeps reads its states, so they may lie as far apart as the sweeps start.  (Not where DKV_out leaves, the sum of longer
-// pieces: without decay up to 1.13 times as far from 64 bits, fp16, b*h = 16, n = 1536, d = 192 1.09e-7 and 0.96e-7.)  Fewer of them are
-// written by the pre-pass, read and written by the scan; the pre-pass's walks are longer and fewer.  The least 20 x blocks of a walk + walks is taken (a block takes some 0.6 us, a state
-// 0.03), for a wide head, whose slices wait for one another's bytes, if it saves a ninth.  Backward with kept states, us, states at the forward's
-// segments and by this rule: b*h = 8, n = 8192, d = 256 102.2 and 94.8 (512 tokens apart, not 256; 1024 97.9), d = 192 93.1 and 87.2;
-// d = 256, b*h = 16, n = 4000 96.6 and 89.0, b*h = 32, n = 2339 113.5 and 105.7, b*h = 4, n = 7593 56.4 and 51.0; d = 128, b*h = 8, n = 3784
-// 30.1 and 28.3, b*h = 4, n = 7521 33.1 and 30.1.
-// b*h = 16, n = 8192 stays at 512 (82.6, 1024 83.3).  Over 53 shapes (b*h = 4 ... 32, n = 1594 ... 14632, six of seven of them with d > 128) that
-// would take fewer states without the ninth 0.96 of the time on average; wide heads that save less came out between 0.96 and 1.02.
-constexpr int kRevBlock = 20;
-Geom rev_pass_geom(const Geom &g, const Geom &gw) {
-  Geom gp = g;
-  const int64_t heads = (int64_t)g.b * g.h * slices_of(g);
-  auto cost = [&](int len) { return kRevBlock * (int64_t)(len / BLK) + heads * ((g.n + len - 1) / len); };
-  const int64_t enough = g.dt > kMaxWidth ? cost(g.pre_len) * 8 / 9 : cost(g.pre_len);
-  for (int len = 2 * g.pre_len; len <= gw.seg_len; len += g.pre_len)
-    if (gw.seg_len % len == 0 && cost(len) < enough && cost(len) < cost(gp.pre_len)) gp.pre_len = len;
-  gp.pre_n = (int)((g.n + gp.pre_len - 1) / gp.pre_len);
-  return pre_pass_geom(gp);
-}
 
 // A wide head (d > 128) is swept one slice of 128 features of q and k after the other, straight from and to their rows
 // (b*h = 8, n = 8192, d = 256, e = 128, forward + backward: 197 us, against 383 with slices copied out and summed outside):
@@ -2008,9 +1978,9 @@ const void *row_slice(const void *p, int i) { return (const elem16_t *)p + i * k
 void *row_slice(void *p, int i) { return (elem16_t *)p + i * kMaxWidth; }
 template <class T>  // of the chunk's d x e states
 T *carry_slice(T *p, const Geom &g, int i) { return p ? p + (int64_t)i * kMaxWidth * g.e : p; }
-template <class T>  // of the workspace, which holds `n` states per (b, h)
-T *state_slice(T *p, const Geom &g, int n, int i) {
-  return p ? p + (int64_t)i * g.b * g.h * n * kMaxWidth * kMaxWidth : p;
+template <class T>  // of the workspace
+T *state_slice(T *p, const Geom &g, int i) {
+  return p ? p + (int64_t)i * g.b * g.h * g.pre_n * kMaxWidth * kMaxWidth : p;
 }
 FwdArgs slice_args(const FwdArgs &a, const Geom &g, int i) {
   FwdArgs r = a;
@@ -2061,7 +2031,7 @@ int fwd_e(const FwdArgs &a, const Geom &g, hipStream_t st) {
   auto sweep = [&](auto mode, int i) {
     const FwdArgs as = slice_args(a, g, i);
     return launch_apply<E, false, false, SRC_SCANNED, decltype(mode)::value, W>(
-        as.q, as.k, as.v, as.s, need_states ? state_slice(as.seg_states, g, g.pre_n, i) : nullptr, as.kv_in, nullptr, as.o,
+        as.q, as.k, as.v, as.s, need_states ? state_slice(as.seg_states, g, i) : nullptr, as.kv_in, nullptr, as.o,
         slice_geom(g, i), st);
   };
   rc = sweep(std::integral_constant<int, MODE>(), 0);
@@ -2145,16 +2115,18 @@ bool whole_fwd_pays(const Geom &g) {
 
 // Segments of the backward sweeps: m of the plan's in a row.  The plan's segments give the forward a workgroup per CU; three roles of them
 // take one round and a half to three, each with its start-up -- the first tiles, the entering state, the last stores -- of about five
-// blocks' time, and half of a last round is empty.  The KV states lie at the plan's segments either way (a sweep takes the one that enters
-// its first), so the forward and the KV pre-pass and scan stay as they are; DKV's lie at them or as rev_pass_geom says, at lengths that
-// divide a sweep's and that the plan's pieces divide: at most as many, so that they fit the workspace, and as few as one.  m is the one with the least rounds x (blocks + 5), a round
-// being 32 workgroups on each XCD, as launch_bwd3 deals items out, if that saves 3 %.  bf16, backward with kept states, us, m = 1 and m:
+// blocks' time, and half of a last round is empty.  The states lie at the plan's segments either way (a sweep takes the one that enters its
+// first), so the forward, the pre-passes and the scans stay as they are but for the states that nothing reads.  m is the one with the least
+// rounds x (blocks + 5), a round being 32 workgroups on each XCD, as launch_bwd3 deals items out, if that saves 3 %.  bf16, backward with kept states, us, m = 1 and m:
 // b*h = 4, n = 8192 38.2 and 34.0 (m = 2: one round of 8 blocks for two of 4), b*h = 8, n = 3784 35.5 and 31.1 (2), b*h = 16, n = 8192 87.9
 // and 81.2 (4: one round of 32 for three of 8), b*h = 20, n = 3757, d = 96 52.7 and 43.3 (3), b*h = 16, n = 1536, d = 192 55.9 and 47.9 (2).
 // A last segment of the plan's less than a fifth full makes no round of its own (b*h = 10, n = 8226: 3.4 % slower with m = 3).  Over 225 shapes
 // (b*h = 3 ... 48, n = 1523 ... 31484) 0.956 of the time on average, 0.954 with the best m of each, none slower.  Slices of a wide head, whose
 // sweeps fetch narrow rows, lose from 28 blocks on (b*h = 32, n = 4096, d = 256 1.012 and up).  Heads of up to 64 features run two workgroups to a
 // CU and lose with any m (1.03 and up on 24 shapes).
+// Tried: DKV states as far apart as the sweeps start, which only they read (b*h = 8, n = 8192, d = 256 102.2 and 94.8 us backwards).  DKV_out is
+// then a sum of longer pieces, without decay up to 1.13 times as far from 64 bits (fp16, b*h = 16, n = 1536, d = 192 1.09e-7 and 0.96e-7), and
+// where that keeps to calls that leave no state, gradients depend on whether one is asked for.
 constexpr int kSweepStart = 5, kSweepBlocks = 40, kSweepBlocksSlice = 24, kSweepRow = 8;
 template <int W>
 Geom bwd_sweep_geom(const Geom &g) {
@@ -2208,11 +2180,7 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
     return launch_bwd3<E, SRC_COMBINE, MODE, W>(a, g.n_seg > 1 ? kv_states : nullptr,
                                                 g.n_seg > 1 ? a.ws_dkv : nullptr, g, st);
   }
-  const Geom gp = pre_pass_geom(g);
-  Geom gw = bwd_sweep_geom<W>(g);
-  const Geom gr = W == kMaxWidth && !a.dkv_out ? rev_pass_geom(g, gw) : gp;
-  gw.rev_len = gr.seg_len;
-  gw.rev_n = gr.n_seg;
+  const Geom gp = pre_pass_geom(g), gw = bwd_sweep_geom<W>(g);
   const int sub = gw.seg_len / g.pre_len;  // pre-pass segments per sweep segment
   const float *kv_states = a.kv_seg_states;
   if (!kv_states && (g.n_seg > 1 || a.kv_in)) {
@@ -2222,13 +2190,13 @@ int bwd_e(const BwdArgs &a, const Geom &g, hipStream_t st) {
   }
   const float *dkv_states = nullptr;
   if (g.n_seg > 1 || a.dkv_in || a.dkv_out) {
-    if ((rc = launch_state<E, true, MODE, W>(a.q, a.d_o, a.s, a.ws_dkv, gr, a.dkv_out != nullptr, gw.seg_len / gr.seg_len, st))) return rc;
-    if ((rc = launch_segment_scan(a.ws_dkv, a.dkv_in, a.dkv_out, a.s, gr, 1, st))) return rc;
+    if ((rc = launch_state<E, true, MODE, W>(a.q, a.d_o, a.s, a.ws_dkv, gp, a.dkv_out != nullptr, sub, st))) return rc;
+    if ((rc = launch_segment_scan(a.ws_dkv, a.dkv_in, a.dkv_out, a.s, gp, 1, st))) return rc;
     dkv_states = a.ws_dkv;
   }
   auto sweep = [&](auto mode, int i) {
-    return launch_bwd3<E, SRC_SCANNED, decltype(mode)::value, W>(slice_args(a, g, i), state_slice(kv_states, g, g.pre_n, i),
-                                                                 state_slice(dkv_states, g, gr.n_seg, i), slice_geom(gw, i), st);
+    return launch_bwd3<E, SRC_SCANNED, decltype(mode)::value, W>(slice_args(a, g, i), state_slice(kv_states, g, i),
+                                                                 state_slice(dkv_states, g, i), slice_geom(gw, i), st);
   };
   rc = sweep(std::integral_constant<int, MODE>(), 0);
   if constexpr (MODE == M_NARROW && W == kMaxWidth)
@@ -2290,12 +2258,9 @@ int mfma_fwd(const FwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
 int mfma_bwd(const BwdArgs &a, const Geom &g, int dtype, hipStream_t st) {
   return dtype == LASP_DTYPE_F16 ? mfma_f16_bwd(a, g, st) : bwd_w<ElemBF16>(a, g, st);
 }
-void mfma_bwd_rows(const Geom &g, bool planned, bool state_leaves, int *row, int *piece) {
-  *row = *piece = 0;
-  if (g.fused || g.combine || (planned && g.width == kMaxWidth && g.dt <= kMaxWidth && whole_bwd_pays(g))) return;
-  const Geom gw = g.width == 64 ? bwd_sweep_geom<64>(g) : bwd_sweep_geom<kMaxWidth>(g);
-  *row = gw.seg_len;
-  *piece = g.width == 64 || state_leaves ? g.pre_len : rev_pass_geom(g, gw).seg_len;
+int mfma_bwd_row(const Geom &g, bool planned) {
+  if (g.fused || g.combine || (planned && g.width == kMaxWidth && g.dt <= kMaxWidth && whole_bwd_pays(g))) return 0;
+  return (g.width == 64 ? bwd_sweep_geom<64>(g) : bwd_sweep_geom<kMaxWidth>(g)).seg_len;
 }
 bool mfma_whole(const Geom &g, bool backward_follows) {
   return !g.fused && g.width == kMaxWidth && g.dt <= kMaxWidth && whole_fwd_pays(g) && (!backward_follows || whole_bwd_pays(g));

@@ -76,14 +76,13 @@ def in_place_bits(inp, s, seg):
     return list(zip(run(True), run(False)))
 
 
-def bwd_rows(b, h, n, d, e, dtype, seg_len, state_leaves):
-    """(tokens of a backward sweep, tokens from one DKV state to the next) as the library has them, see lasp_bwd_rows."""
+def bwd_rows(b, h, n, d, e, dtype, seg_len):
+    """Tokens of a backward sweep as the library has them, see lasp_bwd_rows."""
     import ctypes
 
     from lasp_amd import _abi
 
-    row, piece = ctypes.c_int(-1), ctypes.c_int(-1)
-    rc = _abi.load().lasp_bwd_rows(b, h, ctypes.c_int64(n), d, e, _abi.DTYPE_CODE[dtype], seg_len, int(state_leaves),
-                                   ctypes.byref(row), ctypes.byref(piece))
+    row = ctypes.c_int(-1)
+    rc = _abi.load().lasp_bwd_rows(b, h, ctypes.c_int64(n), d, e, _abi.DTYPE_CODE[dtype], seg_len, ctypes.byref(row))
     assert rc == 0, rc
-    return row.value, piece.value
+    return row.value

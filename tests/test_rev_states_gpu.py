@@ -1,5 +1,5 @@
-"""DKV states that lie further apart than the forward's segments: as far as the sweeps start and half as far, in whole and partial pieces,
-for heads that the scan takes and heads that it leaves out, one piece from the other end of the chunk and many."""
+"""DKV states of backwards whose sweeps go over several of the forward's segments in a row: in whole and partial rows, for heads that the
+scan takes and heads that it leaves out, one row from the other end of the chunk and many."""
 import pytest
 import torch
 
@@ -11,26 +11,19 @@ pytestmark = pytest.mark.gpu
 TOL = {torch.bfloat16: 2e-2, torch.float16: 2e-2 / 8}
 
 
-# (b, h, n, d, e, seg_len): segments from one DKV state to the next where none leaves, as the rule has them, and how many states that are
-SHAPES = {
-    (1, 16, 1088, 128, 128, 64): (4, 5), (2, 8, 1100, 128, 128, 64): (4, 5),  # the last piece one block; one block and 12 tokens
-    (1, 12, 897, 128, 128, 64): (3, 5), (1, 16, 641, 128, 64, 64): (3, 4),    # one token in the last segment
-    (1, 12, 1999, 128, 128, 64): (3, 11),                                     # sweeps over six, pieces of three
-    (2, 16, 449, 128, 128, 64): (4, 2), (1, 20, 520, 128, 128, 64): (3, 3),
-    (1, 8, 700, 256, 128, 64): (2, 6), (1, 10, 1300, 192, 128, 64): (3, 7), (1, 16, 385, 200, 72, 64): (2, 4),  # slices
-    (1, 8, 3784, 128, 128, 0): (2, 10), (1, 16, 1536, 192, 128, 0): (2, 4),   # default plans
-}
-
-
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("b,h,n,d,e,seg_len", SHAPES)
+@pytest.mark.parametrize("b,h,n,d,e,seg_len", [
+    (1, 16, 1088, 128, 128, 64), (2, 8, 1100, 128, 128, 64),  # four of the forward's segments each; the last row one segment, one and 12 tokens
+    (1, 12, 897, 128, 128, 64), (1, 16, 641, 128, 64, 64),    # three; one token in the last one
+    (1, 12, 1999, 128, 128, 64),                              # six
+    (2, 16, 449, 128, 128, 64), (1, 20, 520, 128, 128, 64),   # two rows, three
+    (1, 8, 700, 256, 128, 64), (1, 10, 1300, 192, 128, 64), (1, 16, 385, 200, 72, 64),  # slices
+    (1, 8, 3784, 128, 128, 0), (1, 16, 1536, 192, 128, 0),    # default plans
+])
 @pytest.mark.parametrize("decay", [(0.4, 0.003), (0.9, 0.08), (0.0, 0.0)])
 def test_matches_oracle(gpu_device, b, h, n, d, e, seg_len, dtype, decay):
     from lasp_amd import _abi
 
-    apart, states = SHAPES[b, h, n, d, e, seg_len]
-    piece = bwd_rows(b, h, n, d, e, dtype, seg_len, False)[1]
-    assert (piece, -(-n // piece)) == (apart * _abi.plan(b, h, n, d, e, dtype, seg_len)[0], states)
     inp = make_inputs(b, h, n, d, e, dtype, seed=n + d + e, scale=0.3, state=True, state_std=1.0)
     dev = {k: v.to(gpu_device) for k, v in inp.items()}
     s = torch.linspace(*decay, h)
@@ -58,25 +51,24 @@ def test_matches_oracle(gpu_device, b, h, n, d, e, seg_len, dtype, decay):
                                                (1, 12, 1999, 96, 128, 64)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_a_state_that_leaves_is_a_sum_of_the_same_pieces(gpu_device, b, h, n, d, e, seg_len, dtype):
-    """DKV_out has the bits that a call of few heads gives, whose sweeps go over one segment each: its pieces are the forward's, also where
-    the states that only the sweeps read would lie further apart."""
+    """DKV_out has the bits that a call of few heads gives, whose sweeps go over one segment each: it is a sum of the forward's segments,
+    whatever row the sweeps go over.  The gradients do not depend on whether it is asked for."""
     from lasp_amd import _abi
 
-    row, piece = bwd_rows(b, h, n, d, e, dtype, seg_len, False)
-    assert row >= piece > seg_len and bwd_rows(b, h, n, d, e, dtype, seg_len, True) == (row, seg_len)
-    assert bwd_rows(1, 1, n, d, e, dtype, seg_len, False) == (seg_len, seg_len)
+    assert bwd_rows(b, h, n, d, e, dtype, seg_len) > seg_len and bwd_rows(1, 1, n, d, e, dtype, seg_len) == seg_len
     dev = make_inputs(b, h, n, d, e, dtype, seed=n + d, scale=0.3, state=True, state_std=1.0, device=gpu_device)
     s = torch.linspace(0.05, 0.0, h, device=gpu_device)
 
-    def run(part, s):
-        out = torch.full_like(part["kv"], float("nan"))
-        _abi.chunk_bwd(part["q"], part["k"], part["v"], s, part["do"], part["kv"], part["dkv"], out, None, seg_len)
-        return out
+    def run(part, s, leaves=True):
+        out = torch.full_like(part["kv"], float("nan")) if leaves else None
+        return out, _abi.chunk_bwd(part["q"], part["k"], part["v"], s, part["do"], part["kv"], part["dkv"], out, None, seg_len)
 
-    whole = run(dev, s)
+    whole, grads = run(dev, s)
     for i in range(h):
-        one = run({k: v[:1, i:i + 1].contiguous() for k, v in dev.items()}, s[i:i + 1].contiguous())
+        one, _ = run({k: v[:1, i:i + 1].contiguous() for k, v in dev.items()}, s[i:i + 1].contiguous())
         assert torch.equal(one, whole[:1, i:i + 1]), i
+    for name, x, y in zip(("dq", "dk", "dv"), grads, run(dev, s, leaves=False)[1]):
+        assert torch.equal(x, y), name
 
 
 def chunk_bwd_over(fill, inp, s, kv_in, dkv_in, dkv_out, seg_len):
@@ -103,9 +95,8 @@ def chunk_bwd_over(fill, inp, s, kv_in, dkv_in, dkv_out, seg_len):
     (4, 16, 1536, 512, 128, 0),                              # the library's own plan
 ])
 def test_one_row_of_segments(gpu_device, b, h, n, d, e, seg_len, dtype):
-    """A sweep over the whole chunk, whose DKV states may be a single one: it has no neighbour to take a state from, so no head, whatever
-    the next one or the workspace holds, leaves anything but its own sum."""
-    assert bwd_rows(b, h, n, d, e, dtype, seg_len, False) == (-(-n // seg_len) * seg_len if seg_len else n,) * 2
+    """A sweep over the whole chunk: no head, whatever the next one or the workspace holds, leaves anything but its own sum."""
+    assert bwd_rows(b, h, n, d, e, dtype, seg_len) == (-(-n // seg_len) * seg_len if seg_len else n)
     inp = make_inputs(b, h, n, d, e, dtype, seed=n + d + e, scale=0.3, state=True, state_std=1.0)
     # every state dies within the chunk; the slowest is at 2^-25 after it, which a head 2^20 times as large would show
     s = torch.linspace(0.5, 25 / (1.4427 * n), h)

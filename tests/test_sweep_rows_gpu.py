@@ -36,7 +36,7 @@ def test_matches_oracle(gpu_device, b, h, n, d, e, seg_len, dtype, decay):
     from lasp_amd import _abi
 
     segment = _abi.plan(b, h, n, d, e, dtype, seg_len)[0]
-    assert bwd_rows(b, h, n, d, e, dtype, seg_len, True)[0] == SHAPES[b, h, n, d, e, seg_len] * segment
+    assert bwd_rows(b, h, n, d, e, dtype, seg_len) == SHAPES[b, h, n, d, e, seg_len] * segment
     inp = make_inputs(b, h, n, d, e, dtype, seed=n + d + e, scale=0.3, state=True, state_std=1.0)
     dev = {k: v.to(gpu_device) for k, v in inp.items()}
     s = torch.linspace(0.4, 0.003, h) if decay else torch.zeros(h)  # heads that the scan leaves out, and heads that it does not
