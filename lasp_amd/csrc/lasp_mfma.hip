@@ -877,7 +877,7 @@ sweep_body(const elem16_t *__restrict__ X, const elem16_t *__restrict__ Y, const
     const char *const o_from = smem + L::X + 16 * w * L::ROW + lane * 16;
     u32x4 out[4];
     // Output is not read again here, and its stores say so, but the dV that the next slice of a wide head adds to: where the L2s hold it, it
-    // stays there.  Backward, us, d = 256: b*h = 8, n = 8192 94.5 -> 87.5, b*h = 32, n = 3000 130 -> 120; beyond, b*h = 24, n = 12000 308 -> 313,
+    // stays there.  Backward, us, d = 256: b*h = 8, n = 8192 96.1 -> 89.1, b*h = 32, n = 3000 128.8 -> 120.9; beyond, b*h = 24, n = 12000 308 -> 313,
     // and in the forward, b*h = 4, n = 15761 60.1 -> 61.3, it would lose.
     constexpr int64_t L2_BYTES = (int64_t)32 << 20;
     const bool again = MODE == M_NARROW && REV && !TRANS && g.dt > W && (int64_t)(g.b * g.h) * g.n * g.e * 2 <= L2_BYTES;
@@ -1434,7 +1434,7 @@ la_fused_fwd(const elem16_t *__restrict__ Q, const elem16_t *__restrict__ K, con
   any_body<E, false, false, SRC_WALK, MODE, W>(Q, K, V, S, nullptr, O, g, g.d, g.e, item, smem, kv_in, kv_out);
 }
 
-// The (b, h) from bh0 on are cut into segments of their own (n_seg of seg_len tokens): see launch_fused_bwd.
+// The (b, h) from bh0 on are cut into n_seg segments of their own, unequal ones as `cut` says: see fused_bwd_tail.
 struct Fine {
   int bh0, n_seg;
   Divisor by_seg;
@@ -1765,10 +1765,12 @@ la_seg_state(const elem16_t *__restrict__ Y, const elem16_t *__restrict__ Z, con
 // soon, and it begins at the ends of the segments.  Where they exceed the cache, only the last blocks of the segments are loaded as usual, as
 // many as have 160 MB; the blocks before them, which would not last, are loaded as data that is read once (`nt`), and come faster for it.
 // Forwards, us: b*h = 32, n = 16384 138 -> 126, b*h = 16, n = 65536 245 -> 222, b*h = 64, n = 8192 134 -> 126; with the backward 394 -> 385,
-// 732 -> 698, 384 -> 378.  With every block read once b*h = 32's forward takes 128 and its backward 16 more.  Tensors that fit the cache lose:
-// b*h = 36, n = 5003, d = e = 128, every block read once 164.5 -> 168.1 in both directions, b*h = 16, n = 16384, 160 of 201 MB as usual, 237.7 ->
-// 239.8.  Of 64, 96, 128, 160, 192 and 256 MB the forwards are the faster the less stays (b*h = 32: 0.91 of the time with 64, 0.95 with 192), the
-// backwards the slower (b*h = 64, n = 4096: 1.03 of both with 64, 0.99 to 1.01 from 96 on).
+// 732 -> 698, 384 -> 378.  (Forwards one after the other, some of whose tensors the call before left in the cache; with the backwards between
+// them and two sets of tensors in turn the sweep itself takes 198 -> 176 at b*h = 16, n = 65536, 6.1 TB/s, and 99 -> 91 at b*h = 32.)  With
+// every block read once b*h = 32's forward takes 128 and its backward 16 more.  Tensors that fit the cache lose: b*h = 36, n = 5003, d = e =
+// 128, every block read once 164.5 -> 168.1 in both directions, b*h = 16, n = 16384, 160 of 201 MB as usual, 237.7 -> 239.8.  Of 64, 96, 128,
+// 160, 192 and 256 MB the forwards are the faster the less stays (b*h = 32: 0.91 of the time with 64, 0.95 with 192), the backwards the slower
+// (b*h = 64, n = 4096: 1.03 of both with 64, 0.99 to 1.01 from 96 on).
 // In a backward the three roles' workgroups of a round go over their segments' q, k, v and dO at about the same time, dQ's in the other
 // direction: where these exceed the cache, dQ's loads leave nothing behind (b*h = 16, n = 65536: both directions 718 -> 706; b*h = 32, n = 16384,
 // where they do not, 393 -> 396).
@@ -2103,8 +2105,8 @@ bool whole_bwd(const BwdArgs &a, const Geom &g) {
 // nearest), b*h = 112, n = 3600 115 and 99, b*h = 200, n = 5400 295 and 222; d = 96, b*h = 80, n = 2600 72.9 and 47.1.  Of 160 shapes that
 // take it (four widths, b*h = 13 ... 512, n = 1100 ... 6144) the slowest is at 1.006 of its three kernels, the mean at 0.84.
 // KV_out is one sum over the whole chunk, as DKV_out is backwards: without decay 2.9e-7 off 64 bits at b*h = 24, n = 2048 where sums of
-// segments are 1.0e-7, 5.0e-7 and 3.7e-7 at b*h = 120, n = 6000, so the operators take it only where no state leaves; with decay 1.66e-3 (bf16) and 2.07e-4 (fp16) either way, the rounding
-// of its operand, and O 1.7e-3 to 2.7e-3 either way.
+// segments are 1.0e-7, 5.0e-7 and 3.7e-7 at b*h = 120, n = 6000, so the operators take it only where no state leaves; with decay 1.66e-3
+// (bf16) and 2.07e-4 (fp16) either way, the rounding of its operand, and O 1.7e-3 to 2.7e-3 either way.
 constexpr int64_t kWholeFwdNarrow = 80, kWholeFwdGathered = 64;
 bool whole_fwd_pays(const Geom &g) {
   const int64_t bh = (int64_t)g.b * g.h;
@@ -2117,13 +2119,13 @@ bool whole_fwd_pays(const Geom &g) {
 // take one round and a half to three, each with its start-up -- the first tiles, the entering state, the last stores -- of about five
 // blocks' time, and half of a last round is empty.  The states lie at the plan's segments either way (a sweep takes the one that enters its
 // first), so the forward, the pre-passes and the scans stay as they are but for the states that nothing reads.  m is the one with the least
-// rounds x (blocks + 5), a round being 32 workgroups on each XCD, as launch_bwd3 deals items out, if that saves 3 %.  bf16, backward with kept states, us, m = 1 and m:
-// b*h = 4, n = 8192 38.2 and 34.0 (m = 2: one round of 8 blocks for two of 4), b*h = 8, n = 3784 35.5 and 31.1 (2), b*h = 16, n = 8192 87.9
-// and 81.2 (4: one round of 32 for three of 8), b*h = 20, n = 3757, d = 96 52.7 and 43.3 (3), b*h = 16, n = 1536, d = 192 55.9 and 47.9 (2).
-// A last segment of the plan's less than a fifth full makes no round of its own (b*h = 10, n = 8226: 3.4 % slower with m = 3).  Over 225 shapes
-// (b*h = 3 ... 48, n = 1523 ... 31484) 0.956 of the time on average, 0.954 with the best m of each, none slower.  Slices of a wide head, whose
-// sweeps fetch narrow rows, lose from 28 blocks on (b*h = 32, n = 4096, d = 256 1.012 and up).  Heads of up to 64 features run two workgroups to a
-// CU and lose with any m (1.03 and up on 24 shapes).
+// rounds x (blocks + 5), a round being 32 workgroups on each XCD, as launch_bwd3 deals items out, if that saves 3 %.  bf16, backward with kept
+// states, us, m = 1 and m: b*h = 4, n = 8192 38.2 and 34.0 (m = 2: one round of 8 blocks for two of 4), b*h = 8, n = 3784 35.5 and 31.1 (2),
+// b*h = 16, n = 8192 87.9 and 81.2 (4: one round of 32 for three of 8), b*h = 20, n = 3757, d = 96 52.7 and 43.3 (3), b*h = 16, n = 1536, d =
+// 192 55.9 and 47.9 (2). A last segment of the plan's less than a fifth full makes no round of its own (b*h = 10, n = 8226: 3.4 % slower with
+// m = 3).  Over 225 shapes (b*h = 3 ... 48, n = 1523 ... 31484) 0.956 of the time on average, 0.954 with the best m of each, none slower.
+// Slices of a wide head, whose sweeps fetch narrow rows, lose from 28 blocks on (b*h = 32, n = 4096, d = 256 1.012 and up).  Heads of up to 64
+// features run two workgroups to a CU and lose with any m (1.03 and up on 24 shapes).
 // Tried: DKV states as far apart as the sweeps start, which only they read (b*h = 8, n = 8192, d = 256 102.2 and 94.8 us backwards).  DKV_out is
 // then a sum of longer pieces, without decay up to 1.13 times as far from 64 bits (fp16, b*h = 16, n = 1536, d = 192 1.09e-7 and 0.96e-7), and
 // where that keeps to calls that leave no state, gradients depend on whether one is asked for.
